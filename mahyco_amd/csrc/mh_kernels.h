@@ -2099,6 +2099,44 @@ __device__ __forceinline__ double dual_edge_flux(const MhDev& S, int a, int it1,
   return f;
 }
 
+// The dual state of a node between two sweeps is four words, v and m, read from one buffer and
+// written to the other (psel, as the cells' U): A = Ud, B = Pa for v and Pb for m; the first sweep
+// reads v = u and m = the node mass.  phi is not stored: a node updated by an earlier sweep holds
+// v = U (momentum), and phi = U / m is formed where it is read, from the operands the reference
+// divides (DualPhaseRemap.cc:251-257); a node that every earlier sweep kept (a boundary node of
+// each direction swept so far, hence every node in the first sweep) holds v = phi, which is still
+// u, and U = m u (PrepareRemap.cc:169-178).  prev is the bit mask of the directions already swept.
+// The sweeps are bound by HBM: storing phi besides U moved 6 of 17 words per node and sweep, and
+// the last sweep wrote 7 words that nothing reads.  Without them, per launch: x 157 -> 119 us, y
+// and z 192 -> 168 us on the 256x128x128 tube; 230 -> 169 and 247 -> 204 us on the 192^3 blast.
+struct DualBuf {
+  const double* v[3];
+  const double* m;
+};
+template <int DIM>
+__device__ __forceinline__ DualBuf dual_in(const MhDev& S, int psel, int prev) {
+  DualBuf b;
+  const double* base = psel ? S.Ud : S.Pa;
+#pragma unroll
+  for (int cc = 0; cc < 3; ++cc) b.v[cc] = prev ? base + cc * S.g.nn : S.u[cc];
+  b.m = prev ? (psel ? S.Ud + DIM * S.g.nn : S.Pb) : S.mn;
+  return b;
+}
+__device__ __forceinline__ double* dual_out_v(const MhDev& S, int psel) { return psel ? S.Pa : S.Ud; }
+template <int DIM>
+__device__ __forceinline__ double* dual_out_m(const MhDev& S, int psel) {
+  return psel ? S.Pb : S.Ud + DIM * S.g.nn;
+}
+// Whether every sweep so far kept node (i, j, k).
+template <int DIM>
+__device__ __forceinline__ bool dual_kept(const MhDev& S, int prev, int i, int j, int k) {
+  bool kept = true;
+  if (prev & 1) kept = kept && (i == 0 || i == S.g.nx);
+  if (prev & 2) kept = kept && (j == 0 || j == S.g.ny);
+  if (DIM == 3 && (prev & 4)) kept = kept && (k == 0 || k == S.g.nz);
+  return kept;
+}
+
 // Limited nodal gradient from the edge gradients behind (gb) and ahead (gf)
 // (computeAndLimitGradPhiDual, UtilesRemap.cc:369-400), in the order of k_sweep_node_body.
 template <int LIM>
@@ -2109,17 +2147,34 @@ __device__ __forceinline__ double dual_limited(const MhDev& S, double gb, double
   return g;
 }
 
+// Writes the dual state (v, U[DIM]) of node n, or on the last sweep the velocity U / m
+// (RemapADIFinal.cc:286-297); the mass is still read after it by conservation-energie-totale.
+// A node with no neighbour along D keeps its state: v and m are written as they were read.
+template <int DIM>
+__device__ __forceinline__ void dual_store(const MhDev& S, long n, const double* U, const double* v, int psel,
+                                           int last) {
+  const long nn = S.g.nn;
+  if (!last) {
+    double* __restrict__ V = dual_out_v(S, psel);
+#pragma unroll
+    for (int cc = 0; cc < DIM; ++cc) V[cc * nn + n] = v[cc];
+  }
+  if (!last || S.dec) dual_out_m<DIM>(S, psel)[n] = U[DIM];
+  if (last && U[DIM] != 0.)
+#pragma unroll
+    for (int cc = 0; cc < DIM; ++cc) S.u[cc][n] = U[cc] / U[DIM];
+}
+
 // Dual update of one node from its neighbourhood along D (DualPhaseRemap.cc:110-257):
 // Pm/P0/Pp, Xm/X0/Xp, Gm/G0/Gp are phi, coordinate and limited gradient of the nodes a-1,
-// a, a+1; back/front the dual mass fluxes.  Writes Ud, phi and, on the last sweep, u.
+// a, a+1; back/front the dual mass fluxes.  Writes the dual state or, on the last sweep, u.
 template <int DIM, int D>
 __device__ __forceinline__ void dual_node_update(const MhDev& S, long n, double* U, const double* Pm,
                                                  const double* P0, const double* Pp, double Xm, double X0,
                                                  double Xp, const double* Gm, const double* G0,
-                                                 const double* Gp, double back, double front, double* Pout,
+                                                 const double* Gp, double back, double front, int psel,
                                                  int last) {
   constexpr int NC = DIM;
-  const long nn = S.g.nn;
   const double dt = S.sc->dt;
   U[NC] += back - front;
   const double o2 = (double)S.order2;
@@ -2138,36 +2193,14 @@ __device__ __forceinline__ void dual_node_update(const MhDev& S, long n, double*
 #pragma unroll
   for (int cc = 0; cc < NC; ++cc)
     if (fabs(U[cc]) < 1.e-300) U[cc] = 0.;
-#pragma unroll
-  for (int cc = 0; cc <= NC; ++cc) S.Ud[cc * nn + n] = U[cc];
-#pragma unroll
-  for (int cc = 0; cc < NC; ++cc) {
-    const double ph = U[cc] / U[NC];
-    Pout[cc * nn + n] = ph;
-    if (last && U[NC] != 0.) S.u[cc][n] = ph;
-  }
-}
-
-// A node with no neighbour along D keeps its dual state (k_sweep_node_body).
-template <int DIM>
-__device__ __forceinline__ void dual_node_keep(const MhDev& S, long n, const double* U, const double* P,
-                                               double* Pout, int last) {
-  constexpr int NC = DIM;
-  const long nn = S.g.nn;
-#pragma unroll
-  for (int cc = 0; cc <= NC; ++cc) S.Ud[cc * nn + n] = U[cc];
-#pragma unroll
-  for (int cc = 0; cc < NC; ++cc) Pout[cc * nn + n] = P[cc];
-  if (last && U[NC] != 0.)
-#pragma unroll
-    for (int cc = 0; cc < NC; ++cc) S.u[cc][n] = U[cc] / U[NC];
+  dual_store<DIM>(S, n, U, U, psel, last);
 }
 
 // Dual x sweep with one wavefront per 60 nodes of a node row (lane shuffles carry the
 // neighbours' phi, coordinates, edge gradients and limited gradients; the front flux of
 // node i is the back flux of node i+1).  Lanes 2..61 write their node.
 template <int DIM, int LIM>
-__device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, int psel, int first, int last) {
+__device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, int psel, int prev, int last) {
   constexpr int NC = DIM;
   const int nnx = S.g.nnx, na = S.g.nx;
   const long rows = (long)S.g.nny * S.g.nnz;
@@ -2176,9 +2209,7 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
   const long gw = (long)lb * (MH_BLOCK / 64) + (threadIdx.x >> 6);
   if (gw >= rows * wpr) return;  // whole wavefront
   if (mh_halted(S.sc)) return;
-  const double* __restrict__ Pin = psel ? S.Pa : S.Pb;
-  double* __restrict__ Pout = psel ? S.Pb : S.Pa;
-  const long nn = S.g.nn;
+  const DualBuf in = dual_in<DIM>(S, psel, prev);
   const long row = gw / wpr;
   const int i = (int)(gw % wpr) * MH_ROW_OUT - 2 + lane;
   const bool valid = i >= 0 && i <= na;
@@ -2187,10 +2218,16 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
   const int j = (int)(row % S.g.nny);
   const int k = (int)(row / S.g.nny);
   const long n = row * nnx + i;
-  double P[NC], X = 0.;
+  double v[NC], P[NC], m = 0., X = 0.;
 #pragma unroll
-  for (int cc = 0; cc < NC; ++cc) P[cc] = valid ? (first ? S.u[cc][n] : Pin[cc * nn + n]) : 0.;
-  if (valid) X = S.xlc[0][n];
+  for (int cc = 0; cc < NC; ++cc) v[cc] = valid ? in.v[cc][n] : 0.;
+  if (valid) {
+    m = in.m[n];
+    X = S.xlc[0][n];
+  }
+  const bool kept = dual_kept<DIM>(S, prev, i, j, k);
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc) P[cc] = kept || !valid ? v[cc] : v[cc] / m;
   const bool inner = valid && i >= 1 && i <= na - 1;
   const double Xm = __shfl_up(X, 1), Xp = __shfl_down(X, 1);
   double Pm[NC], Pp[NC], G0[NC], Gm[NC], Gp[NC];
@@ -2208,20 +2245,14 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
   const double back = __shfl_up(front, 1);
   if (!out) return;
   double U[NC + 1];
-  if (first) {
-    const double mass = S.mn[n];
 #pragma unroll
-    for (int cc = 0; cc < NC; ++cc) U[cc] = mass * S.u[cc][n];
-    U[NC] = mass;
-  } else {
-#pragma unroll
-    for (int cc = 0; cc <= NC; ++cc) U[cc] = S.Ud[cc * nn + n];
-  }
+  for (int cc = 0; cc < NC; ++cc) U[cc] = kept ? m * v[cc] : v[cc];
+  U[NC] = m;
   if (!inner) {
-    dual_node_keep<DIM>(S, n, U, P, Pout, last);
+    dual_store<DIM>(S, n, U, v, psel, last);
     return;
   }
-  dual_node_update<DIM, 0>(S, n, U, Pm, P, Pp, Xm, X, Xp, Gm, G0, Gp, back, front, Pout, last);
+  dual_node_update<DIM, 0>(S, n, U, Pm, P, Pp, Xm, X, Xp, Gm, G0, Gp, back, front, psel, last);
 }
 
 // The same sweep for D = y or z, LDS tiles: a block of 64 x 4 threads owns 64 cells along
@@ -2452,12 +2483,10 @@ __device__ __forceinline__ void dual_mass_fluxes(const MhDev& S, int i, int j, i
 }
 
 template <int DIM, int D, int LIM>
-__device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel, int first, int last) {
-  double* __restrict__ Ud = S.Ud;
-  const double* __restrict__ Pin = psel ? S.Pa : S.Pb;
-  double* __restrict__ Pout = psel ? S.Pb : S.Pa;
+__device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel, int prev, int last) {
   constexpr int NC = DIM;  // velocity components carried
   if (mh_halted(S.sc)) return;
+  const DualBuf din = dual_in<DIM>(S, psel, prev);
   const int nnx = S.g.nnx, nny = S.g.nny;
   const int i = (int)(n % nnx);
   const long r = n / nnx;
@@ -2466,21 +2495,19 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
   const int a = D == 0 ? i : D == 1 ? j : k;
   const int na = D == 0 ? S.g.nx : D == 1 ? S.g.ny : S.g.nz;
   const long nD = D == 0 ? 1 : D == 1 ? (long)nnx : (long)nnx * nny;
-  const long nn = S.g.nn;
-  double U[NC + 1];
-  if (first) {
-    const double mass = S.mn[n];
-    for (int cc = 0; cc < NC; ++cc) U[cc] = mass * S.u[cc][n];
-    U[NC] = mass;
-  } else {
-    for (int cc = 0; cc <= NC; ++cc) U[cc] = Ud[cc * nn + n];
-  }
+  // earlier sweeps ran along other directions: the nodes of one line along D were all kept by
+  // them or none was
+  const bool kept = dual_kept<DIM>(S, prev, i, j, k);
   const bool inner = a >= 1 && a <= na - 1;
+  double U[NC + 1], v0[NC];
+  U[NC] = din.m[n];
+#pragma unroll
+  for (int cc = 0; cc < NC; ++cc) {
+    v0[cc] = din.v[cc][n];
+    U[cc] = kept ? U[NC] * v0[cc] : v0[cc];
+  }
   if (!inner) {
-    for (int cc = 0; cc <= NC; ++cc) Ud[cc * nn + n] = U[cc];
-    for (int cc = 0; cc < NC; ++cc) Pout[cc * nn + n] = first ? S.u[cc][n] : Pin[cc * nn + n];
-    if (last && U[NC] != 0.)
-      for (int cc = 0; cc < NC; ++cc) S.u[cc][n] = U[cc] / U[NC];
+    dual_store<DIM>(S, n, U, v0, psel, last);
     return;
   }
   const double dt = S.sc->dt;
@@ -2490,7 +2517,11 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
     const int bb = a + o;
     if (bb >= 0 && bb <= na) {
       const long m2 = n + o * nD;
-      for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = first ? S.u[cc][m2] : Pin[cc * nn + m2];
+      for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = din.v[cc][m2];
+      if (!kept) {
+        const double mm = din.m[m2];
+        for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = P[o + 2][cc] / mm;
+      }
       X[o + 2] = S.xlc[D][m2];
     } else {
       for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = 0.;
@@ -2553,19 +2584,14 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
   }
   for (int cc = 0; cc < NC; ++cc)
     if (fabs(U[cc]) < 1.e-300) U[cc] = 0.;
-  for (int cc = 0; cc <= NC; ++cc) Ud[cc * nn + n] = U[cc];
-  for (int cc = 0; cc < NC; ++cc) {
-    const double ph = U[cc] / U[NC];
-    Pout[cc * nn + n] = ph;
-    if (last && U[NC] != 0.) S.u[cc][n] = ph;
-  }
+  dual_store<DIM>(S, n, U, U, psel, last);
 }
 
 template <int DIM, int D, int LIM>
-__device__ __forceinline__ void k_sweep_node_body(const MhDev& S, int lb, int psel, int first, int last) {
+__device__ __forceinline__ void k_sweep_node_body(const MhDev& S, int lb, int psel, int prev, int last) {
   const long n = lb * (long)blockDim.x + threadIdx.x;
   if (n >= S.g.nn) return;
-  k_sweep_node_at<DIM, D, LIM>(S, n, psel, first, last);
+  k_sweep_node_at<DIM, D, LIM>(S, n, psel, prev, last);
 }
 
 // The y or z dual sweep of one mesh with each thread marching along D over a segment of
@@ -2586,7 +2612,7 @@ MH_HD int march_nseg(int n, int len) { return (n + len - 1) / len; }
 #define MH_NM_MIN_WAVES 1
 #endif
 template <int DIM, int D, int LIM>
-__device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, int psel, int first, int last) {
+__device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, int psel, int prev, int last) {
   constexpr int NC = DIM;
   const int nnx = S.g.nnx, nny = S.g.nny;
   const int na = D == 1 ? S.g.ny : S.g.nz;
@@ -2600,21 +2626,24 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
   const long rem = g - seg * cols;
   const int i = (int)(rem % nnx), t2 = (int)(rem / nnx);
   const int a0 = (int)((long)seg * (na + 1) / nseg), a1 = (int)((long)(seg + 1) * (na + 1) / nseg);  // nodes a0 .. a1-1
-  const long nn = S.g.nn;
   const long nD = D == 1 ? (long)nnx : (long)nnx * nny;
   const long base = D == 1 ? i + (long)nnx * nny * t2 : i + (long)nnx * t2;  // node at a = 0
-  const double* __restrict__ Pin = psel ? S.Pa : S.Pb;
-  double* __restrict__ Pout = psel ? S.Pb : S.Pa;
-  double* __restrict__ Ud = S.Ud;
+  const DualBuf din = dual_in<DIM>(S, psel, prev);
+  // one line along D was kept by the earlier sweeps as a whole or not at all
+  const bool kept = dual_kept<DIM>(S, prev, i, D == 1 ? 0 : t2, D == 1 ? t2 : 0);
   const double* __restrict__ Xd = S.xlc[D];
   const double dt = S.sc->dt;
   const double o2 = (double)S.order2;
   auto loadP = [&](int b, double* P, double& X) {
     if (b >= 0 && b <= na) {
       const long m2 = base + b * nD;
+      const double m = din.m[m2];
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) P[cc] = first ? S.u[cc][m2] : Pin[cc * nn + m2];
+      for (int cc = 0; cc < NC; ++cc) P[cc] = din.v[cc][m2];
       X = Xd[m2];
+      if (!kept)
+#pragma unroll
+        for (int cc = 0; cc < NC; ++cc) P[cc] = P[cc] / m;
     } else {
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) P[cc] = 0.;
@@ -2657,18 +2686,15 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
   double back = 0., front = 0.;
   for (int a = a0; a < a1; ++a) {
     const long n = base + a * nD;
-    double U[NC + 1];
-    if (first) {
-      const double mass = S.mn[n];
+    double U[NC + 1], v0[NC];  // read a second time (from L2): carrying them costs a wave per SIMD
+    U[NC] = din.m[n];
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) U[cc] = mass * S.u[cc][n];
-      U[NC] = mass;
-    } else {
-#pragma unroll
-      for (int cc = 0; cc <= NC; ++cc) U[cc] = Ud[cc * nn + n];
+    for (int cc = 0; cc < NC; ++cc) {
+      v0[cc] = din.v[cc][n];
+      U[cc] = kept ? U[NC] * v0[cc] : v0[cc];
     }
     if (!(a >= 1 && a <= na - 1)) {
-      dual_node_keep<DIM>(S, n, U, P[1], Pout, last);
+      dual_store<DIM>(S, n, U, v0, psel, last);
     } else {
       const int jj = D == 1 ? a : j0, kk = D == 1 ? k0 : a;
       if (a > a0 && a >= 2) {  // the back face of node a is the front face of inner node a-1
@@ -2694,14 +2720,7 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc)
         if (fabs(U[cc]) < 1.e-300) U[cc] = 0.;
-#pragma unroll
-      for (int cc = 0; cc <= NC; ++cc) Ud[cc * nn + n] = U[cc];
-#pragma unroll
-      for (int cc = 0; cc < NC; ++cc) {
-        const double ph = U[cc] / U[NC];
-        Pout[cc * nn + n] = ph;
-        if (last && U[NC] != 0.) S.u[cc][n] = ph;
-      }
+      dual_store<DIM>(S, n, U, U, psel, last);
     }
     if (a + 1 < a1) {  // slide the window one node along D
 #pragma unroll
@@ -2726,24 +2745,23 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
 
 
 // u = mu / m for every node with a non-zero projected mass (RemapADIFinal.cc:286-297), for
-// cycles whose remap has a single sweep (the sweep kernel still reads u) or none.
+// cycles whose remap has a single sweep (the sweep kernel still reads u; prev is its direction)
+// or none (prev 0: u and the node mass).
 template <int DIM>
-__device__ __forceinline__ void k_node_velocity_body(const MhDev& S, int lb, int materialize) {
-  const double* __restrict__ Ud = S.Ud;
+__device__ __forceinline__ void k_node_velocity_body(const MhDev& S, int lb, int prev) {
   const long n = lb * (long)blockDim.x + threadIdx.x;
   if (n >= S.g.nn) return;
   if (mh_halted(S.sc)) return;
-  const long nn = S.g.nn;
-  double U[DIM + 1];
-  if (materialize) {
-    const double mass = S.mn[n];
-    for (int cc = 0; cc < DIM; ++cc) U[cc] = mass * S.u[cc][n];
-    U[DIM] = mass;
-  } else {
-    for (int cc = 0; cc <= DIM; ++cc) U[cc] = Ud[cc * nn + n];
-  }
-  if (U[DIM] != 0.)
-    for (int cc = 0; cc < DIM; ++cc) S.u[cc][n] = U[cc] / U[DIM];
+  const DualBuf din = dual_in<DIM>(S, 1, prev);  // the first sweep writes buffer A
+  const int i = (int)(n % S.g.nnx);
+  const long r = n / S.g.nnx;
+  const bool kept = dual_kept<DIM>(S, prev, i, (int)(r % S.g.nny), (int)(r / S.g.nny));
+  const double m = din.m[n];
+  if (m != 0.)
+    for (int cc = 0; cc < DIM; ++cc) {
+      const double v = din.v[cc][n];
+      S.u[cc][n] = (kept ? m * v : v) / m;
+    }
 }
 
 // ------------------------------------------------- conservation-energie-totale (RemapADI.axl:178)
@@ -2754,14 +2772,14 @@ __device__ __forceinline__ void k_node_velocity_body(const MhDev& S, int lb, int
 // formed (UtilesRemap.cc:369-400 covers the velocity only), so the slope term multiplies 0.
 // phi = U / the node mass the node sweep has just written (:251-257).
 template <int DIM, int D>
-__device__ __forceinline__ void k_sweep_ke_body(const MhDev& S, int lb, int psel, int first) {
+__device__ __forceinline__ void k_sweep_ke_body(const MhDev& S, int lb, int psel, int prev) {
   const long n = lb * (long)blockDim.x + threadIdx.x;
   if (n >= S.g.nn) return;
   if (mh_halted(S.sc)) return;
-  const double* __restrict__ Pin = psel ? S.Pa : S.Pb;
+  const int first = prev == 0;
+  const DualBuf din = dual_in<DIM>(S, psel, prev);
   const double* __restrict__ Kin = psel ? S.ke_Pa : S.ke_Pb;
   double* __restrict__ Kout = psel ? S.ke_Pb : S.ke_Pa;
-  const long nn = S.g.nn;
   const int nnx = S.g.nnx, nny = S.g.nny;
   const int i = (int)(n % nnx);
   const long r = n / nnx;
@@ -2788,7 +2806,8 @@ __device__ __forceinline__ void k_sweep_ke_body(const MhDev& S, int lb, int psel
   const double dt = S.sc->dt;
   const double o2 = (double)S.order2;
   const double zero_slope = 0.;
-  auto vel = [&](long m2) { return first ? S.u[D][m2] : Pin[D * nn + m2]; };
+  const bool kept = dual_kept<DIM>(S, prev, i, j, k);  // of the whole line along D
+  auto vel = [&](long m2) { return kept ? din.v[D][m2] : din.v[D][m2] / din.m[m2]; };
   const double xb = S.xlc[D][n - nD], xn = S.xlc[D][n], xf = S.xlc[D][n + nD];
   const double ufront = 0.5 * (vel(n) + vel(n + nD));
   const int sf = ufront > 0 ? 1 : -1;
@@ -2798,11 +2817,11 @@ __device__ __forceinline__ void k_sweep_ke_body(const MhDev& S, int lb, int psel
   const double BE = phi(back > 0. ? n - nD : n) + o2 * (0.5 * zero_slope * (sb * (xn - xb) - dt * uback));
   U += back * BE - front * FE;
   S.ke_U[n] = U;
-  Kout[n] = U / S.Ud[DIM * nn + n];
+  Kout[n] = U / dual_out_m<DIM>(S, psel)[n];
 }
 
-// The dual state of a remap with no sweep (every direction one cell wide): U = (m u, m) and
-// the kinetic energy 1/2 m |u|^2, untouched by any sweep (PrepareRemap.cc:169-190).
+// The dual state of a remap with no sweep (every direction one cell wide): the mass and the
+// kinetic energy 1/2 m |u|^2, untouched by any sweep (PrepareRemap.cc:169-190).
 template <int DIM>
 __device__ __forceinline__ void k_dual_init_body(const MhDev& S, int lb) {
   const long n = lb * (long)blockDim.x + threadIdx.x;
@@ -2813,7 +2832,6 @@ __device__ __forceinline__ void k_dual_init_body(const MhDev& S, int lb) {
   double v = 0.;
   for (int cc = 0; cc < DIM; ++cc) {
     const double uc = S.u[cc][n];
-    S.Ud[cc * nn + n] = mass * uc;
     v = cc == 0 ? uc * uc : v + uc * uc;
   }
   S.Ud[DIM * nn + n] = mass;
@@ -2825,11 +2843,11 @@ __device__ __forceinline__ void k_dual_init_body(const MhDev& S, int lb) {
 // minus the reconstructed kinetic energy per unit mass, for nodes with a non-zero projected
 // mass; kept if positive (std::max(0., .)).  k_finalize adds it to the internal energies.
 template <int DIM>
-__device__ __forceinline__ void k_cons_ec_body(const MhDev& S, int lb) {
+__device__ __forceinline__ void k_cons_ec_body(const MhDev& S, int lb, int psel) {
   const long c = lb * (long)blockDim.x + threadIdx.x;
   if (c >= S.g.nc) return;
   if (mh_halted(S.sc)) return;
-  const long nn = S.g.nn;
+  const double* __restrict__ mass = dual_out_m<DIM>(S, psel);  // as the last sweep left it
   const int i = (int)(c % S.g.nx);
   const long r = c / S.g.nx;
   const int j = (int)(r % S.g.ny);
@@ -2841,7 +2859,7 @@ __device__ __forceinline__ void k_cons_ec_body(const MhDev& S, int lb) {
 #pragma unroll
   for (int l = 0; l < (DIM == 3 ? 8 : 4); ++l) {
     const long n = b + off[l];
-    const double mp = S.Ud[DIM * nn + n];
+    const double mp = mass[n];
     if (mp != 0.) {
       const double ux = S.u[0][n], uy = S.u[1][n];
       double v = ux * ux + uy * uy;
@@ -3401,8 +3419,8 @@ MH_WRAP(k_cell_length, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_sweep_cell, 1, template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
 MH_WRAP(k_sweep_node, 1, template <int DIM MH_COMMA int D MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA LIM>,
-        MH_COMMA int psel MH_COMMA int first MH_COMMA int last, MH_COMMA psel MH_COMMA first MH_COMMA last)
-MH_WRAP(k_node_velocity, 1, template <int DIM>, <DIM>, MH_COMMA int materialize, MH_COMMA materialize)
+        MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
+MH_WRAP(k_node_velocity, 1, template <int DIM>, <DIM>, MH_COMMA int prev, MH_COMMA prev)
 MH_WRAP(k_finalize, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, MH_COMMA int usel, MH_COMMA usel)
 MH_WRAP(k_sweep_cell_row, 1, template <int DIM MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
@@ -3410,7 +3428,7 @@ MH_WRAP(k_sweep_cell_tile, MH_TILE_MIN_WAVES,
         template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
 MH_WRAP(k_sweep_node_row, 1, template <int DIM MH_COMMA int LIM>, <DIM MH_COMMA LIM>,
-        MH_COMMA int psel MH_COMMA int first MH_COMMA int last, MH_COMMA psel MH_COMMA first MH_COMMA last)
+        MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
 MH_WRAP(k_hcell, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_node_adv, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_node_fwd, 1, template <int DIM>, <DIM>, , )
@@ -3418,13 +3436,13 @@ MH_WRAP(k_sweep_cell_gen, 1, template <int DIM MH_COMMA int D MH_COMMA int M>, <
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
 MH_WRAP(k_sweep_cell3, 1, template <int DIM MH_COMMA int D MH_COMMA int M>, <DIM MH_COMMA D MH_COMMA M>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
-MH_WRAP(k_sweep_ke, 1, template <int DIM MH_COMMA int D>, <DIM MH_COMMA D>, MH_COMMA int psel MH_COMMA int first,
-        MH_COMMA psel MH_COMMA first)
+MH_WRAP(k_sweep_ke, 1, template <int DIM MH_COMMA int D>, <DIM MH_COMMA D>, MH_COMMA int psel MH_COMMA int prev,
+        MH_COMMA psel MH_COMMA prev)
 MH_WRAP(k_dual_init, 1, template <int DIM>, <DIM>, , )
-MH_WRAP(k_cons_ec, 1, template <int DIM>, <DIM>, , )
+MH_WRAP(k_cons_ec, 1, template <int DIM>, <DIM>, MH_COMMA int psel, MH_COMMA psel)
 MH_WRAP(k_prepare_remap, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
 MH_WRAP(k_sweep_node_march, MH_NM_MIN_WAVES, template <int DIM MH_COMMA int D MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA LIM>,
-        MH_COMMA int psel MH_COMMA int first MH_COMMA int last, MH_COMMA psel MH_COMMA first MH_COMMA last)
+        MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
 
 // (the plain kernels are templates with an unused parameter, so that every translation unit
 // that launches one may instantiate it)

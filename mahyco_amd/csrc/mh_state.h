@@ -75,8 +75,8 @@ struct MhDev {
   double* partial;                            // per-block CFL minima
   int* err;                                   // error word raised inside a cycle
   MhScalars* sc;
-  // remap buffers: U ping-pong [nv][nc], mass fluxes [m][nc], dual state [4][nn] (in
-  // place), dual phi ping-pong [3][nn]
+  // remap buffers: U ping-pong [nv][nc], mass fluxes [m][nc], dual state ping-pong: A = Ud
+  // [dim+1][nn], B = Pa [dim][nn] with its masses in Pb [nn] (DualBuf in mh_kernels.h)
   double *Ua, *Ub, *dflux, *Ud, *Pa, *Pb;
   // conservation-energie-totale: the dual kinetic energy [nn] (in place), its phi ping-pong
   // [nn] each, and the energy each cell receives back [nc]; null otherwise

@@ -36,32 +36,32 @@ void launch_cell_part(MhHandle* h, int D, int sel, int first, bool gen, bool o3)
 // Dual part of one sweep direction (computeDualUremap), then the dual kinetic energy when
 // the total energy is conserved.  None in advection mode (withDualProjection, PrepareRemap.cc:211).
 template <int DIM>
-void launch_dual_part(MhHandle* h, int D, int sel, int first, int last, bool gen, bool o3) {
+void launch_dual_part(MhHandle* h, int D, int sel, int prev, int last, bool gen, bool o3) {
   const MhDev& S = h->dev;
   if (S.sans_lagrange) return;
   const bool flat = h->sweep_mode == MH_SWEEP_FLAT;
   if (gen) {
-    if (D == 0) LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, first, last);
-    else if (D == 1) LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, first, last);
-    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, first, last);
+    if (D == 0) LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
+    else if (D == 1) LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
+    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
   } else if (D == 0) {
-    if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, LIM>), h->nblk_n, MH_BLOCK, S, sel, first, last));
-    else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node_row<DIM, LIM>), node_row_blocks(h), MH_BLOCK, S, sel, first, last));
+    if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
+    else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node_row<DIM, LIM>), node_row_blocks(h), MH_BLOCK, S, sel, prev, last));
   } else if (D == 1) {
     if (!flat && !o3)  // threads march along y over segments of nodes
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node_march<DIM, 1, LIM>), node_march_blocks(h, 1), MH_BLOCK, S, sel, first, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node_march<DIM, 1, LIM>), node_march_blocks(h, 1), MH_BLOCK, S, sel, prev, last));
     else
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, LIM>), h->nblk_n, MH_BLOCK, S, sel, first, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
   } else if constexpr (DIM == 3) {
     if (!flat && !o3)  // threads march along z over segments of nodes
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node_march<3, 2, LIM>), node_march_blocks(h, 2), MH_BLOCK, S, sel, first, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node_march<3, 2, LIM>), node_march_blocks(h, 2), MH_BLOCK, S, sel, prev, last));
     else
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, LIM>), h->nblk_n, MH_BLOCK, S, sel, first, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
   }
   if (S.dec) {  // conservation-energie-totale: the dual kinetic energy of this sweep
-    if (D == 0) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 0>), h->nblk_n, MH_BLOCK, S, sel, first);
-    else if (D == 1) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 1>), h->nblk_n, MH_BLOCK, S, sel, first);
-    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<3, 2>), h->nblk_n, MH_BLOCK, S, sel, first);
+    if (D == 0) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 0>), h->nblk_n, MH_BLOCK, S, sel, prev);
+    else if (D == 1) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 1>), h->nblk_n, MH_BLOCK, S, sel, prev);
+    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<3, 2>), h->nblk_n, MH_BLOCK, S, sel, prev);
   }
 }
 
@@ -83,16 +83,18 @@ void launch_sweeps_t(MhHandle* h) {
   const bool gen = !o3 && (S.pb || (S.order2 && S.limiter >= MH_MINMOD_G));
   if (S.csts) LAUNCH(h, KN_NODE_FWD, (k_node_fwd<DIM>), h->nblk_n, MH_BLOCK, S);  // PrepareRemap.cc:210
   if (S.hc && nd > 0) LAUNCH(h, KN_HCELL, (k_hcell<DIM>), h->nblk_c, MH_BLOCK, S);
+  int prev = 0;  // directions swept so far
   for (int s = 0; s < nd; ++s) {
     const int first = s == 0, last = (s == nd - 1) && !first, sel = s & 1;
     const int D = dirs[s];
     launch_cell_part<DIM, M>(h, D, sel, first, gen, o3);
-    launch_dual_part<DIM>(h, D, sel, first, last, gen, o3);
+    launch_dual_part<DIM>(h, D, sel, prev, last, gen, o3);
+    prev |= 1 << D;
   }
   if (S.dec && nd == 0) LAUNCH(h, KN_SWEEP_KE, (k_dual_init<DIM>), h->nblk_n, MH_BLOCK, S);
   if (nd <= 1 && !S.sans_lagrange)
-    LAUNCH(h, KN_NODE_VEL, (k_node_velocity<DIM>), h->nblk_n, MH_BLOCK, S, nd == 0 && !S.dec ? 1 : 0);
-  if (S.dec) LAUNCH(h, KN_CONS_EC, (k_cons_ec<DIM>), h->nblk_c, MH_BLOCK, S);
+    LAUNCH(h, KN_NODE_VEL, (k_node_velocity<DIM>), h->nblk_n, MH_BLOCK, S, prev);
+  if (S.dec) LAUNCH(h, KN_CONS_EC, (k_cons_ec<DIM>), h->nblk_c, MH_BLOCK, S, nd > 0 ? (nd - 1) & 1 : 0);
   LAUNCH(h, KN_FINAL, (k_finalize<DIM, M>), h->nblk_c, MH_BLOCK, S, nd & 1);
   h->sens = (h->sens + 1) % dim;
 }
@@ -102,34 +104,35 @@ void launch_sweeps_t(MhHandle* h) {
 
 // One sweep direction of a batch group (cell part, then dual part).
 template <int DIM, int D, int M, int LIM>
-void ens_sweep(const EnsGroup& g, const MhDev* tab, hipStream_t st, dim3 G, int sel, int first, int last) {
+void ens_sweep(const EnsGroup& g, const MhDev* tab, hipStream_t st, dim3 G, int sel, int prev, int last) {
+  const int first = prev == 0;
   const dim3 B(MH_BLOCK);
   if constexpr (LIM < 0) {  // order 3 or pente-borne / generalised limiters: one thread per item
     if (g.gen) {
       hipLaunchKernelGGL((k_sweep_cell_gen_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(g.cmap), sel, first);
       if (!g.adv)
-        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, MH_LIM_ANY>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, first, last);
+        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, MH_LIM_ANY>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     } else {
       hipLaunchKernelGGL((k_sweep_cell3_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(g.cmap), sel, first);
       if (!g.adv)
-        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, -1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, first, last);
+        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, -1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     }
   } else if (g.rows && D == 0) {
     hipLaunchKernelGGL((k_sweep_cell_row_batch<DIM, M, LIM>), G, B, 0, st, tab, MH_LIST(g.rcmap), sel, first);
     if (!g.adv)
-      hipLaunchKernelGGL((k_sweep_node_row_batch<DIM, LIM>), G, B, 0, st, tab, MH_LIST(g.rnmap), sel, first, last);
+      hipLaunchKernelGGL((k_sweep_node_row_batch<DIM, LIM>), G, B, 0, st, tab, MH_LIST(g.rnmap), sel, prev, last);
   } else if (g.rows) {
     hipLaunchKernelGGL((k_sweep_cell_tile_batch<DIM, D, M, LIM>), G, B, 0, st, tab, MH_LIST(g.tmap[D == 0 ? 0 : D - 1]),
                        sel, first);
     if (!g.adv && !g.o3)  // threads march along D over segments of nodes
       hipLaunchKernelGGL((k_sweep_node_march_batch<DIM, (D == 0 ? 1 : D), LIM>), G, B, 0, st, tab,
-                         MH_LIST(g.mmap[D == 0 ? 0 : D - 1]), sel, first, last);
+                         MH_LIST(g.mmap[D == 0 ? 0 : D - 1]), sel, prev, last);
     else if (!g.adv)
-      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, first, last);
+      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
   } else {
     hipLaunchKernelGGL((k_sweep_cell_batch<DIM, D, M, LIM>), G, B, 0, st, tab, MH_LIST(g.cmap), sel, first);
     if (!g.adv)
-      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, first, last);
+      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
   }
 }
 
@@ -150,19 +153,21 @@ void ens_group_cycle_l(MhEnsembleImpl* E, const EnsGroup& g) {
   if (g.csts) hipLaunchKernelGGL((k_node_fwd_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.nmap));
   const int sens = (int)(E->launched % DIM);
   if (g.o3 || g.gen) hipLaunchKernelGGL((k_hcell_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.cmap));
+  int prev = 0;  // directions swept so far
   for (int s = 0; s < DIM; ++s) {
-    const int D = (s + sens) % DIM, first = s == 0, last = s == DIM - 1, sel = s & 1;
-    if (D == 0) ens_sweep<DIM, 0, M, LIM>(g, tab, st, G, sel, first, last);
-    else if (D == 1) ens_sweep<DIM, 1, M, LIM>(g, tab, st, G, sel, first, last);
-    else if constexpr (DIM == 3) ens_sweep<3, 2, M, LIM>(g, tab, st, G, sel, first, last);
+    const int D = (s + sens) % DIM, last = s == DIM - 1, sel = s & 1;
+    if (D == 0) ens_sweep<DIM, 0, M, LIM>(g, tab, st, G, sel, prev, last);
+    else if (D == 1) ens_sweep<DIM, 1, M, LIM>(g, tab, st, G, sel, prev, last);
+    else if constexpr (DIM == 3) ens_sweep<3, 2, M, LIM>(g, tab, st, G, sel, prev, last);
     if (g.cons) {  // the dual kinetic energy of this sweep
-      if (D == 0) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 0>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, first);
-      else if (D == 1) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, first);
+      if (D == 0) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 0>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
+      else if (D == 1) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
       else if constexpr (DIM == 3)
-        hipLaunchKernelGGL((k_sweep_ke_batch<3, 2>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, first);
+        hipLaunchKernelGGL((k_sweep_ke_batch<3, 2>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
     }
+    prev |= 1 << D;
   }
-  if (g.cons) hipLaunchKernelGGL((k_cons_ec_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.cmap));
+  if (g.cons) hipLaunchKernelGGL((k_cons_ec_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.cmap), (DIM - 1) & 1);
   hipLaunchKernelGGL((k_finalize_batch<DIM, M>), G, B, 0, st, tab, MH_LIST(g.cmap), DIM & 1);
   hipLaunchKernelGGL((k_dt_batch<>), dim3((unsigned)E->ncu), dim3(MH_DT_BLOCK), 0, st, tab, g.d_list, g.d_nlist);
 }

@@ -1,0 +1,58 @@
+"""The remap sweeps at the edges of their launch shapes, bit for bit against the oracle.
+
+Meshes of one to a few cells per direction, one more or less than a row segment (60 lanes), a
+tile (64 x 16) or a marching segment, and directions one cell wide, which are not swept: every
+number of sweeps per remap (one, two, three) and every rotation of their order.  A moving tube
+with walls sends material through every face; the interface lies inside a cell, so pure and
+mixed cells meet."""
+import numpy as np
+import pytest
+
+from mahyco_amd import cases
+from mahyco_amd import types as T
+from tests.helpers import bitwise_equal, fields
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(2, 2, 2), (3, 17, 4), (61, 5, 3), (122, 3, 2), (5, 1, 6), (1, 7, 4), (4, 3, 1), (1, 1, 5), (7, 33, 2),
+          (64, 4, 18), (65, 2, 17), (6, 9, 35)]
+FLAT = [(2, 2), (3, 17), (61, 18), (122, 5), (1, 9), (8, 1), (65, 34)]
+
+
+def moving_tube(n, seed, **kw):
+    rng = np.random.default_rng(seed)
+    c = cases.riemann2d(n[0], n[1], rng, stiffened=bool(seed % 2), name="moving_%s_%d" % ("x".join(map(str, n)), seed))
+    if len(n) == 3:
+        c.dim, c.n, c.length, c.bcs = 3, n, (1., 1., 1.), list(cases.WALLS_3D)
+    c.interface_axis = seed % len(n)
+    c.limiter = (T.MH_MINMOD, T.MH_SUPERBEE, T.MH_VANLEER)[seed % 3]
+    for e in c.envs:
+        e.vitesse_initiale = (.4, -.3, .2)
+    for k, v in kw.items():
+        setattr(c, k, v)
+    return c
+
+
+def check(c, iterations=13):
+    from mahyco_amd.lib import GpuCase
+    from oracle.pyoracle import OracleCase
+    g, o = GpuCase(c), OracleCase(c, pow_mode=1, threads=4)
+    st = g.run(iterations)
+    assert st == o.run(iterations) and g.iteration == o.iteration
+    assert (g.time, g.deltat) == (o.time, o.deltat)
+    a, b = fields(g, len(c.envs), c.dim), fields(o, len(c.envs), c.dim)
+    bad = [k for k in a if not bitwise_equal(a[k], b[k])]
+    g.close()
+    o.close()
+    assert not bad, bad
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+@pytest.mark.parametrize("n", SHAPES + FLAT, ids=lambda n: "x".join(map(str, n)))
+def test_sweeps_at_launch_shape_edges(n, seed):
+    check(moving_tube(n, seed))
+
+
+@pytest.mark.parametrize("n", [(3, 17, 4), (5, 1, 6), (1, 1, 5), (61, 18)], ids=lambda n: "x".join(map(str, n)))
+def test_total_energy_reads_the_last_sweeps_mass(n):
+    check(moving_tube(n, 1, conservation_energie_totale=True))
