@@ -787,16 +787,19 @@ static int create_case(const MhMesh* mesh, const MhEnvironment* envs, int nb_env
   h->astream = copy_stream ? copy_stream : h->stream;
   {
     const char* nk = getenv("MAHYCO_NODE_KERNEL");
-    h->node_tiled = !(nk && strcmp(nk, "flat") == 0);
+    const long nn = (long)h->g.nnx * h->g.nny * (h->g.dim == 3 ? h->g.nnz : 1);
+    h->node_tiled = nk && strcmp(nk, "flat") == 0    ? false
+                    : nk && strcmp(nk, "tiled") == 0 ? true
+                                                     : ext_sc || nn >= MH_NODE_TILE_NODES;
     const char* ck = getenv("MAHYCO_CELL_KERNEL");
     h->cell_tiled = ck && strcmp(ck, "tiled") == 0;
     const char* sw = getenv("MAHYCO_SWEEP");
     h->sweep_mode = (sw && strcmp(sw, "flat") == 0) ? MH_SWEEP_FLAT : MH_SWEEP_TILE;
+    h->sweep_large = sw && strcmp(sw, "tile") == 0;
     const char* ml = getenv("MAHYCO_MARCH_LEN");  // segment length of the marching dual sweeps
-    // 10-node segments where the mesh still fills the GPU with them (about 2.6 M nodes, one round of
-    // waves), 4 on smaller meshes, whose sweeps need the threads
-    const long nn = (long)h->g.nnx * h->g.nny * (h->g.dim == 3 ? h->g.nnz : 1);
-    h->nm_len = ml && atoi(ml) >= 1 ? atoi(ml) : nn >= 10L * 4096 * 64 ? MH_NM_L : 4;
+    // 10-node segments where the mesh still fills the GPU with them, 4 on smaller meshes, whose
+    // sweeps need the threads
+    h->nm_len = ml && atoi(ml) >= 1 ? atoi(ml) : nn >= MH_MARCH_LONG_NODES ? MH_NM_L : 4;
   }
   {
     const int tuned = tune_lookup(case_key_dims(h));
@@ -1755,7 +1758,7 @@ int mahyco_autotune(MhHandle* h, int cycles, int* variant_out, double* ms_per_cy
   }
   // the segment length of the marching y / z dual sweeps, where they run (tiled sweeps, dual
   // phase, order <= 2)
-  if (h->opt.with_projection && !h->opt.sans_lagrange && h->dev.order2 != 2 && !(best & 16)) {
+  if (h->opt.with_projection && !h->opt.sans_lagrange && h->dev.order2 != 2 && !(best & 16) && march_sweep(h)) {
     for (int mc = 0; mc < 5 && st == MH_OK && !stopped; ++mc) {
       const int v = (best & ~(7 << 5)) | (mc << 5);
       if (v != best) st = timed(v);

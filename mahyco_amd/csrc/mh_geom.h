@@ -330,4 +330,36 @@ MH_HD double mh_limiter(int id, double r) {
   return mh_flux_limiter((LIM < 0 || LIM == MH_LIM_ANY) ? id : LIM, r);
 }
 
+// The limited gradient from the gradients behind (gb) and ahead (gf),
+//   g = 1/2 (phi(gf / gb) gb) + 1/2 (phi(gb / gf) gf),  a term dropped where its divisor is 0
+// (computeAndLimitGradPhi, UtilesRemap.cc:325-357), or with DUAL (1/2 phi) gb and (1/2 phi) gf
+// (computeAndLimitGradPhiDual, :369-400; the two differ for subnormal products only).  The two
+// ratios are the inverse of one another, so minmod and superbee need the value of one of them
+// only: with hi the gradient of larger modulus and lo the other, phi is 1 at hi / lo (minmod);
+// for superbee phi is 1 at lo / hi when |hi| < 2 |lo|, and 2 at hi / lo otherwise (a correctly
+// rounded quotient does not cross the threshold).  One division instead of two, the same operands
+// and the same bits; infinities and NaN give what the two-sided form gives.  Other limiters take
+// that form.
+template <int LIM, bool DUAL = false>
+MH_HD double mh_limited_gradient(int id, double gb, double gf) {
+  auto term = [](double phi, double g) { return DUAL ? (0.5 * phi) * g : 0.5 * (phi * g); };
+  if (LIM == 0 || LIM == 1) {
+    const bool back = std::fabs(gf) <= std::fabs(gb);
+    const double hi = back ? gb : gf, lo = back ? gf : gb;
+    const bool opposite = (hi < 0.) != (lo < 0.);
+    if (LIM == 0) {
+      const double t = mh_flux_limiter(0, lo / hi);
+      return term(t, hi) + term(opposite ? 0. : 1., lo);
+    }
+    const bool near = std::fabs(hi) < 2. * std::fabs(lo);
+    const double t = mh_flux_limiter(1, (near ? hi : lo) / (near ? lo : hi));
+    const double s = opposite ? 0. : (near ? 1. : 2.);
+    return term(near ? s : t, hi) + term(near ? t : s, lo);
+  }
+  double g = 0.;
+  if (gb != 0.) g += term(mh_limiter<LIM>(id, gf / gb), gb);
+  if (gf != 0.) g += term(mh_limiter<LIM>(id, gb / gf), gf);
+  return g;
+}
+
 #endif

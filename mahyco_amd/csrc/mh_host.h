@@ -35,6 +35,20 @@ enum {
 
 // sweep variants: one thread per cell / node; row segments along x and LDS tiles along y / z
 enum { MH_SWEEP_FLAT = 0, MH_SWEEP_TILE = 1 };
+// Sizes below which a single mesh takes the variants of the row/tile sweeps that need fewer
+// wavefronts to hide their latency; both sides measured around each line:
+// y / z cell sweeps: 2-cell register segments (k_sweep_cell_seg) below, LDS tiles above.  Tile
+// against segments, two environments: 27 / 10 us on 181x181, 30 / 22 on 512x512, 45 / 33 on 80^3,
+// 37 / 30 on 724x724, 71 / 60 on 101^3, but 45 / 54 on 1024x1024, and 69 / 85 on 128^3 (one).
+#define MH_SEG_CELLS 800000L
+// y / z dual sweeps: one thread per node below, marching segments above.  March (4 nodes) against
+// one per node: 17 / 8.6 us on 181x181, 25 / 20 on 64^3, 30 / 30 on 80^3, 35 / 39 on 128x96x64.
+#define MH_MARCH_NODES 600000L
+// ... and 10-node segments from here on (2.1 M nodes: 94 us with 4, 87 with 10; 1.05 M: 31 / 40)
+#define MH_MARCH_LONG_NODES 1600000L
+// 3D node kernel: one thread per node below, z-marching tiles above.  Tiles (8 planes) against one
+// per node: 39 / 14 us on 16^3, 41 / 35 on 64^3, 54 / 54 on 80^3, 87 / 95 on 101^3.
+#define MH_NODE_TILE_NODES 600000L
 
 struct ProfRec {
   int kind;
@@ -75,6 +89,7 @@ struct MhHandle {
   int nt_kc = MH_NT_KC;     // node planes per block of the tiled node kernel
   int ct_k = MH_CT_K;       // cell planes per block of the tiled cell kernel
   int sweep_mode = MH_SWEEP_TILE;  // MAHYCO_SWEEP=flat selects one thread per cell / node
+  bool sweep_large = false;        // MAHYCO_SWEEP=tile: the large-mesh sweeps at every size
   std::vector<const mh_output::VarSpec*> ens_vars;  // EnSight variables of this case's outputs
   std::vector<double> ens_times;                    // times of the EnSight steps written
   MhScalars* ext_sc = nullptr;  // scalars living in an ensemble's array
@@ -152,6 +167,16 @@ inline int node_march_blocks(MhHandle* h, int D) {
   const long na = D == 1 ? h->g.ny : h->g.nz;
   const long nt2 = D == 1 ? h->g.nnz : h->g.nny;
   const long threads = (long)h->g.nnx * nt2 * march_nseg((int)na + 1, h->nm_len);
+  return (int)(((threads + MH_BLOCK - 1) / MH_BLOCK + 7) / 8 * 8);
+}
+// the y / z variants a single mesh takes (an ensemble's launches are filled by its many cases)
+inline bool seg_sweep(const MhHandle* h) { return !h->sweep_large && h->g.nc < MH_SEG_CELLS; }
+inline bool march_sweep(const MhHandle* h) { return h->sweep_large || h->g.nn >= MH_MARCH_NODES; }
+// blocks of the segment y / z sweep (one thread per len cells of a column), a multiple of 8
+inline int seg_blocks(MhHandle* h, int D, int len) {
+  const long na = D == 1 ? h->g.ny : h->g.nz;
+  const long nt = D == 1 ? (h->g.dim == 3 ? h->g.nz : 1) : h->g.ny;
+  const long threads = (long)h->g.nx * nt * seg_count((int)na, len);
   return (int)(((threads + MH_BLOCK - 1) / MH_BLOCK + 7) / 8 * 8);
 }
 inline int tile_blocks(MhHandle* h, int D) {

@@ -1984,8 +1984,8 @@ __device__ __forceinline__ void row_jk(const MhGrid& g, long r, int& j, int& k) 
   k = kt * MH_ROW_KT + (int)(rem % h);
 }
 template <int DIM, int M, int LIM>
-__device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, int usel, int first) {
-  constexpr int NV = 3 * M + 1;
+__device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, int usel, int first, int v0 = 0,
+                                                      int v1 = 3 * M + 1) {  // slots v0 .. v1-1
   const int nx = S.g.nx;
   const long rows = (long)S.g.ny * S.g.nz;
   const int wpr = (nx + MH_ROW_OUT - 1) / MH_ROW_OUT;
@@ -2008,6 +2008,7 @@ __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, in
   const bool own = !(first && valid && S.mask[c] == 0);  // an empty cell's U starts from 0
   const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
   const double dt = S.sc->dt;
+  double unext = valid ? Uin[v0 * nc + c] : 0.;  // slot loads run one slot ahead
   double den = 1., xc = 0.;
   if (valid) {
     if (first) {
@@ -2028,10 +2029,9 @@ __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, in
   if (inb) face_quant<DIM, 0>(S, b, area, xf, vf);
   const bool upprev = vf * dxb > 0.0;
   const double hb = (double)S.order2 * (xf - (upprev ? xcp : xc));
-  double unext = valid ? Uin[c] : 0.;  // slot loads run one slot ahead
-  for (int v = 0; v < NV; ++v) {
+  for (int v = v0; v < v1; ++v) {
     const double uv = unext;
-    if (v + 1 < NV) unext = valid ? Uin[(v + 1) * nc + c] : 0.;
+    if (v + 1 < v1) unext = valid ? Uin[(v + 1) * nc + c] : 0.;
     const double phi = valid ? uv / den : 0.;
     const double phip = __shfl_up(phi, 1);
     const double gb = (valid && validp) ? (phi - phip) / dxb : 0.;
@@ -2141,10 +2141,7 @@ __device__ __forceinline__ bool dual_kept(const MhDev& S, int prev, int i, int j
 // (computeAndLimitGradPhiDual, UtilesRemap.cc:369-400), in the order of k_sweep_node_body.
 template <int LIM>
 __device__ __forceinline__ double dual_limited(const MhDev& S, double gb, double gf) {
-  double g = 0.;
-  if (gb != 0.) g += 0.5 * mh_limiter<LIM>(S.limiter, gf / gb) * gb;
-  if (gf != 0.) g += 0.5 * mh_limiter<LIM>(S.limiter, gb / gf) * gf;
-  return g;
+  return mh_limited_gradient<LIM, true>(S.limiter, gb, gf);
 }
 
 // Writes the dual state (v, U[DIM]) of node n, or on the last sweep the velocity U / m
@@ -2160,9 +2157,11 @@ __device__ __forceinline__ void dual_store(const MhDev& S, long n, const double*
     for (int cc = 0; cc < DIM; ++cc) V[cc * nn + n] = v[cc];
   }
   if (!last || S.dec) dual_out_m<DIM>(S, psel)[n] = U[DIM];
-  if (last && U[DIM] != 0.)
+  if (last && U[DIM] != 0.) {
+    const MhRecip rm = mh_recip(U[DIM]);
 #pragma unroll
-    for (int cc = 0; cc < DIM; ++cc) S.u[cc][n] = U[cc] / U[DIM];
+    for (int cc = 0; cc < DIM; ++cc) S.u[cc][n] = mh_quot(U[cc], rm);
+  }
 }
 
 // Dual update of one node from its neighbourhood along D (DualPhaseRemap.cc:110-257):
@@ -2227,15 +2226,21 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
   }
   const bool kept = dual_kept<DIM>(S, prev, i, j, k);
 #pragma unroll
-  for (int cc = 0; cc < NC; ++cc) P[cc] = kept || !valid ? v[cc] : v[cc] / m;
+  for (int cc = 0; cc < NC; ++cc) P[cc] = v[cc];
+  if (!kept && valid) {
+    const MhRecip rm = mh_recip(m);
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) P[cc] = mh_quot(v[cc], rm);
+  }
   const bool inner = valid && i >= 1 && i <= na - 1;
   const double Xm = __shfl_up(X, 1), Xp = __shfl_down(X, 1);
   double Pm[NC], Pp[NC], G0[NC], Gm[NC], Gp[NC];
+  const MhRecip rX = mh_recip(X - Xm);
 #pragma unroll
   for (int cc = 0; cc < NC; ++cc) {
     Pm[cc] = __shfl_up(P[cc], 1);
     Pp[cc] = __shfl_down(P[cc], 1);
-    const double eb = (valid && validp) ? (P[cc] - Pm[cc]) / (X - Xm) : 0.;  // edge i-1/2
+    const double eb = (valid && validp) ? mh_quot(P[cc] - Pm[cc], rX) : 0.;  // edge i-1/2
     const double ef = __shfl_down(eb, 1);                                    // edge i+1/2
     G0[cc] = (S.order2 && inner) ? dual_limited<LIM>(S, eb, ef) : 0.;
     Gm[cc] = __shfl_up(G0[cc], 1);
@@ -2438,6 +2443,149 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
   }
 }
 
+// The same sweep for D = y or z on meshes that do not fill the chip with tiles: each thread holds
+// L cells of a column along D (and two halo cells on each side) in registers.  Per remap slot every
+// phi, face gradient, limited slope and face flux of the segment is formed once, without LDS or
+// barriers, and the chains of the L + 4 rows are independent of one another.  What bounds it is the
+// latency of one wavefront (about 2000 instructions and four rounds of loads for seven slots), so
+// the slots are shared out too (v0 .. v1-1 here).  Threads are consecutive along x, then over the
+// segments of a column, then over the columns, so any nx fills the wavefronts and consecutive
+// segments share their halo cells in L2.  Against the tiles, two environments: 15 -> 8 us on
+// 100x5x5 cells, 27 -> 10 us on 181x181, 29 -> 21 us on 512x512x1, 44 -> 39 us on 97x61x83; longer
+// segments are slower there (four cells: 10, 14, 24, 37 us).  Same formulas in the same order as
+// k_sweep_cell_body.
+MH_HD int seg_count(int na, int len) { return (na + len - 1) / len; }
+#ifndef MH_SEG_L
+#define MH_SEG_L 2  // cells along D per thread
+#endif
+template <int DIM, int D, int M, int LIM, int L>
+__device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, int usel, int first, int v0, int v1) {
+  constexpr int R = L + 4;
+  const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
+  const int na = D == 1 ? ny : nz;
+  const int nt = D == 1 ? (DIM == 3 ? nz : 1) : ny;
+  const int nseg = seg_count(na, L);
+  const long g = lb * (long)blockDim.x + threadIdx.x;
+  if (g >= (long)nx * nseg * nt) return;
+  if (mh_halted(S.sc)) return;
+  const int i = (int)(g % nx);
+  const int rest = (int)(g / nx);
+  const int abase = (rest % nseg) * L - 2;  // cell along D of row 0
+  const int t = rest / nseg;
+  const double* __restrict__ Uin = usel ? S.Ub : S.Ua;
+  double* __restrict__ Uout = usel ? S.Ua : S.Ub;
+  double* __restrict__ dflux = S.dflux;
+  const long nc = S.g.nc;
+  const long nnx = S.g.nnx, nny = S.g.nny;
+  const long sD = D == 1 ? (long)nx : (long)nx * ny;
+  const long c0 = (D == 1 ? i + (long)nx * ny * t : i + (long)nx * t) + abase * sD;
+  const long nD = D == 1 ? nnx : nnx * nny;
+  const long n0 = (D == 1 ? i + nnx * nny * t : i + nnx * t) + abase * nD;
+  const double dt = S.sc->dt;
+  const double o2 = (double)S.order2;
+  auto valid = [&](int r) { return abase + r >= 0 && abase + r < na; };
+  auto inner = [&](int f) { return valid(f - 1) && valid(f); };  // face f: between rows f-1 and f
+  double u[R], un[R];  // slot loads run one slot ahead
+#pragma unroll
+  for (int r = 0; r < R; ++r) un[r] = valid(r) ? Uin[v0 * nc + c0 + r * sD] : 0.;
+  unsigned ownm = 0;  // bit r: the cell's own U enters its update
+  MhRecip den[R], dx[R];
+  double xc[R], w[R], hh[R];
+  unsigned upm = 0;  // bit f: the upwind cell of face f is the one behind it
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    double d = 1.;
+    xc[r] = 0.;
+    if (valid(r)) {
+      const long c = c0 + r * sD;
+      if (first) {
+        const bool empty = !S.mask[c];  // an empty cell holds Phi itself and its U starts from 0
+        d = empty ? 1. : S.Vl[c];
+        if (!empty) ownm |= 1u << r;
+      } else {
+        ownm |= 1u << r;
+        double sv = 0.;
+        for (int k = 0; k < M; ++k) sv += Uin[k * nc + c];
+        d = sv;
+      }
+      xc[r] = cell_centre_d<DIM, D>(S, n0 + r * nD);
+    }
+    den[r] = mh_recip(d);
+  }
+#pragma unroll
+  for (int f = 1; f < R; ++f) {
+    const double d = inner(f) ? xc[f] - xc[f - 1] : 1.;
+    dx[f] = mh_recip(d);
+    w[f] = 0.;
+    hh[f] = 0.;
+    if (f >= 2 && f <= R - 2 && inner(f)) {
+      double area, xf, vf;
+      face_quant<DIM, D>(S, n0 + f * nD, area, xf, vf);
+      const bool up = vf * d > 0.0;
+      if (up) upm |= 1u << f;
+      hh[f] = o2 * (xf - (up ? xc[f - 1] : xc[f]));
+      w[f] = 1. * vf * area * dt;
+    }
+  }
+  for (int v = v0; v < v1; ++v) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      u[r] = un[r];
+      if (v + 1 < v1) un[r] = valid(r) ? Uin[(v + 1) * nc + c0 + r * sD] : 0.;
+    }
+    double phi[R], gr[R];
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      bad |= den[r].bad;
+      phi[r] = mh_div(u[r], den[r], bad);
+    }
+    if (__builtin_expect(bad, 0))
+#pragma unroll
+      for (int r = 0; r < R; ++r) phi[r] = u[r] / den[r].b;
+    bad = false;
+#pragma unroll
+    for (int f = 1; f < R; ++f) {
+      bad |= dx[f].bad;
+      gr[f] = mh_div(phi[f] - phi[f - 1], dx[f], bad);
+    }
+    if (__builtin_expect(bad, 0))
+#pragma unroll
+      for (int f = 1; f < R; ++f) gr[f] = (phi[f] - phi[f - 1]) / dx[f].b;
+#pragma unroll
+    for (int f = 1; f < R; ++f)
+      if (!inner(f)) gr[f] = 0.;
+#pragma unroll
+    for (int r = 1; r < R - 1; ++r)  // limited slope of row r in place of its back gradient
+      gr[r] = S.order2 && valid(r) ? mh_limited_gradient<LIM>(S.limiter, gr[r], gr[r + 1]) : 0.;
+    double F[R];
+#pragma unroll
+    for (int f = 2; f <= R - 2; ++f) {
+      const bool up = (upm >> f) & 1u;
+      const double pf = (up ? phi[f - 1] : phi[f]) + hh[f] * (up ? gr[f - 1] : gr[f]);
+      F[f] = inner(f) ? w[f] * pf : 0.;
+    }
+#pragma unroll
+    for (int r = 2; r < R - 2; ++r) {
+      if (!valid(r)) continue;
+      const double fb = -F[r], Ff = F[r + 1];
+      double ff = 0.;
+      if (inner(r)) ff += fb;
+      if (inner(r + 1)) ff += Ff;
+      const long c = c0 + r * sD;
+      double uo = (((ownm >> r) & 1u) ? u[r] : 0.) - ff;
+      if (v >= M && v < 2 * M) {
+        double dd = 0.;
+        if (inner(r)) dd += 0.5 * fb * -1.;
+        if (inner(r + 1)) dd += 0.5 * Ff * 1.;
+        dflux[(v - M) * nc + c] = dd;
+      }
+      if (v >= M && v < 3 * M && uo < 0.) uo = 0.;
+      Uout[v * nc + c] = uo;
+    }
+  }
+}
+
 // One ADI direction, dual part for one node: limited nodal velocity gradients
 // (computeDualGradPhi UtilesRemap.cc:19-72, computeAndLimitGradPhiDual :369-400), back/front
 // mass fluxes gathered from the cells behind/ahead in face order, env order
@@ -2600,8 +2748,8 @@ __device__ __forceinline__ void k_sweep_node_body(const MhDev& S, int lb, int ps
 // its back-side values), so each is formed once per node instead of by each of the three nodes
 // whose update reads it.  Threads of a wave are consecutive along x.  Same formulas and orders
 // as k_sweep_node_at (classical limiters; the generalised ones keep k_sweep_node).  The segment
-// length is per case (the autotuner tries 4-12 nodes): 10 by default from 2.6 M nodes on (fastest
-// on the 256x128x128 tube and the 192^3 Sedov blast), 4 on smaller meshes, which need the threads.
+// length is per case (the autotuner tries 4-12 nodes): 10 by default on large meshes, 4 on smaller
+// ones, which need the threads, and below MH_MARCH_NODES one thread per node (k_sweep_node).
 #ifndef MH_NM_L
 #define MH_NM_L 10  // default target segment length (MhDev::nm_len; variant march code 0, kMarchLen[0])
 #endif
@@ -2641,9 +2789,11 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) P[cc] = din.v[cc][m2];
       X = Xd[m2];
-      if (!kept)
+      if (!kept) {
+        const MhRecip rm = mh_recip(m);
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) P[cc] = P[cc] / m;
+        for (int cc = 0; cc < NC; ++cc) P[cc] = mh_quot(P[cc], rm);
+      }
     } else {
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) P[cc] = 0.;
@@ -2655,19 +2805,15 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
     const bool in = S.order2 && b >= 1 && b <= na - 1;
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) {
-      double gg = 0.;
-      if (in) {
-        if (gb[cc] != 0.) gg += 0.5 * mh_limiter<LIM>(S.limiter, gf[cc] / gb[cc]) * gb[cc];
-        if (gf[cc] != 0.) gg += 0.5 * mh_limiter<LIM>(S.limiter, gb[cc] / gf[cc]) * gf[cc];
-      }
-      G[cc] = gg;
+      G[cc] = in ? dual_limited<LIM>(S, gb[cc], gf[cc]) : 0.;
     }
   };
   // edge gradient between nodes b and b+1 (formed only where a limited gradient reads it)
   auto edge = [&](int b, const double* P0, double X0, const double* P1, double X1, double* E) {
     const bool used = S.order2 && b >= 0 && b + 1 <= na && (b >= 1 || b + 1 <= na - 1);
+    const MhRecip rX = mh_recip(X1 - X0);
 #pragma unroll
-    for (int cc = 0; cc < NC; ++cc) E[cc] = used ? (P1[cc] - P0[cc]) / (X1 - X0) : 0.;
+    for (int cc = 0; cc < NC; ++cc) E[cc] = used ? mh_quot(P1[cc] - P0[cc], rX) : 0.;
   };
   // window: P and X of nodes a-1 .. a+2 (slots 0..3), edges (a-1/2, a+1/2, a+3/2), G of a-1, a, a+1
   double P[4][NC], X[4], E[3][NC], G[3][NC];
@@ -3444,6 +3590,21 @@ MH_WRAP(k_prepare_remap, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>,
 MH_WRAP(k_sweep_node_march, MH_NM_MIN_WAVES, template <int DIM MH_COMMA int D MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA LIM>,
         MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
 
+// Small meshes: the remap slots of a cell are shared out over the gridDim.y rows of the grid, vper
+// each, so that a mesh of a few hundred wavefronts fills the chip and each thread forms the
+// geometry and one or a few slots instead of all 3m+1 one after the other.
+template <int DIM, int M, int LIM>
+__global__ __launch_bounds__(MH_BLOCK) void k_sweep_cell_row_slots(MhDev S, int usel, int first, int vper) {
+  const int v0 = (int)blockIdx.y * vper;
+  k_sweep_cell_row_body<DIM, M, LIM>(S, xcd_block((int)blockIdx.x, (int)gridDim.x), usel, first, v0,
+                                     min(v0 + vper, 3 * M + 1));
+}
+template <int DIM, int D, int M, int LIM, int L>
+__global__ __launch_bounds__(MH_BLOCK) void k_sweep_cell_seg(MhDev S, int usel, int first, int vper) {
+  const int v0 = (int)blockIdx.y * vper;
+  k_sweep_cell_seg_body<DIM, D, M, LIM, L>(S, xcd_block((int)blockIdx.x, (int)gridDim.x), usel, first, v0,
+                                           min(v0 + vper, 3 * M + 1));
+}
 // (the plain kernels are templates with an unused parameter, so that every translation unit
 // that launches one may instantiate it)
 template <int U = 0>

@@ -1,6 +1,8 @@
 // mh_sweep.hip -- launch sequences of the remap (sweeps in the rotated direction order,
 // finalize) for single meshes, and of a whole iteration for a batched ensemble group.
 // Compiled once per environment count: -DMH_TU_M=1..4.
+#include <algorithm>
+
 #include "mh_kernels.h"
 #include "mh_host.h"
 
@@ -9,6 +11,43 @@
 #endif
 
 // Cell part of one sweep direction (computeGradPhiFace ... computeUremap).
+// Slots shared out over gridDim.y groups of vper: as many groups as bring the launch to
+// `target` wavefronts, at least one.
+struct SlotSplit {
+  int groups, vper;
+};
+inline SlotSplit slot_split(long waves, long target, int nv) {
+  const long g = std::max(1L, std::min((long)nv, (target + waves / 2) / std::max(1L, waves)));
+  const int vper = (int)((nv + g - 1) / g);
+  return {(nv + vper - 1) / vper, vper};
+}
+template <int DIM, int M>
+void launch_cell_x(MhHandle* h, int sel, int first) {
+  const MhDev& S = h->dev;
+  // One thread runs a cell's 3m+1 slots one after the other, some 1 us each where nothing else
+  // fills the wait: up to about 4000 wavefronts (4 per SIMD) the slots are shared out (two
+  // environments: 7.9 -> 5.0 us on 100x5x5 cells, 7.7 -> 5.8 us on 181x181, 13.1 -> 11.6 us on
+  // 362x362); beyond that the repeated geometry costs more (512x512: 16.0 us, split 16.2).
+  const SlotSplit p = slot_split((long)row_blocks(h) * (MH_BLOCK / 64), 4000, 3 * M + 1);
+  if (p.groups > 1)
+    MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell_row_slots<DIM, M, LIM>), dim3(row_blocks(h), p.groups), MH_BLOCK,
+                       S, sel, first, p.vper));
+  else
+    MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell_row<DIM, M, LIM>), row_blocks(h), MH_BLOCK, S, sel, first));
+}
+template <int DIM, int D, int M>
+void launch_cell_yz(MhHandle* h, int sel, int first) {
+  const MhDev& S = h->dev;
+  if (seg_sweep(h)) {
+    // the slots of a segment as in launch_cell_x, up to about 2000 wavefronts of 2-cell segments
+    const SlotSplit p = slot_split((long)seg_blocks(h, D, MH_SEG_L) * (MH_BLOCK / 64), 2048, 3 * M + 1);
+    MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + D, (k_sweep_cell_seg<DIM, D, M, LIM, MH_SEG_L>),
+                       dim3(seg_blocks(h, D, MH_SEG_L), p.groups), MH_BLOCK, S, sel, first, p.vper));
+  } else {
+    MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + D, (k_sweep_cell_tile<DIM, D, M, LIM>), tile_blocks(h, D), MH_BLOCK, S, sel,
+                       first));
+  }
+}
 template <int DIM, int M>
 void launch_cell_part(MhHandle* h, int D, int sel, int first, bool gen, bool o3) {
   const MhDev& S = h->dev;
@@ -23,13 +62,13 @@ void launch_cell_part(MhHandle* h, int D, int sel, int first, bool gen, bool o3)
     else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_CELL + 2, (k_sweep_cell3<3, 2, M>), h->nblk_c, MH_BLOCK, S, sel, first);
   } else if (D == 0) {
     if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell<DIM, 0, M, LIM>), h->nblk_c, MH_BLOCK, S, sel, first));
-    else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell_row<DIM, M, LIM>), row_blocks(h), MH_BLOCK, S, sel, first));
+    else launch_cell_x<DIM, M>(h, sel, first);
   } else if (D == 1) {
     if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + 1, (k_sweep_cell<DIM, 1, M, LIM>), h->nblk_c, MH_BLOCK, S, sel, first));
-    else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + 1, (k_sweep_cell_tile<DIM, 1, M, LIM>), tile_blocks(h, 1), MH_BLOCK, S, sel, first));
+    else launch_cell_yz<DIM, 1, M>(h, sel, first);
   } else if constexpr (DIM == 3) {
     if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + 2, (k_sweep_cell<3, 2, M, LIM>), h->nblk_c, MH_BLOCK, S, sel, first));
-    else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + 2, (k_sweep_cell_tile<3, 2, M, LIM>), tile_blocks(h, 2), MH_BLOCK, S, sel, first));
+    else launch_cell_yz<3, 2, M>(h, sel, first);
   }
 }
 
@@ -40,6 +79,7 @@ void launch_dual_part(MhHandle* h, int D, int sel, int prev, int last, bool gen,
   const MhDev& S = h->dev;
   if (S.sans_lagrange) return;
   const bool flat = h->sweep_mode == MH_SWEEP_FLAT;
+  const bool march = !flat && !o3 && march_sweep(h);  // y / z: threads march over segments of nodes
   if (gen) {
     if (D == 0) LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
     else if (D == 1) LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
@@ -48,12 +88,12 @@ void launch_dual_part(MhHandle* h, int D, int sel, int prev, int last, bool gen,
     if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
     else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node_row<DIM, LIM>), node_row_blocks(h), MH_BLOCK, S, sel, prev, last));
   } else if (D == 1) {
-    if (!flat && !o3)  // threads march along y over segments of nodes
+    if (march)
       MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node_march<DIM, 1, LIM>), node_march_blocks(h, 1), MH_BLOCK, S, sel, prev, last));
     else
       MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
   } else if constexpr (DIM == 3) {
-    if (!flat && !o3)  // threads march along z over segments of nodes
+    if (march)
       MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node_march<3, 2, LIM>), node_march_blocks(h, 2), MH_BLOCK, S, sel, prev, last));
     else
       MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));

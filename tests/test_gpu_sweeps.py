@@ -47,10 +47,21 @@ def check(c, iterations=13):
     assert not bad, bad
 
 
+# the variants a mesh takes by its size, and at every size those of the large meshes (tiles,
+# marching segments) and one thread per item
+@pytest.mark.parametrize("sweep,node", [("", ""), ("tile", "tiled"), ("flat", "flat")])
 @pytest.mark.parametrize("seed", [0, 1, 2])
 @pytest.mark.parametrize("n", SHAPES + FLAT, ids=lambda n: "x".join(map(str, n)))
-def test_sweeps_at_launch_shape_edges(n, seed):
+def test_sweeps_at_launch_shape_edges(n, seed, sweep, node, monkeypatch):
+    monkeypatch.setenv("MAHYCO_SWEEP", sweep)
+    monkeypatch.setenv("MAHYCO_NODE_KERNEL", node)
     check(moving_tube(n, seed))
+
+
+@pytest.mark.parametrize("n", [(181, 20), (300, 100), (31, 30, 29), (62, 40, 20)], ids=lambda n: "x".join(map(str, n)))
+def test_slots_shared_out(n):
+    """Meshes around the lines between one, two, four and all slots per thread."""
+    check(moving_tube(n, 2), iterations=5)
 
 
 @pytest.mark.parametrize("n", [(3, 17, 4), (5, 1, 6), (1, 1, 5), (61, 18)], ids=lambda n: "x".join(map(str, n)))
