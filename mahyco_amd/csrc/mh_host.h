@@ -172,11 +172,10 @@ inline int node_march_blocks(MhHandle* h, int D) {
 // the y / z variants a single mesh takes (an ensemble's launches are filled by its many cases)
 inline bool seg_sweep(const MhHandle* h) { return !h->sweep_large && h->g.nc < MH_SEG_CELLS; }
 inline bool march_sweep(const MhHandle* h) { return h->sweep_large || h->g.nn >= MH_MARCH_NODES; }
-// blocks of the segment y / z sweep (one thread per len cells of a column), a multiple of 8
+// blocks of the sweeps over segments (one thread per len cells of a line along D), a multiple of 8
 inline int seg_blocks(MhHandle* h, int D, int len) {
-  const long na = D == 1 ? h->g.ny : h->g.nz;
-  const long nt = D == 1 ? (h->g.dim == 3 ? h->g.nz : 1) : h->g.ny;
-  const long threads = (long)h->g.nx * nt * seg_count((int)na, len);
+  const long na = D == 0 ? h->g.nx : D == 1 ? h->g.ny : h->g.nz;
+  const long threads = h->g.nc / na * seg_count((int)na, len);
   return (int)(((threads + MH_BLOCK - 1) / MH_BLOCK + 7) / 8 * 8);
 }
 inline int tile_blocks(MhHandle* h, int D) {

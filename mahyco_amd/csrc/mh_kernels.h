@@ -1324,6 +1324,9 @@ __device__ __forceinline__ void k_sweep_cell_body(const MhDev& S, int lb, int us
   }
 }
 
+// Segments of `len` cells of a line of na cells.
+MH_HD int seg_count(int na, int len) { return (na + len - 1) / len; }
+
 // ----------------------------------------------------------------------------- order-3 remap
 // Lagrangian centre of the face of direction D whose first node is f0, all three components,
 // summed over the face nodes in Arcane order as computeFaceQuantitesForRemap does
@@ -1398,52 +1401,80 @@ __device__ __forceinline__ void k_hcell_body(const MhDev& S, int lb) {
   }
 }
 
-// Remap-ordre-3.cc:16-112: evaluate_grad, evaluate_ystar, evaluate_fm / evaluate_fp (the
-// piecewise-parabolic reconstruction on a non-uniform 1D stencil).
-__device__ __forceinline__ double o3_grad(double hm, double h0, double hp, double ym, double y0, double yp) {
-  return h0 / (hm + h0 + hp) * ((2. * hm + h0) / (h0 + hp) * (yp - y0) + (h0 + 2. * hp) / (hm + h0) * (y0 - ym));
+// The order-3 face values (ComputeFluxOrdre3, Remap-ordre-3.cc:16-189) on a line of cells: the
+// limited parabola of each cell from the gradients evaluate_grad of the cells and the edge values
+// evaluate_ystar of the faces, a non-uniform 1D stencil.  Every factor that depends on the widths
+// and the velocity alone is formed once per cell or face and serves all remap slots; the products
+// and sums over the values keep the reference's order, so the results have its bits.
+struct O3Grad {  // cell of width h0 between hm and hp
+  double c, cp, cm;
+};
+__device__ __forceinline__ O3Grad o3_grad_coef(double hm, double h0, double hp) {
+  O3Grad g;
+  g.c = h0 / (hm + h0 + hp);
+  g.cp = (2. * hm + h0) / (h0 + hp);
+  g.cm = (h0 + 2. * hp) / (hm + h0);
+  return g;
 }
-__device__ __forceinline__ double o3_ystar(double hmm, double hm, double hp, double hpp, double ymm, double ym,
-                                           double yp, double ypp, double gradm, double gradp) {
-  const double t1 = (2. * hp * hm) / (hm + hp) * ((hmm + hm) / (2. * hm + hp) - (hpp + hp) / (2. * hp + hm)) * (yp - ym);
-  const double t2 = -hm * (hmm + hm) / (2. * hm + hp) * gradp + hp * (hp + hpp) / (hm + 2. * hp) * gradm;
-  return ym + hm / (hm + hp) * (yp - ym) + 1. / (hmm + hm + hp + hpp) * (t1 + t2);
+__device__ __forceinline__ double o3_grad(const O3Grad& g, double ym, double y0, double yp) {
+  return g.c * (g.cp * (yp - y0) + g.cm * (y0 - ym));
 }
-__device__ __forceinline__ double o3_fm(double x, double dx, double up, double du, double u6) {
-  return up - 0.5 * x / dx * (du - (1. - 2. / 3. * x / dx) * u6);
+struct O3Star {  // face between cells of widths hm and hp, their outer neighbours hmm and hpp
+  double t, gp, gm, f, w;
+};
+__device__ __forceinline__ O3Star o3_star_coef(double hmm, double hm, double hp, double hpp) {
+  O3Star c;
+  c.t = (2. * hp * hm) / (hm + hp) * ((hmm + hm) / (2. * hm + hp) - (hpp + hp) / (2. * hp + hm));
+  c.gp = -hm * (hmm + hm) / (2. * hm + hp);
+  c.gm = hp * (hp + hpp) / (hm + 2. * hp);
+  c.f = hm / (hm + hp);
+  c.w = 1. / (hmm + hm + hp + hpp);
+  return c;
 }
-__device__ __forceinline__ double o3_fp(double x, double dx, double um, double du, double u6) {
-  return um + 0.5 * x / dx * (du - (1. - 2. / 3. * x / dx) * u6);
+__device__ __forceinline__ double o3_star(const O3Star& c, double ym, double yp, double gradm, double gradp) {
+  const double d = yp - ym;
+  const double t1 = c.t * d;
+  const double t2 = c.gp * gradp + c.gm * gradm;
+  return ym + c.f * d + c.w * (t1 + t2);
 }
-
-// ComputeFluxOrdre3 (Remap-ordre-3.cc:127-189): face value from the six cells y[0..5]
-// around the face (y[2] behind, y[3] ahead) of widths h[0..5], for the displacement
-// vdt = u_face dt, clipped to the interval the upwind cell and its neighbours allow.
-__device__ __forceinline__ double flux_ordre3(const double* y, const double* h, double vdt) {
-  const double gmm = o3_grad(h[0], h[1], h[2], y[0], y[1], y[2]);
-  const double gm = o3_grad(h[1], h[2], h[3], y[1], y[2], y[3]);
-  const double gp = o3_grad(h[2], h[3], h[4], y[2], y[3], y[4]);
-  const double gpp = o3_grad(h[3], h[4], h[5], y[3], y[4], y[5]);
-  const double ysm = o3_ystar(h[0], h[1], h[2], h[3], y[0], y[1], y[2], y[3], gmm, gm);
-  const double ys = o3_ystar(h[1], h[2], h[3], h[4], y[1], y[2], y[3], y[4], gm, gp);
-  const double ysp = o3_ystar(h[2], h[3], h[4], h[5], y[2], y[3], y[4], y[5], gp, gpp);
-  const double ym = y[2], yp = y[3], hm = h[2], hp = h[3];
-  double flux;
-  if (vdt > 0.) flux = o3_fm(vdt, hm, ys, ys - ysm, 6. * (ym - 0.5 * (ysm + ys)));
-  else if (vdt < 0.) flux = o3_fp(-vdt, hp, ys, ysp - ys, 6. * (yp - 0.5 * (ys + ysp)));
-  else return 0.;
-  const double num = vdt / hm, nup = vdt / hp;
-  const double ym_ym = ym + (1. - num) / num * (ym - y[1]);
-  const double yp_ym = yp - (1. + nup) / nup * (yp - y[4]);
-  const double a0 = amin(ym, yp), a1 = amax(ym, yp);
-  double b0, b1;
-  if (vdt >= 0.) {
-    b0 = amin(ym, ym_ym);
-    b1 = amax(ym, ym_ym);
-  } else {
-    b0 = amin(yp, yp_ym);
-    b1 = amax(yp, yp_ym);
+struct O3Face {  // displacement vdt = u_face dt through a face between widths hm and hp
+  double x, q, k;  // 0.5 |vdt| / h, 1 - 2/3 |vdt| / h of the upwind cell, the weight of its slope limit
+  int dir;         // 1: from behind, -1: from ahead, 0: none
+};
+__device__ __forceinline__ O3Face o3_face_coef(double vdt, double hm, double hp) {
+  O3Face c;
+  c.x = c.q = c.k = 0.;
+  c.dir = vdt > 0. ? 1 : vdt < 0. ? -1 : 0;
+  if (vdt > 0.) {
+    const double num = vdt / hm;
+    c.x = 0.5 * vdt / hm;
+    c.q = 1. - 2. / 3. * vdt / hm;
+    c.k = (1. - num) / num;
+  } else if (vdt < 0.) {
+    const double nup = vdt / hp;
+    c.x = 0.5 * -vdt / hp;
+    c.q = 1. - 2. / 3. * -vdt / hp;
+    c.k = (1. + nup) / nup;
   }
+  return c;
+}
+// The face value from the cells around the face (ymm, ym behind, yp, ypp ahead) and the edge values
+// of the face behind, the face and the face ahead, clipped to the interval the upwind cell and its
+// neighbours allow (Remap-ordre-3.cc:155-189).
+__device__ __forceinline__ double o3_flux(const O3Face& c, double ymm, double ym, double yp, double ypp, double ysm,
+                                          double ys, double ysp) {
+  if (c.dir == 0) return 0.;
+  double flux, b;
+  if (c.dir > 0) {
+    flux = ys - c.x * ((ys - ysm) - c.q * (6. * (ym - 0.5 * (ysm + ys))));
+    b = ym + c.k * (ym - ymm);
+  } else {
+    flux = ys + c.x * ((ysp - ys) - c.q * (6. * (yp - 0.5 * (ys + ysp))));
+    b = yp - c.k * (yp - ypp);
+  }
+  const double yu = c.dir > 0 ? ym : yp;
+  const double a0 = amin(ym, yp), a1 = amax(ym, yp);
+  const double b0 = amin(yu, b), b1 = amax(yu, b);
   double lo, hi;
   if ((a1 < b0) || (b1 < a0)) {
     lo = 0.;
@@ -1458,132 +1489,204 @@ __device__ __forceinline__ double flux_ordre3(const double* y, const double* h, 
 }
 
 // One ADI direction, cell part, order 3 (computeUpwindFaceQuantitiesForProjection,
-// RemapADIService.cc:319-379, then computeUremap :395-575): the face value of each
-// variable comes from the six cells around the face along D, clamped at the mesh boundary
-// (ComputeFluxOrdre3).  Across a face whose two cells are not pure cells of one
-// environment, the mass and energy face values are rebuilt from the upwind cell's
-// ratios.  The flags of the two cells come from the sweep input (volume fractions > 0,
-// :559-573), or in the first sweep of a cycle from the flags remapVariables left
-// (RemapADIFinal.cc:124-145).  Phi as in k_sweep_cell_body.
-template <int DIM, int D, int M>
-__device__ __forceinline__ void k_sweep_cell3_body(const MhDev& S, int lb, int usel, int first) {
+// RemapADIService.cc:319-379, then computeUremap :395-575): the face value of each variable
+// comes from the six cells around the face along D, clamped at the mesh boundary.  Across a face
+// whose two cells are not pure cells of one environment, the mass and energy face values are
+// rebuilt from the upwind cell's ratios.  The flags of the two cells come from the sweep input
+// (volume fractions > 0, :559-573), or in the first sweep of a cycle from the flags
+// remapVariables left (RemapADIFinal.cc:124-145).  Phi as in k_sweep_cell_body.
+//
+// Each thread holds L cells of a line along D and three halo cells on each side in registers; a
+// halo cell beyond the mesh is the boundary cell again, as the reference clamps.  With one cell per
+// thread the kernel was bound by FP64 instructions: every face value was formed by both its cells,
+// from eight gradients and six edge values with their divisions in every slot (7000-8500
+// instructions per cell).  Two cells per thread share them, and the factors of the widths are
+// formed once: 145 / 164 / 164 -> 54 / 64 / 64 us for x / y / z on 128x64x64 cells and two
+// environments, at two wavefronts per SIMD (256 registers), now bound by latency at that occupancy;
+// one cell per thread with the same factors takes 68 / 66 / 66 us.  Slots run environment by
+// environment (volume, mass, energy, then V q), so that the face values the correction needs live
+// for one environment only; groups e0 .. e1-1 of the m environments and V q (a small mesh shares
+// them out over gridDim.y).
+#define MH_O3_L 2  // cells along D per thread
+template <int DIM, int D, int M, int L>
+__device__ __forceinline__ void k_sweep_cell3_body(const MhDev& S, int lb, int usel, int first, int e0, int e1) {
+  constexpr int R = L + 6;
   const double* __restrict__ Uin = usel ? S.Ub : S.Ua;
   double* __restrict__ Uout = usel ? S.Ua : S.Ub;
-  constexpr int NV = 3 * M + 1;
-  const long c = lb * (long)blockDim.x + threadIdx.x;
-  if (c >= S.g.nc) return;
+  const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
+  const int na = D == 0 ? nx : D == 1 ? ny : nz;
+  const int nseg = seg_count(na, L);
+  const long g = lb * (long)blockDim.x + threadIdx.x;
+  if (g >= S.g.nc / na * nseg) return;
   if (mh_halted(S.sc)) return;
-  const bool own = !(first && S.mask[c] == 0);  // an empty cell's U starts from 0 (its Phi is stale)
-  const int nx = S.g.nx, ny = S.g.ny;
-  const int i = (int)(c % nx);
-  const long r = c / nx;
-  const int j = (int)(r % ny);
-  const int k = (int)(r / ny);
-  const int a = D == 0 ? i : D == 1 ? j : k;
-  const int na = D == 0 ? nx : D == 1 ? ny : S.g.nz;
+  // threads run along x first (segments of it for D = 0), then over the segments along D
+  int i, j, k, a0;
+  if (D == 0) {
+    a0 = (int)(g % nseg) * L;
+    const int r = (int)(g / nseg);
+    i = 0;
+    j = r % ny;
+    k = r / ny;
+  } else {
+    i = (int)(g % nx);
+    const int r = (int)(g / nx);
+    a0 = (r % nseg) * L;
+    j = D == 1 ? 0 : r / nseg;
+    k = D == 1 ? r / nseg : 0;
+  }
+  const long nc = S.g.nc;
   const long sD = D == 0 ? 1 : D == 1 ? (long)nx : (long)nx * ny;
   const long nD = D == 0 ? 1 : D == 1 ? (long)S.g.nnx : (long)S.g.nnx * S.g.nny;
-  const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
-  const long nc = S.g.nc;
+  const long line = i + (long)nx * (j + (long)ny * k);  // cell and node of the line at 0
+  const long nline = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
   const double dt = S.sc->dt;
-  // stencil: offsets -3..3 along D, clamped to the mesh (index o + 3)
-  long cs[7];
-  double den[7], hs[7];
+  // row r: the cell at a0 - 3 + r, clamped; face f: between rows f-1 and f
+  int cs[R];  // offset of the row from the line
+  MhRecip den[R];
+  double h[R];
 #pragma unroll
-  for (int o = 0; o < 7; ++o) {
-    const int ao = min(max(a + o - 3, 0), na - 1);
-    cs[o] = c + (ao - a) * sD;
+  for (int r = 0; r < R; ++r) {
+    cs[r] = min(max(a0 - 3 + r, 0), na - 1) * (int)sD;
+    double d;
     if (first) {
-      den[o] = S.mask[cs[o]] ? S.Vl[cs[o]] : 1.;  // an empty cell holds Phi itself
+      d = S.mask[line + cs[r]] ? S.Vl[line + cs[r]] : 1.;  // an empty cell holds Phi itself
     } else {
-      double sv = 0.;
-      for (int kk = 0; kk < M; ++kk) sv += Uin[kk * nc + cs[o]];
-      den[o] = sv;
+      d = 0.;
+      for (int kk = 0; kk < M; ++kk) d += Uin[kk * nc + line + cs[r]];
     }
-    hs[o] = S.hc[D * nc + cs[o]];
+    den[r] = mh_recip(d);
+    h[r] = S.hc[D * nc + line + cs[r]];
   }
-  // the two faces of the cell along D: s = 0 back (cells at offsets -1, 0), s = 1 front (0, +1)
-  bool inner[2];
-  double area[2], vf[2], vdt[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    inner[s] = s == 0 ? (a > 0) : (a < na - 1);
-    area[s] = 0.;
-    vf[s] = 0.;
-    vdt[s] = 0.;
-    if (!inner[s]) continue;
-    double xf;
-    face_quant<DIM, D>(S, b + s * nD, area[s], xf, vf[s]);
-    vdt[s] = vf[s] * dt;
-  }
-  // flags of the cells at offsets -1, 0, +1
-  int code[3] = {0, 0, 0}, cnt[3] = {0, 0, 0}, pur[3] = {-1, -1, -1};
+  // flags of the cells beside the faces: rows 2 .. L+3
+  int code[L + 2];
   if (first) {
 #pragma unroll
-    for (int o = 0; o < 3; ++o) code[o] = S.est[cs[o + 2]];
-  }
-  bool vpure[2] = {true, true};
-  double fv[2][M], pv[2][M], fm[2][M], pm[2][M];
-  bool cor[2][M];
-  const int s0 = (DIM == 2 && D == 0) ? 1 : 0, s1 = 1 - s0;
-  const double od[2] = {-1., 1.};
-  for (int v = 0; v < NV; ++v) {
-    if (v == M) {
-      if (!first) {
+    for (int o = 0; o < L + 2; ++o) code[o] = S.est[line + cs[o + 2]];
+  } else {
 #pragma unroll
-        for (int o = 0; o < 3; ++o) code[o] = cnt[o] > 1 ? MH_EST_MIXED : pur[o];
-      }
-#pragma unroll
-      for (int s = 0; s < 2; ++s) vpure[s] = code[s] == code[s + 1] && code[s] != MH_EST_MIXED;
-    }
-    double phi[7];
-#pragma unroll
-    for (int o = 0; o < 7; ++o) phi[o] = Uin[v * nc + cs[o]] / den[o];
-    if (v < M && !first) {
-#pragma unroll
-      for (int o = 0; o < 3; ++o)
-        if (phi[o + 2] > 0.) {
-          cnt[o]++;
-          pur[o] = v;
+    for (int o = 0; o < L + 2; ++o) {
+      int cnt = 0, pur = -1;
+      for (int v = 0; v < M; ++v)
+        if (mh_quot(Uin[v * nc + line + cs[o + 2]], den[o + 2]) > 0.) {
+          cnt++;
+          pur = v;
         }
+      code[o] = cnt > 1 ? MH_EST_MIXED : pur;
     }
-    double flux[2] = {0., 0.};
+  }
+  O3Grad cg[R];   // rows 1 .. R-2
+  O3Star cst[R];  // faces 2 .. R-2
+  O3Face cf[L + 1];
+  double w[L + 1];
+  bool vpure[L + 1];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if (!inner[s]) continue;
-      double pf = flux_ordre3(&phi[s], &hs[s], vdt[s]);
-      // upwind cell of the face: offset s-1 (vdt > 0) or s (vdt < 0)
-      const double pu = vdt[s] > 0. ? phi[s + 2] : phi[s + 3];
-      if (v < M) {
-        fv[s][v] = pf;
-        pv[s][v] = pu;
-      } else if (v < 2 * M) {
-        const int e = v - M;
-        cor[s][e] = !vpure[s] && (vdt[s] > 0. || vdt[s] < 0.) && pv[s][e] != 0. && pu != 0.;
-        if (cor[s][e]) pf = (pu / pv[s][e]) * fv[s][e];
-        fm[s][e] = pf;
-        pm[s][e] = pu;
-      } else if (v < 3 * M) {
-        const int e = v - 2 * M;
-        if (cor[s][e]) pf = (pu / pm[s][e]) * fm[s][e];
+  for (int r = 1; r < R - 1; ++r) cg[r] = o3_grad_coef(h[r - 1], h[r], h[r + 1]);
+#pragma unroll
+  for (int f = 2; f < R - 1; ++f) cst[f] = o3_star_coef(h[f - 2], h[f - 1], h[f], h[f + 1]);
+#pragma unroll
+  for (int s = 0; s <= L; ++s) {  // face s of the segment: behind cell a0 + s
+    const int a = a0 + s;
+    double vdt = 0.;
+    w[s] = 0.;
+    vpure[s] = code[s] == code[s + 1] && code[s] != MH_EST_MIXED;
+    if (a > 0 && a < na) {
+      double area, xf, vf;
+      face_quant<DIM, D>(S, nline + a * nD, area, xf, vf);
+      vdt = vf * dt;
+      w[s] = vf * area * dt;
+    }
+    cf[s] = o3_face_coef(vdt, h[s + 2], h[s + 3]);
+  }
+  unsigned ownm = 0;  // bit o: the cell's own U enters its update (an empty cell's U starts from 0)
+#pragma unroll
+  for (int o = 0; o < L; ++o)
+    if (!(first && S.mask[line + cs[o + 3]] == 0)) ownm |= 1u << o;
+
+  double pf[L + 1], pu[L + 1];  // face value and upwind phi of the slot
+  auto slot = [&](int v, double* u) {
+    double y[R], gr[R], ys[R];
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const double uv = Uin[v * nc + line + cs[r]];
+      bad |= den[r].bad;
+      y[r] = mh_div(uv, den[r], bad);
+      if (r >= 3 && r < 3 + L) u[r - 3] = uv;
+    }
+    if (__builtin_expect(bad, 0))
+#pragma unroll
+      for (int r = 0; r < R; ++r) y[r] = Uin[v * nc + line + cs[r]] / den[r].b;
+#pragma unroll
+    for (int r = 1; r < R - 1; ++r) gr[r] = o3_grad(cg[r], y[r - 1], y[r], y[r + 1]);
+#pragma unroll
+    for (int f = 2; f < R - 1; ++f) ys[f] = o3_star(cst[f], y[f - 1], y[f], gr[f - 1], gr[f]);
+#pragma unroll
+    for (int s = 0; s <= L; ++s) {
+      pf[s] = o3_flux(cf[s], y[s + 1], y[s + 2], y[s + 3], y[s + 4], ys[s + 2], ys[s + 3], ys[s + 4]);
+      pu[s] = cf[s].dir > 0 ? y[s + 2] : y[s + 3];
+    }
+  };
+  auto store = [&](int v, const double* u, bool mass, bool clamp) {
+#pragma unroll
+    for (int o = 0; o < L; ++o) {
+      const int a = a0 + o;
+      if (a >= na) continue;
+      const bool inb = a > 0, inf = a < na - 1;
+      const double Fb = -(w[o] * pf[o]), Ff = w[o + 1] * pf[o + 1];
+      double ff = 0., dd = 0.;
+      if (DIM == 2 && D == 0) {  // cell faces in Arcane order: 2D x has the max face first
+        if (inf) ff += Ff;
+        if (inb) ff += Fb;
+        if (inf) dd += 0.5 * Ff * 1.;
+        if (inb) dd += 0.5 * Fb * -1.;
+      } else {
+        if (inb) ff += Fb;
+        if (inf) ff += Ff;
+        if (inb) dd += 0.5 * Fb * -1.;
+        if (inf) dd += 0.5 * Ff * 1.;
       }
-      flux[s] = od[s] * vf[s] * area[s] * dt * pf;
+      const long c = line + a * sD;
+      double un = (((ownm >> o) & 1u) ? u[o] : 0.) - ff;
+      if (mass) S.dflux[(v - M) * nc + c] = dd;
+      if (clamp && un < 0.) un = 0.;  // computeUremap clamps, :465-485
+      Uout[v * nc + c] = un;
     }
-    double ff = 0.;
-    if (inner[s0]) ff += flux[s0];
-    if (inner[s1]) ff += flux[s1];
-    double un = (own ? Uin[v * nc + c] : 0.) - ff;
-    if (v >= M && v < 2 * M) {
-      double dd = 0.;
-      if (inner[s0]) dd += 0.5 * flux[s0] * od[s0];
-      if (inner[s1]) dd += 0.5 * flux[s1] * od[s1];
-      S.dflux[(v - M) * nc + c] = dd;
+  };
+  for (int e = e0; e < e1; ++e) {
+    double u[L];
+    if (e == M) {
+      slot(3 * M, u);
+      store(3 * M, u, false, false);
+      break;
     }
-    if (v >= M && v < 3 * M && un < 0.) un = 0.;  // computeUremap clamps, :465-485
-    Uout[v * nc + c] = un;
+    double fv[L + 1], pv[L + 1];
+    bool cor[L + 1];
+    slot(e, u);
+    store(e, u, false, false);
+#pragma unroll
+    for (int s = 0; s <= L; ++s) {
+      fv[s] = pf[s];
+      pv[s] = pu[s];
+    }
+    slot(M + e, u);
+#pragma unroll
+    for (int s = 0; s <= L; ++s) {
+      cor[s] = !vpure[s] && cf[s].dir != 0 && pv[s] != 0. && pu[s] != 0.;
+      if (cor[s]) pf[s] = (pu[s] / pv[s]) * fv[s];
+    }
+    store(M + e, u, true, true);
+#pragma unroll
+    for (int s = 0; s <= L; ++s) {
+      fv[s] = pf[s];
+      pv[s] = pu[s];
+    }
+    slot(2 * M + e, u);
+#pragma unroll
+    for (int s = 0; s <= L; ++s)
+      if (cor[s]) pf[s] = (pu[s] / pv[s]) * fv[s];
+    store(2 * M + e, u, false, true);
   }
 }
-
 
 // ----------------------------------------------------------------------------- generalised
 // limiters and pente-borne fluxes (UtilesRemap.cc), in the reference's operation order.
@@ -2454,7 +2557,6 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
 // 100x5x5 cells, 27 -> 10 us on 181x181, 29 -> 21 us on 512x512x1, 44 -> 39 us on 97x61x83; longer
 // segments are slower there (four cells: 10, 14, 24, 37 us).  Same formulas in the same order as
 // k_sweep_cell_body.
-MH_HD int seg_count(int na, int len) { return (na + len - 1) / len; }
 #ifndef MH_SEG_L
 #define MH_SEG_L 2  // cells along D per thread
 #endif
@@ -3580,8 +3682,6 @@ MH_WRAP(k_node_adv, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_node_fwd, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_sweep_cell_gen, 1, template <int DIM MH_COMMA int D MH_COMMA int M>, <DIM MH_COMMA D MH_COMMA M>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
-MH_WRAP(k_sweep_cell3, 1, template <int DIM MH_COMMA int D MH_COMMA int M>, <DIM MH_COMMA D MH_COMMA M>,
-        MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
 MH_WRAP(k_sweep_ke, 1, template <int DIM MH_COMMA int D>, <DIM MH_COMMA D>, MH_COMMA int psel MH_COMMA int prev,
         MH_COMMA psel MH_COMMA prev)
 MH_WRAP(k_dual_init, 1, template <int DIM>, <DIM>, , )
@@ -3604,6 +3704,24 @@ __global__ __launch_bounds__(MH_BLOCK) void k_sweep_cell_seg(MhDev S, int usel, 
   const int v0 = (int)blockIdx.y * vper;
   k_sweep_cell_seg_body<DIM, D, M, LIM, L>(S, xcd_block((int)blockIdx.x, (int)gridDim.x), usel, first, v0,
                                            min(v0 + vper, 3 * M + 1));
+}
+// The order-3 sweep: gridDim.y rows of the grid share out the environments and V q, eper each.
+template <int DIM, int D, int M>
+__global__ __launch_bounds__(MH_BLOCK, 2) void k_sweep_cell3(MhDev S, int usel, int first, int eper) {
+  const int e0 = (int)blockIdx.y * eper;
+  k_sweep_cell3_body<DIM, D, M, MH_O3_L>(S, xcd_block((int)blockIdx.x, (int)gridDim.x), usel, first, e0,
+                                         min(e0 + eper, M + 1));
+}
+template <int DIM, int D, int M>
+__global__ __launch_bounds__(MH_BLOCK, 2) void k_sweep_cell3_batch(const MhDev* __restrict__ tab,
+                                                                const int2* __restrict__ bmap,
+                                                                const int* __restrict__ nwork, int usel, int first) {
+  const int n = *nwork;
+  for (int w = (int)blockIdx.x; w < n; w += (int)gridDim.x) {
+    const int2 bm = bmap[w];
+    k_sweep_cell3_body<DIM, D, M, MH_O3_L>(tab[bm.x], bm.y, usel, first, 0, M + 1);
+    __syncthreads();
+  }
 }
 // (the plain kernels are templates with an unused parameter, so that every translation unit
 // that launches one may instantiate it)

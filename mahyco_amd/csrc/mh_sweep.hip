@@ -48,6 +48,12 @@ void launch_cell_yz(MhHandle* h, int sel, int first) {
                        first));
   }
 }
+template <int DIM, int D, int M>
+void launch_cell3(MhHandle* h, int sel, int first) {
+  const int nb = seg_blocks(h, D, MH_O3_L);
+  const SlotSplit p = slot_split((long)nb * (MH_BLOCK / 64), 2048, M + 1);
+  LAUNCH(h, KN_SWEEP_CELL + D, (k_sweep_cell3<DIM, D, M>), dim3(nb, p.groups), MH_BLOCK, h->dev, sel, first, p.vper);
+}
 template <int DIM, int M>
 void launch_cell_part(MhHandle* h, int D, int sel, int first, bool gen, bool o3) {
   const MhDev& S = h->dev;
@@ -57,9 +63,9 @@ void launch_cell_part(MhHandle* h, int D, int sel, int first, bool gen, bool o3)
     else if (D == 1) LAUNCH(h, KN_SWEEP_CELL + 1, (k_sweep_cell_gen<DIM, 1, M>), h->nblk_c, MH_BLOCK, S, sel, first);
     else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_CELL + 2, (k_sweep_cell_gen<3, 2, M>), h->nblk_c, MH_BLOCK, S, sel, first);
   } else if (o3) {
-    if (D == 0) LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell3<DIM, 0, M>), h->nblk_c, MH_BLOCK, S, sel, first);
-    else if (D == 1) LAUNCH(h, KN_SWEEP_CELL + 1, (k_sweep_cell3<DIM, 1, M>), h->nblk_c, MH_BLOCK, S, sel, first);
-    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_CELL + 2, (k_sweep_cell3<3, 2, M>), h->nblk_c, MH_BLOCK, S, sel, first);
+    if (D == 0) launch_cell3<DIM, 0, M>(h, sel, first);
+    else if (D == 1) launch_cell3<DIM, 1, M>(h, sel, first);
+    else if constexpr (DIM == 3) launch_cell3<3, 2, M>(h, sel, first);
   } else if (D == 0) {
     if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell<DIM, 0, M, LIM>), h->nblk_c, MH_BLOCK, S, sel, first));
     else launch_cell_x<DIM, M>(h, sel, first);
@@ -153,7 +159,9 @@ void ens_sweep(const EnsGroup& g, const MhDev* tab, hipStream_t st, dim3 G, int 
       if (!g.adv)
         hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, MH_LIM_ANY>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     } else {
-      hipLaunchKernelGGL((k_sweep_cell3_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(g.cmap), sel, first);
+      hipLaunchKernelGGL((k_sweep_cell3_batch<DIM, D, M>), G, B, 0, st, tab,
+                         D == 0 ? g.rcmap.d : g.tmap[D == 0 ? 0 : D - 1].d,
+                         D == 0 ? g.rcmap.d_n : g.tmap[D == 0 ? 0 : D - 1].d_n, sel, first);
       if (!g.adv)
         hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, -1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     }

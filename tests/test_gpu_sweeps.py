@@ -67,3 +67,15 @@ def test_slots_shared_out(n):
 @pytest.mark.parametrize("n", [(3, 17, 4), (5, 1, 6), (1, 1, 5), (61, 18)], ids=lambda n: "x".join(map(str, n)))
 def test_total_energy_reads_the_last_sweeps_mass(n):
     check(moving_tube(n, 1, conservation_energie_totale=True))
+
+
+@pytest.mark.parametrize("seed", [0, 1])
+@pytest.mark.parametrize("n", SHAPES + FLAT, ids=lambda n: "x".join(map(str, n)))
+def test_order3_segments(n, seed):
+    """The order-3 sweep at odd and even line lengths, lines shorter than its stencil included."""
+    check(moving_tube(n, seed, ordre_projection=3))
+
+
+def test_order3_three_materials():
+    check(moving_tube((61, 18), 2, ordre_projection=3, envs=[cases.Env(d, p, 1.4, vitesse_initiale=(.4, -.3, 0.))
+                                                             for d, p in ((1., 1.), (.5, .3), (.2, .1))]))
