@@ -556,6 +556,10 @@ void ens_lists_add(EnsGroup& g, MhHandle* h, int sl) {
     ens_list_add(g.rcmap, sl, seg_blocks(h, 0, MH_O3_L));
     for (int D = 1; D < g.dim; ++D) ens_list_add(g.tmap[D - 1], sl, seg_blocks(h, D, MH_O3_L));
   }
+  if (g.gen) {  // tiles of faces along each direction
+    ens_list_add(g.rcmap, sl, gen_blocks(h, 0));
+    for (int D = 1; D < g.dim; ++D) ens_list_add(g.tmap[D - 1], sl, gen_blocks(h, D));
+  }
   if (g.ntile) ens_list_add(g.ntmap, sl, node_tile_blocks(h));
   g.slots.push_back(sl);
   g.list_dirty = true;

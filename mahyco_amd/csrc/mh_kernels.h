@@ -1834,235 +1834,238 @@ __device__ __forceinline__ double pb_flux(int type, double y0, double yplus, dou
 // face carries the flux leaving the cell behind it minus the flux leaving the cell ahead,
 // each computed from that cell and its two neighbours, then adjusted by the debar fix
 // (UtilesRemap.cc:577-623, :782-826).  Boundary cells are their own missing neighbour.
+//
+// One thread per face: the fluxes of all 3m+1 slots through the back face of its cell, left in LDS,
+// then the update of its cell from its own face and the next one.  A flux leaves through a face
+// from one side only, so a face forms the slope and the flux of its upwind cell alone (of both
+// cells where the face velocity is not a number).  A block takes MH_BLOCK faces: 255 cells in
+// memory order for D = x, 32 x 7 cells of a plane for y and z.  Bound by the FP64 instructions and
+// the latency of one face's chain of slots, whose loads run one slot ahead; with a thread per cell,
+// four fluxes per slot and all slots in registers (354: one wavefront per SIMD) it took 76 / 74 us for
+// y / x on 420x180 cells and three environments, now 25 / 29.
+#define MH_GEN_TX 32  // y / z: cells along x of a block's tile
+#define MH_GEN_TY (MH_BLOCK / MH_GEN_TX)  // faces along D, one more than cells
 template <int DIM, int D, int M>
 __device__ __forceinline__ void k_sweep_cell_gen_body(const MhDev& S, int lb, int usel, int first) {
+  constexpr int NV = 3 * M + 1;
+  __shared__ double F[NV][MH_BLOCK];  // of the face behind the thread's cell, in the direction +D
+  __shared__ double Fv[M][MH_BLOCK];  // volume fluxes of the side being formed, for the debar fix
   const double* __restrict__ Uin = usel ? S.Ub : S.Ua;
   double* __restrict__ Uout = usel ? S.Ua : S.Ub;
-  constexpr int NV = 3 * M + 1;
-  const long c = lb * (long)blockDim.x + threadIdx.x;
-  if (c >= S.g.nc) return;
   if (mh_halted(S.sc)) return;
-  const bool own = !(first && S.mask[c] == 0);  // an empty cell's U starts from 0 (its Phi is stale)
-  const int nx = S.g.nx, ny = S.g.ny;
-  const int i = (int)(c % nx);
-  const long r = c / nx;
-  const int j = (int)(r % ny);
-  const int k = (int)(r / ny);
-  const int a = D == 0 ? i : D == 1 ? j : k;
-  const int na = D == 0 ? nx : D == 1 ? ny : S.g.nz;
-  const long sD = D == 0 ? 1 : D == 1 ? (long)nx : (long)nx * ny;
-  const long nD = D == 0 ? 1 : D == 1 ? (long)S.g.nnx : (long)S.g.nnx * S.g.nny;
-  const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
+  const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
+  const int na = D == 0 ? nx : D == 1 ? ny : nz;
   const long nc = S.g.nc;
-  const double dt = S.sc->dt;
+  const int tid = threadIdx.x;
+  // the thread's cell (i, j, k), and whether it has one (a face only: the last row of the tile)
+  int i, j, k;
+  bool face, cell;
+  constexpr int next = D == 0 ? 1 : MH_GEN_TX;  // thread of the face ahead
+  if (D == 0) {
+    const long c = (long)lb * (MH_BLOCK - 1) + tid;
+    face = c < nc;
+    cell = face && tid < MH_BLOCK - 1;
+    i = (int)(c % nx);
+    const long r = c / nx;
+    j = (int)(r % ny);
+    k = (int)(r / ny);
+  } else {
+    const int tilesx = (nx + MH_GEN_TX - 1) / MH_GEN_TX, tilesd = (na + MH_GEN_TY - 2) / (MH_GEN_TY - 1);
+    i = lb % tilesx * MH_GEN_TX + tid % MH_GEN_TX;
+    const int r = lb / tilesx;
+    const int ad = r % tilesd * (MH_GEN_TY - 1) + tid / MH_GEN_TX, t = r / tilesd;
+    j = D == 1 ? ad : t;
+    k = D == 1 ? t : ad;
+    face = i < nx && ad < na && t < (D == 1 ? nz : ny);
+    cell = face && tid / MH_GEN_TX < MH_GEN_TY - 1;
+  }
+  const int a = D == 0 ? i : D == 1 ? j : k;
+  const long c = i + (long)nx * (j + (long)ny * k);
+  const long sD = D == 0 ? 1 : D == 1 ? (long)nx : (long)nx * ny;
   const bool pb = S.pb != 0;
   const double thr = S.thr_remap;
-  const int sp = S.simple_pente;
-  // stencil offsets -2..2 (index o + 2), clamped to the mesh
-  long cs[5];
-  bool valid[5];
-  double den[5], xc[5], hs[5];
+  if (face && a > 0) {
+    const long nD = D == 0 ? 1 : D == 1 ? (long)S.g.nnx : (long)S.g.nnx * S.g.nny;
+    const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
+    const double dt = S.sc->dt;
+    const int sp = S.simple_pente;
+    const bool order2 = S.order2 != 0;
+    const int debar = S.debar;
+    // cells at offsets -2 .. 1 (index o + 2), clamped to the mesh: the two beside the face and one
+    // more on each side
+    long cs[4];
+    bool valid[4];
+    double den[4], xc[4], hs[4];
 #pragma unroll
-  for (int o = 0; o < 5; ++o) {
-    const int bb = a + o - 2;
-    valid[o] = bb >= 0 && bb < na;
-    const int ao = min(max(bb, 0), na - 1);
-    cs[o] = c + (ao - a) * sD;
-    hs[o] = S.hc[D * nc + cs[o]];
-    xc[o] = valid[o] ? cell_centre_d<DIM, D>(S, b + (o - 2) * nD) : 0.;
-    if (first && !pb) {
-      den[o] = S.mask[cs[o]] ? S.Vl[cs[o]] : 1.;  // an empty cell holds Phi itself
-    } else {
-      double sv = 0.;
-      if (!first)
-        for (int kk = 0; kk < M; ++kk) sv += Uin[kk * nc + cs[o]];
-      den[o] = sv;
-    }
-  }
-  double dxf[4];
-#pragma unroll
-  for (int f = 0; f < 4; ++f) dxf[f] = (valid[f] && valid[f + 1]) ? xc[f + 1] - xc[f] : 0.;
-  // the two faces of the cell along D: s = 0 back (outer normal -e_D), s = 1 front (+e_D)
-  bool inner[2], upprev[2];
-  double area[2], vf[2], hup[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    inner[s] = s == 0 ? (a > 0) : (a < na - 1);
-    area[s] = 0.;
-    vf[s] = 0.;
-    hup[s] = 0.;
-    upprev[s] = false;
-    if (!inner[s]) continue;
-    double xf;
-    face_quant<DIM, D>(S, b + s * nD, area[s], xf, vf[s]);
-    upprev[s] = vf[s] * dxf[s + 1] > 0.0;
-    hup[s] = (double)S.order2 * (xf - (upprev[s] ? xc[s + 1] : xc[s + 2]));
-  }
-  // pure neighbourhoods of the cells at offsets -1, 0, +1 (index x = 1, 2, 3)
-  bool vpure[5] = {false, false, false, false, false};
-  if (S.pb_mixte) {
-    int code[5];
-#pragma unroll
-    for (int o = 0; o < 5; ++o) {
-      if (first) {
-        code[o] = S.est[cs[o]];
+    for (int o = 0; o < 4; ++o) {
+      const int bb = a + o - 2;
+      valid[o] = bb >= 0 && bb < na;
+      const int ao = min(max(bb, 0), na - 1);
+      cs[o] = c + (ao - a) * sD;
+      hs[o] = S.hc[D * nc + cs[o]];
+      xc[o] = valid[o] ? cell_centre_d<DIM, D>(S, b + (o - 2) * nD) : 0.;
+      if (first && !pb) {
+        den[o] = S.mask[cs[o]] ? S.Vl[cs[o]] : 1.;  // an empty cell holds Phi itself
       } else {
-        int cnt = 0, pu = -1;
-        for (int kk = 0; kk < M; ++kk)
-          if (Uin[kk * nc + cs[o]] / den[o] > 0.) {
-            cnt++;
-            pu = kk;
-          }
-        code[o] = cnt > 1 ? MH_EST_MIXED : pu;
+        double sv = 0.;
+        if (!first)
+          for (int kk = 0; kk < M; ++kk) sv += Uin[kk * nc + cs[o]];
+        den[o] = sv;
       }
     }
+    double area, xf, vf;
+    face_quant<DIM, D>(S, b, area, xf, vf);
+    // pure neighbourhoods of the cells behind and ahead of the face
+    bool vpure[2] = {false, false};
+    if (S.pb_mixte) {
+      int code[4];
 #pragma unroll
-    for (int x = 1; x <= 3; ++x)
-      vpure[x] = code[x] != MH_EST_MIXED && code[x - 1] != MH_EST_MIXED && code[x + 1] != MH_EST_MIXED &&
-                 code[x] == code[x + 1] && code[x] == code[x - 1];
-  }
-  int lim[5], limY[5];
-#pragma unroll
-  for (int x = 0; x < 5; ++x) {
-    lim[x] = (S.lim_pure == 1 && vpure[x]) ? S.lim_pure : S.limiter;
-    limY[x] = vpure[x] ? S.lim_pure : S.limiter;
-  }
-  // pente-borne combinations q: (cell -1, front), (cell 0, back), (cell 0, front), (cell +1, back)
-  const int qx[4] = {1, 2, 2, 3}, qt[4] = {1, 0, 1, 0};
-  double ppv[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int s = q < 2 ? 0 : 1;
-    const double vout = qt[q] == 1 ? vf[s] : -vf[s];
-    ppv[q] = 0.5 * (vout + fabs(vout)) * dt;
-  }
-  const bool order2 = S.order2 != 0;
-  // phi and limited slopes of variable v at the five stencil cells
-  auto load_phi = [&](int v, double* phi) {
-#pragma unroll
-    for (int o = 0; o < 5; ++o) {
-      const long cc = cs[o];
-      double p;
-      if (!pb) {
-        p = Uin[v * nc + cc] / den[o];
-      } else if (first || v == 3 * M) {
-        p = S.phi0[v * nc + cc];
-      } else if (v < M) {
-        p = Uin[v * nc + cc] / den[o];
-      } else {
-        const double d = Uin[(v - M) * nc + cc];
-        p = d != 0. ? Uin[v * nc + cc] / d : 0.;
-      }
-      phi[o] = p;
-    }
-  };
-  auto slopes = [&](const double* phi, double* gr) {
-    double gface[4];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) gface[f] = (valid[f] && valid[f + 1]) ? (phi[f + 1] - phi[f]) / dxf[f] : 0.;
-#pragma unroll
-    for (int x = 1; x <= 3; ++x)
-      gr[x] = order2 ? limited_grad(lim[x], gface[x - 1], gface[x], phi[x + 1], phi[x - 1], hs[x], hs[x + 1], hs[x - 1], sp)
-                     : 0.;
-  };
-  auto pb_raw = [&](const double* phi, const double* gr, int q) {
-    const int x = qx[q];
-    return pb_flux(qt[q], phi[x], phi[x + 1], phi[x - 1], hs[x], hs[x + 1], hs[x - 1], gr[x], ppv[q], limY[x], thr, sp);
-  };
-  // pente-borne volume fluxes first: the debar fix and the zero tests need their sums
-  double Fv[4][M], Fm[4][M], sfv[4] = {0., 0., 0., 0.};
-  bool zero[4] = {true, true, true, true};
-  if (pb && order2) {
-    for (int v = 0; v < M; ++v) {
-      double phi[5], gr[5];
-      load_phi(v, phi);
-      slopes(phi, gr);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        Fv[q][v] = inner[q < 2 ? 0 : 1] ? pb_raw(phi, gr, q) : 0.;
-        sfv[q] += Fv[q][v];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) zero[q] = ppv[q] == 0. || (S.debar == 1 && !(fabs(sfv[q]) > thr));
-  }
-  const int s0 = (DIM == 2 && D == 0) ? 1 : 0, s1 = 1 - s0;
-  const double od[2] = {-1., 1.};
-  double un[NV];
-  for (int v = 0; v < NV; ++v) {
-    double phi[5], gr[5];
-    double face[2] = {0., 0.};
-    if (pb) {
-      double F[4] = {0., 0., 0., 0.};
-      if (order2) {
-        if (v >= M) {
-          load_phi(v, phi);
-          slopes(phi, gr);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          if (!inner[q < 2 ? 0 : 1] || zero[q]) continue;
-          const int x = qx[q];
-          if (v < M) {
-            F[q] = Fv[q][v];
-          } else if (v < 2 * M) {
-            const int e = v - M;
-            double f = pb_raw(phi, gr, q);
-            if (!vpure[x]) {
-              if (S.debar == 1) f = (f / sfv[q]) * Fv[q][e];
-              else if (S.debar == 2) f = phi[x] * Fv[q][e];
+      for (int o = 0; o < 4; ++o) {
+        if (first) {
+          code[o] = S.est[cs[o]];
+        } else {
+          int cnt = 0, pu = -1;
+          for (int kk = 0; kk < M; ++kk)
+            if (Uin[kk * nc + cs[o]] / den[o] > 0.) {
+              cnt++;
+              pu = kk;
             }
-            F[q] = Fm[q][e] = f;
-          } else if (v < 3 * M) {
-            const int e = v - 2 * M;
-            double f = pb_raw(phi, gr, q);
-            if (S.debar == 1) f = (f / sfv[q]) * Fm[q][e];
-            else if (S.debar == 2) f = phi[x] * Fm[q][e];
-            F[q] = f;
+          code[o] = cnt > 1 ? MH_EST_MIXED : pu;
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+        vpure[x] = code[x + 1] != MH_EST_MIXED && code[x] != MH_EST_MIXED && code[x + 2] != MH_EST_MIXED &&
+                   code[x + 1] == code[x + 2] && code[x + 1] == code[x];
+    }
+    // slots in the order volumes, then mass and energy of each environment, then V q: the debar
+    // fix and the zero test need the sum of the volume fluxes
+    auto slot_of = [](int t) {
+      if (t < M) return t;
+      if (t == 3 * M) return 3 * M;
+      const int e = (t - M) >> 1;
+      return ((t - M) & 1) ? 2 * M + e : M + e;
+    };
+    const double ppA = 0.5 * (vf + fabs(vf)) * dt, ppB = 0.5 * (-vf + fabs(-vf)) * dt;  // leaving the cell behind, ahead
+    int side = pb ? (ppA != 0. ? 0 : 1) : (vf * (xc[2] - xc[1]) > 0.0 ? 0 : 1);  // 0: upwind cell behind the face
+    for (int v = 0; v < NV; ++v) F[v][tid] = 0.;
+    for (;;) {
+      const double pp = side ? ppB : ppA;
+      if ((!pb || order2) && !(pb && pp == 0.)) {
+        const bool sd = side != 0;
+        const long cc[3] = {sd ? cs[1] : cs[0], sd ? cs[2] : cs[1], sd ? cs[3] : cs[2]};
+        const double dn[3] = {sd ? den[1] : den[0], sd ? den[2] : den[1], sd ? den[3] : den[2]};
+        const double hm = sd ? hs[1] : hs[0], h0 = sd ? hs[2] : hs[1], hp = sd ? hs[3] : hs[2];
+        const double xm = sd ? xc[1] : xc[0], x0 = sd ? xc[2] : xc[1], xp = sd ? xc[3] : xc[2];
+        const bool okb = sd ? valid[1] : valid[0], okf = sd ? valid[3] : valid[2];  // the upwind cell exists
+        const bool vp = sd ? vpure[1] : vpure[0];
+        const int lim = (S.lim_pure == 1 && vp) ? S.lim_pure : S.limiter;
+        const int limY = vp ? S.lim_pure : S.limiter;
+        const double hup = (double)S.order2 * (xf - x0);
+        const double dxb = okb ? x0 - xm : 0., dxf = okf ? xp - x0 : 0.;
+        // phi of a slot: numerators and denominators, loaded one slot ahead
+        auto fetch = [&](int v, double* n, double* d) {
+          const bool ratio = pb && !first && v >= M && v < 3 * M;
+          const double* src = pb && (first || v == 3 * M) ? S.phi0 : Uin;
+#pragma unroll
+          for (int o = 0; o < 3; ++o) {
+            n[o] = src[v * nc + cc[o]];
+            if (ratio) d[o] = Uin[(v - M) * nc + cc[o]];
+          }
+        };
+        double n1[3], d1[3] = {1., 1., 1.};
+        fetch(slot_of(0), n1, d1);
+        double sfv = 0., Fm = 0.;
+#pragma unroll 1
+        for (int t = 0; t < NV; ++t) {
+          const int v = slot_of(t);
+          double y[3];
+          if (pb && (first || v == 3 * M)) {
+#pragma unroll
+            for (int o = 0; o < 3; ++o) y[o] = n1[o];
+          } else if (!pb || v < M) {
+#pragma unroll
+            for (int o = 0; o < 3; ++o) y[o] = n1[o] / dn[o];
           } else {
-            F[q] = pb_raw(phi, gr, q);
+#pragma unroll
+            for (int o = 0; o < 3; ++o) y[o] = d1[o] != 0. ? n1[o] / d1[o] : 0.;
+          }
+          if (t + 1 < NV) fetch(slot_of(t + 1), n1, d1);
+          double g = 0.;
+          if (order2) {
+            const double gb = okb ? (y[1] - y[0]) / dxb : 0.;
+            const double gf = okf ? (y[2] - y[1]) / dxf : 0.;
+            g = limited_grad(lim, gb, gf, y[2], y[0], h0, hp, hm, sp);
+          }
+          double f;
+          if (!pb) {
+            f = y[1] + hup * g;
+          } else {
+            f = pb_flux(side == 0 ? 1 : 0, y[1], y[2], y[0], h0, hp, hm, g, pp, limY, thr, sp);
+            if (v >= M && v < 3 * M) {
+              const bool energy = v >= 2 * M;
+              const double Fr = energy ? Fm : Fv[v - M][tid];  // the volume or the mass flux
+              if (energy || !vp) {
+                if (debar == 1) f = (f / sfv) * Fr;
+                else if (debar == 2) f = y[1] * Fr;
+              }
+              if (!energy) Fm = f;
+            }
+          }
+          auto add = [&](int q, double x) { F[q][tid] = pb && side ? F[q][tid] - x : x; };
+          if (t >= M) {
+            add(v, f);
+          } else {
+            sfv += f;
+            Fv[v][tid] = f;
+            if (t == M - 1) {
+              if (pb && debar == 1 && !(fabs(sfv) > thr)) break;  // nothing leaves from this side
+              for (int q = 0; q < M; ++q) add(q, Fv[q][tid]);
+            }
           }
         }
       }
-      face[0] = F[0] - F[1];
-      face[1] = F[2] - F[3];
+      if (!(pb && side == 0 && ppB != 0.)) break;
+      side = 1;
+    }
+    const double w = pb ? area : vf * area * dt;
+    for (int v = 0; v < NV; ++v) F[v][tid] = w * F[v][tid];
+  }
+  __syncthreads();
+  if (!cell) return;
+  const bool inb = a > 0, inf = a < na - 1;
+  const bool own = !(first && S.mask[c] == 0);  // an empty cell's U starts from 0 (its Phi is stale)
+  auto update = [&](int v, bool mass) {
+    const double Fb = inb ? -F[v][tid] : 0., Ff = inf ? F[v][tid + next] : 0.;
+    double ff = 0., dd = 0.;
+    if (DIM == 2 && D == 0) {  // cell faces in Arcane order: 2D x has the max face first
+      if (inf) ff += Ff;
+      if (inb) ff += Fb;
+      if (inf) dd += 0.5 * Ff * 1.;
+      if (inb) dd += 0.5 * Fb * -1.;
     } else {
-      load_phi(v, phi);
-      slopes(phi, gr);
+      if (inb) ff += Fb;
+      if (inf) ff += Ff;
+      if (inb) dd += 0.5 * Fb * -1.;
+      if (inf) dd += 0.5 * Ff * 1.;
+    }
+    if (mass) S.dflux[(v - M) * nc + c] = dd;
+    return (own ? Uin[v * nc + c] : 0.) - ff;
+  };
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int up = upprev[s] ? s + 1 : s + 2;
-        face[s] = phi[up] + hup[s] * gr[up];
-      }
+  for (int e = 0; e < M; ++e) {
+    double un[3] = {update(e, false), update(M + e, true), update(2 * M + e, false)};
+    if (pb && !S.sans_lagrange) {  // with the dual phase, tiny partial volumes, masses or energies drop the environment (:441-463)
+      if (un[0] < 1. * thr) un[0] = un[1] = un[2] = 0.;
+      if (un[1] < 1. * thr) un[0] = un[1] = un[2] = 0.;
+      if (un[2] < 1. * thr) un[0] = un[1] = un[2] = 0.;
     }
-    double flux[2] = {0., 0.};
+    if (un[1] < 0.) un[1] = 0.;  // computeUremap clamps, :465-485
+    if (un[2] < 0.) un[2] = 0.;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if (!inner[s]) continue;
-      flux[s] = pb ? od[s] * area[s] * face[s] : od[s] * vf[s] * area[s] * dt * face[s];
-    }
-    double ff = 0.;
-    if (inner[s0]) ff += flux[s0];
-    if (inner[s1]) ff += flux[s1];
-    un[v] = (own ? Uin[v * nc + c] : 0.) - ff;
-    if (v >= M && v < 2 * M) {
-      double dd = 0.;
-      if (inner[s0]) dd += 0.5 * flux[s0] * od[s0];
-      if (inner[s1]) dd += 0.5 * flux[s1] * od[s1];
-      S.dflux[(v - M) * nc + c] = dd;
-    }
+    for (int q = 0; q < 3; ++q) Uout[(q * M + e) * nc + c] = un[q];
   }
-  if (pb && !S.sans_lagrange)  // with the dual phase, tiny partial volumes, masses or energies drop the environment (:441-463)
-    for (int kk = 0; kk < M; ++kk) {
-      if (un[kk] < 1. * thr) un[kk] = un[M + kk] = un[2 * M + kk] = 0.;
-      if (un[M + kk] < 1. * thr) un[kk] = un[M + kk] = un[2 * M + kk] = 0.;
-      if (un[2 * M + kk] < 1. * thr) un[kk] = un[M + kk] = un[2 * M + kk] = 0.;
-    }
-  for (int v = 0; v < NV; ++v) {
-    double w = un[v];
-    if (v >= M && v < 3 * M && w < 0.) w = 0.;  // computeUremap clamps, :465-485
-    Uout[v * nc + c] = w;
-  }
+  Uout[3 * M * nc + c] = update(3 * M, false);
 }
 
 // The x sweep with one wavefront per row segment: lane l holds cell i = 60 s - 2 + l of a

@@ -59,9 +59,9 @@ void launch_cell_part(MhHandle* h, int D, int sel, int first, bool gen, bool o3)
   const MhDev& S = h->dev;
   const bool flat = h->sweep_mode == MH_SWEEP_FLAT;
   if (gen) {
-    if (D == 0) LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell_gen<DIM, 0, M>), h->nblk_c, MH_BLOCK, S, sel, first);
-    else if (D == 1) LAUNCH(h, KN_SWEEP_CELL + 1, (k_sweep_cell_gen<DIM, 1, M>), h->nblk_c, MH_BLOCK, S, sel, first);
-    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_CELL + 2, (k_sweep_cell_gen<3, 2, M>), h->nblk_c, MH_BLOCK, S, sel, first);
+    if (D == 0) LAUNCH(h, KN_SWEEP_CELL + 0, (k_sweep_cell_gen<DIM, 0, M>), gen_blocks(h, 0), MH_BLOCK, S, sel, first);
+    else if (D == 1) LAUNCH(h, KN_SWEEP_CELL + 1, (k_sweep_cell_gen<DIM, 1, M>), gen_blocks(h, 1), MH_BLOCK, S, sel, first);
+    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_CELL + 2, (k_sweep_cell_gen<3, 2, M>), gen_blocks(h, 2), MH_BLOCK, S, sel, first);
   } else if (o3) {
     if (D == 0) launch_cell3<DIM, 0, M>(h, sel, first);
     else if (D == 1) launch_cell3<DIM, 1, M>(h, sel, first);
@@ -153,15 +153,14 @@ template <int DIM, int D, int M, int LIM>
 void ens_sweep(const EnsGroup& g, const MhDev* tab, hipStream_t st, dim3 G, int sel, int prev, int last) {
   const int first = prev == 0;
   const dim3 B(MH_BLOCK);
-  if constexpr (LIM < 0) {  // order 3 or pente-borne / generalised limiters: one thread per item
+  if constexpr (LIM < 0) {  // order 3 or pente-borne / generalised limiters
+    const EnsList& dir = D == 0 ? g.rcmap : g.tmap[D == 0 ? 0 : D - 1];
     if (g.gen) {
-      hipLaunchKernelGGL((k_sweep_cell_gen_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(g.cmap), sel, first);
+      hipLaunchKernelGGL((k_sweep_cell_gen_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(dir), sel, first);
       if (!g.adv)
         hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, MH_LIM_ANY>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     } else {
-      hipLaunchKernelGGL((k_sweep_cell3_batch<DIM, D, M>), G, B, 0, st, tab,
-                         D == 0 ? g.rcmap.d : g.tmap[D == 0 ? 0 : D - 1].d,
-                         D == 0 ? g.rcmap.d_n : g.tmap[D == 0 ? 0 : D - 1].d_n, sel, first);
+      hipLaunchKernelGGL((k_sweep_cell3_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(dir), sel, first);
       if (!g.adv)
         hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, -1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     }

@@ -79,3 +79,17 @@ def test_order3_segments(n, seed):
 def test_order3_three_materials():
     check(moving_tube((61, 18), 2, ordre_projection=3, envs=[cases.Env(d, p, 1.4, vitesse_initiale=(.4, -.3, 0.))
                                                              for d, p in ((1., 1.), (.5, .3), (.2, .1))]))
+
+
+@pytest.mark.parametrize("debar", [0, 1, 2])
+@pytest.mark.parametrize("n", [(3, 17, 4), (1, 7, 4), (61, 18), (2, 2)], ids=lambda n: "x".join(map(str, n)))
+def test_pente_borne_groups(n, debar):
+    """Pente-borne fluxes with each debar fix: every group of environments on its own."""
+    check(moving_tube(n, debar, pente_borne=True, debar_fix=debar, pente_borne_mixte=debar != 2,
+                      limiter=T.MH_SUPERBEE_G if debar else T.MH_MINMOD, simple_pente=debar == 1,
+                      limiter_pure=T.MH_VANLEER_G))
+
+
+@pytest.mark.parametrize("limiter", [T.MH_MINMOD_G, T.MH_VANLEER_G, T.MH_ARITHMETIC_G, T.MH_ULTRABEE_G])
+def test_generalised_limiters(limiter):
+    check(moving_tube((9, 5, 4), 1, limiter=limiter))
