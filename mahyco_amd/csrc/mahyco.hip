@@ -957,6 +957,12 @@ static int create_case(const MhMesh* mesh, const MhEnvironment* envs, int nb_env
   S.Ud = h->Ud;
   S.Pa = h->Pa;
   S.Pb = h->Pb;
+  // the presence bytes of the two U buffers lie behind the dual masses in Pb (3 nn words, of which
+  // the masses take nn); large single meshes and ensembles of two environments or more keep them
+  if (presence_bytes(h)) {
+    S.pm[0] = (uint8_t*)(h->Pb + nn);
+    S.pm[1] = S.pm[0] + nc;
+  }
   S.nblk_c = h->nblk_c;
   S.nt_kc = h->nt_kc;
   S.ct_k = h->ct_k;
@@ -1040,6 +1046,7 @@ static int create_case(const MhMesh* mesh, const MhEnvironment* envs, int nb_env
     S.rev_cos = h->rev_cos;
     S.rev_n = (long)I.rev_cos.size();
   }
+  if (S.pm[0]) fill(S.pm[0], 2 * nc, (uint8_t)0xff);  // the buffers hold no zeros yet
   if (S.phi0) fill(S.phi0, (long)S.nv * nc, 0.);  // pente-borne phi: Arcane starts m_phi_lagrange at 0
   // the scalars may sit in an ensemble's array, which the iterations' stream writes: set them in
   // that stream's order (a kernel argument, no host buffer)
@@ -2001,6 +2008,12 @@ int mahyco_checkpoint_read(MhHandle* h, const char* path) {
   HIPCHK(hipStreamSynchronize(h->stream));
   for (size_t i = 0; i < h->allocs.size(); ++i)
     HIPCHK(hipMemcpy(h->allocs[i], data[i].data(), data[i].size(), hipMemcpyHostToDevice));
+  // another program's file may hold other data in place of the presence bytes
+  if (h->dev.pm[0]) {
+    hipLaunchKernelGGL(k_fill_value<uint8_t>, dim3(fill_blocks(2 * h->g.nc)), dim3(MH_BLOCK), 0, h->stream,
+                       h->dev.pm[0], 2 * h->g.nc, (uint8_t)0xff);
+    HIPCHK(hipGetLastError());
+  }
   h->launched = hd.launched;
   h->sens = hd.sens;
   h->dev.max_iter = hd.max_iter;

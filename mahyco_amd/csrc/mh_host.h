@@ -172,6 +172,13 @@ inline int node_march_blocks(MhHandle* h, int D) {
 // the y / z variants a single mesh takes (an ensemble's launches are filled by its many cases)
 inline bool seg_sweep(const MhHandle* h) { return !h->sweep_large && h->g.nc < MH_SEG_CELLS; }
 inline bool march_sweep(const MhHandle* h) { return h->sweep_large || h->g.nn >= MH_MARCH_NODES; }
+// whether the case keeps presence bytes (MhDev::pm): its sweeps are the row and tile ones.  Small
+// meshes are bound by latency, and their segment sweeps do not use them.
+inline bool presence_bytes(const MhHandle* h) {
+  const MhDev& S = h->dev;
+  return h->m > 1 && h->opt.with_projection && S.order2 != 2 && !S.pb && !(S.order2 && S.limiter >= MH_MINMOD_G) &&
+         (h->ext_sc || !seg_sweep(h));
+}
 // blocks of the sweeps over segments (one thread per len cells of a line along D), a multiple of 8
 inline int seg_blocks(MhHandle* h, int D, int len) {
   const long na = D == 0 ? h->g.nx : D == 1 ? h->g.ny : h->g.nz;

@@ -33,6 +33,19 @@ __device__ __forceinline__ bool mh_halted(const MhScalars* sc) { return sc->stat
 // so each XCD sweeps one contiguous slab and the neighbours of a stencil stay in its L2.
 __device__ __forceinline__ int xcd_block(int b, int nb) { return (b & 7) * (nb >> 3) + (b >> 3); }
 
+// The value of the lane behind / ahead (a shift of the whole wavefront by one lane; the lane at the
+// end gets 0): a register move, where a shuffle goes through LDS.
+__device__ __forceinline__ double lane_back(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x138, 0xf, 0xf, true);  // wave_shr:1
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x138, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane_front(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x130, 0xf, 0xf, true);  // wave_shl:1
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x130, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
 // Arcane math::min / math::max
 __device__ __forceinline__ double amin(double a, double b) { return (a < b) ? a : b; }
 __device__ __forceinline__ double amax(double a, double b) { return (a < b) ? b : a; }
@@ -668,6 +681,15 @@ __device__ __forceinline__ double char_length_alt(int lc, const D3* x) {
   return fabs(x[2].z - x[0].z);
 }
 
+// Which environments a cell's remap vector holds anything of.  Most cells of a multi-material mesh
+// hold one material, and the volume, mass and energy slots of the others are zeros that every sweep
+// would read, divide, limit and write.  Beside each U buffer one byte per cell (MhDev::pm, null for
+// meshes whose sweeps do not use it) keeps the invariant: bit k clear => the buffer's three slots of
+// environment k are 0 in that cell.  The buffers always hold those zeros, so code that ignores the
+// bytes reads the same values; a writer stores a zero only where the bit was set.
+__device__ __forceinline__ bool mh_finite_nonzero(double x) { return __builtin_amdgcn_class(x, 0x198); }
+__device__ __forceinline__ bool mh_finite(double x) { return __builtin_amdgcn_class(x, 0x1f8); }
+
 // A cell that no environment occupies gets no remap values from computeVariablesForRemap
 // (PrepareRemap.cc:100-166 loop over environment cells): its U is 0 and its Phi is the one
 // the last sweep of the previous remap left, U / sum V_k (RemapADIService.cc:493-538).
@@ -680,6 +702,25 @@ __device__ __forceinline__ void empty_cell_phi(const MhDev& S, long c, double* u
   double sv = 0.;
   for (int kk = 0; kk < M; ++kk) sv += Ulast[kk * nc + c];
   for (int v = 0; v <= 3 * M; ++v) u_out[v] = Ulast[v * nc + c] / sv;
+}
+
+// The remap vector of cell c (environments mk) to the first buffer.
+template <int M>
+__device__ __forceinline__ void store_remap_vector(const MhDev& S, long c, unsigned mk, const double* u) {
+  double* __restrict__ U = S.Ua;
+  const long nc = S.g.nc;
+  if (M > 1 && S.pm[0]) {
+    const unsigned held = mk ? mk : (1u << M) - 1u;  // an empty cell holds a phi of every slot
+    const unsigned old = S.pm[0][c];
+#pragma unroll
+    for (int v = 0; v < 3 * M; ++v)
+      if (((held | old) >> (v % M)) & 1u) U[v * nc + c] = u[v];
+    U[3 * M * nc + c] = u[3 * M];
+    S.pm[0][c] = (uint8_t)held;
+  } else {
+#pragma unroll
+    for (int v = 0; v <= 3 * M; ++v) U[v * nc + c] = u[v];
+  }
 }
 
 // ComputeGeometricValues (:1097-1253) + UpdateDensity (:1267-1316) +
@@ -712,7 +753,6 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
   // Lagrange-only branch (state and EOS written back) and k_prepare_remap forms U later.
   const bool with_proj = REMAP ? true : (S.with_proj != 0 && !S.staged);
   const bool sans_lagrange = REMAP ? false : (S.sans_lagrange != 0);
-  double* __restrict__ U = S.Ua;
   constexpr int NV = 3 * M + 1;
   double dxs = 1.79769313486231570815e+308;
   {
@@ -773,7 +813,7 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
       u_out[3 * M] = V * S.q[c];
       if (S.pb && mk) S.phi0[3 * M * nc + c] = S.q[c];
       if (!mk && !S.pb && S.nsweep > 0) empty_cell_phi<M>(S, c, u_out);
-      for (int v = 0; v < NV; ++v) U[v * nc + c] = u_out[v];
+      store_remap_vector<M>(S, c, mk, u_out);
       S.Vl[c] = V;
       S.L[c] = L;
       return dxs;
@@ -907,8 +947,7 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
       }
     }
     if (with_proj && !mk && !S.pb && S.nsweep > 0) empty_cell_phi<M>(S, c, u_out);
-    if (with_proj)
-      for (int v = 0; v < NV; ++v) U[v * nc + c] = u_out[v];
+    if (with_proj) store_remap_vector<M>(S, c, mk, u_out);
     S.Vl[c] = V;
     S.L[c] = L;
   }
@@ -989,7 +1028,7 @@ __device__ __forceinline__ void k_prepare_remap_body(const MhDev& S, int lb) {
   }
   u_out[3 * M] = V * q;
   if (!mk && !S.pb && S.nsweep > 0) empty_cell_phi<M>(S, c, u_out);
-  for (int v = 0; v < NV; ++v) S.Ua[v * nc + c] = u_out[v];
+  store_remap_vector<M>(S, c, mk, u_out);
 }
 
 // 3D cell kernel of the remap loop with the node neighbourhood staged in LDS: a block owns
@@ -1322,6 +1361,7 @@ __device__ __forceinline__ void k_sweep_cell_body(const MhDev& S, int lb, int us
     if (v >= M && v < 3 * M && un < 0.) un = 0.;  // computeUremap clamps, :465-485
     Uout[v * nc + c] = un;
   }
+  if (S.pm[0]) S.pm[usel ? 0 : 1][c] = 0xff;
 }
 
 // Segments of `len` cells of a line of na cells.
@@ -2092,13 +2132,13 @@ __device__ __forceinline__ void row_jk(const MhGrid& g, long r, int& j, int& k) 
 template <int DIM, int M, int LIM>
 __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, int usel, int first, int v0 = 0,
                                                       int v1 = 3 * M + 1) {  // slots v0 .. v1-1
+  constexpr int NV = 3 * M + 1;
   const int nx = S.g.nx;
   const long rows = (long)S.g.ny * S.g.nz;
   const int wpr = (nx + MH_ROW_OUT - 1) / MH_ROW_OUT;
   const int lane = threadIdx.x & 63;
   const long gw = (long)lb * (MH_BLOCK / 64) + (threadIdx.x >> 6);
   if (gw >= rows * wpr) return;  // whole wavefront
-  if (mh_halted(S.sc)) return;
   const double* __restrict__ Uin = usel ? S.Ub : S.Ua;
   double* __restrict__ Uout = usel ? S.Ua : S.Ub;
   double* __restrict__ dflux = S.dflux;
@@ -2109,51 +2149,89 @@ __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, in
   const bool valid = i >= 0 && i < nx;
   const bool validp = i - 1 >= 0 && i - 1 < nx;
   const bool out = valid && lane >= 2 && lane < 2 + MH_ROW_OUT;
+  const bool inb = valid && i > 0;       // back face (node column i): inner when 0 < i < nx
+  const bool inf = valid && i < nx - 1;
   const long nc = S.g.nc;
   const long c = row * nx + i;
-  const bool own = !(first && valid && S.mask[c] == 0);  // an empty cell's U starts from 0
   const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
+  const bool sparse = M > 1 && S.pm[0] != nullptr;
+  unsigned slots = ((1u << v1) - 1u) & ~((1u << v0) - 1u);  // the slots to run
+  // every load that depends on the kernel arguments alone goes out before anything waits (the stop
+  // flag included): a wavefront's time here is that of its load rounds
+  const unsigned here = sparse && valid ? S.pm[usel ? 1 : 0][c] : 0u;
+  const unsigned old = sparse && out ? S.pm[usel ? 0 : 1][c] : ~0u;
+  const uint8_t mk = first && valid ? S.mask[c] : (uint8_t)1;
+  double den = first && valid ? S.Vl[c] : 1.;
+  double u[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const bool now = !sparse || v == 3 * M || (v < M && !first);
+    u[v] = now && valid && (((slots >> v) & 1u) || (v < M && !first)) ? Uin[v * nc + c] : 0.;
+  }
   const double dt = S.sc->dt;
-  double unext = valid ? Uin[v0 * nc + c] : 0.;  // slot loads run one slot ahead
-  double den = 1., xc = 0.;
+  const bool halted = mh_halted(S.sc);
+  double xc = 0., area = 0., xf = 0., vf = 0.;
+  if (valid) xc = cell_centre_d<DIM, 0>(S, b);
+  if (inb) face_quant<DIM, 0>(S, b, area, xf, vf);
+  if (halted) return;
+  const bool own = mk != 0;  // an empty cell's U starts from 0
   if (valid) {
     if (first) {
-      den = S.mask[c] ? S.Vl[c] : 1.;  // an empty cell holds Phi itself
+      if (!own) den = 1.;  // an empty cell holds Phi itself
     } else {
       double sv = 0.;
-      for (int kk = 0; kk < M; ++kk) sv += Uin[kk * nc + c];
+#pragma unroll
+      for (int kk = 0; kk < M; ++kk) sv += u[kk];
       den = sv;
     }
-    xc = cell_centre_d<DIM, 0>(S, b);
   }
-  const double xcp = __shfl_up(xc, 1);
+  const double xcp = lane_back(xc);
   const double dxb = (valid && validp) ? xc - xcp : 0.;
-  // back face (node column i): inner when 0 < i < nx
-  const bool inb = valid && i > 0;
-  const bool inf = valid && i < nx - 1;
-  double area = 0., xf = 0., vf = 0.;
-  if (inb) face_quant<DIM, 0>(S, b, area, xf, vf);
   const bool upprev = vf * dxb > 0.0;
   const double hb = (double)S.order2 * (xf - (upprev ? xcp : xc));
-  for (int v = v0; v < v1; ++v) {
-    const double uv = unext;
-    if (v + 1 < v1) unext = valid ? Uin[(v + 1) * nc + c] : 0.;
-    const double phi = valid ? uv / den : 0.;
-    const double phip = __shfl_up(phi, 1);
+  const double w = 1. * vf * area * dt;
+  // with presence bytes the slots to run are those of the environments some cell of the wavefront
+  // holds, and V q.  Where no cell of a stencil holds an environment its slots stay 0, unless a
+  // factor is zero, infinite or not a number, and then they all run.
+  unsigned held = 0;
+  if (sparse) {
+    const bool irregular = valid && (!mh_finite_nonzero(den) || (validp && lane > 0 && !mh_finite_nonzero(dxb)) ||
+                                     (inb && (!mh_finite(w) || !mh_finite(hb))));
+    const unsigned in = irregular ? (1u << M) - 1u : here;
+#pragma unroll
+    for (int e = 0; e < M; ++e)
+      if (__ballot((in >> e) & 1u) == 0) slots &= ~((1u << e) | (1u << (M + e)) | (1u << (2 * M + e)));
+#pragma unroll
+    for (int v = 0; v < 3 * M; ++v)
+      if (((slots >> v) & 1u) && (v >= M || first)) u[v] = valid ? Uin[v * nc + c] : 0.;
+    if (out) {
+#pragma unroll
+      for (int e = 0; e < M; ++e)
+        if (!((slots >> e) & 1u)) {  // zeros, stored where the buffer holds anything else
+          dflux[e * nc + c] = 0.;
+          if ((old >> e) & 1u) Uout[e * nc + c] = Uout[(M + e) * nc + c] = Uout[(2 * M + e) * nc + c] = 0.;
+        }
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    if (!((slots >> v) & 1u)) continue;
+    const double phi = valid ? u[v] / den : 0.;
+    const double phip = lane_back(phi);
     const double gb = (valid && validp) ? (phi - phip) / dxb : 0.;
-    const double gf = __shfl_down(gb, 1);
+    const double gf = lane_front(gb);
     double g = 0.;
     if (S.order2 && valid) {
       if (gb != 0.) g += 0.5 * (mh_limiter<LIM>(S.limiter, gf / gb) * gb);
       if (gf != 0.) g += 0.5 * (mh_limiter<LIM>(S.limiter, gb / gf) * gf);
     }
-    const double gp = __shfl_up(g, 1);
+    const double gp = lane_back(g);
     double F = 0.;  // flux of the back face with outer normal +e_x (for cell i-1)
     if (inb) {
       const double pf = (upprev ? phip : phi) + hb * (upprev ? gp : g);
-      F = 1. * vf * area * dt * pf;
+      F = w * pf;
     }
-    const double Ff = __shfl_down(F, 1);
+    const double Ff = lane_front(F);
     const double fb = -F;  // the back face seen from cell i (outer normal -e_x)
     double ff = 0.;
     double dd = 0.;
@@ -2169,12 +2247,18 @@ __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, in
       if (inf) dd += 0.5 * Ff * 1.;
     }
     if (out) {
-      double un = (own ? uv : 0.) - ff;
+      double un = (own ? u[v] : 0.) - ff;
       if (v >= M && v < 2 * M) dflux[(v - M) * nc + c] = dd;
       if (v >= M && v < 3 * M && un < 0.) un = 0.;
-      Uout[v * nc + c] = un;
+      if (M > 1 && v < 3 * M) {
+        if (un != 0.) held |= 1u << (v % M);
+        if (un != 0. || ((old >> (v % M)) & 1u)) Uout[v * nc + c] = un;
+      } else {
+        Uout[v * nc + c] = un;
+      }
     }
   }
+  if (sparse && out) S.pm[usel ? 0 : 1][c] = (uint8_t)held;
 }
 
 // Mass flux through the dual faces between node position a and a+1 along D: the sum, in
@@ -2339,21 +2423,21 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
     for (int cc = 0; cc < NC; ++cc) P[cc] = mh_quot(v[cc], rm);
   }
   const bool inner = valid && i >= 1 && i <= na - 1;
-  const double Xm = __shfl_up(X, 1), Xp = __shfl_down(X, 1);
+  const double Xm = lane_back(X), Xp = lane_front(X);
   double Pm[NC], Pp[NC], G0[NC], Gm[NC], Gp[NC];
   const MhRecip rX = mh_recip(X - Xm);
 #pragma unroll
   for (int cc = 0; cc < NC; ++cc) {
-    Pm[cc] = __shfl_up(P[cc], 1);
-    Pp[cc] = __shfl_down(P[cc], 1);
+    Pm[cc] = lane_back(P[cc]);
+    Pp[cc] = lane_front(P[cc]);
     const double eb = (valid && validp) ? mh_quot(P[cc] - Pm[cc], rX) : 0.;  // edge i-1/2
-    const double ef = __shfl_down(eb, 1);                                    // edge i+1/2
+    const double ef = lane_front(eb);                                    // edge i+1/2
     G0[cc] = (S.order2 && inner) ? dual_limited<LIM>(S, eb, ef) : 0.;
-    Gm[cc] = __shfl_up(G0[cc], 1);
-    Gp[cc] = __shfl_down(G0[cc], 1);
+    Gm[cc] = lane_back(G0[cc]);
+    Gp[cc] = lane_front(G0[cc]);
   }
   const double front = valid ? dual_edge_flux<DIM, 0>(S, i, j, k) : 0.;
-  const double back = __shfl_up(front, 1);
+  const double back = lane_back(front);
   if (!out) return;
   double U[NC + 1];
 #pragma unroll
@@ -2471,10 +2555,47 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
       w[q] = 1. * vf * area * dt;
     }
   }
+  // the slots to run, as in k_sweep_cell_row_body: those of the environments some cell of the tile
+  // holds, and V q
+  const bool sparse = M > 1 && S.pm[0] != nullptr;
+  unsigned slots = (1u << NV) - 1u, held = 0, olds = ~0u;  // held, olds: M bits per row q
+  if (sparse) {
+    static_assert(MH_TILE_Q * M <= 32, "the presence bits of a thread's rows fit a word");
+    unsigned in = 0;
+    olds = 0;
+#pragma unroll
+    for (int q = 0; q < MH_TILE_Q; ++q) {
+      const int r = ly + 4 * q;
+      if (!val[q]) continue;
+      const long c = c_base + (abase + r) * sD;
+      const bool irregular = !mh_finite_nonzero(den[q]) ||
+                             (inner[q] && (!mh_finite_nonzero(dx[q]) || !mh_finite(w[q]) || !mh_finite(hh[q])));
+      in |= irregular ? (1u << M) - 1u : (unsigned)S.pm[usel ? 1 : 0][c];
+      if (r >= 2 && r < 2 + MH_TILE_L) olds |= (S.pm[usel ? 0 : 1][c] & ((1u << M) - 1u)) << (M * q);
+    }
+#pragma unroll
+    for (int e = 0; e < M; ++e)
+      if (!__syncthreads_or((in >> e) & 1u)) slots &= ~((1u << e) | (1u << (M + e)) | (1u << (2 * M + e)));
+#pragma unroll
+    for (int q = 0; q < MH_TILE_Q; ++q) {
+      const int r = ly + 4 * q;
+      if (!val[q] || r < 2 || r >= 2 + MH_TILE_L) continue;
+      const long c = c_base + (abase + r) * sD;
+#pragma unroll
+      for (int e = 0; e < M; ++e)
+        if (!((slots >> e) & 1u)) {
+          dflux[e * nc + c] = 0.;
+          if ((olds >> (M * q + e)) & 1u) Uout[e * nc + c] = Uout[(M + e) * nc + c] = Uout[(2 * M + e) * nc + c] = 0.;
+        }
+    }
+  }
   double un_next[MH_TILE_Q];  // slot loads run one slot ahead
 #pragma unroll
-  for (int q = 0; q < MH_TILE_Q; ++q) un_next[q] = val[q] ? Uin[c_base + (abase + ly + 4 * q) * sD] : 0.;
-  for (int v = 0; v < NV; ++v) {
+  for (int q = 0; q < MH_TILE_Q; ++q)
+    un_next[q] = val[q] ? Uin[(__ffs(slots) - 1) * nc + c_base + (abase + ly + 4 * q) * sD] : 0.;
+  while (slots) {
+    const int v = __ffs(slots) - 1;
+    slots &= slots - 1;
     // barriers: the previous slot read sphi and ssl before its last barrier, and reads
     // sgf (fluxes) before the first barrier of this slot
     double uq[MH_TILE_Q];
@@ -2482,7 +2603,7 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
     for (int q = 0; q < MH_TILE_Q; ++q) {
       const int a = abase + ly + 4 * q;
       uq[q] = un_next[q];
-      if (v + 1 < NV) un_next[q] = val[q] ? Uin[(v + 1) * nc + c_base + a * sD] : 0.;
+      if (slots) un_next[q] = val[q] ? Uin[(__ffs(slots) - 1) * nc + c_base + a * sD] : 0.;
       sphi[ly + 4 * q][lx] = val[q] ? uq[q] / den[q] : 0.;
     }
     __syncthreads();
@@ -2544,7 +2665,21 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
         dflux[(v - M) * nc + c] = dd;
       }
       if (v >= M && v < 3 * M && un < 0.) un = 0.;
-      Uout[v * nc + c] = un;
+      if (M > 1 && v < 3 * M) {
+        const int e = v < M ? v : v < 2 * M ? v - M : v - 2 * M;
+        if (un != 0.) held |= 1u << (M * q + e);
+        if (un != 0. || ((olds >> (M * q + e)) & 1u)) Uout[v * nc + c] = un;
+      } else {
+        Uout[v * nc + c] = un;
+      }
+    }
+  }
+  if (sparse) {
+#pragma unroll
+    for (int q = 0; q < MH_TILE_Q; ++q) {
+      const int r = ly + 4 * q;
+      if (val[q] && r >= 2 && r < 2 + MH_TILE_L)
+        S.pm[usel ? 0 : 1][c_base + (abase + r) * sD] = (uint8_t)((held >> (M * q)) & ((1u << M) - 1u));
     }
   }
 }
@@ -3138,7 +3273,9 @@ __device__ __forceinline__ void k_finalize_body(const MhDev& S, int lb, int usel
     const long nc = S.g.nc;
     const double thr = S.thr_remap;
     double U[3 * M + 1];
-    for (int v = 0; v <= 3 * M; ++v) U[v] = Uin[v * nc + c];
+    const unsigned held = M > 1 && S.pm[0] ? S.pm[usel ? 1 : 0][c] : ~0u;
+    for (int v = 0; v < 3 * M; ++v) U[v] = ((held >> (v % M)) & 1u) ? Uin[v * nc + c] : 0.;
+    U[3 * M] = Uin[3 * M * nc + c];
     if (S.pb && S.nsweep > 0) {  // phi the last sweep left (RemapADIService.cc:493-538): what the
                                   // next cycle's first sweep sees for non-member environments
       double sv = 0.;

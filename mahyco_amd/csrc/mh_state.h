@@ -78,6 +78,7 @@ struct MhDev {
   // remap buffers: U ping-pong [nv][nc], mass fluxes [m][nc], dual state ping-pong: A = Ud
   // [dim+1][nn], B = Pa [dim][nn] with its masses in Pb [nn] (DualBuf in mh_kernels.h)
   double *Ua, *Ub, *dflux, *Ud, *Pa, *Pb;
+  uint8_t* pm[2];  // environments each cell's slots of Ua / Ub hold anything of [nc] (k_cell_lag), or null
   // conservation-energie-totale: the dual kinetic energy [nn] (in place), its phi ping-pong
   // [nn] each, and the energy each cell receives back [nc]; null otherwise
   double *ke_U, *ke_Pa, *ke_Pb, *dec;

@@ -29,7 +29,7 @@ void launch_cell_x(MhHandle* h, int sel, int first) {
   // environments: 7.9 -> 5.0 us on 100x5x5 cells, 7.7 -> 5.8 us on 181x181, 13.1 -> 11.6 us on
   // 362x362); beyond that the repeated geometry costs more (512x512: 16.0 us, split 16.2).
   const SlotSplit p = slot_split((long)row_blocks(h) * (MH_BLOCK / 64), 4000, 3 * M + 1);
-  if (p.groups > 1)
+  if (p.groups > 1 && !S.pm[0])  // (the presence byte of a cell is written with its last slot)
     MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL, (k_sweep_cell_row_slots<DIM, M, LIM>), dim3(row_blocks(h), p.groups), MH_BLOCK,
                        S, sel, first, p.vper));
   else

@@ -93,3 +93,41 @@ def test_pente_borne_groups(n, debar):
 @pytest.mark.parametrize("limiter", [T.MH_MINMOD_G, T.MH_VANLEER_G, T.MH_ARITHMETIC_G, T.MH_ULTRABEE_G])
 def test_generalised_limiters(limiter):
     check(moving_tube((9, 5, 4), 1, limiter=limiter))
+
+
+@pytest.mark.parametrize("name", ["served114", "served162"])
+def test_emptying_cells_with_presence_bytes(name, monkeypatch):
+    """Runs whose cells empty out (phi of an empty cell, zero denominators), with the sweeps that
+    skip the slots of environments a stencil does not hold."""
+    from tests.test_gpu_paths import test_full_size_bitwise_vs_oracle
+    monkeypatch.setenv("MAHYCO_SWEEP", "tile")
+    test_full_size_bitwise_vs_oracle(name)
+
+
+@pytest.mark.parametrize("sweep", ["tile", "flat"])
+def test_presence_bytes_three_materials(sweep, monkeypatch):
+    monkeypatch.setenv("MAHYCO_SWEEP", sweep)
+    c = cases.bitriplepoint()
+    c.n = (130, 67, 1)
+    check(c, iterations=60)
+
+
+def test_presence_bytes_over_variants_and_checkpoint(tmp_path, monkeypatch):
+    """Sweep variants that keep the presence bytes and variants that do not, in turn on one case, and
+    a restart in between."""
+    from mahyco_amd.lib import GpuCase
+    from oracle.pyoracle import OracleCase
+    monkeypatch.setenv("MAHYCO_SWEEP", "tile")
+    c = moving_tube((70, 33), 1)
+    g, o = GpuCase(c), OracleCase(c, pow_mode=1, threads=4)
+    v = g.variant
+    for k, code in enumerate((v, v | 16, v)):
+        g.set_variant(code)
+        g.run(7)
+        o.run(7)
+        if k == 1:
+            g.checkpoint_write(tmp_path / "dump")
+            g.run(3)
+            g.checkpoint_read(tmp_path / "dump")
+    a, b = fields(g, 2, 2), fields(o, 2, 2)
+    assert not [k for k in a if not bitwise_equal(a[k], b[k])]
