@@ -1198,6 +1198,9 @@ __device__ __forceinline__ void face_quant(const MhDev& S, long f0, double& area
     if (D == 0) { nd[0] = f0; nd[1] = f0 + nnx; nd[2] = f0 + nnx + nnxy; nd[3] = f0 + nnxy; }
     else if (D == 1) { nd[0] = f0; nd[1] = f0 + 1; nd[2] = f0 + 1 + nnxy; nd[3] = f0 + nnxy; }
     else { nd[0] = f0; nd[1] = f0 + 1; nd[2] = f0 + 1 + nnx; nd[3] = f0 + nnx; }
+    // every load first: the branch below would split them into two rounds
+    const double* ud = S.u[D];
+    const double u0 = ud[nd[0]], u1 = ud[nd[1]], u2 = ud[nd[2]], u3 = ud[nd[3]];
     const D3 x0 = load3(S.xlc, nd[0]), x1 = load3(S.xlc, nd[1]);
     const D3 x2 = load3(S.xlc, nd[2]), x3 = load3(S.xlc, nd[3]);
     const D3 v1 = x2 - x0, v2 = x3 - x1;
@@ -1214,20 +1217,23 @@ __device__ __forceinline__ void face_quant(const MhDev& S, long f0, double& area
     s += 0.25 * xc;
     s += 0.25 * xd;
     xf = s;
-    const double* ud = S.u[D];
     double us = 0.;
     if (S.csts) {  // the mean of n and n+1 (PrepareRemap.cc:236-240)
       const double* vd = S.un[D];
-      for (int l = 0; l < 4; ++l) us += 0.5 * (ud[nd[l]] + vd[nd[l]]);
+      us += 0.5 * (u0 + vd[nd[0]]);
+      us += 0.5 * (u1 + vd[nd[1]]);
+      us += 0.5 * (u2 + vd[nd[2]]);
+      us += 0.5 * (u3 + vd[nd[3]]);
     } else {
-      us += ud[nd[0]];
-      us += ud[nd[1]];
-      us += ud[nd[2]];
-      us += ud[nd[3]];
+      us += u0;
+      us += u1;
+      us += u2;
+      us += u3;
     }
     vf = 0.25 * us;
   } else {
     const long n1 = D == 0 ? f0 + nnx : f0 + 1;
+    const double u0 = S.u[D][f0], u1 = S.u[D][n1];
     const double dxv = S.xlc[0][n1] - S.xlc[0][f0];
     const double dyv = S.xlc[1][n1] - S.xlc[1][f0];
     area = D == 0 ? fabs(dyv) : fabs(dxv);
@@ -1236,15 +1242,14 @@ __device__ __forceinline__ void face_quant(const MhDev& S, long f0, double& area
     s += 0.5 * xd[f0];
     s += 0.5 * xd[n1];
     xf = s;
-    const double* ud = S.u[D];
     double us = 0.;
     if (S.csts) {
       const double* vd = S.un[D];
-      us += 0.5 * (ud[f0] + vd[f0]);
-      us += 0.5 * (ud[n1] + vd[n1]);
+      us += 0.5 * (u0 + vd[f0]);
+      us += 0.5 * (u1 + vd[n1]);
     } else {
-      us += ud[f0];
-      us += ud[n1];
+      us += u0;
+      us += u1;
     }
     vf = 0.5 * us;
   }
@@ -2152,38 +2157,38 @@ __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, in
   const bool inb = valid && i > 0;       // back face (node column i): inner when 0 < i < nx
   const bool inf = valid && i < nx - 1;
   const long nc = S.g.nc;
-  const long c = row * nx + i;
-  const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
+  // lanes beyond the row load its end cell again (unused), so that no branch parts the loads
+  const int ic = min(max(i, 0), nx - 1);
+  const long c = row * nx + ic;
+  const long b = ic + (long)S.g.nnx * (j + (long)S.g.nny * k);
   const bool sparse = M > 1 && S.pm[0] != nullptr;
   unsigned slots = ((1u << v1) - 1u) & ~((1u << v0) - 1u);  // the slots to run
   // every load that depends on the kernel arguments alone goes out before anything waits (the stop
   // flag included): a wavefront's time here is that of its load rounds
-  const unsigned here = sparse && valid ? S.pm[usel ? 1 : 0][c] : 0u;
-  const unsigned old = sparse && out ? S.pm[usel ? 0 : 1][c] : ~0u;
-  const uint8_t mk = first && valid ? S.mask[c] : (uint8_t)1;
-  double den = first && valid ? S.Vl[c] : 1.;
+  const unsigned here = sparse ? S.pm[usel ? 1 : 0][c] : 0u;
+  const unsigned old = sparse ? S.pm[usel ? 0 : 1][c] : ~0u;
+  const uint8_t mk = first ? S.mask[c] : (uint8_t)1;
+  double den = first ? S.Vl[c] : 1.;
   double u[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const bool now = !sparse || v == 3 * M || (v < M && !first);
-    u[v] = now && valid && (((slots >> v) & 1u) || (v < M && !first)) ? Uin[v * nc + c] : 0.;
+    u[v] = now && (((slots >> v) & 1u) || (v < M && !first)) ? Uin[v * nc + c] : 0.;
   }
   const double dt = S.sc->dt;
   const bool halted = mh_halted(S.sc);
-  double xc = 0., area = 0., xf = 0., vf = 0.;
-  if (valid) xc = cell_centre_d<DIM, 0>(S, b);
-  if (inb) face_quant<DIM, 0>(S, b, area, xf, vf);
+  const double xc = cell_centre_d<DIM, 0>(S, b);
+  double area, xf, vf;
+  face_quant<DIM, 0>(S, b, area, xf, vf);
   if (halted) return;
   const bool own = mk != 0;  // an empty cell's U starts from 0
-  if (valid) {
-    if (first) {
-      if (!own) den = 1.;  // an empty cell holds Phi itself
-    } else {
-      double sv = 0.;
+  if (first) {
+    if (!own) den = 1.;  // an empty cell holds Phi itself
+  } else {
+    double sv = 0.;
 #pragma unroll
-      for (int kk = 0; kk < M; ++kk) sv += u[kk];
-      den = sv;
-    }
+    for (int kk = 0; kk < M; ++kk) sv += u[kk];
+    den = sv;
   }
   const double xcp = lane_back(xc);
   const double dxb = (valid && validp) ? xc - xcp : 0.;
@@ -2197,13 +2202,13 @@ __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, in
   if (sparse) {
     const bool irregular = valid && (!mh_finite_nonzero(den) || (validp && lane > 0 && !mh_finite_nonzero(dxb)) ||
                                      (inb && (!mh_finite(w) || !mh_finite(hb))));
-    const unsigned in = irregular ? (1u << M) - 1u : here;
+    const unsigned in = irregular ? (1u << M) - 1u : valid ? here : 0u;
 #pragma unroll
     for (int e = 0; e < M; ++e)
       if (__ballot((in >> e) & 1u) == 0) slots &= ~((1u << e) | (1u << (M + e)) | (1u << (2 * M + e)));
 #pragma unroll
     for (int v = 0; v < 3 * M; ++v)
-      if (((slots >> v) & 1u) && (v >= M || first)) u[v] = valid ? Uin[v * nc + c] : 0.;
+      if (((slots >> v) & 1u) && (v >= M || first)) u[v] = Uin[v * nc + c];
     if (out) {
 #pragma unroll
       for (int e = 0; e < M; ++e)
@@ -2265,28 +2270,41 @@ __device__ __forceinline__ void k_sweep_cell_row_body(const MhDev& S, int lb, in
 // the order of k_sweep_node_body, of the cell mass fluxes of the 2^(d-1) cells at
 // position a around the node line (it1, it2) -- the "front" flux of node a and the "back"
 // flux of node a+1 (DualPhaseRemap.cc:75-108).  0 when position a holds no cells.
-template <int DIM, int D>
+template <int DIM, int D, int M>
 __device__ __forceinline__ double dual_edge_flux(const MhDev& S, int a, int it1, int it2) {
   const int na = D == 0 ? S.g.nx : D == 1 ? S.g.ny : S.g.nz;
-  if (a < 0 || a >= na) return 0.;
   const double w = DIM == 3 ? 0.25 : 0.5;
   const long nc = S.g.nc;
   const int n1 = D == 0 ? S.g.ny : S.g.nx;
   const int n2 = D == 2 ? S.g.ny : S.g.nz;
   const long st1 = D == 0 ? (long)S.g.nx : 1;
   const long st2 = D == 2 ? (long)S.g.nx : (long)S.g.nx * S.g.ny;
-  const long cbase = D == 0 ? (long)a : D == 1 ? (long)a * S.g.nx : (long)a * S.g.nx * S.g.ny;
-  const int lo2 = DIM == 3 ? it2 - 1 : 0, hi2 = DIM == 3 ? it2 : 0;
-  double f = 0.;
-  for (int p2 = lo2; p2 <= hi2; ++p2) {
-    if (DIM == 3 && (p2 < 0 || p2 >= n2)) continue;
-    for (int p1 = it1 - 1; p1 <= it1; ++p1) {
-      if (p1 < 0 || p1 >= n1) continue;
+  const int ac = min(max(a, 0), na - 1);
+  const long cbase = D == 0 ? (long)ac : D == 1 ? (long)ac * S.g.nx : (long)ac * S.g.nx * S.g.ny;
+  constexpr int N2 = DIM == 3 ? 2 : 1;
+  // all cells are loaded before the first is added: a cell beyond the mesh is its neighbour again,
+  // left out of the sum (one wait instead of one per cell and environment)
+  double d[N2][2][M];
+#pragma unroll
+  for (int q2 = 0; q2 < N2; ++q2)
+#pragma unroll
+    for (int q1 = 0; q1 < 2; ++q1) {
+      const int p1 = min(max(it1 - 1 + q1, 0), n1 - 1), p2 = DIM == 3 ? min(max(it2 - 1 + q2, 0), n2 - 1) : 0;
       const long cf = cbase + p1 * st1 + (DIM == 3 ? p2 * st2 : 0);
-      for (int kk = 0; kk < S.m; ++kk) f += w * S.dflux[kk * nc + cf];
+#pragma unroll
+      for (int kk = 0; kk < M; ++kk) d[q2][q1][kk] = S.dflux[kk * nc + cf];
     }
-  }
-  return f;
+  double f = 0.;
+#pragma unroll
+  for (int q2 = 0; q2 < N2; ++q2)
+#pragma unroll
+    for (int q1 = 0; q1 < 2; ++q1) {
+      const int p1 = it1 - 1 + q1, p2 = it2 - 1 + q2;
+      const bool in = p1 >= 0 && p1 < n1 && (DIM == 2 || (p2 >= 0 && p2 < n2));
+#pragma unroll
+      for (int kk = 0; kk < M; ++kk) f = in ? f + w * d[q2][q1][kk] : f;
+    }
+  return a < 0 || a >= na ? 0. : f;
 }
 
 // The dual state of a node between two sweeps is four words, v and m, read from one buffer and
@@ -2388,7 +2406,7 @@ __device__ __forceinline__ void dual_node_update(const MhDev& S, long n, double*
 // Dual x sweep with one wavefront per 60 nodes of a node row (lane shuffles carry the
 // neighbours' phi, coordinates, edge gradients and limited gradients; the front flux of
 // node i is the back flux of node i+1).  Lanes 2..61 write their node.
-template <int DIM, int LIM>
+template <int DIM, int M, int LIM>
 __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, int psel, int prev, int last) {
   constexpr int NC = DIM;
   const int nnx = S.g.nnx, na = S.g.nx;
@@ -2397,7 +2415,6 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
   const int lane = threadIdx.x & 63;
   const long gw = (long)lb * (MH_BLOCK / 64) + (threadIdx.x >> 6);
   if (gw >= rows * wpr) return;  // whole wavefront
-  if (mh_halted(S.sc)) return;
   const DualBuf in = dual_in<DIM>(S, psel, prev);
   const long row = gw / wpr;
   const int i = (int)(gw % wpr) * MH_ROW_OUT - 2 + lane;
@@ -2406,17 +2423,19 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
   const bool out = valid && lane >= 2 && lane < 2 + MH_ROW_OUT;
   const int j = (int)(row % S.g.nny);
   const int k = (int)(row / S.g.nny);
-  const long n = row * nnx + i;
-  double v[NC], P[NC], m = 0., X = 0.;
+  // lanes beyond the row load its end node again (unused); one round of loads, the stop flag included
+  const long n = row * nnx + min(max(i, 0), na);
+  double v[NC], P[NC];
 #pragma unroll
-  for (int cc = 0; cc < NC; ++cc) v[cc] = valid ? in.v[cc][n] : 0.;
-  if (valid) {
-    m = in.m[n];
-    X = S.xlc[0][n];
-  }
+  for (int cc = 0; cc < NC; ++cc) v[cc] = in.v[cc][n];
+  const double m = in.m[n];
+  const double X = S.xlc[0][n];
+  const double flux = dual_edge_flux<DIM, 0, M>(S, i, j, k);
+  if (mh_halted(S.sc)) return;
+  const double front = valid ? flux : 0.;
   const bool kept = dual_kept<DIM>(S, prev, i, j, k);
 #pragma unroll
-  for (int cc = 0; cc < NC; ++cc) P[cc] = v[cc];
+  for (int cc = 0; cc < NC; ++cc) P[cc] = valid ? v[cc] : 0.;
   if (!kept && valid) {
     const MhRecip rm = mh_recip(m);
 #pragma unroll
@@ -2431,12 +2450,11 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
     Pm[cc] = lane_back(P[cc]);
     Pp[cc] = lane_front(P[cc]);
     const double eb = (valid && validp) ? mh_quot(P[cc] - Pm[cc], rX) : 0.;  // edge i-1/2
-    const double ef = lane_front(eb);                                    // edge i+1/2
+    const double ef = lane_front(eb);                                        // edge i+1/2
     G0[cc] = (S.order2 && inner) ? dual_limited<LIM>(S, eb, ef) : 0.;
     Gm[cc] = lane_back(G0[cc]);
     Gp[cc] = lane_front(G0[cc]);
   }
-  const double front = valid ? dual_edge_flux<DIM, 0>(S, i, j, k) : 0.;
   const double back = lane_back(front);
   if (!out) return;
   double U[NC + 1];
@@ -2835,45 +2853,17 @@ __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, in
 // The mass fluxes through an inner node's back and front dual faces along D
 // (DualPhaseRemap.cc:75-108): 1/2 (2D) or 1/4 (3D) of the dual mass fluxes of the cells
 // behind / ahead of the node, over those cells in face order and the environments in order.
-template <int DIM, int D, bool BACK = true>
+template <int DIM, int D, int M>
 __device__ __forceinline__ void dual_mass_fluxes(const MhDev& S, int i, int j, int k, int a, double& back,
                                                  double& front) {
-  const double* __restrict__ dflux = S.dflux;
-  const long nc = S.g.nc;
-  const double w = DIM == 3 ? 0.25 : 0.5;
-  const int M = S.m;
-  back = 0.;
-  front = 0.;
-  const long sD = D == 0 ? 1 : D == 1 ? (long)S.g.nx : (long)S.g.nx * S.g.ny;
-  // transverse axes (t1 fastest, t2 slowest) and their cell counts
-  const int t1 = D == 0 ? 1 : 0;
-  const int t2 = D == 2 ? 1 : 2;
-  const int it1 = t1 == 0 ? i : j;
-  const int it2 = t2 == 1 ? j : k;
-  const int n1 = t1 == 0 ? S.g.nx : S.g.ny;
-  const int n2 = t2 == 1 ? S.g.ny : S.g.nz;
-  const long st1 = t1 == 0 ? 1 : (long)S.g.nx;
-  const long st2 = t2 == 1 ? (long)S.g.nx : (long)S.g.nx * S.g.ny;
-  const int lo2 = DIM == 3 ? it2 - 1 : 0, hi2 = DIM == 3 ? it2 : 0;
-  // cell at position a along D and (p1, p2) along the transverse axes
-  const long cbase = D == 0 ? (long)a : D == 1 ? (long)a * S.g.nx : (long)a * S.g.nx * S.g.ny;
-  for (int p2 = lo2; p2 <= hi2; ++p2) {
-    if (DIM == 3 && (p2 < 0 || p2 >= n2)) continue;
-    for (int p1 = it1 - 1; p1 <= it1; ++p1) {
-      if (p1 < 0 || p1 >= n1) continue;
-      const long cf = cbase + p1 * st1 + (DIM == 3 ? p2 * st2 : 0);
-      const long cb = cf - sD;
-      if (BACK)
-        for (int kk = 0; kk < M; ++kk) back += w * dflux[kk * nc + cb];
-      for (int kk = 0; kk < M; ++kk) front += w * dflux[kk * nc + cf];
-    }
-  }
+  const int it1 = D == 0 ? j : i, it2 = D == 2 ? j : k;
+  back = dual_edge_flux<DIM, D, M>(S, a - 1, it1, it2);
+  front = dual_edge_flux<DIM, D, M>(S, a, it1, it2);
 }
 
-template <int DIM, int D, int LIM>
+template <int DIM, int D, int M, int LIM>
 __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel, int prev, int last) {
   constexpr int NC = DIM;  // velocity components carried
-  if (mh_halted(S.sc)) return;
   const DualBuf din = dual_in<DIM>(S, psel, prev);
   const int nnx = S.g.nnx, nny = S.g.nny;
   const int i = (int)(n % nnx);
@@ -2887,11 +2877,23 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
   // them or none was
   const bool kept = dual_kept<DIM>(S, prev, i, j, k);
   const bool inner = a >= 1 && a <= na - 1;
+  // one round of loads, the stop flag included: a node beyond the mesh is its end node again (unused)
+  double P[5][NC], X[5], mm[5], fl[2];
+#pragma unroll
+  for (int o = -2; o <= 2; ++o) {
+    const long m2 = n + (min(max(a + o, 0), na) - a) * nD;
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = din.v[cc][m2];
+    mm[o + 2] = din.m[m2];
+    X[o + 2] = S.xlc[D][m2];
+  }
+  dual_mass_fluxes<DIM, D, M>(S, i, j, k, a, fl[0], fl[1]);
+  if (mh_halted(S.sc)) return;
   double U[NC + 1], v0[NC];
-  U[NC] = din.m[n];
+  U[NC] = mm[2];
 #pragma unroll
   for (int cc = 0; cc < NC; ++cc) {
-    v0[cc] = din.v[cc][n];
+    v0[cc] = P[2][cc];
     U[cc] = kept ? U[NC] * v0[cc] : v0[cc];
   }
   if (!inner) {
@@ -2899,19 +2901,16 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
     return;
   }
   const double dt = S.sc->dt;
-  double P[5][NC], X[5];
 #pragma unroll
   for (int o = -2; o <= 2; ++o) {
     const int bb = a + o;
-    if (bb >= 0 && bb <= na) {
-      const long m2 = n + o * nD;
-      for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = din.v[cc][m2];
-      if (!kept) {
-        const double mm = din.m[m2];
-        for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = P[o + 2][cc] / mm;
-      }
-      X[o + 2] = S.xlc[D][m2];
-    } else {
+    if (!kept) {
+      const MhRecip rm = mh_recip(mm[o + 2]);
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = mh_quot(P[o + 2][cc], rm);
+    }
+    if (bb < 0 || bb > na) {
+#pragma unroll
       for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = 0.;
       X[o + 2] = 0.;
     }
@@ -2948,15 +2947,13 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
         if (LIM == MH_LIM_ANY && S.limiter >= MH_MINMOD_G) {
           g = flux_limiter_g(S.limiter, gf, gb, P[o + 3][cc], P[o + 1][cc], h0, hp, hm, S.simple_pente);
         } else {
-          if (gb != 0.) g += 0.5 * mh_limiter<LIM>(S.limiter, gf / gb) * gb;
-          if (gf != 0.) g += 0.5 * mh_limiter<LIM>(S.limiter, gb / gf) * gf;
+          g = mh_limited_gradient<LIM, true>(S.limiter, gb, gf);
         }
       }
       G[o + 1][cc] = g;
     }
   }
-  double back, front;
-  dual_mass_fluxes<DIM, D>(S, i, j, k, a, back, front);
+  const double back = fl[0], front = fl[1];
   U[NC] += back - front;
   const double o2 = (double)S.order2;
   const double ufront = 0.5 * (P[2][D] + P[3][D]);
@@ -2975,19 +2972,23 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
   dual_store<DIM>(S, n, U, U, psel, last);
 }
 
-template <int DIM, int D, int LIM>
+template <int DIM, int D, int M, int LIM>
 __device__ __forceinline__ void k_sweep_node_body(const MhDev& S, int lb, int psel, int prev, int last) {
   const long n = lb * (long)blockDim.x + threadIdx.x;
   if (n >= S.g.nn) return;
-  k_sweep_node_at<DIM, D, LIM>(S, n, psel, prev, last);
+  k_sweep_node_at<DIM, D, M, LIM>(S, n, psel, prev, last);
 }
 
 // The y or z dual sweep of one mesh with each thread marching along D over a segment of
-// MH_NM_L nodes: the window of phi and coordinates, the edge gradients, the limited gradients
+// nm_len nodes: the window of phi and coordinates, the edge gradients, the limited gradients
 // and the mass flux through the node's front dual face are carried to the next node (they are
 // its back-side values), so each is formed once per node instead of by each of the three nodes
 // whose update reads it.  Threads of a wave are consecutive along x.  Same formulas and orders
-// as k_sweep_node_at (classical limiters; the generalised ones keep k_sweep_node).  The segment
+// as k_sweep_node_at (classical limiters; the generalised ones keep k_sweep_node).  What bounds it
+// is the latency of a node's loads at 3 waves per SIMD: with the next node's loads issued together
+// ahead of this node's arithmetic, y / z take 116 / 114 us on the 256x128x128 tube (2.9 TB/s of the
+// bytes it cannot do without) and 166 / 161 us on the 192^3 blast; with one load round per cell of
+// a mass flux, waited for where it is added, 165 / 162 and 201 / 198 us at 4 waves.  The segment
 // length is per case (the autotuner tries 4-12 nodes): 10 by default on large meshes, 4 on smaller
 // ones, which need the threads, and below MH_MARCH_NODES one thread per node (k_sweep_node).
 #ifndef MH_NM_L
@@ -2999,7 +3000,7 @@ MH_HD int march_nseg(int n, int len) { return (n + len - 1) / len; }
 #ifndef MH_NM_MIN_WAVES
 #define MH_NM_MIN_WAVES 1
 #endif
-template <int DIM, int D, int LIM>
+template <int DIM, int D, int M, int LIM>
 __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, int psel, int prev, int last) {
   constexpr int NC = DIM;
   const int nnx = S.g.nnx, nny = S.g.nny;
@@ -3009,7 +3010,6 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
   const long g = lb * (long)blockDim.x + threadIdx.x;
   const int nseg = march_nseg(na + 1, S.nm_len);  // na + 1 nodes along D
   if (g >= cols * nseg) return;
-  if (mh_halted(S.sc)) return;
   const int seg = (int)(g / cols);
   const long rem = g - seg * cols;
   const int i = (int)(rem % nnx), t2 = (int)(rem / nnx);
@@ -3022,19 +3022,23 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
   const double* __restrict__ Xd = S.xlc[D];
   const double dt = S.sc->dt;
   const double o2 = (double)S.order2;
-  auto loadP = [&](int b, double* P, double& X) {
-    if (b >= 0 && b <= na) {
-      const long m2 = base + b * nD;
-      const double m = din.m[m2];
+  // a node of the line (beyond its ends the end node again, then set to 0)
+  auto fetch = [&](int b, double* v, double& m, double& X) {
+    const long m2 = base + min(max(b, 0), na) * nD;
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) P[cc] = din.v[cc][m2];
-      X = Xd[m2];
-      if (!kept) {
-        const MhRecip rm = mh_recip(m);
+    for (int cc = 0; cc < NC; ++cc) v[cc] = din.v[cc][m2];
+    m = din.m[m2];
+    X = Xd[m2];
+  };
+  auto phi = [&](int b, const double* v, double m, double* P, double& X) {
 #pragma unroll
-        for (int cc = 0; cc < NC; ++cc) P[cc] = mh_quot(P[cc], rm);
-      }
-    } else {
+    for (int cc = 0; cc < NC; ++cc) P[cc] = v[cc];
+    if (!kept) {
+      const MhRecip rm = mh_recip(m);
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) P[cc] = mh_quot(v[cc], rm);
+    }
+    if (b < 0 || b > na) {
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) P[cc] = 0.;
       X = 0.;
@@ -3057,39 +3061,58 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
   };
   // window: P and X of nodes a-1 .. a+2 (slots 0..3), edges (a-1/2, a+1/2, a+3/2), G of a-1, a, a+1
   double P[4][NC], X[4], E[3][NC], G[3][NC];
+  double U1[NC + 1], back, front;  // U of the next node, and the fluxes through its dual faces
+  const int j0 = D == 1 ? 0 : t2, k0 = D == 1 ? t2 : 0;  // transverse node position (the D one is a)
+  const int it1 = i, it2 = D == 1 ? k0 : j0;  // transverse cells: x, and z or y
   {
-    double Pm2[NC], Xm2;
-    loadP(a0 - 2, Pm2, Xm2);
-    for (int o = 0; o < 4; ++o) loadP(a0 - 1 + o, P[o], X[o]);
+    double v[5][NC], m[5], Xs[5];
+#pragma unroll
+    for (int o = 0; o < 5; ++o) fetch(a0 - 2 + o, v[o], m[o], Xs[o]);
+    back = dual_edge_flux<DIM, D, M>(S, a0 - 1, it1, it2);
+    front = dual_edge_flux<DIM, D, M>(S, a0, it1, it2);
+    if (mh_halted(S.sc)) return;
+    double Pm2[NC];
+    phi(a0 - 2, v[0], m[0], Pm2, Xs[0]);
+#pragma unroll
+    for (int o = 0; o < 4; ++o) {
+      X[o] = Xs[o + 1];
+      phi(a0 - 1 + o, v[o + 1], m[o + 1], P[o], X[o]);
+    }
+#pragma unroll
+    for (int cc = 0; cc < NC; ++cc) U1[cc] = v[2][cc];
+    U1[NC] = m[2];
     double Em[NC];  // edge a0 - 3/2
-    edge(a0 - 2, Pm2, Xm2, P[0], X[0], Em);
+    edge(a0 - 2, Pm2, Xs[0], P[0], X[0], Em);
+#pragma unroll
     for (int o = 0; o < 3; ++o) edge(a0 - 1 + o, P[o], X[o], P[o + 1], X[o + 1], E[o]);
     limited(a0 - 1, Em, E[0], G[0]);
     limited(a0, E[0], E[1], G[1]);
     limited(a0 + 1, E[1], E[2], G[2]);
   }
-  const int j0 = D == 1 ? 0 : t2, k0 = D == 1 ? t2 : 0;  // transverse node position (the D one is a)
-  double back = 0., front = 0.;
   for (int a = a0; a < a1; ++a) {
     const long n = base + a * nD;
-    double U[NC + 1], v0[NC];  // read a second time (from L2): carrying them costs a wave per SIMD
-    U[NC] = din.m[n];
+    // the next node's loads go out before this one's arithmetic: its U and front flux, and the node
+    // three ahead that enters the window (the state of node a + 1 is read a second time, from L2:
+    // carrying it costs a wave per SIMD)
+    const bool more = a + 1 < a1;
+    double U2[NC + 1], v3[NC], m3 = 0., X3 = 0., front2 = 0.;
+    if (more) {
+#pragma unroll
+      for (int cc = 0; cc < NC; ++cc) U2[cc] = din.v[cc][n + nD];
+      U2[NC] = din.m[n + nD];
+      fetch(a + 3, v3, m3, X3);
+      front2 = dual_edge_flux<DIM, D, M>(S, a + 1, it1, it2);
+    }
+    double U[NC + 1], v0[NC];
+    U[NC] = U1[NC];
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) {
-      v0[cc] = din.v[cc][n];
+      v0[cc] = U1[cc];
       U[cc] = kept ? U[NC] * v0[cc] : v0[cc];
     }
     if (!(a >= 1 && a <= na - 1)) {
       dual_store<DIM>(S, n, U, v0, psel, last);
     } else {
-      const int jj = D == 1 ? a : j0, kk = D == 1 ? k0 : a;
-      if (a > a0 && a >= 2) {  // the back face of node a is the front face of inner node a-1
-        back = front;
-        double unused = 0.;
-        dual_mass_fluxes<DIM, D, false>(S, i, jj, kk, a, unused, front);
-      } else {
-        dual_mass_fluxes<DIM, D>(S, i, jj, kk, a, back, front);
-      }
       U[NC] += back - front;
       const double ufront = 0.5 * (P[1][D] + P[2][D]);
       const int sf = ufront > 0 ? 1 : -1;
@@ -3108,14 +3131,15 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
         if (fabs(U[cc]) < 1.e-300) U[cc] = 0.;
       dual_store<DIM>(S, n, U, U, psel, last);
     }
-    if (a + 1 < a1) {  // slide the window one node along D
+    if (more) {  // slide the window one node along D
 #pragma unroll
       for (int o = 0; o < 3; ++o) {
         X[o] = X[o + 1];
 #pragma unroll
         for (int cc = 0; cc < NC; ++cc) P[o][cc] = P[o + 1][cc];
       }
-      loadP(a + 3, P[3], X[3]);
+      X[3] = X3;
+      phi(a + 3, v3, m3, P[3], X[3]);
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) {
         E[0][cc] = E[1][cc];
@@ -3125,6 +3149,10 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
       }
       edge(a + 2, P[2], X[2], P[3], X[3], E[2]);
       limited(a + 2, E[1], E[2], G[2]);
+#pragma unroll
+      for (int cc = 0; cc <= NC; ++cc) U1[cc] = U2[cc];
+      back = front;
+      front = front2;
     }
   }
 }
@@ -3157,7 +3185,7 @@ __device__ __forceinline__ void k_node_velocity_body(const MhDev& S, int lb, int
 // mass fluxes and upwind choices (DualPhaseRemap.cc:132-238).  Its limited gradient is never
 // formed (UtilesRemap.cc:369-400 covers the velocity only), so the slope term multiplies 0.
 // phi = U / the node mass the node sweep has just written (:251-257).
-template <int DIM, int D>
+template <int DIM, int D, int M>
 __device__ __forceinline__ void k_sweep_ke_body(const MhDev& S, int lb, int psel, int prev) {
   const long n = lb * (long)blockDim.x + threadIdx.x;
   if (n >= S.g.nn) return;
@@ -3188,7 +3216,7 @@ __device__ __forceinline__ void k_sweep_ke_body(const MhDev& S, int lb, int psel
     return;
   }
   double back, front;
-  dual_mass_fluxes<DIM, D>(S, i, j, k, a, back, front);
+  dual_mass_fluxes<DIM, D, M>(S, i, j, k, a, back, front);
   const double dt = S.sc->dt;
   const double o2 = (double)S.order2;
   const double zero_slope = 0.;
@@ -3806,7 +3834,8 @@ MH_WRAP(k_cell_lag_csts, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>,
 MH_WRAP(k_cell_length, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_sweep_cell, 1, template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
-MH_WRAP(k_sweep_node, 1, template <int DIM MH_COMMA int D MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA LIM>,
+MH_WRAP(k_sweep_node, 1, template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>,
+        <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
 MH_WRAP(k_node_velocity, 1, template <int DIM>, <DIM>, MH_COMMA int prev, MH_COMMA prev)
 MH_WRAP(k_finalize, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, MH_COMMA int usel, MH_COMMA usel)
@@ -3815,19 +3844,20 @@ MH_WRAP(k_sweep_cell_row, 1, template <int DIM MH_COMMA int M MH_COMMA int LIM>,
 MH_WRAP(k_sweep_cell_tile, MH_TILE_MIN_WAVES,
         template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
-MH_WRAP(k_sweep_node_row, 1, template <int DIM MH_COMMA int LIM>, <DIM MH_COMMA LIM>,
+MH_WRAP(k_sweep_node_row, 1, template <int DIM MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
 MH_WRAP(k_hcell, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_node_adv, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_node_fwd, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_sweep_cell_gen, 1, template <int DIM MH_COMMA int D MH_COMMA int M>, <DIM MH_COMMA D MH_COMMA M>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
-MH_WRAP(k_sweep_ke, 1, template <int DIM MH_COMMA int D>, <DIM MH_COMMA D>, MH_COMMA int psel MH_COMMA int prev,
+MH_WRAP(k_sweep_ke, 1, template <int DIM MH_COMMA int D MH_COMMA int M>, <DIM MH_COMMA D MH_COMMA M>, MH_COMMA int psel MH_COMMA int prev,
         MH_COMMA psel MH_COMMA prev)
 MH_WRAP(k_dual_init, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_cons_ec, 1, template <int DIM>, <DIM>, MH_COMMA int psel, MH_COMMA psel)
 MH_WRAP(k_prepare_remap, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
-MH_WRAP(k_sweep_node_march, MH_NM_MIN_WAVES, template <int DIM MH_COMMA int D MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA LIM>,
+MH_WRAP(k_sweep_node_march, MH_NM_MIN_WAVES, template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>,
+        <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
 
 // Small meshes: the remap slots of a cell are shared out over the gridDim.y rows of the grid, vper

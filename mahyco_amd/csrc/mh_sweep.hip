@@ -80,34 +80,34 @@ void launch_cell_part(MhHandle* h, int D, int sel, int first, bool gen, bool o3)
 
 // Dual part of one sweep direction (computeDualUremap), then the dual kinetic energy when
 // the total energy is conserved.  None in advection mode (withDualProjection, PrepareRemap.cc:211).
-template <int DIM>
+template <int DIM, int M>
 void launch_dual_part(MhHandle* h, int D, int sel, int prev, int last, bool gen, bool o3) {
   const MhDev& S = h->dev;
   if (S.sans_lagrange) return;
   const bool flat = h->sweep_mode == MH_SWEEP_FLAT;
   const bool march = !flat && !o3 && march_sweep(h);  // y / z: threads march over segments of nodes
   if (gen) {
-    if (D == 0) LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
-    else if (D == 1) LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
-    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
+    if (D == 0) LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, M, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
+    else if (D == 1) LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, M, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
+    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, M, MH_LIM_ANY>), h->nblk_n, MH_BLOCK, S, sel, prev, last);
   } else if (D == 0) {
-    if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
-    else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node_row<DIM, LIM>), node_row_blocks(h), MH_BLOCK, S, sel, prev, last));
+    if (flat) MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node<DIM, 0, M, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
+    else MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE, (k_sweep_node_row<DIM, M, LIM>), node_row_blocks(h), MH_BLOCK, S, sel, prev, last));
   } else if (D == 1) {
     if (march)
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node_march<DIM, 1, LIM>), node_march_blocks(h, 1), MH_BLOCK, S, sel, prev, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node_march<DIM, 1, M, LIM>), node_march_blocks(h, 1), MH_BLOCK, S, sel, prev, last));
     else
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 1, (k_sweep_node<DIM, 1, M, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
   } else if constexpr (DIM == 3) {
     if (march)
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node_march<3, 2, LIM>), node_march_blocks(h, 2), MH_BLOCK, S, sel, prev, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node_march<3, 2, M, LIM>), node_march_blocks(h, 2), MH_BLOCK, S, sel, prev, last));
     else
-      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_NODE + 2, (k_sweep_node<3, 2, M, LIM>), h->nblk_n, MH_BLOCK, S, sel, prev, last));
   }
   if (S.dec) {  // conservation-energie-totale: the dual kinetic energy of this sweep
-    if (D == 0) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 0>), h->nblk_n, MH_BLOCK, S, sel, prev);
-    else if (D == 1) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 1>), h->nblk_n, MH_BLOCK, S, sel, prev);
-    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<3, 2>), h->nblk_n, MH_BLOCK, S, sel, prev);
+    if (D == 0) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 0, M>), h->nblk_n, MH_BLOCK, S, sel, prev);
+    else if (D == 1) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<DIM, 1, M>), h->nblk_n, MH_BLOCK, S, sel, prev);
+    else if constexpr (DIM == 3) LAUNCH(h, KN_SWEEP_KE, (k_sweep_ke<3, 2, M>), h->nblk_n, MH_BLOCK, S, sel, prev);
   }
 }
 
@@ -134,7 +134,7 @@ void launch_sweeps_t(MhHandle* h) {
     const int first = s == 0, last = (s == nd - 1) && !first, sel = s & 1;
     const int D = dirs[s];
     launch_cell_part<DIM, M>(h, D, sel, first, gen, o3);
-    launch_dual_part<DIM>(h, D, sel, prev, last, gen, o3);
+    launch_dual_part<DIM, M>(h, D, sel, prev, last, gen, o3);
     prev |= 1 << D;
   }
   if (S.dec && nd == 0) LAUNCH(h, KN_SWEEP_KE, (k_dual_init<DIM>), h->nblk_n, MH_BLOCK, S);
@@ -158,28 +158,28 @@ void ens_sweep(const EnsGroup& g, const MhDev* tab, hipStream_t st, dim3 G, int 
     if (g.gen) {
       hipLaunchKernelGGL((k_sweep_cell_gen_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(dir), sel, first);
       if (!g.adv)
-        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, MH_LIM_ANY>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
+        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, M, MH_LIM_ANY>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     } else {
       hipLaunchKernelGGL((k_sweep_cell3_batch<DIM, D, M>), G, B, 0, st, tab, MH_LIST(dir), sel, first);
       if (!g.adv)
-        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, -1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
+        hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, M, -1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
     }
   } else if (g.rows && D == 0) {
     hipLaunchKernelGGL((k_sweep_cell_row_batch<DIM, M, LIM>), G, B, 0, st, tab, MH_LIST(g.rcmap), sel, first);
     if (!g.adv)
-      hipLaunchKernelGGL((k_sweep_node_row_batch<DIM, LIM>), G, B, 0, st, tab, MH_LIST(g.rnmap), sel, prev, last);
+      hipLaunchKernelGGL((k_sweep_node_row_batch<DIM, M, LIM>), G, B, 0, st, tab, MH_LIST(g.rnmap), sel, prev, last);
   } else if (g.rows) {
     hipLaunchKernelGGL((k_sweep_cell_tile_batch<DIM, D, M, LIM>), G, B, 0, st, tab, MH_LIST(g.tmap[D == 0 ? 0 : D - 1]),
                        sel, first);
     if (!g.adv && !g.o3)  // threads march along D over segments of nodes
-      hipLaunchKernelGGL((k_sweep_node_march_batch<DIM, (D == 0 ? 1 : D), LIM>), G, B, 0, st, tab,
+      hipLaunchKernelGGL((k_sweep_node_march_batch<DIM, (D == 0 ? 1 : D), M, LIM>), G, B, 0, st, tab,
                          MH_LIST(g.mmap[D == 0 ? 0 : D - 1]), sel, prev, last);
     else if (!g.adv)
-      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
+      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, M, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
   } else {
     hipLaunchKernelGGL((k_sweep_cell_batch<DIM, D, M, LIM>), G, B, 0, st, tab, MH_LIST(g.cmap), sel, first);
     if (!g.adv)
-      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
+      hipLaunchKernelGGL((k_sweep_node_batch<DIM, D, M, LIM>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev, last);
   }
 }
 
@@ -207,10 +207,10 @@ void ens_group_cycle_l(MhEnsembleImpl* E, const EnsGroup& g) {
     else if (D == 1) ens_sweep<DIM, 1, M, LIM>(g, tab, st, G, sel, prev, last);
     else if constexpr (DIM == 3) ens_sweep<3, 2, M, LIM>(g, tab, st, G, sel, prev, last);
     if (g.cons) {  // the dual kinetic energy of this sweep
-      if (D == 0) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 0>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
-      else if (D == 1) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 1>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
+      if (D == 0) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 0, M>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
+      else if (D == 1) hipLaunchKernelGGL((k_sweep_ke_batch<DIM, 1, M>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
       else if constexpr (DIM == 3)
-        hipLaunchKernelGGL((k_sweep_ke_batch<3, 2>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
+        hipLaunchKernelGGL((k_sweep_ke_batch<3, 2, M>), G, B, 0, st, tab, MH_LIST(g.nmap), sel, prev);
     }
     prev |= 1 << D;
   }
