@@ -444,6 +444,33 @@ int node_tile_blocks(const MhHandle* h) {
          ((h->g.nnz + h->dev.nt_kc - 1) / h->dev.nt_kc);
 }
 
+// Node planes per block of the z-marching node kernel for one mesh: the depth of 2 to 16 whose blocks
+// finish first when 512 run at a time (two on each of 256 CUs) and each takes one step per plane and
+// one more for the cell plane below it.  Deep blocks repeat fewer planes, shallow ones fill the chip:
+// node kernel with 8 planes / with this depth 38 / 16 us on 24^3, 39 / 31 on 64^3, 71 / 59 on 128x96x64,
+// 79 / 74 on 101^3, 134 / 137 on 128^3, 384 / 361 on 192^3.
+int node_tile_depth(const MhGrid& g) {
+  const long slots = 512;
+  const long tiles = ((g.nnx + MH_NTX - 1L) / MH_NTX) * ((g.nny + MH_NTY - 1) / MH_NTY);
+  int best = MH_NT_KC;
+  long best_steps = -1;
+  for (int kc = 2; kc <= 16; ++kc) {
+    const long full = tiles * (g.nnz / kc), over = full % slots;
+    // `over` slots are free again after the step late, the others after early
+    const long early = full / slots * (kc + 1), late = early + (over ? kc + 1 : 0);
+    long steps = late;
+    if (g.nnz % kc) {  // the last blocks of the columns are shallower: until they fit into the slots
+      const long len = g.nnz % kc + 1;
+      while ((slots - over) * ((steps - early) / len) + over * ((steps - late) / len) < tiles) ++steps;
+    }
+    if (best_steps < 0 || steps <= best_steps) {  // the deeper of two equals
+      best = kc;
+      best_steps = steps;
+    }
+  }
+  return best;
+}
+
 // Launch shapes chosen by the autotuners, per kind of work (process-wide, so that a later
 // case or ensemble of the same kind starts with them).
 std::mutex g_tune_mu;
@@ -467,7 +494,7 @@ void tune_store(const std::string& k, int v) {
 
 // Kernel variants of a single case as one number v = node + 4 cell + 16 sweep, every one of
 // which gives the same bits: node 0 the flat node kernel, 1 / 2 / 3 the z-marching one with 12 /
-// 8 / 16 node planes per block; cell 0 the flat cell kernel, 1 / 2 / 3 the LDS-staged one with
+// the mesh's own (node_tile_depth) / 16 node planes per block; cell 0 the flat cell kernel, 1 / 2 / 3 the LDS-staged one with
 // 12 / 8 / 16 cell planes per block; sweep 0 row segments and tiles, 1 one thread per item.
 const int kTileDepth[4] = {0, 12, 8, 16};
 // target segment lengths of the marching y / z dual sweeps, by variant code bits 5-7
@@ -477,7 +504,7 @@ void set_variant(MhHandle* h, int v) {
   h->nm_len = kMarchLen[mc < 5 ? mc : 0];
   h->dev.nm_len = h->nm_len;
   h->node_tiled = node != 0;
-  if (node) h->nt_kc = kTileDepth[node];
+  if (node) h->nt_kc = node == 2 ? h->nt_auto : kTileDepth[node];
   h->cell_tiled = cell != 0;
   if (cell) h->ct_k = kTileDepth[cell];
   h->sweep_mode = (v >> 4) & 1 ? MH_SWEEP_FLAT : MH_SWEEP_TILE;
@@ -799,6 +826,8 @@ static int create_case(const MhMesh* mesh, const MhEnvironment* envs, int nb_env
     h->node_tiled = nk && strcmp(nk, "flat") == 0    ? false
                     : nk && strcmp(nk, "tiled") == 0 ? true
                                                      : ext_sc || nn >= MH_NODE_TILE_NODES;
+    // (an ensemble's many meshes fill the chip with any depth)
+    if (h->g.dim == 3 && !ext_sc) h->nt_kc = h->nt_auto = node_tile_depth(h->g);
     const char* ck = getenv("MAHYCO_CELL_KERNEL");
     h->cell_tiled = ck && strcmp(ck, "tiled") == 0;
     const char* sw = getenv("MAHYCO_SWEEP");
@@ -1759,7 +1788,7 @@ int mahyco_autotune(MhHandle* h, int cycles, int* variant_out, double* ms_per_cy
   };
   // one coordinate at a time: the sweep variant, then (3D) the node kernel and its tile depth,
   // then the cell kernel and its tile depth, each with the best of the others so far
-  const int dflt = h->g.dim == 3 ? 2 : 0;  // tiled node kernel with 8 planes, flat cell kernel, tiled sweeps
+  const int dflt = h->g.dim == 3 ? 2 : 0;  // tiled node kernel of the mesh's depth, flat cell kernel, tiled sweeps
   for (int sw = 0; sw < 2 && st == MH_OK && !stopped; ++sw) st = timed((dflt & 15) | (sw << 4));
   if (h->g.dim == 3 && h->opt.with_projection) {
     for (int node = 0; node < 4 && st == MH_OK && !stopped; ++node) {

@@ -33,6 +33,34 @@ MH_HD D3 hex_fc3(const D3* x) { return 0.25 * (x[4] + x[5] + x[6] + x[7]); }
 MH_HD D3 hex_fc4(const D3* x) { return 0.25 * (x[1] + x[2] + x[6] + x[5]); }
 MH_HD D3 hex_fc5(const D3* x) { return 0.25 * (x[2] + x[3] + x[7] + x[6]); }
 
+// The same geometry in units that spare the multiplications by 1/4 and 1/2: with the face centre
+// 1/4 s, a difference to it is 1/4 (4 x - s), so hex_arm = 4 x - s is four times cqs_hex's
+// difference (4 x is exact: one rounding, one fma), hex_cross32 = 32 times its half cross product,
+// and the corner sums are scaled back by their last factor, 1/12 / 32.  Scaling by a power of two
+// commutes with every rounding, so the corner vectors have cqs_hex's bits; 12 % fewer operations.
+MH_HD double hex_arm(double x, double s) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_fma(4., x, -s);
+#else
+  return 4. * x - s;
+#endif
+}
+MH_HD D3 hex_arm(D3 x, D3 s) { return d3(hex_arm(x.x, s.x), hex_arm(x.y, s.y), hex_arm(x.z, s.z)); }
+MH_HD D3 hex_cross32(D3 a, D3 b) {
+  return d3(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
+}
+// the four cross products of the face with nodes p0..p3 in the order of its centre sum, of the
+// edges p0p1, p1p2, p2p3, p3p0
+MH_HD void hex_face32(D3 p0, D3 p1, D3 p2, D3 p3, D3& e0, D3& e1, D3& e2, D3& e3) {
+  const D3 s = p0 + p1 + p2 + p3;
+  const D3 a0 = hex_arm(p0, s), a1 = hex_arm(p1, s), a2 = hex_arm(p2, s), a3 = hex_arm(p3, s);
+  e0 = hex_cross32(a0, a1);
+  e1 = hex_cross32(a1, a2);
+  e2 = hex_cross32(a2, a3);
+  e3 = hex_cross32(a3, a0);
+}
+#define MH_HEX_T32 ((1. / 12.) * 0.03125)  // cqs_hex's factor 1/12, over the 32 of the terms
+
 // All eight corner vectors of a hexahedron.
 MH_HD void cqs_hex(const D3* x, D3* q) {
   const D3 c0 = hex_fc0(x), c1 = hex_fc1(x), c2 = hex_fc2(x);
@@ -66,29 +94,23 @@ MH_HD void cqs_hex(const D3* x, D3* q) {
 // six.  Every term and sum is the one of cqs_hex, so each q_l has the same bits.
 template <class F>
 MH_HD void cqs_hex_each(const D3* x, F&& f) {
-  const double t = 1. / 12.;
-  const D3 c0 = hex_fc0(x);
-  const D3 n1a04 = hcross(x[0] - c0, x[3] - c0), n1a03 = hcross(x[3] - c0, x[2] - c0);
-  const D3 n1a02 = hcross(x[2] - c0, x[1] - c0), n1a01 = hcross(x[1] - c0, x[0] - c0);
-  const D3 c1 = hex_fc1(x);
-  const D3 n2a05 = hcross(x[0] - c1, x[4] - c1), n2a12 = hcross(x[4] - c1, x[7] - c1);
-  const D3 n2a08 = hcross(x[7] - c1, x[3] - c1), n2a04 = hcross(x[3] - c1, x[0] - c1);
-  const D3 c2 = hex_fc2(x);
-  const D3 n3a01 = hcross(x[0] - c2, x[1] - c2), n3a06 = hcross(x[1] - c2, x[5] - c2);
-  const D3 n3a09 = hcross(x[5] - c2, x[4] - c2), n3a05 = hcross(x[4] - c2, x[0] - c2);
+  const double t = MH_HEX_T32;
+  D3 n1a04, n1a03, n1a02, n1a01;
+  hex_face32(x[0], x[3], x[2], x[1], n1a04, n1a03, n1a02, n1a01);
+  D3 n2a05, n2a12, n2a08, n2a04;
+  hex_face32(x[0], x[4], x[7], x[3], n2a05, n2a12, n2a08, n2a04);
+  D3 n3a01, n3a06, n3a09, n3a05;
+  hex_face32(x[0], x[1], x[5], x[4], n3a01, n3a06, n3a09, n3a05);
   f(0, t * (5. * (n1a01 + n1a04 + n2a04 + n2a05 + n3a05 + n3a01) + (n1a02 + n1a03 + n2a08 + n2a12 + n3a06 + n3a09)));
-  const D3 c4 = hex_fc4(x);
-  const D3 n5a02 = hcross(x[1] - c4, x[2] - c4), n5a07 = hcross(x[2] - c4, x[6] - c4);
-  const D3 n5a10 = hcross(x[6] - c4, x[5] - c4), n5a06 = hcross(x[5] - c4, x[1] - c4);
+  D3 n5a02, n5a07, n5a10, n5a06;
+  hex_face32(x[1], x[2], x[6], x[5], n5a02, n5a07, n5a10, n5a06);
   f(1, t * (5. * (n1a01 + n1a02 + n3a01 + n3a06 + n5a06 + n5a02) + (n1a04 + n1a03 + n3a09 + n3a05 + n5a10 + n5a07)));
-  const D3 c5 = hex_fc5(x);
-  const D3 n6a03 = hcross(x[2] - c5, x[3] - c5), n6a08 = hcross(x[3] - c5, x[7] - c5);
-  const D3 n6a11 = hcross(x[7] - c5, x[6] - c5), n6a07 = hcross(x[6] - c5, x[2] - c5);
+  D3 n6a03, n6a08, n6a11, n6a07;
+  hex_face32(x[2], x[3], x[7], x[6], n6a03, n6a08, n6a11, n6a07);
   f(2, t * (5. * (n1a02 + n1a03 + n5a07 + n5a02 + n6a07 + n6a03) + (n1a01 + n1a04 + n5a06 + n5a10 + n6a11 + n6a08)));
   f(3, t * (5. * (n1a03 + n1a04 + n2a08 + n2a04 + n6a08 + n6a03) + (n1a01 + n1a02 + n2a05 + n2a12 + n6a07 + n6a11)));
-  const D3 c3 = hex_fc3(x);
-  const D3 n4a09 = hcross(x[4] - c3, x[5] - c3), n4a10 = hcross(x[5] - c3, x[6] - c3);
-  const D3 n4a11 = hcross(x[6] - c3, x[7] - c3), n4a12 = hcross(x[7] - c3, x[4] - c3);
+  D3 n4a09, n4a10, n4a11, n4a12;
+  hex_face32(x[4], x[5], x[6], x[7], n4a09, n4a10, n4a11, n4a12);
   f(4, t * (5. * (n2a05 + n2a12 + n3a05 + n3a09 + n4a09 + n4a12) + (n2a08 + n2a04 + n3a01 + n3a06 + n4a10 + n4a11)));
   f(5, t * (5. * (n3a06 + n3a09 + n4a09 + n4a10 + n5a10 + n5a06) + (n3a01 + n3a05 + n4a12 + n4a11 + n5a07 + n5a02)));
   f(6, t * (5. * (n4a11 + n4a10 + n5a10 + n5a07 + n6a07 + n6a11) + (n4a12 + n4a09 + n5a06 + n5a02 + n6a03 + n6a08)));
@@ -108,36 +130,24 @@ MH_HD D3 cqs_hex_corner(const D3* x) {
   D3 n1a04, n1a03, n1a02, n1a01, n2a05, n2a12, n2a08, n2a04, n3a01, n3a06, n3a09, n3a05;
   D3 n4a09, n4a10, n4a11, n4a12, n5a02, n5a07, n5a10, n5a06, n6a03, n6a08, n6a11, n6a07;
   if (F1) {
-    const D3 c0 = hex_fc0(x);
-    n1a04 = hcross(x[0] - c0, x[3] - c0); n1a03 = hcross(x[3] - c0, x[2] - c0);
-    n1a02 = hcross(x[2] - c0, x[1] - c0); n1a01 = hcross(x[1] - c0, x[0] - c0);
+    hex_face32(x[0], x[3], x[2], x[1], n1a04, n1a03, n1a02, n1a01);
   }
   if (F2) {
-    const D3 c1 = hex_fc1(x);
-    n2a05 = hcross(x[0] - c1, x[4] - c1); n2a12 = hcross(x[4] - c1, x[7] - c1);
-    n2a08 = hcross(x[7] - c1, x[3] - c1); n2a04 = hcross(x[3] - c1, x[0] - c1);
+    hex_face32(x[0], x[4], x[7], x[3], n2a05, n2a12, n2a08, n2a04);
   }
   if (F3) {
-    const D3 c2 = hex_fc2(x);
-    n3a01 = hcross(x[0] - c2, x[1] - c2); n3a06 = hcross(x[1] - c2, x[5] - c2);
-    n3a09 = hcross(x[5] - c2, x[4] - c2); n3a05 = hcross(x[4] - c2, x[0] - c2);
+    hex_face32(x[0], x[1], x[5], x[4], n3a01, n3a06, n3a09, n3a05);
   }
   if (F4) {
-    const D3 c3 = hex_fc3(x);
-    n4a09 = hcross(x[4] - c3, x[5] - c3); n4a10 = hcross(x[5] - c3, x[6] - c3);
-    n4a11 = hcross(x[6] - c3, x[7] - c3); n4a12 = hcross(x[7] - c3, x[4] - c3);
+    hex_face32(x[4], x[5], x[6], x[7], n4a09, n4a10, n4a11, n4a12);
   }
   if (F5) {
-    const D3 c4 = hex_fc4(x);
-    n5a02 = hcross(x[1] - c4, x[2] - c4); n5a07 = hcross(x[2] - c4, x[6] - c4);
-    n5a10 = hcross(x[6] - c4, x[5] - c4); n5a06 = hcross(x[5] - c4, x[1] - c4);
+    hex_face32(x[1], x[2], x[6], x[5], n5a02, n5a07, n5a10, n5a06);
   }
   if (F6) {
-    const D3 c5 = hex_fc5(x);
-    n6a03 = hcross(x[2] - c5, x[3] - c5); n6a08 = hcross(x[3] - c5, x[7] - c5);
-    n6a11 = hcross(x[7] - c5, x[6] - c5); n6a07 = hcross(x[6] - c5, x[2] - c5);
+    hex_face32(x[2], x[3], x[7], x[6], n6a03, n6a08, n6a11, n6a07);
   }
-  const double t = 1. / 12.;
+  const double t = MH_HEX_T32;
   if (L == 0) return t * (5. * (n1a01 + n1a04 + n2a04 + n2a05 + n3a05 + n3a01) + (n1a02 + n1a03 + n2a08 + n2a12 + n3a06 + n3a09));
   if (L == 1) return t * (5. * (n1a01 + n1a02 + n3a01 + n3a06 + n5a06 + n5a02) + (n1a04 + n1a03 + n3a09 + n3a05 + n5a10 + n5a07));
   if (L == 2) return t * (5. * (n1a02 + n1a03 + n5a07 + n5a02 + n6a07 + n6a03) + (n1a01 + n1a04 + n5a06 + n5a10 + n6a11 + n6a08));
@@ -202,18 +212,18 @@ MH_HD void cqs_hex_comp_fm(const D3* x, double* q) {
   constexpr int U = (C + 1) % 3, W = (C + 2) % 3;
   auto cmp = [](const D3& v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : v.z); };
   auto face = [&](int p0, int p1, int p2, int p3, double& e0, double& e1, double& e2, double& e3) {
-    const double cu = 0.25 * (((cmp(x[p0], U) + cmp(x[p1], U)) + cmp(x[p2], U)) + cmp(x[p3], U));
-    const double cw = 0.25 * (((cmp(x[p0], W) + cmp(x[p1], W)) + cmp(x[p2], W)) + cmp(x[p3], W));
-    const double au0 = cmp(x[p0], U) - cu, aw0 = cmp(x[p0], W) - cw;
-    const double au1 = cmp(x[p1], U) - cu, aw1 = cmp(x[p1], W) - cw;
-    const double au2 = cmp(x[p2], U) - cu, aw2 = cmp(x[p2], W) - cw;
-    const double au3 = cmp(x[p3], U) - cu, aw3 = cmp(x[p3], W) - cw;
-    e0 = 0.5 * (au0 * aw1 - aw0 * au1);
-    e1 = 0.5 * (au1 * aw2 - aw1 * au2);
-    e2 = 0.5 * (au2 * aw3 - aw2 * au3);
-    e3 = 0.5 * (au3 * aw0 - aw3 * au0);
+    const double su = ((cmp(x[p0], U) + cmp(x[p1], U)) + cmp(x[p2], U)) + cmp(x[p3], U);
+    const double sw = ((cmp(x[p0], W) + cmp(x[p1], W)) + cmp(x[p2], W)) + cmp(x[p3], W);
+    const double au0 = hex_arm(cmp(x[p0], U), su), aw0 = hex_arm(cmp(x[p0], W), sw);
+    const double au1 = hex_arm(cmp(x[p1], U), su), aw1 = hex_arm(cmp(x[p1], W), sw);
+    const double au2 = hex_arm(cmp(x[p2], U), su), aw2 = hex_arm(cmp(x[p2], W), sw);
+    const double au3 = hex_arm(cmp(x[p3], U), su), aw3 = hex_arm(cmp(x[p3], W), sw);
+    e0 = au0 * aw1 - aw0 * au1;
+    e1 = au1 * aw2 - aw1 * au2;
+    e2 = au2 * aw3 - aw2 * au3;
+    e3 = au3 * aw0 - aw3 * au0;
   };
-  const double t = 1. / 12.;
+  const double t = MH_HEX_T32;
   double A[8], B[8];  // the 5 x part and the 1 x part of each corner sum
   double a, b, c, d;
   face(0, 3, 2, 1, a, b, c, d);  // n1a04, n1a03, n1a02, n1a01
@@ -256,20 +266,56 @@ MH_HD void cqs_hex_comp_fm(const D3* x, double* q) {
   q[7] = t * (5. * A[7] + B[7]);
 }
 
-// Volume of a hexahedron, sum_l x_l . CQS_l / 3 (MahycoModule.cc:1149-1162), one corner-vector
-// component at a time: dot3 rounds (x.x q.x + x.y q.y) + x.z q.z, so the products of the x and
-// y passes are summed before the z pass, and the corner terms are added in corner order.  Same
-// bits as cell_volume<8>(x, q) after cqs_hex(x, q).
-MH_HD double hex_volume_lowreg(const D3* x) {
-  double q[8], d[8];
-  cqs_hex_comp<0>(x, q);
-  for (int l = 0; l < 8; ++l) d[l] = x[l].x * q[l];
-  cqs_hex_comp<1>(x, q);
-  for (int l = 0; l < 8; ++l) d[l] = d[l] + x[l].y * q[l];
-  cqs_hex_comp<2>(x, q);
+// Volume of a hexahedron, sum_l x_l . CQS_l / 3 (MahycoModule.cc:1149-1162), with the corner sums
+// accumulated face by face as in cqs_hex_comp_fm, all components together: each face's centre and
+// arms are formed once, and a corner's sums die with its last face.  Same bits as
+// cell_volume<8>(x, q) after cqs_hex(x, q).  The division by 3 is taken by its reciprocal.
+MH_HD double hex_volume(const D3* x) {
+  const double t = MH_HEX_T32;
+  D3 A[8], B[8];  // the 5 x part and the 1 x part of each corner sum
+  D3 a, b, c, d;
+  double e[8];
+  hex_face32(x[0], x[3], x[2], x[1], a, b, c, d);  // n1a04, n1a03, n1a02, n1a01
+  A[0] = d + a; B[0] = c + b;
+  A[1] = d + c; B[1] = a + b;
+  A[2] = c + b; B[2] = d + a;
+  A[3] = b + a; B[3] = d + c;
+  hex_face32(x[0], x[4], x[7], x[3], a, b, c, d);  // n2a05, n2a12, n2a08, n2a04
+  A[0] = (A[0] + d) + a; B[0] = (B[0] + c) + b;
+  A[3] = (A[3] + c) + d; B[3] = (B[3] + a) + b;
+  A[4] = a + b; B[4] = c + d;
+  A[7] = c + b; B[7] = d + a;
+  hex_face32(x[0], x[1], x[5], x[4], a, b, c, d);  // n3a01, n3a06, n3a09, n3a05
+  A[0] = (A[0] + d) + a; B[0] = (B[0] + b) + c;
+  A[1] = (A[1] + a) + b; B[1] = (B[1] + c) + d;
+  A[4] = (A[4] + d) + c; B[4] = (B[4] + a) + b;
+  A[5] = b + c; B[5] = a + d;
+  e[0] = dot3(x[0], t * (5. * A[0] + B[0]));
+  hex_face32(x[4], x[5], x[6], x[7], a, b, c, d);  // n4a09, n4a10, n4a11, n4a12
+  A[4] = (A[4] + a) + d; B[4] = (B[4] + b) + c;
+  A[5] = (A[5] + a) + b; B[5] = (B[5] + d) + c;
+  A[6] = c + b; B[6] = d + a;
+  A[7] = (A[7] + d) + c; B[7] = (B[7] + a) + b;
+  e[4] = dot3(x[4], t * (5. * A[4] + B[4]));
+  hex_face32(x[1], x[2], x[6], x[5], a, b, c, d);  // n5a02, n5a07, n5a10, n5a06
+  A[1] = (A[1] + d) + a; B[1] = (B[1] + c) + b;
+  A[2] = (A[2] + b) + a; B[2] = (B[2] + d) + c;
+  A[5] = (A[5] + c) + d; B[5] = (B[5] + b) + a;
+  A[6] = (A[6] + c) + b; B[6] = (B[6] + d) + a;
+  e[1] = dot3(x[1], t * (5. * A[1] + B[1]));
+  e[5] = dot3(x[5], t * (5. * A[5] + B[5]));
+  hex_face32(x[2], x[3], x[7], x[6], a, b, c, d);  // n6a03, n6a08, n6a11, n6a07
+  A[2] = (A[2] + d) + a; B[2] = (B[2] + c) + b;
+  A[3] = (A[3] + b) + a; B[3] = (B[3] + d) + c;
+  A[6] = (A[6] + d) + c; B[6] = (B[6] + a) + b;
+  A[7] = (A[7] + c) + b; B[7] = (B[7] + d) + a;
+  e[2] = dot3(x[2], t * (5. * A[2] + B[2]));
+  e[3] = dot3(x[3], t * (5. * A[3] + B[3]));
+  e[6] = dot3(x[6], t * (5. * A[6] + B[6]));
+  e[7] = dot3(x[7], t * (5. * A[7] + B[7]));
   double v = 0.;
-  for (int l = 0; l < 8; ++l) v += d[l] + x[l].z * q[l];
-  return v / 3;
+  for (int l = 0; l < 8; ++l) v += e[l];
+  return mh_quot(v, MhRecip{3., 1. / 3., false});
 }
 
 // Quadrangle corner vectors: half edge normals of the two edges at each corner

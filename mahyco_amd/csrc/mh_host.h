@@ -46,9 +46,10 @@ enum { MH_SWEEP_FLAT = 0, MH_SWEEP_TILE = 1 };
 #define MH_MARCH_NODES 600000L
 // ... and 10-node segments from here on (2.1 M nodes: 94 us with 4, 87 with 10; 1.05 M: 31 / 40)
 #define MH_MARCH_LONG_NODES 1600000L
-// 3D node kernel: one thread per node below, z-marching tiles above.  Tiles (8 planes) against one
-// per node: 39 / 14 us on 16^3, 41 / 35 on 64^3, 54 / 54 on 80^3, 87 / 95 on 101^3.
-#define MH_NODE_TILE_NODES 600000L
+// 3D node kernel: the cells of a node over four wavefronts below, z-marching tiles above.  Tiles (of the
+// mesh's depth) against wavefronts: 16 / 9.3 us on 24^3, 22 / 21 on 50^3, 31 / 34 on 64^3, 41 / 54 on
+// 97x61x83, 138 / 226 on 128^3.
+#define MH_NODE_TILE_NODES 200000L
 
 struct ProfRec {
   int kind;
@@ -82,11 +83,12 @@ struct MhHandle {
   std::vector<hipGraph_t> graph_defs;
   long graph_captures = 0;  // graphs captured and instantiated so far
   bool owns_stream = true;
-  bool node_tiled = true;   // 3D: z-marching node kernel (MAHYCO_NODE_KERNEL=flat selects the flat one)
+  bool node_tiled = true;   // 3D: z-marching node kernel (MAHYCO_NODE_KERNEL=flat: k_node_lag3_split)
   bool cell_tiled = false;  // 3D remap loop: LDS-staged cell kernel (MAHYCO_CELL_KERNEL=tiled; an autotuner candidate)
   bool staged = false;      // Lagrangian state written before the remap, U formed from it (mahyco_set_staged)
   int nm_len = MH_NM_L;     // target segment length of the marching dual sweeps (MAHYCO_MARCH_LEN)
   int nt_kc = MH_NT_KC;     // node planes per block of the tiled node kernel
+  int nt_auto = MH_NT_KC;   // the depth node_tile_depth gives the mesh
   int ct_k = MH_CT_K;       // cell planes per block of the tiled cell kernel
   int sweep_mode = MH_SWEEP_TILE;  // MAHYCO_SWEEP=flat selects one thread per cell / node
   bool sweep_large = false;        // MAHYCO_SWEEP=tile: the large-mesh sweeps at every size

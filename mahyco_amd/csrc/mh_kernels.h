@@ -20,6 +20,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mh_geom.h"
 #include "mh_state.h"
 
@@ -146,56 +148,113 @@ __device__ __forceinline__ void block_min_store(double v, bool active, double* o
 }
 
 // ----------------------------------------------------------------------------- nodes
-// Corner L of cell (ii,jj,kk) seen from node (i,j,k); accumulates mass and force in the
-// order of a cell-order scatter (MahycoModule.cc:247-262 and :455-462).
+// Node mass and corner forces of node (i,j,k) over its cells, in the order of a cell-order scatter
+// (MahycoModule.cc:247-262 and :455-462).
 // FWD: the corner vectors at this cycle's Lagrangian positions (updateVelocityForward,
 // :638-690) instead of the previous cycle's.
-template <int DIM, int DI, int DJ, int DK, int FWD = 0>
-__device__ __forceinline__ void node_gather(const MhDev& S, int i, int j, int k, double& mass,
-                                            double& fx, double& fy, double& fz) {
-  double* const* X = FWD ? S.xlc : S.xlp;
-  const int ii = i - DI, jj = j - DJ, kk = k - DK;
-  if (ii < 0 || ii >= S.g.nx || jj < 0 || jj >= S.g.ny) return;
-  if (DIM == 3 && (kk < 0 || kk >= S.g.nz)) return;
-  const long c = ii + (long)S.g.nx * (jj + (long)S.g.ny * kk);
-  const double w = DIM == 3 ? 0.125 : 0.25;
-  mass += w * S.M[c];
-  const double pr = S.p[c] + S.q[c];
-  const long nnx = S.g.nnx, nnxy = (long)S.g.nnx * S.g.nny;
-  const long b = ii + nnx * (jj + (long)S.g.nny * kk);
-  constexpr int L = 4 * DK + (DJ ? (DI ? 2 : 3) : (DI ? 1 : 0));
-  D3 q;
-  if (DIM == 3) {
-    D3 x[8];
-    x[0] = load3(X, b);
-    x[1] = load3(X, b + 1);
-    x[2] = load3(X, b + 1 + nnx);
-    x[3] = load3(X, b + nnx);
-    x[4] = load3(X, b + nnxy);
-    x[5] = load3(X, b + 1 + nnxy);
-    x[6] = load3(X, b + 1 + nnx + nnxy);
-    x[7] = load3(X, b + nnx + nnxy);
-    q = cqs_hex_corner<L>(x);
+// The 3x3(x3) nodes around are read once each; indices past the mesh are clamped and the terms of a
+// cell outside it are dropped by a select, so no branch parts the loads: they are all in flight
+// together (3D: those of one cell plane), where a branch per cell waited for each cell in turn: 28.5 ->
+// 26 us on 1023x1021, 6.2 -> 5.4 us on 200x10, 146 -> 128 us for 64 meshes of 64^2 to 512^2.
+template <int DIM, int A, int B, int DZ>  // this node's corner vector of cell (A,B,DZ) around it
+__device__ __forceinline__ D3 node_corner(const D3 (*lo)[3], const D3 (*hi)[3]) {
+  constexpr int L = 4 * (1 - DZ) + (B ? (A ? 0 : 1) : (A ? 3 : 2));
+  if constexpr (DIM == 3) {
+    const D3 x[8] = {lo[B][A], lo[B][A + 1], lo[B + 1][A + 1], lo[B + 1][A],
+                     hi[B][A], hi[B][A + 1], hi[B + 1][A + 1], hi[B + 1][A]};
+    return cqs_hex_corner<L>(x);
   } else {
-    D3 x[4];
-    x[0] = d3(X[0][b], X[1][b], 0.);
-    x[1] = d3(X[0][b + 1], X[1][b + 1], 0.);
-    x[2] = d3(X[0][b + 1 + nnx], X[1][b + 1 + nnx], 0.);
-    x[3] = d3(X[0][b + nnx], X[1][b + nnx], 0.);
-    q = cqs_quad_corner<L & 3>(x);
+    const D3 x[4] = {lo[B][A], lo[B][A + 1], lo[B + 1][A + 1], lo[B + 1][A]};
+    return cqs_quad_corner<L & 3>(x);
   }
-  fx += pr * q.x;
-  fy += pr * q.y;
-  if (DIM == 3) fz += pr * q.z;
+}
+template <int DIM, int A, int B, int DZ>
+__device__ __forceinline__ void node_add(const D3 (*lo)[3], const D3 (*hi)[3], double M, double p, double q, bool ok,
+                                         double& mass, double& fx, double& fy, double& fz) {
+  const D3 v = node_corner<DIM, A, B, DZ>(lo, hi);
+  const double pr = p + q;
+  mass = ok ? mass + (DIM == 3 ? 0.125 : 0.25) * M : mass;
+  fx = ok ? fx + pr * v.x : fx;
+  fy = ok ? fy + pr * v.y : fy;
+  if (DIM == 3) fz = ok ? fz + pr * v.z : fz;
+}
+template <int DIM, int FWD = 0>
+__device__ __forceinline__ void node_gather(const MhDev& S, int i, int j, int k, double& mass, double& fx, double& fy,
+                                            double& fz) {
+  double* const* X = FWD ? S.xlc : S.xlp;
+  const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
+  const long nnx = S.g.nnx, nny = S.g.nny;
+  const int ni[3] = {max(i - 1, 0), i, min(i + 1, nx)}, nj[3] = {max(j - 1, 0), j, min(j + 1, ny)};
+  const int ci[2] = {max(i - 1, 0), min(i, nx - 1)}, cj[2] = {max(j - 1, 0), min(j, ny - 1)};
+  const bool oi[2] = {i > 0, i < nx}, oj[2] = {j > 0, j < ny};
+  D3 lo[3][3], hi[3][3];
+  auto plane = [&](D3 (*P)[3], int kz) {
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const long n = ni[a] + nnx * (nj[b] + nny * kz);
+        P[b][a] = d3(X[0][n], X[1][n], DIM == 3 ? X[2][n] : 0.);
+      }
+  };
+  // the four cells of cell plane kc, as members of the mesh where ok
+  auto cells = [&](auto dz, int kc, bool ok) {
+    constexpr int DZ = decltype(dz)::value;
+    double M[4], p[4], q[4];
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+      const long c = ci[l & 1] + (long)nx * (cj[l >> 1] + (long)ny * kc);
+      M[l] = S.M[c];
+      p[l] = S.p[c];
+      q[l] = S.q[c];
+    }
+    node_add<DIM, 0, 0, DZ>(lo, hi, M[0], p[0], q[0], ok && oi[0] && oj[0], mass, fx, fy, fz);
+    node_add<DIM, 1, 0, DZ>(lo, hi, M[1], p[1], q[1], ok && oi[1] && oj[0], mass, fx, fy, fz);
+    node_add<DIM, 0, 1, DZ>(lo, hi, M[2], p[2], q[2], ok && oi[0] && oj[1], mass, fx, fy, fz);
+    node_add<DIM, 1, 1, DZ>(lo, hi, M[3], p[3], q[3], ok && oi[1] && oj[1], mass, fx, fy, fz);
+  };
+  if constexpr (DIM == 3) {
+    plane(lo, max(k - 1, 0));
+    plane(hi, k);
+    cells(std::integral_constant<int, 0>{}, max(k - 1, 0), k > 0);
+    asm volatile("" ::: "memory");  // the next plane's loads would take the registers of this one's corners
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) lo[b][a] = hi[b][a];
+    plane(hi, min(k + 1, nz));
+    cells(std::integral_constant<int, 1>{}, min(k, nz - 1), k < nz);
+  } else {
+    plane(lo, 0);
+    cells(std::integral_constant<int, 1>{}, 0, true);
+  }
 }
 
 // UpdateVelocity tail (u += dt_half / m F), ApplyBoundaryCondition (Vx/Vy/Vz on the
 // XMIN..ZMAX node groups, in option order) and UpdatePosition (x += dt u) for node n.
+// The node's own state, u and the position the step starts from (the Eulerian one with remap), is
+// loaded by the caller ahead of the forces.
+struct NodePre {
+  double u[3], x[3];
+};
 template <int DIM>
-__device__ __forceinline__ void node_finish(const MhDev& S, long n, int i, int j, int k, double dt,
-                                            double dth, double mass, double fx, double fy, double fz) {
+__device__ __forceinline__ void node_pre_load(const MhDev& S, long n, int i, int j, int k, NodePre& pre) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) pre.u[d] = d < DIM ? S.u[d][n] : 0.;
+  if (S.with_proj) {
+    pre.x[0] = S.ax[i];
+    pre.x[1] = S.ay[j];
+    pre.x[2] = DIM == 3 ? S.az[k] : 0.;
+  } else {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) pre.x[d] = d < DIM ? S.xlp[d][n] : 0.;
+  }
+}
+template <int DIM>
+__device__ __forceinline__ void node_finish(const MhDev& S, long n, int i, int j, int k, double dt, double dth,
+                                            const NodePre& pre, double mass, double fx, double fy, double fz) {
   const double s = dth / mass;
-  double ux = S.u[0][n], uy = S.u[1][n], uz = DIM == 3 ? S.u[2][n] : 0.;
+  double ux = pre.u[0], uy = pre.u[1], uz = pre.u[2];
   if (S.csts) {  // SaveValuesAtN of the velocity
     S.un[0][n] = ux;
     S.un[1][n] = uy;
@@ -228,23 +287,13 @@ __device__ __forceinline__ void node_finish(const MhDev& S, long n, int i, int j
       else if (DIM == 3) uz = S.bc_val[b];
     }
   }
-  double x0, y0, z0;
-  if (S.with_proj) {
-    x0 = S.ax[i];
-    y0 = S.ay[j];
-    z0 = DIM == 3 ? S.az[k] : 0.;
-  } else {
-    x0 = S.xlp[0][n];
-    y0 = S.xlp[1][n];
-    z0 = DIM == 3 ? S.xlp[2][n] : 0.;
-  }
   S.u[0][n] = ux;
   S.u[1][n] = uy;
-  S.xlc[0][n] = x0 + dt * ux;
-  S.xlc[1][n] = y0 + dt * uy;
+  S.xlc[0][n] = pre.x[0] + dt * ux;
+  S.xlc[1][n] = pre.x[1] + dt * uy;
   if (DIM == 3) {
     S.u[2][n] = uz;
-    S.xlc[2][n] = z0 + dt * uz;
+    S.xlc[2][n] = pre.x[2] + dt * uz;
   }
   S.mn[n] = mass;
 }
@@ -256,7 +305,7 @@ template <int DIM>
 __device__ __forceinline__ void k_node_lag_body(const MhDev& S, int lb) {
   const long n = lb * (long)blockDim.x + threadIdx.x;
   if (n >= S.g.nn) return;
-  if (mh_halted(S.sc)) return;
+  const bool halted = mh_halted(S.sc);
   const int nnx = S.g.nnx, nny = S.g.nny;
   const int i = (int)(n % nnx);
   const long r = n / nnx;
@@ -264,20 +313,96 @@ __device__ __forceinline__ void k_node_lag_body(const MhDev& S, int lb) {
   const int k = (int)(r / nny);
   const double dt = S.sc->dt;
   const double dth = 0.5 * (S.sc->dt_old + dt);
+  NodePre pre;
+  node_pre_load<DIM>(S, n, i, j, k, pre);
   double mass = 0., fx = 0., fy = 0., fz = 0.;
-  if (DIM == 3) {
-    node_gather<3, 1, 1, 1>(S, i, j, k, mass, fx, fy, fz);
-    node_gather<3, 0, 1, 1>(S, i, j, k, mass, fx, fy, fz);
-    node_gather<3, 1, 0, 1>(S, i, j, k, mass, fx, fy, fz);
-    node_gather<3, 0, 0, 1>(S, i, j, k, mass, fx, fy, fz);
-  }
-  node_gather<DIM, 1, 1, 0>(S, i, j, k, mass, fx, fy, fz);
-  node_gather<DIM, 0, 1, 0>(S, i, j, k, mass, fx, fy, fz);
-  node_gather<DIM, 1, 0, 0>(S, i, j, k, mass, fx, fy, fz);
-  node_gather<DIM, 0, 0, 0>(S, i, j, k, mass, fx, fy, fz);
-  node_finish<DIM>(S, n, i, j, k, dt, dth, mass, fx, fy, fz);
+  node_gather<DIM>(S, i, j, k, mass, fx, fy, fz);
+  if (halted) return;
+  node_finish<DIM>(S, n, i, j, k, dt, dth, pre, mass, fx, fy, fz);
 }
 
+
+// The same in 3D with the cells shared out over the wavefronts: a block owns 64 nodes, each of its
+// four wavefronts the two cells (one below, one above) of one quadrant around them, and the first
+// one adds the eight terms from LDS in cell order.  A thread of the kernel above forms eight corner
+// vectors of some 200 operations each one after the other, and waits for its two cell planes in
+// turn; a mesh of a few hundred wavefronts has the processors free to do that at once: 12.6 -> 7.2 us
+// on 100x5x5, one thread per node against this.
+template <int A, int B>
+__device__ __forceinline__ void node_quadrant(const MhDev& S, int i, int j, int k, double* out) {
+  const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
+  const long nnx = S.g.nnx, nny = S.g.nny;
+  const int ni[2] = {A ? i : max(i - 1, 0), A ? min(i + 1, nx) : i}, nj[2] = {B ? j : max(j - 1, 0), B ? min(j + 1, ny) : j};
+  const int nk[3] = {max(k - 1, 0), k, min(k + 1, nz)};
+  D3 P[3][3][3];  // rows and columns A, A + 1 of the 3x3 neighbourhood are used
+#pragma unroll
+  for (int z = 0; z < 3; ++z)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int a = 0; a < 2; ++a) P[z][B + b][A + a] = load3(S.xlp, ni[a] + nnx * (nj[b] + nny * nk[z]));
+  const int ci = A ? min(i, nx - 1) : max(i - 1, 0), cj = B ? min(j, ny - 1) : max(j - 1, 0);
+  double M[2], p[2], q[2];
+#pragma unroll
+  for (int z = 0; z < 2; ++z) {
+    const long c = ci + (long)nx * (cj + (long)ny * (z ? min(k, nz - 1) : max(k - 1, 0)));
+    M[z] = S.M[c];
+    p[z] = S.p[c];
+    q[z] = S.q[c];
+  }
+  auto corner = [&](auto dz) {
+    constexpr int DZ = decltype(dz)::value;
+    const D3 v = node_corner<3, A, B, DZ>(P[DZ], P[DZ + 1]);
+    const double pr = p[DZ] + q[DZ];
+    double* o = out + DZ * (4 * 4 * 64);
+    o[0] = 0.125 * M[DZ];
+    o[64] = pr * v.x;
+    o[128] = pr * v.y;
+    o[192] = pr * v.z;
+  };
+  corner(std::integral_constant<int, 0>{});
+  corner(std::integral_constant<int, 1>{});
+}
+__device__ __forceinline__ void k_node_lag3_split_body(const MhDev& S, int lb) {
+  static_assert(MH_BLOCK == 256, "one wavefront per quadrant");
+  __shared__ double part[2][4][4][64];  // cells below / above, quadrant, (mass, force), node
+  const bool halted = mh_halted(S.sc);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long n = min(lb * 64L + lane, S.g.nn - 1);
+  const int nnx = S.g.nnx, nny = S.g.nny;
+  const int i = (int)(n % nnx);
+  const long r = n / nnx;
+  const int j = (int)(r % nny);
+  const int k = (int)(r / nny);
+  const double dt = S.sc->dt;
+  const double dth = 0.5 * (S.sc->dt_old + dt);
+  NodePre pre;
+  if (w == 0) {
+    node_pre_load<3>(S, n, i, j, k, pre);
+    node_quadrant<0, 0>(S, i, j, k, &part[0][0][0][lane]);
+  } else if (w == 1) {
+    node_quadrant<1, 0>(S, i, j, k, &part[0][1][0][lane]);
+  } else if (w == 2) {
+    node_quadrant<0, 1>(S, i, j, k, &part[0][2][0][lane]);
+  } else {
+    node_quadrant<1, 1>(S, i, j, k, &part[0][3][0][lane]);
+  }
+  __syncthreads();
+  if (w || halted || lb * 64L + lane >= S.g.nn) return;
+  double sum[4] = {0., 0., 0., 0.};
+  const bool okz[2] = {k > 0, k < S.g.nz};
+  const bool okq[4] = {i > 0 && j > 0, i < S.g.nx && j > 0, i > 0 && j < S.g.ny, i < S.g.nx && j < S.g.ny};
+#pragma unroll
+  for (int z = 0; z < 2; ++z)
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const double t = sum[v] + part[z][l][v][lane];
+        sum[v] = okz[z] && okq[l] ? t : sum[v];
+      }
+  node_finish<3>(S, n, i, j, k, dt, dth, pre, sum[0], sum[1], sum[2], sum[3]);
+}
 
 // updateVelocityForward (:638-690), before a CSTS remap: u += (dt/2) / m F with the force of
 // this cycle's pressure array, pseudo-viscosity and corner vectors (no boundary condition).
@@ -292,16 +417,7 @@ __device__ __forceinline__ void k_node_fwd_body(const MhDev& S, int lb) {
   const int j = (int)(r % nny);
   const int k = (int)(r / nny);
   double mass = 0., fx = 0., fy = 0., fz = 0.;
-  if (DIM == 3) {
-    node_gather<3, 1, 1, 1, 1>(S, i, j, k, mass, fx, fy, fz);
-    node_gather<3, 0, 1, 1, 1>(S, i, j, k, mass, fx, fy, fz);
-    node_gather<3, 1, 0, 1, 1>(S, i, j, k, mass, fx, fy, fz);
-    node_gather<3, 0, 0, 1, 1>(S, i, j, k, mass, fx, fy, fz);
-  }
-  node_gather<DIM, 1, 1, 0, 1>(S, i, j, k, mass, fx, fy, fz);
-  node_gather<DIM, 0, 1, 0, 1>(S, i, j, k, mass, fx, fy, fz);
-  node_gather<DIM, 1, 0, 0, 1>(S, i, j, k, mass, fx, fy, fz);
-  node_gather<DIM, 0, 0, 0, 1>(S, i, j, k, mass, fx, fy, fz);
+  node_gather<DIM, 1>(S, i, j, k, mass, fx, fy, fz);
   const double s = (0.5 * S.sc->dt) / S.mn[n];
   S.u[0][n] = S.u[0][n] + s * fx;
   S.u[1][n] = S.u[1][n] + s * fy;
@@ -356,14 +472,17 @@ __device__ __forceinline__ void k_node_adv_body(const MhDev& S, int lb) {
   if (DIM == 2) S.u[2][n] = u[2];
 }
 
-// 3D node kernel, z-marching tiles: a block owns MH_NTX x MH_NTY node columns over
-// MH_NT_KC node planes, so each cell plane of the tile is (MH_NTX+1) x (MH_NTY+1) = 256
-// cells, one per thread.  Each cell plane
-// is processed once: its corner vectors (cqs_hex, computed once per cell instead of once
-// per corner) are multiplied by p+q and kept in LDS with M/8 -- the bottom corners for
-// the node plane it sits on, the top ones (held in registers meanwhile) for the next
-// plane.  Every node then adds its 8 cells in cell order, as k_node_lag does, so both
+// 3D node kernel, z-marching tiles: a block owns MH_NTX x MH_NTY node columns over MhDev::nt_kc node
+// planes, so each cell plane of the tile is (MH_NTX+1) x (MH_NTY+1) = 256 cells, one per thread.  Each
+// cell plane is processed once: its corner vectors (cqs_hex, computed once per cell instead of once
+// per corner) are multiplied by p+q and go to LDS with M/8.  The node threads then finish node plane k
+// with the bottom corners, on top of the sums they hold of the cells below, and start the sums of
+// plane k + 1 with the top corners: the 8 cells are added in cell order, as in k_node_lag, so both
 // kernels give the same bits.
+// Bound by FP64 issue, at two wavefronts per SIMD (the corner vectors take 240 registers), 60 % busy:
+// so the geometry is formed in the units of hex_face32, and all that a plane reads (the next cell, the
+// node's own velocity) is in flight before the corner vectors are formed.  267 -> 234 us on
+// 256x128x128, 433 -> 361 us on 192^3, with node_tile_depth 79 -> 59 us on 128x96x64.
 #ifndef MH_NTX
 #define MH_NTX 31  // node columns of a tile along x
 #endif
@@ -392,48 +511,37 @@ __device__ __forceinline__ void nt_load_cell(const MhDev& S, int ii, int jj, int
   in.q = S.q[c];
   in.M = S.M[c];
 }
-// corner force contributions (p + q) CQS_l and the node-mass share M/8 of one cell: lower
-// corners to LDS slot s, upper corners to keep
-__device__ __forceinline__ void nt_cell(const D3* bot, const NtCellIn& in, double* lds, int s, double* keep) {
-  D3 x[8];
-  x[0] = bot[0];
-  x[1] = bot[1];
-  x[2] = bot[2];
-  x[3] = bot[3];
-  x[4] = in.top[0];
-  x[5] = in.top[1];
-  x[6] = in.top[2];
-  x[7] = in.top[3];
+// corner force contributions (p + q) CQS_l and the node-mass share M/8 of one cell to slot s: lower
+// corners to up, upper corners to lo
+__device__ __forceinline__ void nt_cell(const D3* bot, const NtCellIn& in, double* up, double* lo, int s) {
+  const D3 x[8] = {bot[0], bot[1], bot[2], bot[3], in.top[0], in.top[1], in.top[2], in.top[3]};
   const double pr = in.p + in.q;
   const double wm = 0.125 * in.M;
   cqs_hex_each(x, [&](int l, const D3& q) {
-    if (l < 4) {
-      lds[(3 * l + 0) * MH_NT_CELLS + s] = pr * q.x;
-      lds[(3 * l + 1) * MH_NT_CELLS + s] = pr * q.y;
-      lds[(3 * l + 2) * MH_NT_CELLS + s] = pr * q.z;
-    } else {
-      keep[3 * (l - 4) + 0] = pr * q.x;
-      keep[3 * (l - 4) + 1] = pr * q.y;
-      keep[3 * (l - 4) + 2] = pr * q.z;
-    }
+    double* P = l < 4 ? up : lo;
+    P[(3 * (l & 3) + 0) * MH_NT_CELLS + s] = pr * q.x;
+    P[(3 * (l & 3) + 1) * MH_NT_CELLS + s] = pr * q.y;
+    P[(3 * (l & 3) + 2) * MH_NT_CELLS + s] = pr * q.z;
   });
-  lds[12 * MH_NT_CELLS + s] = wm;
-  keep[12] = wm;
+  up[12 * MH_NT_CELLS + s] = wm;
 }
 
-__device__ __forceinline__ void nt_add(const double* P, int s, int corner, bool ok, double& mass, double& fx,
-                                       double& fy, double& fz) {
-  if (!ok) return;
-  mass += P[12 * MH_NT_CELLS + s];
-  fx += P[(3 * corner + 0) * MH_NT_CELLS + s];
-  fy += P[(3 * corner + 1) * MH_NT_CELLS + s];
-  fz += P[(3 * corner + 2) * MH_NT_CELLS + s];
+__device__ __forceinline__ void nt_add(const double* P, const double* W, int s, int corner, bool ok, double& mass,
+                                       double& fx, double& fy, double& fz) {
+  const double m = mass + W[12 * MH_NT_CELLS + s];
+  const double x = fx + P[(3 * corner + 0) * MH_NT_CELLS + s];
+  const double y = fy + P[(3 * corner + 1) * MH_NT_CELLS + s];
+  const double z = fz + P[(3 * corner + 2) * MH_NT_CELLS + s];
+  mass = ok ? m : mass;
+  fx = ok ? x : fx;
+  fy = ok ? y : fy;
+  fz = ok ? z : fz;
 }
 
 __device__ __forceinline__ void k_node_lag3_tiled_body(const MhDev& S, int bx, int by, int bz) {
   static_assert(MH_NT_CELLS == MH_BLOCK, "one cell of the tile plane per thread");
-  __shared__ double lo[13 * MH_NT_CELLS];  // top corners (4..7) of the cell plane below
-  __shared__ double up[13 * MH_NT_CELLS];  // bottom corners (0..3) of the cell plane above
+  __shared__ double up[13 * MH_NT_CELLS];  // bottom corners (0..3) and M/8 of the cell plane
+  __shared__ double lo[12 * MH_NT_CELLS];  // its top corners (4..7)
   if (mh_halted(S.sc)) return;
   const int tid = threadIdx.x;
   const int i0 = bx * MH_NTX, j0 = by * MH_NTY, k0 = bz * S.nt_kc;
@@ -441,114 +549,70 @@ __device__ __forceinline__ void k_node_lag3_tiled_body(const MhDev& S, int bx, i
   const int kend = min(k0 + S.nt_kc, S.g.nnz);
   const double dt = S.sc->dt;
   const double dth = 0.5 * (S.sc->dt_old + dt);
-  // this thread's cell column of the tile
-  const int ci = i0 - 1 + tid % (MH_NTX + 1), cj = j0 - 1 + tid / (MH_NTX + 1);
-  const bool cell_ok = ci >= 0 && ci < nx && cj >= 0 && cj < ny;
-  double keep[13];
-  // the thread's cell column: lower face carried from plane to plane, the next cell's
-  // loads issued one plane ahead
+  // this thread's cell column of the tile; a column outside the mesh reads the nearest one inside
+  const int ci = min(max(i0 - 1 + tid % (MH_NTX + 1), 0), nx - 1);
+  const int cj = min(max(j0 - 1 + tid / (MH_NTX + 1), 0), ny - 1);
+  // this thread's node column (threads below MH_NTX * MH_NTY)
+  const int tx = tid % MH_NTX, ty = tid / MH_NTX;
+  const int i = i0 + tx, j = j0 + ty;
+  const bool node_ok = tid < MH_NTX * MH_NTY && i < S.g.nnx && j < S.g.nny;
+  const int s00 = min(ty * (MH_NTX + 1) + tx, MH_NT_CELLS - MH_NTX - 3);  // cell (i-1, j-1)
+  const int in = min(i, nx), jn = min(j, ny);
+  const long n0 = in + (long)S.g.nnx * jn, nplane = (long)S.g.nnx * S.g.nny;
+  const bool okx0 = i >= 1, okx1 = i < nx, oky0 = j >= 1, oky1 = j < ny;
+  auto add4 = [&](const double* P, double& mass, double& fx, double& fy, double& fz) {
+    nt_add(P, up, s00, 2, okx0 && oky0, mass, fx, fy, fz);
+    nt_add(P, up, s00 + 1, 3, okx1 && oky0, mass, fx, fy, fz);
+    nt_add(P, up, s00 + MH_NTX + 1, 1, okx0 && oky1, mass, fx, fy, fz);
+    nt_add(P, up, s00 + MH_NTX + 2, 0, okx1 && oky1, mass, fx, fy, fz);
+  };
+  // the lower face of the thread's cell is carried from plane to plane; the next cell's loads and
+  // the loads of the node's own state go out one plane ahead
   D3 bot[4];
   NtCellIn cur, nxt;
-  const int kc_end = min(kend, nz);  // cell planes k0 .. kc_end-1
-  if (cell_ok) {
-    if (k0 >= 1) {  // prologue: top corners of the cell plane k0 - 1
-      nt_load_face(S, ci, cj, k0 - 1, bot);
-      nt_load_cell(S, ci, cj, k0 - 1, cur);
-      nt_cell(bot, cur, up, tid, keep);
-      for (int v = 0; v < 13; ++v) lo[v * MH_NT_CELLS + tid] = keep[v];
-      for (int l = 0; l < 4; ++l) bot[l] = cur.top[l];
-    } else {
-      nt_load_face(S, ci, cj, k0, bot);
-    }
-    if (k0 < kc_end) nt_load_cell(S, ci, cj, k0, nxt);
-  }
-  // this thread's node column (threads below MH_NTX * MH_NTY)
-  const int i = i0 + tid % MH_NTX, j = j0 + tid / MH_NTX;
-  const bool node_ok = tid < MH_NTX * MH_NTY && i < S.g.nnx && j < S.g.nny;
-  const int tx = tid % MH_NTX, ty = tid / MH_NTX;
-  for (int k = k0; k < kend; ++k) {
-    // cell plane k: bottom corners to LDS now, top corners kept for node plane k + 1
-    if (k < nz && cell_ok) {
+  NodePre pre;
+  const int kc_end = min(kend, nz);  // cell planes kb .. kc_end - 1
+  const int kb = max(k0 - 1, 0);
+  nt_load_face(S, ci, cj, kb, bot);
+  nt_load_cell(S, ci, cj, kb, nxt);
+  // sums of the node over the cells below it
+  double mass = 0., fx = 0., fy = 0., fz = 0.;
+  for (int k = kb; k < kend; ++k) {
+    const bool cells = k < nz;  // a cell plane sits on this node plane
+    node_pre_load<3>(S, n0 + nplane * k, in, jn, k, pre);
+    if (cells) {
       cur = nxt;
       if (k + 1 < kc_end) nt_load_cell(S, ci, cj, k + 1, nxt);
-      nt_cell(bot, cur, up, tid, keep);
+      nt_cell(bot, cur, up, lo, tid);
       for (int l = 0; l < 4; ++l) bot[l] = cur.top[l];
     }
     __syncthreads();
-    if (node_ok) {
-      double mass = 0., fx = 0., fy = 0., fz = 0.;
-      const int s00 = ty * (MH_NTX + 1) + tx;  // cell (i-1, j-1)
-      const bool okx0 = i >= 1, okx1 = i < nx, oky0 = j >= 1, oky1 = j < ny;
-      if (k >= 1) {  // cells k-1, corners 4..7 -> slots 0..3 of lo
-        nt_add(lo, s00, 2, okx0 && oky0, mass, fx, fy, fz);
-        nt_add(lo, s00 + 1, 3, okx1 && oky0, mass, fx, fy, fz);
-        nt_add(lo, s00 + MH_NTX + 1, 1, okx0 && oky1, mass, fx, fy, fz);
-        nt_add(lo, s00 + MH_NTX + 2, 0, okx1 && oky1, mass, fx, fy, fz);
-      }
-      if (k < nz) {  // cells k, corners 0..3
-        nt_add(up, s00, 2, okx0 && oky0, mass, fx, fy, fz);
-        nt_add(up, s00 + 1, 3, okx1 && oky0, mass, fx, fy, fz);
-        nt_add(up, s00 + MH_NTX + 1, 1, okx0 && oky1, mass, fx, fy, fz);
-        nt_add(up, s00 + MH_NTX + 2, 0, okx1 && oky1, mass, fx, fy, fz);
-      }
-      const long n = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
-      node_finish<3>(S, n, i, j, k, dt, dth, mass, fx, fy, fz);
+    if (k >= k0) {
+      if (cells) add4(up, mass, fx, fy, fz);
+      if (node_ok) node_finish<3>(S, n0 + nplane * k, i, j, k, dt, dth, pre, mass, fx, fy, fz);
     }
+    mass = fx = fy = fz = 0.;
+    if (cells) add4(lo, mass, fx, fy, fz);
     __syncthreads();
-    if (k < nz && cell_ok)
-      for (int v = 0; v < 13; ++v) lo[v * MH_NT_CELLS + tid] = keep[v];
   }
 }
 
 // ----------------------------------------------------------------------------- cells
 
-// Volume of the hexahedron whose node 0 is b (hex_volume_lowreg's three component passes):
-// the node coordinates are read again for each pass, and a compiler fence between the passes
-// keeps their values from being shared, so one component's terms are live at a time; each pass
-// adds its corner sums face by face (cqs_hex_comp_fm), so only the running sums and one face's
-// terms are live and the cell kernel fits 128 registers (4 waves per SIMD).  Same bits as
-// cqs_hex + cell_volume<8>.
-__device__ __forceinline__ double hex_volume_passes(const MhDev& S, long b) {
-  D3 x[8];
-  double q[8], d[8];
-  cell_nodes<3>(S, b, S.xlc, x);
-  cqs_hex_comp_fm<0>(x, q);
-#pragma unroll
-  for (int l = 0; l < 8; ++l) d[l] = x[l].x * q[l];
-  asm volatile("" ::: "memory");
-  cell_nodes<3>(S, b, S.xlc, x);
-  cqs_hex_comp_fm<1>(x, q);
-#pragma unroll
-  for (int l = 0; l < 8; ++l) d[l] = d[l] + x[l].y * q[l];
-  asm volatile("" ::: "memory");
-  cell_nodes<3>(S, b, S.xlc, x);
-  cqs_hex_comp_fm<2>(x, q);
-  double v = 0.;
-#pragma unroll
-  for (int l = 0; l < 8; ++l) v += d[l] + x[l].z * q[l];
-  return v / 3;
-}
-
-__device__ __forceinline__ double node_speed(const MhDev& S, long n, int dim) {
-  const double ux = S.u[0][n], uy = S.u[1][n];
-  const double uz = dim == 3 ? S.u[2][n] : 0.;
-  return sqrt(ux * ux + uy * uy + uz * uz);
-}
-
-// max over the cell's nodes of |u| (MahycoModule.cc:1771-1774)
+// max over the cell's nodes of |u| (MahycoModule.cc:1771-1774).  The root is taken of the largest
+// square: sqrt is monotonic and correctly rounded, so that is the largest root, and amax hands on
+// the same operand of squares as of roots, NaN included.
 template <int DIM>
-__device__ __forceinline__ double cell_vmax(const MhDev& S, long b) {
+__device__ __forceinline__ double cell_vmax2(const MhDev& S, long b) {
   const long nnx = S.g.nnx, nnxy = (long)S.g.nnx * S.g.nny;
+  const long off[8] = {0, 1, 1 + nnx, nnx, nnxy, 1 + nnxy, 1 + nnx + nnxy, nnx + nnxy};
   double v = 0.;
-  v = amax(node_speed(S, b, DIM), v);
-  v = amax(node_speed(S, b + 1, DIM), v);
-  v = amax(node_speed(S, b + 1 + nnx, DIM), v);
-  v = amax(node_speed(S, b + nnx, DIM), v);
-  if (DIM == 3) {
-    v = amax(node_speed(S, b + nnxy, DIM), v);
-    v = amax(node_speed(S, b + 1 + nnxy, DIM), v);
-    v = amax(node_speed(S, b + 1 + nnx + nnxy, DIM), v);
-    v = amax(node_speed(S, b + nnx + nnxy, DIM), v);
+#pragma unroll
+  for (int l = 0; l < (DIM == 3 ? 8 : 4); ++l) {
+    const long n = b + off[l];
+    const double ux = S.u[0][n], uy = S.u[1][n];
+    const double uz = DIM == 3 ? S.u[2][n] : 0.;
+    v = amax(ux * ux + uy * uy + uz * uz, v);
   }
   return v;
 }
@@ -569,7 +633,13 @@ __device__ __forceinline__ double gp_energy(double e_n, double p, double rho, do
 // MahycoModule.h:378-386, with the EOS of applyOneCellEOS at each iterate) or
 // updateEnergyAndPressureExplicite (:1484-1502).  Newton's last pressure and sound speed are
 // replaced by the EOS call that follows the update (or the remap), so only e is returned.
-__device__ __forceinline__ double lag_energy(const MhDev& S, const MhEnvParam& ep, double e_n, double p_n, double rho,
+// What the Lagrange step takes from an environment's parameters (MhEnvParam has the same names).
+struct MhEosCoef {
+  double gamma, pinf, a1, a2;
+  int stiffened;
+};
+template <class EnvP>
+__device__ __forceinline__ double lag_energy(const MhDev& S, const EnvP& ep, double e_n, double p_n, double rho,
                                              double rho_n, double q) {
   if (S.p_explicit) return e_n - (p_n + q) * (1.0 / rho - 1.0 / rho_n);
   if (!S.newton) return gp_energy(e_n, p_n, rho, rho_n, q, ep.gamma);
@@ -588,7 +658,8 @@ __device__ __forceinline__ double lag_energy(const MhDev& S, const MhEnvParam& e
 }
 
 // applyEOS (PerfectGasEOSService.cc:45-67, StiffenedGasEOSService.cc:43-63)
-__device__ __forceinline__ void eos(const MhEnvParam& ep, double rho, double e, double& p, double& c) {
+template <class EnvP>
+__device__ __forceinline__ void eos(const EnvP& ep, double rho, double e, double& p, double& c) {
   const double g = ep.gamma;
   if (ep.stiffened) {
     p = ((g - 1.) * rho * e) - (g * ep.pinf);
@@ -640,7 +711,8 @@ __device__ __forceinline__ void csts_work(const MhDev& S, long b, const D3* qv, 
   }
 }
 // ... priced per environment with its own mass, density, pressure and pseudo-viscosities
-__device__ __forceinline__ double csts_e(const MhEnvParam& ep, double e, double M, double rho, double pn, double qn,
+template <class EnvP>
+__device__ __forceinline__ double csts_e(const EnvP& ep, double e, double M, double rho, double pn, double qn,
                                          double qnm1, double q, double cn1, double cn, double cdn, double cvon) {
   const double denom = 1 + 0.5 * (ep.gamma - 1.0) * rho * cn1 / M;
   const double numer = e - (0.5 * (pn + qn) * cn / M) - (0.5 * q * cn1 / M) + (0.25 * (pn + qn) * cdn / M) -
@@ -729,11 +801,14 @@ __device__ __forceinline__ void store_remap_vector(const MhDev& S, long c, unsig
 // Without: applies the EOS and the mean pressure and writes the CFL candidate.
 // The cell's work once its node coordinates x (at this cycle's Lagrangian positions) are
 // in registers; returns the CFL candidate of the Lagrange-only loop.
-// The cell's own state read by the Lagrange step, loaded ahead of the geometry so that its
-// latency is hidden behind the corner-vector arithmetic.
+// The cell's own state read by the Lagrange step.  2D kernels are latency-bound: all loads go out
+// together (33.9 -> 27.3 us on 1023x1021, 8.9 -> 7.3 us on 200x10).  3D ones are bound by the FP64 issue
+// of the volume, which takes all 160 registers of three wavefronts per SIMD, so the state is read
+// after it (216 -> 192 us on 256x128x128, 304 -> 257 us on 192^3, 55 -> 46 us on 128x96x64 without remap).
 struct CellPre {
   uint8_t mk;
   double cs, rho_n, Mc, e_c, p_c;
+  double vmax2;  // Lagrange-only loop: the square of the largest node speed, for the CFL candidate
 };
 __device__ __forceinline__ void cell_pre_load(const MhDev& S, long c, CellPre& pr) {
   pr.mk = S.mask[c];
@@ -744,14 +819,15 @@ __device__ __forceinline__ void cell_pre_load(const MhDev& S, long c, CellPre& p
   pr.p_c = S.p[c];
 }
 
-// VGIVEN: the volume Vgiven was formed by the caller (the LDS-tiled kernel); x is unused.
+// VGIVEN: the volume Vgiven was formed by the caller (the 3D kernels but CSTS); x is unused.
 template <int DIM, int M, int CSTS = 0, int VGIVEN = 0, int REMAP = 0>
 __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, const D3* x, const CellPre& pre,
                                                 double Vgiven = 0.) {
-  // REMAP: known at compile time to be the Lagrange step of the remap loop (with_proj set,
-  // sans_lagrange not), so the other branches are not compiled.  Staged mode takes the
+  // REMAP: known at compile time to be the Lagrange step of the remap loop (1: with_proj set,
+  // sans_lagrange and staged not) or of the Lagrange-only loop (2), so the other branches are
+  // not compiled.  Staged mode takes the
   // Lagrange-only branch (state and EOS written back) and k_prepare_remap forms U later.
-  const bool with_proj = REMAP ? true : (S.with_proj != 0 && !S.staged);
+  const bool with_proj = REMAP == 1 ? true : (REMAP == 2 ? false : S.with_proj != 0 && !S.staged);
   const bool sans_lagrange = REMAP ? false : (S.sans_lagrange != 0);
   constexpr int NV = 3 * M + 1;
   double dxs = 1.79769313486231570815e+308;
@@ -766,8 +842,6 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
     double V;
     if constexpr (VGIVEN) {
       V = Vgiven;
-    } else if constexpr (DIM == 3 && !CSTS) {
-      V = hex_volume_passes(S, b);  // the corner vectors themselves are not needed (x unused)
     } else if (DIM == 3) {
       cqs_hex(x, qv);
       V = cell_volume<8>(x, qv, 3);
@@ -827,7 +901,17 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
     for (int v = 0; v < NV; ++v) u_out[v] = 0.;
     if (__popc(mk) == 1) {
       const int ke = __ffs(mk) - 1;
-      const MhEnvParam& ep = S.env[ke];
+      // by selects: an index that varies over the lanes would be another load to wait for
+      MhEosCoef ep{S.env[0].gamma, S.env[0].pinf, S.env[0].a1, S.env[0].a2, S.env[0].stiffened};
+#pragma unroll
+      for (int kk = 1; kk < M; ++kk) {
+        const MhEnvParam& o = S.env[kk];
+        ep.gamma = kk == ke ? o.gamma : ep.gamma;
+        ep.pinf = kk == ke ? o.pinf : ep.pinf;
+        ep.a1 = kk == ke ? o.a1 : ep.a1;
+        ep.a2 = kk == ke ? o.a2 : ep.a2;
+        ep.stiffened = kk == ke ? o.stiffened : ep.stiffened;
+      }
       double q = 0.;
       if (divu < 0.0) q = 1. / tau * (-ep.a1 * L * cs * divu + ep.a2 * L * L * divu * divu);
       double e;
@@ -866,7 +950,7 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
         S.p[c] = p;
         S.c[c] = cc;
         S.q[c] = q;
-        if (!S.staged) dxs = L / (cc + cell_vmax<DIM>(S, b));
+        if (REMAP == 2 || !S.staged) dxs = L / (cc + sqrt(pre.vmax2));
       }
     } else {
       double fk[M], rk[M], qk[M], ek[M], Vk[M];
@@ -943,7 +1027,7 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
         S.p[c] = ps;
         S.c[c] = cmix;
         S.q[c] = qsum;
-        if (!S.staged) dxs = L / (cmix + cell_vmax<DIM>(S, b));
+        if (REMAP == 2 || !S.staged) dxs = L / (cmix + sqrt(pre.vmax2));
       }
     }
     if (with_proj && !mk && !S.pb && S.nsweep > 0) empty_cell_phi<M>(S, c, u_out);
@@ -954,12 +1038,13 @@ __device__ __forceinline__ double cell_lag_core(const MhDev& S, long c, long b, 
   return dxs;
 }
 
-template <int DIM, int M, int CSTS = 0>
+template <int DIM, int M, int CSTS = 0, int REMAP = 0>
 __device__ __forceinline__ void k_cell_lag_body(const MhDev& S, int lb) {
   const long c = lb * (long)blockDim.x + threadIdx.x;
-  const bool active = c < S.g.nc && !mh_halted(S.sc);
+  const bool halted = mh_halted(S.sc);
+  const bool active = c < S.g.nc && !halted;
   double dxs = 1.79769313486231570815e+308;
-  if (active) {
+  if (c < S.g.nc) {
     const int nx = S.g.nx, ny = S.g.ny;
     const int i = (int)(c % nx);
     const long r = c / nx;
@@ -967,16 +1052,16 @@ __device__ __forceinline__ void k_cell_lag_body(const MhDev& S, int lb) {
     const int k = (int)(r / ny);
     const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
     CellPre pre;
+    constexpr bool VOL = DIM == 3 && !CSTS;
+    double V = 0.;
+    D3 x[8];
+    cell_nodes<DIM>(S, b, S.xlc, x);
+    if (VOL) V = hex_volume(x);
     cell_pre_load(S, c, pre);
-    if constexpr (DIM == 3 && !CSTS) {
-      dxs = cell_lag_core<DIM, M, CSTS>(S, c, b, nullptr, pre);  // the volume reads its nodes itself
-    } else {
-      D3 x[8];
-      cell_nodes<DIM>(S, b, S.xlc, x);
-      dxs = cell_lag_core<DIM, M, CSTS>(S, c, b, x, pre);
-    }
+    if (REMAP == 2 || (!REMAP && !S.with_proj)) pre.vmax2 = cell_vmax2<DIM>(S, b);
+    if (active) dxs = cell_lag_core<DIM, M, CSTS, VOL, REMAP>(S, c, b, x, pre, V);
   }
-  if (!S.with_proj) block_min_store(dxs, active, S.partial, lb);
+  if (REMAP == 2 || (!REMAP && !S.with_proj)) block_min_store(dxs, active, S.partial, lb);
 }
 // computeVariablesForRemap (PrepareRemap.cc:100-155) from the stored Lagrangian state, for
 // staged mode: the cell kernel wrote the state of UpdateEnergyAndPressure and the caller may
@@ -1037,7 +1122,7 @@ __device__ __forceinline__ void k_prepare_remap_body(const MhDev& S, int lb) {
 // per tile instead of by each of its cells) go to a rolling set of three LDS planes: the two a
 // cell plane needs, and the next one, whose global loads are issued before the cell plane's
 // arithmetic and written to LDS after it.  The cell's own state is also loaded one plane ahead.
-// The volume takes its three component passes from LDS; everything else is cell_lag_core.
+// The volume takes its nodes from LDS; everything else is cell_lag_core.
 #define MH_CT_X 64
 #define MH_CT_Y (MH_BLOCK / MH_CT_X)
 #define MH_CT_K 8  // cell planes per tile by default (MhDev::ct_k)
@@ -1045,38 +1130,19 @@ __device__ __forceinline__ void k_prepare_remap_body(const MhDev& S, int lb) {
 #define MH_CT_NP (MH_CT_NX * (MH_CT_Y + 1))  // nodes of a tile plane
 #define MH_CT_PER ((MH_CT_NP + MH_BLOCK - 1) / MH_BLOCK)  // node entries loaded per thread
 #ifndef MH_CT_MIN_WAVES
-#define MH_CT_MIN_WAVES 3
+#define MH_CT_MIN_WAVES 2
 #endif
 
-// Volume of the cell whose node 0 is entry s of the bottom plane (hex_volume_passes with the
-// nodes read from LDS; same bits).
+// Volume of the cell whose node 0 is entry s of the bottom plane.
 __device__ __forceinline__ double hex_volume_lds(const double* bot, const double* top, int s) {
   const int o[4] = {s, s + 1, s + 1 + MH_CT_NX, s + MH_CT_NX};
-  auto load = [&](D3* x) {
-#pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      x[l] = d3(bot[o[l]], bot[MH_CT_NP + o[l]], bot[2 * MH_CT_NP + o[l]]);
-      x[l + 4] = d3(top[o[l]], top[MH_CT_NP + o[l]], top[2 * MH_CT_NP + o[l]]);
-    }
-  };
   D3 x[8];
-  double q[8], d[8];
-  load(x);
-  cqs_hex_comp<0>(x, q);
 #pragma unroll
-  for (int l = 0; l < 8; ++l) d[l] = x[l].x * q[l];
-  asm volatile("" ::: "memory");
-  load(x);
-  cqs_hex_comp<1>(x, q);
-#pragma unroll
-  for (int l = 0; l < 8; ++l) d[l] = d[l] + x[l].y * q[l];
-  asm volatile("" ::: "memory");
-  load(x);
-  cqs_hex_comp<2>(x, q);
-  double v = 0.;
-#pragma unroll
-  for (int l = 0; l < 8; ++l) v += d[l] + x[l].z * q[l];
-  return v / 3;
+  for (int l = 0; l < 4; ++l) {
+    x[l] = d3(bot[o[l]], bot[MH_CT_NP + o[l]], bot[2 * MH_CT_NP + o[l]]);
+    x[l + 4] = d3(top[o[l]], top[MH_CT_NP + o[l]], top[2 * MH_CT_NP + o[l]]);
+  }
+  return hex_volume(x);
 }
 
 template <int M>
@@ -1159,8 +1225,18 @@ __device__ __forceinline__ void k_cell_length_body(const MhDev& S, int lb) {
   S.L[c] = char_length_alt<DIM>(S.lc, x);
 }
 
+// The Lagrange step of the remap loop and that of the Lagrange-only loop: an instance each, without
+// one another's registers and those of staged mode and advection, which k_cell_lag keeps.
 // CSTS (with remap): its own instance, so that the other cell kernels do not carry the
 // corner-work registers
+template <int DIM, int M>
+__device__ __forceinline__ void k_cell_lag_remap_body(const MhDev& S, int lb) {
+  k_cell_lag_body<DIM, M, 0, 1>(S, lb);
+}
+template <int DIM, int M>
+__device__ __forceinline__ void k_cell_lag_only_body(const MhDev& S, int lb) {
+  k_cell_lag_body<DIM, M, 0, 2>(S, lb);
+}
 template <int DIM, int M>
 __device__ __forceinline__ void k_cell_lag_csts_body(const MhDev& S, int lb) {
   k_cell_lag_body<DIM, M, 1>(S, lb);
@@ -3295,15 +3371,25 @@ template <int DIM, int M>
 __device__ __forceinline__ void k_finalize_body(const MhDev& S, int lb, int usel) {
   const double* __restrict__ Uin = usel ? S.Ub : S.Ua;
   const long c = lb * (long)blockDim.x + threadIdx.x;
-  const bool active = c < S.g.nc && !mh_halted(S.sc);
+  const bool halted = mh_halted(S.sc);
+  const bool active = c < S.g.nc && !halted;
   double dxs = 1.79769313486231570815e+308;
-  if (active) {
+  if (c < S.g.nc) {
+    // everything the cell reads goes out together: the node velocities and L of the CFL candidate,
+    // the membership and VE, then the slots, which wait for the presence byte (35.5 -> 32.6 us on
+    // 1023x1021, 165 -> 147 us for 64 meshes of 64^2 to 512^2; large 3D meshes are as before)
     const long nc = S.g.nc;
     const double thr = S.thr_remap;
     double U[3 * M + 1];
     const unsigned held = M > 1 && S.pm[0] ? S.pm[usel ? 1 : 0][c] : ~0u;
-    for (int v = 0; v < 3 * M; ++v) U[v] = ((held >> (v % M)) & 1u) ? Uin[v * nc + c] : 0.;
+    const double VE = S.VE[c];
+    const uint8_t om = S.mask[c];
+    const double Lc = S.L[c];
     U[3 * M] = Uin[3 * M * nc + c];
+    const int ci = (int)(c % S.g.nx), cj = (int)(c / S.g.nx % S.g.ny), ck = (int)(c / S.g.nx / S.g.ny);
+    const double vmax2 = cell_vmax2<DIM>(S, ci + (long)S.g.nnx * (cj + (long)S.g.nny * ck));
+    for (int v = 0; v < 3 * M; ++v) U[v] = ((held >> (v % M)) & 1u) ? Uin[v * nc + c] : 0.;
+    if (active) {
     if (S.pb && S.nsweep > 0) {  // phi the last sweep left (RemapADIService.cc:493-538): what the
                                   // next cycle's first sweep sees for non-member environments
       double sv = 0.;
@@ -3314,9 +3400,7 @@ __device__ __forceinline__ void k_finalize_body(const MhDev& S, int lb, int usel
       }
       for (int kk = 0; kk < M; ++kk) S.phi0[(2 * M + kk) * nc + c] = U[M + kk] != 0. ? U[2 * M + kk] / U[M + kk] : 0.;
     }
-    const double VE = S.VE[c];
     // environment membership (:29-78)
-    const uint8_t om = S.mask[c];
     uint8_t nm = om;
     for (int kk = 0; kk < M; ++kk) {
       const bool was = (om >> kk) & 1;
@@ -3529,13 +3613,8 @@ __device__ __forceinline__ void k_finalize_body(const MhDev& S, int lb, int usel
     S.c[c] = c_g;
     S.q[c] = q_g;
     S.M[c] = M_g;
-    const int nx = S.g.nx, ny = S.g.ny;
-    const int i = (int)(c % nx);
-    const long r = c / nx;
-    const int j = (int)(r % ny);
-    const int k = (int)(r / ny);
-    const long b = i + (long)S.g.nnx * (j + (long)S.g.nny * k);
-    dxs = S.L[c] / (c_g + cell_vmax<DIM>(S, b));
+    dxs = Lc / (c_g + sqrt(vmax2));
+    }
   }
   block_min_store(dxs, active, S.partial, lb);
 }
@@ -3805,8 +3884,11 @@ __global__ __launch_bounds__(MH_BLOCK) void k_hist_final(MhDev S) { k_hist_final
 // is tab[bmap[b].x] (meshes of one launch share DIM, M and the sweep direction).
 // Single-mesh grids use the XCD-contiguous block order of xcd_block.
 
+#ifndef MH_NODE_FLAT_MIN_WAVES
+#define MH_NODE_FLAT_MIN_WAVES 2  // register budget of k_node_lag, in waves per SIMD
+#endif
 #ifndef MH_CELL_MIN_WAVES
-#define MH_CELL_MIN_WAVES 4  // register budget of k_cell_lag, in waves per SIMD
+#define MH_CELL_MIN_WAVES 3  // register budget of k_cell_lag, in waves per SIMD
 #endif
 #ifndef MH_NODE_MIN_WAVES
 #define MH_NODE_MIN_WAVES 1  // register budget of k_node_lag3_tiled, in waves per SIMD
@@ -3828,8 +3910,10 @@ __global__ __launch_bounds__(MH_BLOCK) void k_hist_final(MhDev S) { k_hist_final
     }                                                                                        \
   }
 #define MH_COMMA ,
-MH_WRAP(k_node_lag, 1, template <int DIM>, <DIM>, , )
+MH_WRAP(k_node_lag, MH_NODE_FLAT_MIN_WAVES, template <int DIM>, <DIM>, , )
 MH_WRAP(k_cell_lag, MH_CELL_MIN_WAVES, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
+MH_WRAP(k_cell_lag_remap, MH_CELL_MIN_WAVES, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
+MH_WRAP(k_cell_lag_only, MH_CELL_MIN_WAVES, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
 MH_WRAP(k_cell_lag_csts, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
 MH_WRAP(k_cell_length, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_sweep_cell, 1, template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
@@ -3898,6 +3982,11 @@ __global__ __launch_bounds__(MH_BLOCK, 2) void k_sweep_cell3_batch(const MhDev* 
 template <int U = 0>
 __global__ __launch_bounds__(MH_BLOCK, MH_NODE_MIN_WAVES) void k_node_lag3_tiled(MhDev S) {
   k_node_lag3_tiled_body(S, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+template <int U = 0>
+__global__ __launch_bounds__(MH_BLOCK) void k_node_lag3_split(MhDev S) {
+  k_node_lag3_split_body(S, xcd_block((int)blockIdx.x, (int)gridDim.x));
 }
 
 template <int U = 0>

@@ -10,8 +10,10 @@ void launch_node_t(MhHandle* h) {
     const dim3 grid((h->g.nnx + MH_NTX - 1) / MH_NTX, (h->g.nny + MH_NTY - 1) / MH_NTY,
                     (h->g.nnz + h->dev.nt_kc - 1) / h->dev.nt_kc);
     LAUNCH(h, KN_NODE, k_node_lag3_tiled<>, grid, MH_BLOCK, h->dev);
+  } else if (DIM == 3) {
+    LAUNCH(h, KN_NODE, k_node_lag3_split<>, (int)((h->g.nn + 511) / 512 * 8), MH_BLOCK, h->dev);
   } else {
-    LAUNCH(h, KN_NODE, (k_node_lag<DIM>), h->nblk_n, MH_BLOCK, h->dev);
+    LAUNCH(h, KN_NODE, (k_node_lag<2>), h->nblk_n, MH_BLOCK, h->dev);
   }
 }
 template <int DIM, int M>
@@ -19,13 +21,17 @@ void launch_cell_t(MhHandle* h) {
   if (h->dev.lc != MH_L_RACINE_CUBIQUE_VOLUME) LAUNCH(h, KN_CELL, (k_cell_length<DIM>), h->nblk_c, MH_BLOCK, h->dev);
   if (h->dev.csts) {
     LAUNCH(h, KN_CELL, (k_cell_lag_csts<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
-  } else if (DIM == 3 && h->dev.with_proj && !h->dev.sans_lagrange && !h->staged && h->cell_tiled) {
+  } else if (!h->dev.with_proj) {
+    LAUNCH(h, KN_CELL, (k_cell_lag_only<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
+  } else if (h->dev.sans_lagrange || h->staged) {
+    LAUNCH(h, KN_CELL, (k_cell_lag<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
+  } else if (DIM == 3 && h->cell_tiled) {
     // the Lagrange-only loop keeps k_cell_lag: its CFL candidates are folded per block in cell order
     const dim3 grid((h->g.nx + MH_CT_X - 1) / MH_CT_X, (h->g.ny + MH_CT_Y - 1) / MH_CT_Y,
                     (h->g.nz + h->dev.ct_k - 1) / h->dev.ct_k);
     LAUNCH(h, KN_CELL, (k_cell_lag3_tiled<M>), grid, MH_BLOCK, h->dev);
   } else {
-    LAUNCH(h, KN_CELL, (k_cell_lag<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
+    LAUNCH(h, KN_CELL, (k_cell_lag_remap<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
   }
 }
 

@@ -196,7 +196,8 @@ void ens_group_cycle_l(MhEnsembleImpl* E, const EnsGroup& g) {
   else hipLaunchKernelGGL((k_node_lag_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.nmap));
   if (g.lc) hipLaunchKernelGGL((k_cell_length_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.cmap));
   if (g.csts) hipLaunchKernelGGL((k_cell_lag_csts_batch<DIM, M>), G, B, 0, st, tab, MH_LIST(g.cmap));
-  else hipLaunchKernelGGL((k_cell_lag_batch<DIM, M>), G, B, 0, st, tab, MH_LIST(g.cmap));
+  else if (g.adv) hipLaunchKernelGGL((k_cell_lag_batch<DIM, M>), G, B, 0, st, tab, MH_LIST(g.cmap));
+  else hipLaunchKernelGGL((k_cell_lag_remap_batch<DIM, M>), G, B, 0, st, tab, MH_LIST(g.cmap));
   if (g.csts) hipLaunchKernelGGL((k_node_fwd_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.nmap));
   const int sens = (int)(E->launched % DIM);
   if (g.o3 || g.gen) hipLaunchKernelGGL((k_hcell_batch<DIM>), G, B, 0, st, tab, MH_LIST(g.cmap));

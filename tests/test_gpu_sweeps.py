@@ -131,3 +131,20 @@ def test_presence_bytes_over_variants_and_checkpoint(tmp_path, monkeypatch):
             g.checkpoint_read(tmp_path / "dump")
     a, b = fields(g, 2, 2), fields(o, 2, 2)
     assert not [k for k in a if not bitwise_equal(a[k], b[k])]
+
+
+# node kernels: blocks of 64 nodes (64, 65 and 128 of them), tiles of 31 x 7 columns and one more,
+# depths that end on, before and after the last node plane; then the remap's other Lagrange steps
+@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+@pytest.mark.parametrize("kw", [{}, dict(with_projection=False)], ids=["remap", "lagrange"])
+@pytest.mark.parametrize("n", [(3, 3, 3), (4, 12, 1), (7, 7, 1), (30, 6, 11), (31, 7, 12), (32, 8, 15), (5, 3, 16)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_node_kernels_at_block_edges(n, kw, variant):
+    from mahyco_amd.lib import GpuCase
+    from oracle.pyoracle import OracleCase
+    c = moving_tube(n, variant, **kw)
+    g, o = GpuCase(c), OracleCase(c, pow_mode=1, threads=4)
+    g.set_variant(variant)
+    assert g.run(7) == o.run(7)
+    a, b = fields(g, 2, 3), fields(o, 2, 3)
+    assert not [k for k in a if not bitwise_equal(a[k], b[k])]
