@@ -18,6 +18,7 @@
 #include "mh_host.h"
 #include "mh_kernels.h"
 #include "mh_output.h"
+#include "mh_readback.h"
 
 namespace {
 
@@ -1196,16 +1197,19 @@ long mahyco_nb_cells(MhHandle* h) { return h ? h->g.nc : -1; }
 long mahyco_graph_captures(MhHandle* h) { return h ? h->graph_captures : -1; }
 long mahyco_nb_nodes(MhHandle* h) { return h ? h->g.nn : -1; }
 
-int mahyco_get_field(MhHandle* h, int field, int env, int comp, double* out) {
-  if (!h || !out) return MH_ERR_INVALID;
+static int get_field(MhHandle* h, HostStage& stage, int field, int env, int comp, double* out) {
   MhScalars sc;
   int st = read_scalars(h, &sc);
   if (st != MH_OK) return st;
   const long nc = h->g.nc, nn = h->g.nn;
   MhDev& S = h->dev;
+  // (the stream is idle: read_scalars waited for it)
   auto d2h = [&](const double* d, double* hst, long n) -> int {
-    HIPCHK(hipMemcpy(hst, d, n * sizeof(double), hipMemcpyDeviceToHost));
-    return MH_OK;
+    return hip_check(read_back(stage, h->stream, (char*)hst, n * sizeof(double),
+                               [&](char* pin, size_t off, size_t len) {
+                                 return hipMemcpyAsync(pin, (const char*)d + off, len, hipMemcpyDeviceToHost, h->stream);
+                               }),
+                     "read back");
   };
   if (field >= 100) {
     if (comp < 0 || comp > 2) return MH_ERR_INVALID;
@@ -1251,10 +1255,9 @@ int mahyco_get_field(MhHandle* h, int field, int env, int comp, double* out) {
     return MH_ERR_INVALID;
   }
   if (env >= h->m || env < -1) return MH_ERR_INVALID;
-  std::vector<uint8_t> mask(nc);
-  HIPCHK(hipMemcpy(mask.data(), S.mask, nc, hipMemcpyDeviceToHost));
   const double* gsrc = nullptr;
   const double* esrc = nullptr;
+  bool formed = env >= 0;  // per cell, from more than one array
   switch (field) {
     case MH_F_DENSITY: gsrc = S.rho; esrc = S.rhok; break;
     case MH_F_PRESSURE: gsrc = S.p; esrc = S.pk; break;
@@ -1263,67 +1266,29 @@ int mahyco_get_field(MhHandle* h, int field, int env, int comp, double* out) {
     case MH_F_PSEUDO_VISCOSITY: gsrc = S.q; break;
     case MH_F_CELL_MASS: gsrc = S.M; esrc = S.Mk; break;
     case MH_F_FRACVOL: gsrc = S.fg; esrc = S.fk; break;
-    case MH_F_MASS_FRACTION: gsrc = nullptr; esrc = S.chik; break;
     case MH_F_CARACTERISTIC_LENGTH: gsrc = S.L; break;
-    case MH_F_CELL_VOLUME: gsrc = S.VE; break;
-    default: break;
+    case MH_F_CELL_VOLUME: gsrc = !h->opt.with_projection && sc.iteration > 0 ? S.Vl : S.VE; break;
+    case MH_F_MASS_FRACTION:
+    case MH_F_MATERIAU:
+    case MH_F_ENV_MASK: formed = true; break;
+    default: return MH_ERR_INVALID;
   }
-  if (field == MH_F_ENV_MASK) {
-    for (long c = 0; c < nc; ++c) out[c] = mask[c];
-    return MH_OK;
-  }
-  if (field == MH_F_MATERIAU || field == MH_F_CELL_VOLUME || field == MH_F_FRACVOL ||
-      field == MH_F_MASS_FRACTION) {
-    std::vector<double> fg(nc), fk((size_t)h->m * nc), V(nc);
-    if ((st = d2h(S.fg, fg.data(), nc)) != MH_OK) return st;
-    if ((st = d2h(S.fk, fk.data(), (long)h->m * nc)) != MH_OK) return st;
-    const bool lagv = !h->opt.with_projection && sc.iteration > 0;
-    if ((st = d2h(lagv ? S.Vl : S.VE, V.data(), nc)) != MH_OK) return st;
-    std::vector<double> chik, chig;
-    if (field == MH_F_MASS_FRACTION) {
-      chik.resize((size_t)h->m * nc);
-      chig.resize(nc);
-      if ((st = d2h(S.chik, chik.data(), (long)h->m * nc)) != MH_OK) return st;
-      if ((st = d2h(S.chig, chig.data(), nc)) != MH_OK) return st;
-    }
-    for (long c = 0; c < nc; ++c) {
-      const uint8_t b = mask[c];
-      const bool pure = __builtin_popcount(b) == 1;
-      const int kp = __builtin_ctz(b ? b : 1);
-      double val = 0.;
-      if (field == MH_F_MATERIAU) {
-        if (pure) val = kp * fg[c];
-        else
-          for (int k = 0; k < h->m; ++k)
-            if ((b >> k) & 1) val += k * fk[k * nc + c];
-      } else if (field == MH_F_CELL_VOLUME) {
-        if (env < 0) val = V[c];
-        else if ((b >> env) & 1) val = pure ? V[c] : fk[env * nc + c] * V[c];
-      } else if (field == MH_F_FRACVOL) {
-        if (env < 0) val = fg[c];
-        else if ((b >> env) & 1) val = pure ? fg[c] : fk[env * nc + c];
-      } else {
-        if (env < 0) val = 0.;
-        else if ((b >> env) & 1) val = pure ? chig[c] : chik[env * nc + c];
-      }
-      out[c] = val;
-    }
-    return MH_OK;
-  }
-  if (!gsrc) return MH_ERR_INVALID;
-  if ((st = d2h(gsrc, out, nc)) != MH_OK) return st;
-  if (env < 0) return MH_OK;
-  std::vector<double> ev;
-  if (esrc) {
-    ev.resize(nc);
-    if ((st = d2h(esrc + (size_t)env * nc, ev.data(), nc)) != MH_OK) return st;
-  }
-  for (long c = 0; c < nc; ++c) {
-    const uint8_t b = mask[c];
-    if (!((b >> env) & 1)) out[c] = 0.;
-    else if (__builtin_popcount(b) != 1) out[c] = esrc ? ev[c] : out[c];
-  }
-  return MH_OK;
+  if (!formed) return d2h(gsrc, out, nc);
+  const double* ek = esrc && env >= 0 ? esrc + (size_t)env * nc : nullptr;
+  return hip_check(read_back(stage, h->stream, (char*)out, nc * sizeof(double),
+                             [&](char* pin, size_t off, size_t len) {
+                               const long n = (long)(len / sizeof(double));
+                               hipLaunchKernelGGL(k_read_field<>, dim3((unsigned)((n + MH_BLOCK - 1) / MH_BLOCK)),
+                                                  dim3(MH_BLOCK), 0, h->stream, S, field, env, gsrc, ek, (double*)pin,
+                                                  (long)(off / sizeof(double)), n);
+                               return hipGetLastError();
+                             }),
+                   "read back");
+}
+
+int mahyco_get_field(MhHandle* h, int field, int env, int comp, double* out) {
+  if (!h || !out) return MH_ERR_INVALID;
+  return get_field(h, h->stage, field, env, comp, out);
 }
 
 static void drop_graphs(MhHandle* h);
@@ -1650,8 +1615,9 @@ int mahyco_ensemble_poll(MhEnsemble* e, int* status, double* time, int* iteratio
 int mahyco_ensemble_get_field(MhEnsemble* e, int slot, int field, int env, int comp, double* out) {
   MhEnsembleImpl* E = (MhEnsembleImpl*)e;
   if (!E || slot < 0 || slot >= E->max_slots || !E->slot[slot]) return MH_ERR_INVALID;
+  if (!out) return MH_ERR_INVALID;
   HIPCHK(hipStreamSynchronize(E->stream));
-  return mahyco_get_field(E->slot[slot], field, env, comp, out);
+  return get_field(E->slot[slot], E->field_stage, field, env, comp, out);
 }
 
 double mahyco_ensemble_used_bytes(MhEnsemble* e) {

@@ -15,6 +15,7 @@
 #include "../../include/mahyco.h"
 #include "mh_kernels.h"
 #include "mh_output.h"
+#include "mh_readback.h"
 
 // profiled kernel groups (sweeps separately per direction: they run different code)
 enum {
@@ -83,6 +84,7 @@ struct MhHandle {
   std::vector<hipGraph_t> graph_defs;
   long graph_captures = 0;  // graphs captured and instantiated so far
   bool owns_stream = true;
+  HostStage stage;  // pinned slots of mahyco_get_field
   bool node_tiled = true;   // 3D: z-marching node kernel (MAHYCO_NODE_KERNEL=flat: k_node_lag3_split)
   bool cell_tiled = false;  // 3D remap loop: LDS-staged cell kernel (MAHYCO_CELL_KERNEL=tiled; an autotuner candidate)
   bool staged = false;      // Lagrangian state written before the remap, U formed from it (mahyco_set_staged)
@@ -273,6 +275,7 @@ struct MhEnsembleImpl {
   MhScalars* snap = nullptr;       // pinned, max_slots entries
   hipEvent_t snap_done = nullptr;
   bool snap_pending = false;
+  HostStage field_stage;           // pinned slots of mahyco_ensemble_get_field
   std::vector<int> snap_state;     // slot state when the snapshot was taken: -100 empty, 2 pending, 1 active
 };
 
