@@ -289,7 +289,12 @@ void set_parity(MhHandle* h) {
     }                                                           \
   } while (0)
 
-void launch_dt(MhHandle* h) { LAUNCH(h, KN_DT, k_dt<>, 1, MH_DT_BLOCK, h->dev); }
+// One wavefront while it holds all partials in one round of loads (8 per lane): a block of 16 wavefronts
+// takes longer to start and to meet twice than to read them.
+void launch_dt(MhHandle* h) {
+  const int threads = h->nblk_c <= 512 ? 64 : h->nblk_c <= 2048 ? 256 : MH_DT_BLOCK;
+  LAUNCH(h, KN_DT, k_dt<>, 1, threads, h->dev);
+}
 
 // Phase functions shared by mahyco_cycle and the per-entry-point calls.
 void phase_node(MhHandle* h) {
@@ -543,12 +548,13 @@ int ens_group_of(MhEnsembleImpl* E, MhHandle* h) {
   k.lc = h->dev.lc != 0;
   k.rows = !k.o3 && !k.gen && h->sweep_mode == MH_SWEEP_TILE;
   k.ntile = k.dim == 3 && h->node_tiled && !k.adv;
+  k.cmarch = k.rows && cell_march(h);
   k.lim = (k.o3 || k.gen) ? -1 : (h->dev.order2 ? h->dev.limiter : 3);
   k.cons = h->dev.dec != nullptr;
   for (size_t i = 0; i < E->groups.size(); ++i) {
     const EnsGroup& g = E->groups[i];
     if (g.dim == k.dim && g.m == k.m && g.o3 == k.o3 && g.gen == k.gen && g.csts == k.csts && g.adv == k.adv &&
-        g.lc == k.lc && g.rows == k.rows && g.ntile == k.ntile && g.lim == k.lim && g.cons == k.cons)
+        g.lc == k.lc && g.rows == k.rows && g.ntile == k.ntile && g.cmarch == k.cmarch && g.lim == k.lim && g.cons == k.cons)
       return (int)i;
   }
   const int cached = tune_lookup(group_key(k));
@@ -577,7 +583,8 @@ void ens_lists_add(EnsGroup& g, MhHandle* h, int sl) {
   if (g.rows) {
     ens_list_add(g.rcmap, sl, row_blocks(h));
     ens_list_add(g.rnmap, sl, node_row_blocks(h));
-    for (int D = 1; D < g.dim; ++D) ens_list_add(g.tmap[D - 1], sl, tile_blocks(h, D));
+    for (int D = 1; D < g.dim; ++D)
+      ens_list_add(g.tmap[D - 1], sl, g.cmarch ? cell_march_blocks(h, D) : tile_blocks(h, D));
     for (int D = 1; D < g.dim; ++D) ens_list_add(g.mmap[D - 1], sl, node_march_blocks(h, D));
   }
   if (g.o3) {  // segments along each direction

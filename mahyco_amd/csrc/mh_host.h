@@ -38,7 +38,8 @@ enum {
 enum { MH_SWEEP_FLAT = 0, MH_SWEEP_TILE = 1 };
 // Sizes below which a single mesh takes the variants of the row/tile sweeps that need fewer
 // wavefronts to hide their latency; both sides measured around each line:
-// y / z cell sweeps: 2-cell register segments (k_sweep_cell_seg) below, LDS tiles above.  Tile
+// y / z cell sweeps: 2-cell register segments (k_sweep_cell_seg) below, marching threads or LDS tiles
+// (k_sweep_cell_march) above.  Tile
 // against segments, two environments: 27 / 10 us on 181x181, 30 / 22 on 512x512, 45 / 33 on 80^3,
 // 37 / 30 on 724x724, 71 / 60 on 101^3, but 45 / 54 on 1024x1024, and 69 / 85 on 128^3 (one).
 #define MH_SEG_CELLS 800000L
@@ -173,6 +174,14 @@ inline int node_march_blocks(MhHandle* h, int D) {
   const long threads = (long)h->g.nnx * nt2 * march_nseg((int)na + 1, h->nm_len);
   return (int)(((threads + MH_BLOCK - 1) / MH_BLOCK + 7) / 8 * 8);
 }
+// k_sweep_cell_march: one thread per (x cell, other transverse cell, segment of about MH_CM_L cells along D),
+// for the meshes of its environment counts whose offsets fit 32 bits
+inline bool cell_march(const MhHandle* h) { return MH_CM_HAS(h->g.dim, h->m) && h->g.nn < MH_CM_NODES; }
+inline int cell_march_blocks(const MhHandle* h, int D) {
+  const long na = D == 1 ? h->g.ny : h->g.nz;
+  const long threads = h->g.nc / na * march_nseg((int)na, MH_CM_L(h->g.dim));
+  return (int)(((threads + MH_BLOCK - 1) / MH_BLOCK + 7) / 8 * 8);
+}
 // the y / z variants a single mesh takes (an ensemble's launches are filled by its many cases)
 inline bool seg_sweep(const MhHandle* h) { return !h->sweep_large && h->g.nc < MH_SEG_CELLS; }
 inline bool march_sweep(const MhHandle* h) { return h->sweep_large || h->g.nn >= MH_MARCH_NODES; }
@@ -230,6 +239,7 @@ struct EnsGroup {
   bool lc = false;   // characteristic length other than V^(1/d): k_cell_length first
   bool rows = false; // row-segment x sweeps and LDS-tiled y / z cell sweeps (else one thread per item)
   bool ntile = false;  // 3D: z-marching node kernel
+  bool cmarch = false; // marching y / z cell sweeps instead of tiles
   bool cons = false;   // conservation-energie-totale: dual kinetic energy and its return to the cells
   int lim = -1;
   int bpc = 4;         // persistent blocks per CU of the group's launches (autotuned)

@@ -1445,6 +1445,9 @@ __device__ __forceinline__ void k_sweep_cell_body(const MhDev& S, int lb, int us
   if (S.pm[0]) S.pm[usel ? 0 : 1][c] = 0xff;
 }
 
+// Segments of one line of a marching sweep: n cells or nodes split into ceil(n / len) segments whose
+// lengths differ by at most one, so that no line ends in a short segment that costs a whole pass of threads.
+MH_HD int march_nseg(int n, int len) { return (n + len - 1) / len; }
 // Segments of `len` cells of a line of na cells.
 MH_HD int seg_count(int na, int len) { return (na + len - 1) / len; }
 
@@ -2554,9 +2557,6 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
 #define MH_TILE_L 16  // cells along the sweep direction written per tile (a multiple of 4)
 #endif
 #define MH_TILE_R (MH_TILE_L + 4)  // rows held, halos included
-#ifndef MH_TILE_3SYNC
-#define MH_TILE_3SYNC 1  // one environment: three barriers per remap slot instead of four
-#endif
 #define MH_TILE_Q (MH_TILE_R / 4)  // rows per thread
 #ifndef MH_TILE_MIN_WAVES
 #define MH_TILE_MIN_WAVES 4  // waves per SIMD the register allocation must allow
@@ -2597,11 +2597,6 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
   // (between rows r-1 and r) and the upwind data of that face
   bool val[MH_TILE_Q], inner[MH_TILE_Q], up[MH_TILE_Q];
   double den[MH_TILE_Q], dx[MH_TILE_Q], w[MH_TILE_Q], hh[MH_TILE_Q], xcq[MH_TILE_Q];
-  // one environment: the face gradients are formed where the slopes are (three barriers per
-  // slot); with more, the registers this takes cost more than the barrier saves
-  constexpr bool THREE = MH_TILE_3SYNC != 0 && M == 1;
-  bool innern[THREE ? MH_TILE_Q : 1];  // face r+1 (rows r and r+1) and its Delta x
-  double dxn[THREE ? MH_TILE_Q : 1];
   unsigned ownm = 0;  // bit q: the cell's own U enters its update
 #pragma unroll
   for (int q = 0; q < MH_TILE_Q; ++q) {
@@ -2633,11 +2628,6 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
     const double xcp = r >= 1 ? ssl[r - 1][lx] : 0.;
     dx[q] = (val[q] && valp) ? xcq[q] - xcp : 0.;
     inner[q] = val[q] && valp;  // face between cells a-1 and a
-    if constexpr (THREE) {  // face r+1 as the thread of row r+1 forms it
-      const bool valn = r + 1 < MH_TILE_R && i < nx && a + 1 >= 0 && a + 1 < na;
-      innern[q] = valn && val[q];
-      dxn[q] = innern[q] ? ssl[r + 1][lx] - xcq[q] : 0.;
-    }
     up[q] = false;
     w[q] = 0.;
     hh[q] = 0.;
@@ -2701,28 +2691,18 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
       sphi[ly + 4 * q][lx] = val[q] ? uq[q] / den[q] : 0.;
     }
     __syncthreads();
-    if constexpr (!THREE) {
 #pragma unroll
-      for (int q = 0; q < MH_TILE_Q; ++q) {
-        const int r = ly + 4 * q;
-        sgf[r][lx] = (r >= 1 && inner[q]) ? (sphi[r][lx] - sphi[r - 1][lx]) / dx[q] : 0.;
-      }
-      __syncthreads();
+    for (int q = 0; q < MH_TILE_Q; ++q) {
+      const int r = ly + 4 * q;
+      sgf[r][lx] = (r >= 1 && inner[q]) ? (sphi[r][lx] - sphi[r - 1][lx]) / dx[q] : 0.;
     }
+    __syncthreads();
 #pragma unroll
     for (int q = 0; q < MH_TILE_Q; ++q) {
       const int r = ly + 4 * q;
       double g = 0.;
       if (S.order2 && val[q] && r >= 1 && r <= MH_TILE_R - 2) {
-        double gb, gf;
-        if constexpr (THREE) {  // both face gradients of the row from Phi (the front one is also
-                                // formed by the next row's thread, with the same operands)
-          gb = inner[q] ? (sphi[r][lx] - sphi[r - 1][lx]) / dx[q] : 0.;
-          gf = innern[q] ? (sphi[r + 1][lx] - sphi[r][lx]) / dxn[q] : 0.;
-        } else {
-          gb = sgf[r][lx];
-          gf = sgf[r + 1][lx];
-        }
+        const double gb = sgf[r][lx], gf = sgf[r + 1][lx];
         if (gb != 0.) g += 0.5 * (mh_limiter<LIM>(S.limiter, gf / gb) * gb);
         if (gf != 0.) g += 0.5 * (mh_limiter<LIM>(S.limiter, gb / gf) * gf);
       }
@@ -2775,6 +2755,258 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
       if (val[q] && r >= 2 && r < 2 + MH_TILE_L)
         S.pm[usel ? 0 : 1][c_base + (abase + r) * sD] = (uint8_t)((held >> (M * q)) & ((1u << M) - 1u));
     }
+  }
+}
+
+// The same sweep for D = y or z on large meshes, of one environment or (2D) two: each thread marches
+// along D over a segment.  A row's phi, face gradient, limited slope, face flux and centre are formed
+// once and carried to the next rows in registers (the flux and the U of two rows in LDS, so that 3
+// wavefronts fit a SIMD in 3D and in 2D of one environment 4), without a barrier; a row's U, membership
+// and upper face nodes are in flight while the row before is worked on.  An environment's slots are
+// skipped where no lane holds it in the rows a-3 .. a that the update of row a-2 reaches.  What
+// bounds it is memory: 193 us on the 192^3 blast is 4.6 TB/s of its traffic (two halo rows on each
+// side are read again), and 46 us on 1023x1021; the tiles take 215 and 53 us.  Segments of 8, 24
+// cells: 201, 191 us in 3D, 46 and 80 us in 2D, which runs out of threads.  Two environments in 3D
+// hold 220 registers (187 us on the 256x128x128 tube, tiles 182; with 168 they spill: 690 us), so
+// they and more environments keep the tiles.  Same formulas in the same order as k_sweep_cell_body.
+#define MH_CM_L(DIM) ((DIM) == 3 ? 16 : 8)  // cells along D per segment, about
+#define MH_CM_HAS(DIM, M) ((M) == 1 || ((DIM) == 2 && (M) == 2))
+#define MH_CM_NODES (1L << 29)  // meshes of fewer nodes: 32-bit byte offsets
+template <int DIM, int D, int M, int LIM>
+__device__ __forceinline__ void k_sweep_cell_march_body(const MhDev& S, int lb, int usel, int first) {
+  constexpr int NV = 3 * M + 1, FN = DIM == 3 ? 4 : 2;
+  const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
+  const int na = D == 1 ? ny : nz;
+  const int nt = D == 1 ? (DIM == 3 ? nz : 1) : ny;
+  const int nseg = march_nseg(na, MH_CM_L(DIM));
+  const long g = lb * (long)blockDim.x + threadIdx.x;
+  if (g >= (long)nx * nseg * nt) return;
+  if (mh_halted(S.sc)) return;
+  const int i = (int)(g % nx);
+  const int rest = (int)(g / nx);
+  const int seg = rest % nseg, t = rest / nseg;
+  const int a0 = (int)((long)seg * na / nseg), a1 = (int)((long)(seg + 1) * na / nseg);  // cells a0 .. a1-1
+  const int steps = (na + nseg - 1) / nseg + 4;  // the longest segment and two halo rows on each side
+  const double* __restrict__ Uin = usel ? S.Ub : S.Ua;
+  double* __restrict__ Uout = usel ? S.Ua : S.Ub;
+  double* __restrict__ dflux = S.dflux;
+  const long nc = S.g.nc;
+  const unsigned nnx = S.g.nnx, nny = S.g.nny;
+  // cells and nodes as 32-bit offsets, so that an access is one base in scalar registers and one
+  // offset (the launch sees to it that 8 bytes per node stay below 4 GB)
+  const unsigned sD = D == 1 ? nx : nx * ny, c0 = D == 1 ? i + nx * ny * t : i + nx * t;
+  const unsigned nD = D == 1 ? nnx : nnx * nny, n0 = D == 1 ? i + nnx * nny * t : i + nnx * t;
+  const unsigned fN = D == 1 ? nnx * nny : nnx;  // from a face's first two nodes to the others
+  auto at = [](const double* p, unsigned o) { return *(const double*)((const char*)p + 8u * o); };
+  auto put = [](double* p, unsigned o, double v) { *(double*)((char*)p + 8u * o) = v; };
+  auto node = [&](const double* p, unsigned f, int l) {  // node l of the face whose first node is f
+    const unsigned o = f + (l >= 2 ? fN : 0u);
+    return *(const double*)((const char*)p + 8u * o + (l == 1 || l == 2 ? 8 : 0));
+  };
+  const double dt = S.sc->dt;
+  const double o2 = (double)S.order2;
+  const bool sparse = M > 1 && S.pm[0] != nullptr;
+  const uint8_t* __restrict__ pin = S.pm[usel ? 1 : 0];
+  uint8_t* __restrict__ pout = S.pm[usel ? 0 : 1];
+  auto crow = [&](int a) { return c0 + (unsigned)min(max(a, 0), na - 1) * sD; };
+  auto face = [&](int a) { return n0 + (unsigned)min(max(a, 0), na) * nD; };
+  auto presence = [&](int a) { return sparse ? (unsigned)pin[crow(a)] : 0u; };
+  auto anyof = [&](unsigned b) {  // the environments some lane of the wavefront holds
+    unsigned m = (1u << M) - 1u;
+    if (sparse) {
+#pragma unroll
+      for (int e = 0; e < M; ++e)
+        if (__ballot((b >> e) & 1u) == 0) m &= ~(1u << e);
+    }
+    return m;
+  };
+  // the row in flight: U, membership and volume, and the nodes of its upper face
+  double Un[NV], vl = 1., x[FN][DIM], ux[FN];
+  unsigned mk = 1, held = 0;
+  auto load = [&](int a) {
+    const unsigned c = crow(a);
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+      Un[e] = Un[M + e] = Un[2 * M + e] = 0.;
+      if ((held >> e) & 1u) {
+        Un[e] = at(Uin + e * nc, c);
+        Un[M + e] = at(Uin + (M + e) * nc, c);
+        Un[2 * M + e] = at(Uin + (2 * M + e) * nc, c);
+      }
+    }
+    Un[3 * M] = at(Uin + 3 * M * nc, c);
+    if (first) {
+      mk = S.mask[c];
+      vl = at(S.Vl, c);
+    }
+    const unsigned f = face(a + 1);
+#pragma unroll
+    for (int l = 0; l < FN; ++l) {
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) x[l][d] = node(S.xlc[d], f, l);
+      ux[l] = node(S.u[D], f, l);
+    }
+  };
+  // carried values of the slots: row a-1's phi, the gradient of face a-1, the upwind value of face a-1
+  // where it comes from row a-2; in LDS, U of rows a-1 and a-2 (in turn in 0 and 1) and the flux of face a-2
+  double phiP[NV], gP[NV], pfb[NV];
+  __shared__ double keep[3 * NV][MH_BLOCK];
+  auto kept = [&](int v, int q) -> double& { return keep[3 * v + q][threadIdx.x]; };
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    phiP[v] = gP[v] = pfb[v] = 0.;
+    kept(v, 0) = kept(v, 1) = kept(v, 2) = 0.;
+  }
+  unsigned hist[M];
+#pragma unroll
+  for (int e = 0; e < M; ++e) hist[e] = 0;
+  bool innA = false, upA = false, own1 = false, own2 = false;
+  double wA = 0., hhA = 0., xcP = 0., xfP = 0., vfP = 0., wP = 0., lo[FN];
+#pragma unroll
+  for (int l = 0; l < FN; ++l) lo[l] = node(S.xlc[D], face(a0 - 2), l);
+  unsigned pnext = presence(a0 - 2), old1 = 0, old2 = 0;
+  held = anyof(pnext);
+  load(a0 - 2);
+  pnext = presence(a0 - 1);
+  for (int st = 0; st < steps; ++st) {
+    const int a = a0 - 2 + st;
+    const bool val = a >= 0 && a < na, valp = a - 1 >= 0 && a - 1 < na;
+    const bool inn = val && valp && st > 0;  // face a
+    // row a: U, denominator and centre; the face above it
+    double U[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) U[v] = val ? Un[v] : 0.;
+    double den = 1.;
+    bool own = false;
+    if (val) {
+      if (first) {
+        own = mk != 0;  // an empty cell holds Phi itself and its U starts from 0
+        den = own ? vl : 1.;
+      } else {
+        own = true;
+        den = 0.;
+#pragma unroll
+        for (int k = 0; k < M; ++k) den += Un[k];
+      }
+    }
+    double hi[FN];
+#pragma unroll
+    for (int l = 0; l < FN; ++l) hi[l] = x[l][D];
+    double xc = 0.;
+    if constexpr (DIM == 3 && D == 2) {
+      xc += lo[0]; xc += lo[1]; xc += lo[2]; xc += lo[3];
+      xc += hi[0]; xc += hi[1]; xc += hi[2]; xc += hi[3];
+      xc = 0.125 * xc;
+    } else if constexpr (DIM == 3) {
+      xc += lo[0]; xc += lo[1]; xc += hi[1]; xc += hi[0];
+      xc += lo[3]; xc += lo[2]; xc += hi[2]; xc += hi[3];
+      xc = 0.125 * xc;
+    } else {
+      xc += lo[0]; xc += lo[1]; xc += hi[1]; xc += hi[0];
+      xc = 0.25 * xc;
+    }
+#pragma unroll
+    for (int l = 0; l < FN; ++l) lo[l] = hi[l];
+    double area, xfn = 0., us = 0.;
+    if constexpr (DIM == 3) {
+      const D3 x0 = d3(x[0][0], x[0][1], x[0][2]), x1 = d3(x[1][0], x[1][1], x[1][2]);
+      const D3 x2 = d3(x[2][0], x[2][1], x[2][2]), x3 = d3(x[3][0], x[3][1], x[3][2]);
+      const D3 v1 = x2 - x0, v2 = x3 - x1;
+      if (D == 1) area = 0.5 * fabs(v2.x * v1.z - v2.z * v1.x);
+      else area = 0.5 * fabs(v1.x * v2.y - v1.y * v2.x);
+    } else {
+      area = fabs(x[1][0] - x[0][0]);
+    }
+    const double wf = DIM == 3 ? 0.25 : 0.5;
+#pragma unroll
+    for (int l = 0; l < FN; ++l) xfn += wf * hi[l];
+    if (S.csts) {  // the mean of n and n+1 (PrepareRemap.cc:236-240)
+#pragma unroll
+      for (int l = 0; l < FN; ++l) us += 0.5 * (ux[l] + node(S.un[D], face(a + 1), l));
+    } else {
+#pragma unroll
+      for (int l = 0; l < FN; ++l) us += ux[l];
+    }
+    const double vfn = wf * us, wn = 1. * vfn * area * dt;
+    const unsigned heldc = held;
+    old2 = old1;
+    if (st + 1 < steps) {  // the next row's loads
+      held = anyof(pnext);
+      load(a + 1);
+      pnext = presence(a + 2);
+      if (sparse) old1 = pout[crow(a - 1)];
+    }
+    const double dxr = inn ? xc - xcP : 1.;
+    const bool up = inn && vfP * dxr > 0.0;
+    const double hh = inn ? o2 * (xfP - (up ? xcP : xc)) : 0.;
+    const double w = inn ? wP : 0.;
+    const bool irregular = val && (!mh_finite_nonzero(den) || (inn && (!mh_finite_nonzero(dxr) || !mh_finite(w) || !mh_finite(hh))));
+    const unsigned here = sparse && __ballot(irregular) == 0 ? heldc : (1u << M) - 1u;
+    const MhRecip rden = mh_recip(den), rdx = mh_recip(dxr);
+    const bool out = a - 2 >= a0 && a - 2 < a1;
+    const bool inb = a - 2 > 0, inf = a - 2 < na - 1;
+    const unsigned c = crow(a - 2);
+    unsigned holds = 0;
+    auto slot = [&](int v) {
+      const double phi = mh_quot(U[v], rden);
+      const double gf = inn ? mh_quot(phi - phiP[v], rdx) : 0.;
+      const double sl = S.order2 && valp ? mh_limited_gradient<LIM>(S.limiter, gP[v], gf) : 0.;
+      const double F = innA ? wA * (upA ? pfb[v] : phiP[v] + hhA * sl) : 0.;
+      const double fb = -kept(v, 2), U2 = kept(v, st & 1);
+      if (out) {
+        double ff = 0.;
+        if (inb) ff += fb;
+        if (inf) ff += F;
+        double un = (own2 ? U2 : 0.) - ff;
+        if (v >= M && v < 2 * M) {
+          double dd = 0.;
+          if (inb) dd += 0.5 * fb * -1.;
+          if (inf) dd += 0.5 * F * 1.;
+          put(dflux + (v - M) * nc, c, dd);
+        }
+        if (v >= M && v < 3 * M && un < 0.) un = 0.;
+        if (M > 1 && v < 3 * M) {
+          const int e = v < M ? v : v < 2 * M ? v - M : v - 2 * M;
+          if (un != 0.) holds |= 1u << e;
+          if (!sparse || un != 0. || ((old2 >> e) & 1u)) put(Uout + v * nc, c, un);
+        } else {
+          put(Uout + v * nc, c, un);
+        }
+      }
+      pfb[v] = phiP[v] + hh * sl;
+      kept(v, 2) = F;
+      kept(v, st & 1) = U[v];
+      phiP[v] = phi;
+      gP[v] = gf;
+    };
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+      hist[e] = ((hist[e] << 1) | ((here >> e) & 1u)) & 15u;
+      if (hist[e]) {
+        slot(e);
+        slot(M + e);
+        slot(2 * M + e);
+      } else if (out) {
+        put(dflux + e * nc, c, 0.);
+        if ((old2 >> e) & 1u) {
+          put(Uout + e * nc, c, 0.);
+          put(Uout + (M + e) * nc, c, 0.);
+          put(Uout + (2 * M + e) * nc, c, 0.);
+        }
+      }
+    }
+    slot(3 * M);
+    if (sparse && out) pout[c] = (uint8_t)holds;
+    xfP = xfn;
+    vfP = vfn;
+    wP = wn;
+    innA = inn;
+    upA = up;
+    wA = w;
+    hhA = hh;
+    xcP = xc;
+    own2 = own1;
+    own1 = own;
   }
 }
 
@@ -3070,9 +3302,6 @@ __device__ __forceinline__ void k_sweep_node_body(const MhDev& S, int lb, int ps
 #ifndef MH_NM_L
 #define MH_NM_L 10  // default target segment length (MhDev::nm_len; variant march code 0, kMarchLen[0])
 #endif
-// Segments of one node line: the n nodes split into ceil(n / len) segments whose lengths differ
-// by at most one, so that no line ends in a short segment that costs a whole pass of threads.
-MH_HD int march_nseg(int n, int len) { return (n + len - 1) / len; }
 #ifndef MH_NM_MIN_WAVES
 #define MH_NM_MIN_WAVES 1
 #endif
@@ -3695,28 +3924,25 @@ __device__ __forceinline__ bool cfl_fold(const double* __restrict__ partial, int
   // without a NaN candidate anywhere the fold is a plain minimum, in any order
   if (threadIdx.x == 0) any_nan = 0;
   __syncthreads();
-  // four independent running minima keep four loads in flight per thread (the minimum of
-  // non-NaN values does not depend on the order)
-  const double qnan = __longlong_as_double(0x7ff8000000000000LL);
-  double pm = qnan, pm1 = qnan, pm2 = qnan, pm3 = qnan;
+  // eight partials in flight per thread, the last one again where there are fewer (the minimum of
+  // non-NaN values depends neither on the order nor on a repetition)
+  double pm = __longlong_as_double(0x7ff8000000000000LL);
   int pn = 0;
   const int bd = (int)blockDim.x;
-  int b = threadIdx.x;
-  for (; b + 3 * bd < nblocks; b += 4 * bd) {
-    const double a0 = partial[2 * b], a1 = partial[2 * (b + bd)];
-    const double a2 = partial[2 * (b + 2 * bd)], a3 = partial[2 * (b + 3 * bd)];
-    pn |= (partial[2 * b + 1] != 0.) | (partial[2 * (b + bd) + 1] != 0.) |
-          (partial[2 * (b + 2 * bd) + 1] != 0.) | (partial[2 * (b + 3 * bd) + 1] != 0.);
-    pm = min_skip_nan(pm, a0);
-    pm1 = min_skip_nan(pm1, a1);
-    pm2 = min_skip_nan(pm2, a2);
-    pm3 = min_skip_nan(pm3, a3);
+  for (int b = threadIdx.x; b < nblocks; b += 8 * bd) {
+    double m[8], f[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int o = min(b + u * bd, nblocks - 1);
+      m[u] = partial[2 * o];
+      f[u] = partial[2 * o + 1];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      pm = min_skip_nan(pm, m[u]);
+      pn |= f[u] != 0.;
+    }
   }
-  for (; b < nblocks; b += bd) {
-    pm = min_skip_nan(pm, partial[2 * b]);
-    pn |= partial[2 * b + 1] != 0.;
-  }
-  pm = min_skip_nan(min_skip_nan(pm, pm1), min_skip_nan(pm2, pm3));
   for (int off = 32; off > 0; off >>= 1) pm = min_skip_nan(pm, __shfl_xor(pm, off, 64));
   if (__ballot(pn) != 0 && lane == 0) any_nan = 1;
   if (lane == 0) rm[wid] = pm;
@@ -3767,19 +3993,21 @@ __device__ __forceinline__ bool cfl_fold(const double* __restrict__ partial, int
 // of the iteration and the final-time stop rule.  One block.
 __device__ __forceinline__ void k_dt_body(const MhDev& S) {
   MhScalars* sc = S.sc;
-  if (mh_halted(sc)) return;
+  // the scalars are read ahead of the fold: one round of loads instead of three
+  const bool halted = mh_halted(sc);
+  const double dt = sc->dt, t0 = sc->t;
+  const int it = sc->iteration + 1;
+  int status = S.err[0];
   double mn;
-  if (!cfl_fold(S.partial, S.nblk_c, &mn)) return;
-  const double dt = sc->dt;
-  const double t = sc->t + dt;
+  if (!cfl_fold(S.partial, S.nblk_c, &mn) || halted) return;
+  const double t = t0 + dt;
   double new_dt = S.cfl * mn;
   new_dt = amin(new_dt, 1.05 * dt);
   new_dt = amin(new_dt, S.dtmax);
-  int status = S.err[0];
   if (S.sans_lagrange) new_dt = S.dt_init;  // advection mode keeps deltat-init (:1751-1753)
   else if (status == 0 && new_dt < S.dtmin) status = MH_ERR_DT_MIN;
   sc->t = t;
-  sc->iteration = sc->iteration + 1;
+  sc->iteration = it;
   sc->dxmin = mn;
   if (status != 0) {
     sc->status = status;
@@ -3789,7 +4017,7 @@ __device__ __forceinline__ void k_dt_body(const MhDev& S) {
   sc->dt = new_dt;
   const double T = S.tfinal;
   if ((t < T && t + new_dt > T) || t > T) sc->stopped = 1;
-  if (S.max_iter > 0 && sc->iteration >= S.max_iter) sc->stopped = 1;
+  if (S.max_iter > 0 && it >= S.max_iter) sc->stopped = 1;
 }
 
 
@@ -3928,6 +4156,8 @@ MH_WRAP(k_sweep_cell_row, 1, template <int DIM MH_COMMA int M MH_COMMA int LIM>,
 MH_WRAP(k_sweep_cell_tile, MH_TILE_MIN_WAVES,
         template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
+MH_WRAP(k_sweep_cell_march, 1, template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>,
+        <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>, MH_COMMA int usel MH_COMMA int first, MH_COMMA usel MH_COMMA first)
 MH_WRAP(k_sweep_node_row, 1, template <int DIM MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA M MH_COMMA LIM>,
         MH_COMMA int psel MH_COMMA int prev MH_COMMA int last, MH_COMMA psel MH_COMMA prev MH_COMMA last)
 MH_WRAP(k_hcell, 1, template <int DIM>, <DIM>, , )

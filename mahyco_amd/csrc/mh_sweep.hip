@@ -43,6 +43,10 @@ void launch_cell_yz(MhHandle* h, int sel, int first) {
     const SlotSplit p = slot_split((long)seg_blocks(h, D, MH_SEG_L) * (MH_BLOCK / 64), 2048, 3 * M + 1);
     MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + D, (k_sweep_cell_seg<DIM, D, M, LIM, MH_SEG_L>),
                        dim3(seg_blocks(h, D, MH_SEG_L), p.groups), MH_BLOCK, S, sel, first, p.vper));
+  } else if (MH_CM_HAS(DIM, M) && cell_march(h)) {
+    if constexpr (MH_CM_HAS(DIM, M))
+      MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + D, (k_sweep_cell_march<DIM, D, M, LIM>), cell_march_blocks(h, D), MH_BLOCK,
+                         S, sel, first));
   } else {
     MH_LIMSW(h, LAUNCH(h, KN_SWEEP_CELL + D, (k_sweep_cell_tile<DIM, D, M, LIM>), tile_blocks(h, D), MH_BLOCK, S, sel,
                        first));
@@ -169,8 +173,13 @@ void ens_sweep(const EnsGroup& g, const MhDev* tab, hipStream_t st, dim3 G, int 
     if (!g.adv)
       hipLaunchKernelGGL((k_sweep_node_row_batch<DIM, M, LIM>), G, B, 0, st, tab, MH_LIST(g.rnmap), sel, prev, last);
   } else if (g.rows) {
-    hipLaunchKernelGGL((k_sweep_cell_tile_batch<DIM, D, M, LIM>), G, B, 0, st, tab, MH_LIST(g.tmap[D == 0 ? 0 : D - 1]),
-                       sel, first);
+    constexpr int DT = D == 0 ? 1 : D;
+    if (MH_CM_HAS(DIM, M) && g.cmarch) {
+      if constexpr (MH_CM_HAS(DIM, M))
+        hipLaunchKernelGGL((k_sweep_cell_march_batch<DIM, DT, M, LIM>), G, B, 0, st, tab, MH_LIST(g.tmap[DT - 1]), sel, first);
+    } else {
+      hipLaunchKernelGGL((k_sweep_cell_tile_batch<DIM, DT, M, LIM>), G, B, 0, st, tab, MH_LIST(g.tmap[DT - 1]), sel, first);
+    }
     if (!g.adv && !g.o3)  // threads march along D over segments of nodes
       hipLaunchKernelGGL((k_sweep_node_march_batch<DIM, (D == 0 ? 1 : D), M, LIM>), G, B, 0, st, tab,
                          MH_LIST(g.mmap[D == 0 ? 0 : D - 1]), sel, prev, last);

@@ -148,3 +148,16 @@ def test_node_kernels_at_block_edges(n, kw, variant):
     assert g.run(7) == o.run(7)
     a, b = fields(g, 2, 3), fields(o, 2, 3)
     assert not [k for k in a if not bitwise_equal(a[k], b[k])]
+
+
+# the marching cell sweeps: lines shorter than a segment, segments of unequal length, wavefronts
+# that span lines, one environment (2D, 3D) and two (2D, above with MAHYCO_SWEEP=tile)
+@pytest.mark.parametrize("sweep", ["tile", "flat"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (5, 17, 33), (61, 16, 15), (3, 47, 1), (70, 34, 5), (2, 2), (65, 9), (7, 41)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_one_environment_marching_sweeps(n, sweep, monkeypatch):
+    monkeypatch.setenv("MAHYCO_SWEEP", sweep)
+    c = moving_tube(n, n[0] % 3)
+    # a single-material tube along one of the axes
+    c.envs, c.cas_model, c.cas_test = c.envs[:1], T.MH_CASE_SOD, 3 + (n[0] + n[1]) % len(n)
+    check(c)
