@@ -161,3 +161,13 @@ def test_one_environment_marching_sweeps(n, sweep, monkeypatch):
     # a single-material tube along one of the axes
     c.envs, c.cas_model, c.cas_test = c.envs[:1], T.MH_CASE_SOD, 3 + (n[0] + n[1]) % len(n)
     check(c)
+
+
+@pytest.mark.parametrize("envs", [1, 2])
+@pytest.mark.parametrize("n", [(7, 41), (5, 17, 33)], ids=lambda n: "x".join(map(str, n)))
+def test_csts_velocities_in_the_large_mesh_sweeps(n, envs, monkeypatch):
+    monkeypatch.setenv("MAHYCO_SWEEP", "tile")
+    c = moving_tube(n, 0, schema_csts=True)
+    if envs == 1:
+        c.envs, c.cas_model, c.cas_test = c.envs[:1], T.MH_CASE_SOD, 4
+    check(c)
