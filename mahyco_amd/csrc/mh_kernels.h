@@ -3019,21 +3019,25 @@ __device__ __forceinline__ void k_sweep_cell_march_body(const MhDev& S, int lb, 
 // segments of a column, then over the columns, so any nx fills the wavefronts and consecutive
 // segments share their halo cells in L2.  Against the tiles, two environments: 15 -> 8 us on
 // 100x5x5 cells, 27 -> 10 us on 181x181, 29 -> 21 us on 512x512x1, 44 -> 39 us on 97x61x83; longer
-// segments are slower there (four cells: 10, 14, 24, 37 us).  Same formulas in the same order as
-// k_sweep_cell_body.
+// segments are slower there (four cells: 10, 14, 24, 37 us).  In 2D no branch parts the loads of the
+// prologue (y sweep with its events 12.2 -> 11.1 us on 181x181, 21.7 -> 20.4 on 512x512, 41.4 -> 39.9
+// on 850x850); in 3D those loads take 214 registers instead of 126: no gain on 16^3 to 64^3, and 33 ->
+// 39 us on 80^3.  Same formulas in the same order as k_sweep_cell_body.
 #ifndef MH_SEG_L
 #define MH_SEG_L 2  // cells along D per thread
 #endif
 template <int DIM, int D, int M, int LIM, int L>
 __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, int usel, int first, int v0, int v1) {
   constexpr int R = L + 4;
+  constexpr bool FEW = DIM == 2;  // all loads of the prologue in flight together
   const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
   const int na = D == 1 ? ny : nz;
   const int nt = D == 1 ? (DIM == 3 ? nz : 1) : ny;
   const int nseg = seg_count(na, L);
   const long g = lb * (long)blockDim.x + threadIdx.x;
   if (g >= (long)nx * nseg * nt) return;
-  if (mh_halted(S.sc)) return;
+  const bool halted = mh_halted(S.sc);
+  if (!FEW && halted) return;
   const int i = (int)(g % nx);
   const int rest = (int)(g / nx);
   const int abase = (rest % nseg) * L - 2;  // cell along D of row 0
@@ -3044,60 +3048,71 @@ __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, in
   const long nc = S.g.nc;
   const long nnx = S.g.nnx, nny = S.g.nny;
   const long sD = D == 1 ? (long)nx : (long)nx * ny;
-  const long c0 = (D == 1 ? i + (long)nx * ny * t : i + (long)nx * t) + abase * sD;
+  const long cl = D == 1 ? i + (long)nx * ny * t : i + (long)nx * t;  // the column's cell and node at 0
+  const long c0 = cl + abase * sD;
   const long nD = D == 1 ? nnx : nnx * nny;
-  const long n0 = (D == 1 ? i + nnx * nny * t : i + nnx * t) + abase * nD;
+  const long nl = D == 1 ? i + nnx * nny * t : i + nnx * t;
   const double dt = S.sc->dt;
   const double o2 = (double)S.order2;
   auto valid = [&](int r) { return abase + r >= 0 && abase + r < na; };
   auto inner = [&](int f) { return valid(f - 1) && valid(f); };  // face f: between rows f-1 and f
+  // FEW: a row beyond the mesh is its end row again (unused), so that no branch parts the loads
+  auto row = [&](int r) { return min(max(abase + r, 0), na - 1); };
+  auto slot_of = [&](int v, int r) {
+    if (FEW) return Uin[v * nc + cl + row(r) * sD];
+    return valid(r) ? Uin[v * nc + c0 + r * sD] : 0.;
+  };
   double u[R], un[R];  // slot loads run one slot ahead
 #pragma unroll
-  for (int r = 0; r < R; ++r) un[r] = valid(r) ? Uin[v0 * nc + c0 + r * sD] : 0.;
+  for (int r = 0; r < R; ++r) un[r] = slot_of(v0, r);
   unsigned ownm = 0;  // bit r: the cell's own U enters its update
   MhRecip den[R], dx[R];
-  double xc[R], w[R], hh[R];
+  double xc[R], w[R], hh[R], d[R], area[R], xf[R], vf[R];
   unsigned upm = 0;  // bit f: the upwind cell of face f is the one behind it
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    double d = 1.;
+    d[r] = 1.;
     xc[r] = 0.;
-    if (valid(r)) {
-      const long c = c0 + r * sD;
+    if (FEW || valid(r)) {
+      const long c = cl + row(r) * sD;
       if (first) {
         const bool empty = !S.mask[c];  // an empty cell holds Phi itself and its U starts from 0
-        d = empty ? 1. : S.Vl[c];
+        d[r] = empty ? 1. : S.Vl[c];
         if (!empty) ownm |= 1u << r;
       } else {
         ownm |= 1u << r;
         double sv = 0.;
+#pragma unroll
         for (int k = 0; k < M; ++k) sv += Uin[k * nc + c];
-        d = sv;
+        d[r] = sv;
       }
-      xc[r] = cell_centre_d<DIM, D>(S, n0 + r * nD);
+      xc[r] = cell_centre_d<DIM, D>(S, nl + row(r) * nD);
     }
-    den[r] = mh_recip(d);
   }
 #pragma unroll
+  for (int f = 2; f <= R - 2; ++f)
+    if (FEW || inner(f)) face_quant<DIM, D>(S, nl + row(f) * nD, area[f], xf[f], vf[f]);
+  if (FEW && halted) return;
+#pragma unroll
+  for (int r = 0; r < R; ++r) den[r] = mh_recip(valid(r) ? d[r] : 1.);
+#pragma unroll
   for (int f = 1; f < R; ++f) {
-    const double d = inner(f) ? xc[f] - xc[f - 1] : 1.;
-    dx[f] = mh_recip(d);
+    const double dxf = inner(f) ? xc[f] - xc[f - 1] : 1.;
+    dx[f] = mh_recip(dxf);
     w[f] = 0.;
     hh[f] = 0.;
     if (f >= 2 && f <= R - 2 && inner(f)) {
-      double area, xf, vf;
-      face_quant<DIM, D>(S, n0 + f * nD, area, xf, vf);
-      const bool up = vf * d > 0.0;
+      const bool up = vf[f] * dxf > 0.0;
       if (up) upm |= 1u << f;
-      hh[f] = o2 * (xf - (up ? xc[f - 1] : xc[f]));
-      w[f] = 1. * vf * area * dt;
+      hh[f] = o2 * (xf[f] - (up ? xc[f - 1] : xc[f]));
+      w[f] = 1. * vf[f] * area[f] * dt;
     }
   }
   for (int v = v0; v < v1; ++v) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       u[r] = un[r];
-      if (v + 1 < v1) un[r] = valid(r) ? Uin[(v + 1) * nc + c0 + r * sD] : 0.;
+      if (v + 1 < v1) un[r] = slot_of(v + 1, r);
     }
     double phi[R], gr[R];
     bool bad = false;
