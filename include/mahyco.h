@@ -60,7 +60,8 @@ long mahyco_graph_captures(MhHandle* h);
 
 /* Copies one field (MhField) to host memory `out` (nb_cells or nb_nodes doubles).
  * Cell fields: env = -1 (cell value) or environment index (0 outside the env).
- * Node fields: comp = 0,1,2.  Replaces reading the Arcane variables by name. */
+ * Node fields: comp = 0,1,2.  Replaces reading the Arcane variables by name.  Several threads may read
+ * fields of one case, or of the members of one ensemble, at the same time. */
 int mahyco_get_field(MhHandle* h, int field, int env, int comp, double* out);
 
 /* Writes one field of the state from host memory (nb_cells or nb_nodes doubles); replaces a

@@ -6,7 +6,8 @@
 // formed per cell, by a kernel that writes it there, and emptied by the calling thread and up to
 // seven more: 68 us and 2.0 ms.  One thread below 4 MB (two copy 1 MB no faster than one), one more
 // per 2 MB, eight at most (12 are slower); 4 MB slots at most (2 MB ones take 3.4 ms for 57 MB).
-// The slots belong to a case or an ensemble, at most 16 MB, and are freed with it.
+// The slots belong to a case or an ensemble, at most 16 MB, and are freed with it.  Threads that read
+// fields of one case, or of the members of one ensemble, take turns.
 #ifndef MH_READBACK_H
 #define MH_READBACK_H
 
@@ -15,12 +16,14 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
 #include <thread>
 
 #include "mh_state.h"
 
 struct HostStage {
   static constexpr int kSlots = 4;
+  std::mutex mu;  // held by a read from its first use of the slots to its last
   char* pin = nullptr;
   size_t slot = 0;  // bytes of a slot
   int slots = 0;
@@ -77,6 +80,7 @@ struct HostStage {
 template <class Fill>
 hipError_t read_back(HostStage& st, hipStream_t stream, char* dst, size_t n, Fill fill) {
   if (!n) return hipSuccess;
+  std::lock_guard<std::mutex> turn(st.mu);
   hipError_t err = st.reserve(n);
   if (err != hipSuccess) return err;
   const int R = st.slots;

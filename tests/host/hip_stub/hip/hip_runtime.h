@@ -1,0 +1,61 @@
+// Stand-in for the HIP calls of mh_readback.h, so that its host side runs on a CPU: streams run
+// everything at once, pinned memory is ordinary memory and is overwritten before it is freed.
+#ifndef MH_HIP_STUB_H
+#define MH_HIP_STUB_H
+#include <cstddef>
+#include <cstdint>
+#include <cstdlib>
+#include <cstring>
+
+#define __global__
+#define __device__
+#define __host__
+#define __launch_bounds__(...)
+
+enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorInvalidHandle = 400 };
+struct StubStream {
+  int device = 0;
+};
+struct StubEvent {
+  int device = 0;
+};
+typedef StubStream* hipStream_t;
+typedef StubEvent* hipEvent_t;
+enum { hipEventDisableTiming = 2, hipHostMallocDefault = 0 };
+
+struct StubDim {
+  unsigned x = 0, y = 0, z = 0;
+};
+static thread_local StubDim blockIdx, threadIdx;
+static inline int __popc(unsigned x) { return __builtin_popcount(x); }
+static inline int __ffs(unsigned x) { return __builtin_ffs((int)x); }
+
+static size_t stub_head = 64;  // the size of an allocation lies ahead of it
+static inline hipError_t hipHostMalloc(void** p, size_t n, unsigned = 0) {
+  char* b = (char*)std::malloc(n + stub_head);
+  if (!b) return hipErrorOutOfMemory;
+  std::memcpy(b, &n, sizeof n);
+  *p = b + stub_head;
+  return hipSuccess;
+}
+static inline hipError_t hipHostFree(void* p) {
+  char* b = (char*)p - stub_head;
+  size_t n;
+  std::memcpy(&n, b, sizeof n);
+  std::memset(p, 0xee, n);
+  std::free(b);
+  return hipSuccess;
+}
+static inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = new StubEvent;
+  return hipSuccess;
+}
+static inline hipError_t hipEventDestroy(hipEvent_t e) {
+  delete e;
+  return hipSuccess;
+}
+static inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+static inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+static inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+static inline hipError_t hipGetLastError() { return hipSuccess; }
+#endif

@@ -1,0 +1,30 @@
+"""The host side of the pinned read-back (mahyco_amd/csrc/mh_readback.h) on the CPU, over stand-ins of
+the HIP calls (tests/host/hip_stub)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def checker(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = str(tmp_path_factory.mktemp("readback") / "readback_check")
+    subprocess.run(["g++", "-O2", "-g", "-std=c++17", "-pthread", "-I", os.path.join(HERE, "host", "hip_stub"),
+                    os.path.join(HERE, "host", "readback_check.cpp"), "-o", exe], check=True)
+    return exe
+
+
+def _run(checker, check):
+    r = subprocess.run([checker, check], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    return tuple(map(int, r.stdout.split()))
+
+
+def test_threads_share_one_stage(checker):
+    """Reads of one case by several threads: each gets its own field, whatever the others read."""
+    assert _run(checker, "threads") == (48, 0)
