@@ -9,7 +9,9 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -1204,27 +1206,57 @@ long mahyco_nb_cells(MhHandle* h) { return h ? h->g.nc : -1; }
 long mahyco_graph_captures(MhHandle* h) { return h ? h->graph_captures : -1; }
 long mahyco_nb_nodes(MhHandle* h) { return h ? h->g.nn : -1; }
 
-static int get_field(MhHandle* h, HostStage& stage, int field, int env, int comp, double* out) {
+inline unsigned read_blocks(long n) { return (unsigned)((n + MH_BLOCK - 1) / MH_BLOCK); }
+// One array of n doubles to host memory (its stream is idle).
+static int read_array(MhHandle* h, const double* d, double* out, long n) {
+  const size_t bytes = n * sizeof(double);
+  auto fill = [&](char* pin, size_t off, size_t len) {
+    const long k = (long)(len / sizeof(double));
+    hipLaunchKernelGGL(k_read_array<>, dim3(read_blocks(k)), dim3(MH_BLOCK), 0, h->stream, d + off / sizeof(double),
+                       (double*)pin, k);
+    return hipGetLastError();
+  };
+  auto plain = [&] { return hipMemcpy(out, d, bytes, hipMemcpyDeviceToHost); };
+  return hip_check(read_back(read_pool(), h->stream, (char*)out, bytes, array_gain(bytes), fill, plain), "read back");
+}
+// Values formed per cell (field_value) from the membership, g [nc] and e [ne].
+static int read_formed(MhHandle* h, int field, int env, const double* g, const double* e, long ne, double* out) {
+  const long nc = h->g.nc;
+  const size_t bytes = nc * sizeof(double);
+  auto fill = [&](char* pin, size_t off, size_t len) {
+    const long n = (long)(len / sizeof(double));
+    hipLaunchKernelGGL(k_read_field<>, dim3(read_blocks(n)), dim3(MH_BLOCK), 0, h->stream, field, env, h->m, nc,
+                       h->dev.mask, g, e, (double*)pin, (long)(off / sizeof(double)), n);
+    return hipGetLastError();
+  };
+  auto plain = [&]() -> hipError_t {
+    std::unique_ptr<uint8_t[]> mask(new (std::nothrow) uint8_t[nc]);
+    std::unique_ptr<double[]> hg(new (std::nothrow) double[g ? nc : 1]), he(new (std::nothrow) double[e ? ne : 1]);
+    if (!mask || !hg || !he) return hipErrorOutOfMemory;
+    hipError_t r = hipMemcpy(mask.get(), h->dev.mask, nc, hipMemcpyDeviceToHost);
+    if (r == hipSuccess && g) r = hipMemcpy(hg.get(), g, bytes, hipMemcpyDeviceToHost);
+    if (r == hipSuccess && e) r = hipMemcpy(he.get(), e, ne * sizeof(double), hipMemcpyDeviceToHost);
+    if (r != hipSuccess) return r;
+    for (long c = 0; c < nc; ++c) out[c] = field_value(field, env, h->m, nc, mask[c], hg.get(), e ? he.get() : nullptr, c);
+    return hipSuccess;
+  };
+  return hip_check(read_back(read_pool(), h->stream, (char*)out, bytes, formed_gain(bytes), fill, plain), "read back");
+}
+
+int mahyco_get_field(MhHandle* h, int field, int env, int comp, double* out) {
+  if (!h || !out) return MH_ERR_INVALID;
   MhScalars sc;
   int st = read_scalars(h, &sc);
   if (st != MH_OK) return st;
   const long nc = h->g.nc, nn = h->g.nn;
   MhDev& S = h->dev;
-  // (the stream is idle: read_scalars waited for it)
-  auto d2h = [&](const double* d, double* hst, long n) -> int {
-    return hip_check(read_back(stage, h->stream, (char*)hst, n * sizeof(double),
-                               [&](char* pin, size_t off, size_t len) {
-                                 return hipMemcpyAsync(pin, (const char*)d + off, len, hipMemcpyDeviceToHost, h->stream);
-                               }),
-                     "read back");
-  };
   if (field >= 100) {
     if (comp < 0 || comp > 2) return MH_ERR_INVALID;
-    if (field == MH_N_VELOCITY) return d2h(S.u[comp], out, nn);
+    if (field == MH_N_VELOCITY) return read_array(h, S.u[comp], out, nn);
     if (field == MH_N_NODE_MASS) {
       // m_node_mass after the iteration: sum over cells of M / 2^dim, in cell order
       std::vector<double> M(nc);
-      st = d2h(S.M, M.data(), nc);
+      st = read_array(h, S.M, M.data(), nc);
       if (st != MH_OK) return st;
       const MhGrid& g = h->g;
       const double w = g.dim == 3 ? .125 : .25;
@@ -1256,46 +1288,38 @@ static int get_field(MhHandle* h, HostStage& stage, int field, int env, int comp
         }
         return MH_OK;
       }
-      return d2h(h->xl[sc.iteration & 1][comp], out, nn);
+      return read_array(h, h->xl[sc.iteration & 1][comp], out, nn);
     }
-    if (field == MH_N_COORD_LAGRANGE) return d2h(h->xl[sc.iteration & 1][comp], out, nn);
+    if (field == MH_N_COORD_LAGRANGE) return read_array(h, h->xl[sc.iteration & 1][comp], out, nn);
     return MH_ERR_INVALID;
   }
   if (env >= h->m || env < -1) return MH_ERR_INVALID;
-  const double* gsrc = nullptr;
-  const double* esrc = nullptr;
-  bool formed = env >= 0;  // per cell, from more than one array
+  const double* g = nullptr;
+  const double* e = nullptr;
   switch (field) {
-    case MH_F_DENSITY: gsrc = S.rho; esrc = S.rhok; break;
-    case MH_F_PRESSURE: gsrc = S.p; esrc = S.pk; break;
-    case MH_F_INTERNAL_ENERGY: gsrc = S.e; esrc = S.ek; break;
-    case MH_F_SOUND_SPEED: gsrc = S.c; break;
-    case MH_F_PSEUDO_VISCOSITY: gsrc = S.q; break;
-    case MH_F_CELL_MASS: gsrc = S.M; esrc = S.Mk; break;
-    case MH_F_FRACVOL: gsrc = S.fg; esrc = S.fk; break;
-    case MH_F_CARACTERISTIC_LENGTH: gsrc = S.L; break;
-    case MH_F_CELL_VOLUME: gsrc = !h->opt.with_projection && sc.iteration > 0 ? S.Vl : S.VE; break;
+    case MH_F_DENSITY: g = S.rho; e = S.rhok; break;
+    case MH_F_PRESSURE: g = S.p; e = S.pk; break;
+    case MH_F_INTERNAL_ENERGY: g = S.e; e = S.ek; break;
+    case MH_F_SOUND_SPEED: g = S.c; break;
+    case MH_F_PSEUDO_VISCOSITY: g = S.q; break;
+    case MH_F_CELL_MASS: g = S.M; e = S.Mk; break;
+    case MH_F_FRACVOL: g = S.fg; e = S.fk; break;
+    case MH_F_CARACTERISTIC_LENGTH: g = S.L; break;
+    case MH_F_CELL_VOLUME: g = !h->opt.with_projection && sc.iteration > 0 ? S.Vl : S.VE; e = S.fk; break;
     case MH_F_MASS_FRACTION:
-    case MH_F_MATERIAU:
-    case MH_F_ENV_MASK: formed = true; break;
+      if (env < 0) {
+        std::fill(out, out + nc, 0.);
+        return MH_OK;
+      }
+      g = S.chig;
+      e = S.chik;
+      break;
+    case MH_F_MATERIAU: return read_formed(h, field, env, S.fg, S.fk, h->m * nc, out);
+    case MH_F_ENV_MASK: return read_formed(h, field, env, nullptr, nullptr, 0, out);
     default: return MH_ERR_INVALID;
   }
-  if (!formed) return d2h(gsrc, out, nc);
-  const double* ek = esrc && env >= 0 ? esrc + (size_t)env * nc : nullptr;
-  return hip_check(read_back(stage, h->stream, (char*)out, nc * sizeof(double),
-                             [&](char* pin, size_t off, size_t len) {
-                               const long n = (long)(len / sizeof(double));
-                               hipLaunchKernelGGL(k_read_field<>, dim3((unsigned)((n + MH_BLOCK - 1) / MH_BLOCK)),
-                                                  dim3(MH_BLOCK), 0, h->stream, S, field, env, gsrc, ek, (double*)pin,
-                                                  (long)(off / sizeof(double)), n);
-                               return hipGetLastError();
-                             }),
-                   "read back");
-}
-
-int mahyco_get_field(MhHandle* h, int field, int env, int comp, double* out) {
-  if (!h || !out) return MH_ERR_INVALID;
-  return get_field(h, h->stage, field, env, comp, out);
+  if (env < 0) return read_array(h, g, out, nc);
+  return read_formed(h, field, env, g, e ? e + (size_t)env * nc : nullptr, nc, out);
 }
 
 static void drop_graphs(MhHandle* h);
@@ -1624,7 +1648,7 @@ int mahyco_ensemble_get_field(MhEnsemble* e, int slot, int field, int env, int c
   if (!E || slot < 0 || slot >= E->max_slots || !E->slot[slot]) return MH_ERR_INVALID;
   if (!out) return MH_ERR_INVALID;
   HIPCHK(hipStreamSynchronize(E->stream));
-  return get_field(E->slot[slot], E->field_stage, field, env, comp, out);
+  return mahyco_get_field(E->slot[slot], field, env, comp, out);
 }
 
 double mahyco_ensemble_used_bytes(MhEnsemble* e) {

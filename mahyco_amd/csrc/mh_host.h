@@ -85,7 +85,7 @@ struct MhHandle {
   std::vector<hipGraph_t> graph_defs;
   long graph_captures = 0;  // graphs captured and instantiated so far
   bool owns_stream = true;
-  HostStage stage;  // pinned slots of mahyco_get_field
+  ReadPoolUser reads;       // keeps the pinned slots that fields are read through
   bool node_tiled = true;   // 3D: z-marching node kernel (MAHYCO_NODE_KERNEL=flat: k_node_lag3_split)
   bool cell_tiled = false;  // 3D remap loop: LDS-staged cell kernel (MAHYCO_CELL_KERNEL=tiled; an autotuner candidate)
   bool staged = false;      // Lagrangian state written before the remap, U formed from it (mahyco_set_staged)
@@ -285,7 +285,7 @@ struct MhEnsembleImpl {
   MhScalars* snap = nullptr;       // pinned, max_slots entries
   hipEvent_t snap_done = nullptr;
   bool snap_pending = false;
-  HostStage field_stage;           // pinned slots of mahyco_ensemble_get_field
+  ReadPoolUser reads;              // keeps the pinned slots that fields are read through
   std::vector<int> snap_state;     // slot state when the snapshot was taken: -100 empty, 2 pending, 1 active
 };
 

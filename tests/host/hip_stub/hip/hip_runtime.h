@@ -2,6 +2,7 @@
 // everything at once, pinned memory is ordinary memory and is overwritten before it is freed.
 #ifndef MH_HIP_STUB_H
 #define MH_HIP_STUB_H
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <cstdlib>
@@ -27,15 +28,16 @@ struct StubDim {
   unsigned x = 0, y = 0, z = 0;
 };
 static thread_local StubDim blockIdx, threadIdx;
-static inline int __popc(unsigned x) { return __builtin_popcount(x); }
-static inline int __ffs(unsigned x) { return __builtin_ffs((int)x); }
 
 static size_t stub_head = 64;  // the size of an allocation lies ahead of it
+static std::atomic<long> stub_pins{0}, stub_pinned{0};  // allocations made, bytes held
 static inline hipError_t hipHostMalloc(void** p, size_t n, unsigned = 0) {
   char* b = (char*)std::malloc(n + stub_head);
   if (!b) return hipErrorOutOfMemory;
   std::memcpy(b, &n, sizeof n);
   *p = b + stub_head;
+  ++stub_pins;
+  stub_pinned += (long)n;
   return hipSuccess;
 }
 static inline hipError_t hipHostFree(void* p) {
@@ -43,6 +45,7 @@ static inline hipError_t hipHostFree(void* p) {
   size_t n;
   std::memcpy(&n, b, sizeof n);
   std::memset(p, 0xee, n);
+  stub_pinned -= (long)n;
   std::free(b);
   return hipSuccess;
 }

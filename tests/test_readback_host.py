@@ -25,6 +25,11 @@ def _run(checker, check):
     return tuple(map(int, r.stdout.split()))
 
 
-def test_threads_share_one_stage(checker):
-    """Reads of one case by several threads: each gets its own field, whatever the others read."""
+def test_threads_share_the_slots(checker):
+    """Reads by several threads: each gets its own field, whatever the others read."""
     assert _run(checker, "threads") == (48, 0)
+
+
+def test_what_reads_pin(checker):
+    """A single read pins no more than it gains; pinned memory is bounded and given back."""
+    assert _run(checker, "pinning") == (66, 0)
