@@ -54,7 +54,7 @@ struct HostStage {
     if (holds(n)) return hipSuccess;
     release();
     hipError_t e = hipErrorOutOfMemory;
-    for (size_t s = size(n); s >= 4096; s /= 2) {  // with less where pinned memory is short
+    for (size_t s = size(n); s >= (64u << 10); s /= 2) {  // with less where pinned memory is short
       e = hipHostMalloc((void**)&pin, count(n) * s, hipHostMallocDefault);
       if (e == hipSuccess) {
         slot = s;
@@ -131,12 +131,12 @@ struct ReadPoolUser {
 inline double array_gain(size_t n) { return n < HostStage::kArray ? 0. : n / 1048576. * 80.; }
 inline double formed_gain(size_t n) { return 40. + n / 1048576. * 450.; }
 
-// n bytes to dst through the ring: fill(pinned, offset, length) enqueues one slot's worth on the
+// n bytes to dst through the ring's slots: fill(pinned, offset, length) enqueues one slot's worth on the
 // stream.  Returns when dst is written.
 template <class Fill>
 hipError_t read_ring(HostStage& st, hipStream_t stream, char* dst, size_t n, Fill fill) {
   hipEvent_t ev[HostStage::kSlots] = {};
-  hipError_t err = st.reserve(n);
+  hipError_t err = hipSuccess;
   for (int i = 0; i < st.slots && err == hipSuccess; ++i) err = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
   const int R = st.slots;
   const long nch = err == hipSuccess ? (long)((n + st.slot - 1) / st.slot) : 0;
@@ -207,6 +207,10 @@ hipError_t read_back(ReadPool& pool, hipStream_t stream, char* dst, size_t n, do
   if (!n) return hipSuccess;
   HostStage* r = gain > 0. ? pool.take(n, gain) : nullptr;
   if (!r) return plain();
+  if (r->reserve(n) != hipSuccess) {  // pinned memory is not to be had
+    pool.give(r);
+    return plain();
+  }
   const hipError_t e = read_ring(*r, stream, dst, n, fill);
   pool.give(r);
   return e;

@@ -31,8 +31,9 @@ static thread_local StubDim blockIdx, threadIdx;
 
 static size_t stub_head = 64;  // the size of an allocation lies ahead of it
 static std::atomic<long> stub_pins{0}, stub_pinned{0};  // allocations made, bytes held
+static size_t stub_most = ~(size_t)0;  // bytes that can be pinned at once
 static inline hipError_t hipHostMalloc(void** p, size_t n, unsigned = 0) {
-  char* b = (char*)std::malloc(n + stub_head);
+  char* b = n <= stub_most ? (char*)std::malloc(n + stub_head) : nullptr;
   if (!b) return hipErrorOutOfMemory;
   std::memcpy(b, &n, sizeof n);
   *p = b + stub_head;

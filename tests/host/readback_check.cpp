@@ -86,6 +86,18 @@ int main(int argc, char** argv) {
     }
     reads = 66;
   }
+  if (check == "short") {  // no pinned memory to be had, then some
+    pool.owed = 1e9;
+    ReadPoolUser user(pool);
+    const size_t sizes[3] = {8 * 1000, 8 * 600000, 8 * 2500000 + 8};
+    for (size_t most : {(size_t)0, (size_t)(20u << 10), (size_t)(1u << 20)}) {
+      stub_most = most;
+      for (size_t n : sizes) bad += read_field(pool, stream, field(n, (unsigned)n), 100.);
+      bad += expect(stub_pinned <= (long)most, "more than can be pinned");
+    }
+    for (HostStage& r : pool.ring) bad += expect(!r.busy, "a ring was not given back");
+    reads = 9;
+  }
   std::printf("%ld %ld\n", reads, bad.load());
   return 0;
 }

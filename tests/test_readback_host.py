@@ -33,3 +33,8 @@ def test_threads_share_the_slots(checker):
 def test_what_reads_pin(checker):
     """A single read pins no more than it gains; pinned memory is bounded and given back."""
     assert _run(checker, "pinning") == (66, 0)
+
+
+def test_pinned_memory_is_short(checker):
+    """Where pinned memory is not to be had, or not enough, the field is read all the same."""
+    assert _run(checker, "short") == (9, 0)
