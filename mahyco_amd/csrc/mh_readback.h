@@ -55,7 +55,7 @@ struct HostStage {
     release();
     hipError_t e = hipErrorOutOfMemory;
     for (size_t s = size(n); s >= (64u << 10); s /= 2) {  // with less where pinned memory is short
-      e = hipHostMalloc((void**)&pin, count(n) * s, hipHostMallocDefault);
+      e = hipHostMalloc((void**)&pin, count(n) * s, hipHostMallocPortable);  // for every device
       if (e == hipSuccess) {
         slot = s;
         slots = count(n);
@@ -201,12 +201,31 @@ hipError_t read_ring(HostStage& st, hipStream_t stream, char* dst, size_t n, Fil
   return err;
 }
 
+// Makes a stream's device current for the calling thread (a new thread's is device 0): events are made
+// and kernels launched there.
+struct OnDeviceOf {
+  int before = -1;
+  explicit OnDeviceOf(hipStream_t s) {
+    hipDevice_t d;
+    int cur;
+    if (hipStreamGetDevice(s, &d) == hipSuccess && hipGetDevice(&cur) == hipSuccess && d != cur &&
+        hipSetDevice(d) == hipSuccess)
+      before = cur;
+  }
+  OnDeviceOf(const OnDeviceOf&) = delete;
+  OnDeviceOf& operator=(const OnDeviceOf&) = delete;
+  ~OnDeviceOf() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
 // n bytes to dst: by fill through a ring, or by plain().  `gain` as above; a gain of 0 is the plain route.
 template <class Fill, class Plain>
 hipError_t read_back(ReadPool& pool, hipStream_t stream, char* dst, size_t n, double gain, Fill fill, Plain plain) {
   if (!n) return hipSuccess;
   HostStage* r = gain > 0. ? pool.take(n, gain) : nullptr;
   if (!r) return plain();
+  OnDeviceOf dev(stream);
   if (r->reserve(n) != hipSuccess) {  // pinned memory is not to be had
     pool.give(r);
     return plain();

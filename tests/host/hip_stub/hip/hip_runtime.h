@@ -22,7 +22,24 @@ struct StubEvent {
 };
 typedef StubStream* hipStream_t;
 typedef StubEvent* hipEvent_t;
-enum { hipEventDisableTiming = 2, hipHostMallocDefault = 0 };
+typedef int hipDevice_t;
+enum { hipEventDisableTiming = 2, hipHostMallocDefault = 0, hipHostMallocPortable = 1 };
+
+// Each thread has a current device, 0 at first; an event belongs to the device that was current when it
+// was made, and only a stream of that device can record it.
+static thread_local int stub_device = 0;
+static inline hipError_t hipGetDevice(int* d) {
+  *d = stub_device;
+  return hipSuccess;
+}
+static inline hipError_t hipSetDevice(int d) {
+  stub_device = d;
+  return hipSuccess;
+}
+static inline hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) {
+  *d = s ? s->device : stub_device;
+  return hipSuccess;
+}
 
 struct StubDim {
   unsigned x = 0, y = 0, z = 0;
@@ -51,14 +68,16 @@ static inline hipError_t hipHostFree(void* p) {
   return hipSuccess;
 }
 static inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
-  *e = new StubEvent;
+  *e = new StubEvent{stub_device};
   return hipSuccess;
 }
 static inline hipError_t hipEventDestroy(hipEvent_t e) {
   delete e;
   return hipSuccess;
 }
-static inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+static inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  return e->device == s->device ? hipSuccess : hipErrorInvalidHandle;
+}
 static inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 static inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 static inline hipError_t hipGetLastError() { return hipSuccess; }

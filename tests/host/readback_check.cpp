@@ -98,6 +98,18 @@ int main(int argc, char** argv) {
     for (HostStage& r : pool.ring) bad += expect(!r.busy, "a ring was not given back");
     reads = 9;
   }
+  if (check == "device") {  // a case of device 1, read by a thread whose current device is 0
+    pool.owed = 1e9;
+    ReadPoolUser user(pool);
+    StubStream other{1};
+    for (size_t n : {(size_t)8 * 1000, (size_t)8 * 600000}) {
+      bad += read_field(pool, other, field(n, 7), 100.);
+      bad += read_field(pool, stream, field(n, 8), 100.);
+    }
+    bad += expect(rings == 4, "the rings were not used");
+    bad += expect(stub_device == 0, "the thread's device was changed");
+    reads = 4;
+  }
   std::printf("%ld %ld\n", reads, bad.load());
   return 0;
 }

@@ -38,3 +38,8 @@ def test_what_reads_pin(checker):
 def test_pinned_memory_is_short(checker):
     """Where pinned memory is not to be had, or not enough, the field is read all the same."""
     assert _run(checker, "short") == (9, 0)
+
+
+def test_thread_of_another_device(checker):
+    """A case is read by threads whose current device is another than the case's (a new thread's is 0)."""
+    assert _run(checker, "device") == (4, 0)
