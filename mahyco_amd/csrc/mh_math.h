@@ -71,7 +71,7 @@ MH_HD double mh_div(double a, const MhRecip& r, bool& bad) {
   const double q = a * r.y;
   const double e = std::fma(-r.b, q, a);
   bad |= mh_unsafe(e) | mh_tiny(a);
-  return std::fma(e, r.y, q);
+  return std::copysign(std::fma(e, r.y, q), q);  // for a = -0, where e is +0
 }
 // one quotient, formed again by division where it has to be
 MH_HD double mh_quot(double a, const MhRecip& r) {

@@ -1,0 +1,43 @@
+// Host check of the signs of zero: the shared-denominator quotients (mh_math.h) and the one-division
+// limited gradients (mh_geom.h) give the bits of plain division and of the two-sided limiter formula.
+// Reads pairs of doubles (hexadecimal bit patterns) on stdin; prints the pairs read and the mismatches
+// of the quotients and of the gradients.  (A NaN matches any NaN.)
+#include <cinttypes>
+#include <cstdio>
+#include <cstring>
+#include "../../mahyco_amd/csrc/mh_geom.h"
+
+static double from_bits(uint64_t u) { double v; std::memcpy(&v, &u, 8); return v; }
+static uint64_t bits(double v) { uint64_t u; std::memcpy(&u, &v, 8); return u; }
+static bool same(double a, double b) { return bits(a) == bits(b) || (a != a && b != b); }
+
+template <int LIM, bool DUAL>
+static double two_sided(double gb, double gf) {
+  auto term = [](double phi, double g) { return DUAL ? (0.5 * phi) * g : 0.5 * (phi * g); };
+  double g = 0.;
+  if (gb != 0.) g += term(mh_flux_limiter(LIM, gf / gb), gb);
+  if (gf != 0.) g += term(mh_flux_limiter(LIM, gb / gf), gf);
+  return g;
+}
+template <int LIM>
+static bool gradient(double x, double y) {
+  return same(mh_limited_gradient<LIM>(LIM, x, y), two_sided<LIM, false>(x, y)) &&
+         same(mh_limited_gradient<LIM, true>(LIM, x, y), two_sided<LIM, true>(x, y));
+}
+
+int main() {
+  long pairs = 0, div = 0, lim = 0;
+  uint64_t a, b;
+  while (std::scanf("%" SCNx64 " %" SCNx64, &a, &b) == 2) {
+    const double x = from_bits(a), y = from_bits(b);
+    div += !same(mh_quot(x, mh_recip(y)), x / y);
+    bool bad = false;
+    const MhRecip r = mh_recip(y);
+    const double q = mh_div(x, r, bad);
+    if (!bad && !r.bad) div += !same(q, x / y);
+    lim += !gradient<0>(x, y) + !gradient<1>(x, y) + !gradient<2>(x, y) + !gradient<3>(x, y);
+    ++pairs;
+  }
+  std::printf("%ld %ld %ld\n", pairs, div, lim);
+  return 0;
+}
