@@ -1733,7 +1733,7 @@ __device__ __forceinline__ void k_sweep_cell3_body(const MhDev& S, int lb, int u
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const double uv = Uin[v * nc + line + cs[r]];
-      bad |= den[r].bad;
+      bad |= mh_doubt(den[r]);
       y[r] = mh_div(uv, den[r], bad);
       if (r >= 3 && r < 3 + L) u[r - 3] = uv;
     }
@@ -3118,7 +3118,7 @@ __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, in
     bool bad = false;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      bad |= den[r].bad;
+      bad |= mh_doubt(den[r]);
       phi[r] = mh_div(u[r], den[r], bad);
     }
     if (__builtin_expect(bad, 0))
@@ -3127,7 +3127,7 @@ __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, in
     bad = false;
 #pragma unroll
     for (int f = 1; f < R; ++f) {
-      bad |= dx[f].bad;
+      bad |= mh_doubt(dx[f]);
       gr[f] = mh_div(phi[f] - phi[f - 1], dx[f], bad);
     }
     if (__builtin_expect(bad, 0))

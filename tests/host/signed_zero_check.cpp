@@ -1,7 +1,8 @@
-// Host check of the signs of zero: the shared-denominator quotients (mh_math.h) and the one-division
-// limited gradients (mh_geom.h) give the bits of plain division and of the two-sided limiter formula.
-// Reads pairs of doubles (hexadecimal bit patterns) on stdin; prints the pairs read and the mismatches
-// of the quotients and of the gradients.  (A NaN matches any NaN.)
+// Host check of the shared-denominator quotients (mh_math.h) and the one-division limited gradients
+// (mh_geom.h): mh_quot gives the bits of plain division, signs of zero included; mh_div where it is
+// taken, and the gradients against the two-sided formula, but for the sign of a zero.  Reads pairs of
+// doubles (hexadecimal bit patterns) on stdin; prints the pairs read and the mismatches of the quotients
+// and of the gradients.  (A NaN matches any NaN.)
 #include <cinttypes>
 #include <cstdio>
 #include <cstring>
@@ -10,6 +11,7 @@
 static double from_bits(uint64_t u) { double v; std::memcpy(&v, &u, 8); return v; }
 static uint64_t bits(double v) { uint64_t u; std::memcpy(&u, &v, 8); return u; }
 static bool same(double a, double b) { return bits(a) == bits(b) || (a != a && b != b); }
+static bool equal(double a, double b) { return a == b || (a != a && b != b); }
 
 template <int LIM, bool DUAL>
 static double two_sided(double gb, double gf) {
@@ -21,8 +23,8 @@ static double two_sided(double gb, double gf) {
 }
 template <int LIM>
 static bool gradient(double x, double y) {
-  return same(mh_limited_gradient<LIM>(LIM, x, y), two_sided<LIM, false>(x, y)) &&
-         same(mh_limited_gradient<LIM, true>(LIM, x, y), two_sided<LIM, true>(x, y));
+  return equal(mh_limited_gradient<LIM>(LIM, x, y), two_sided<LIM, false>(x, y)) &&
+         equal(mh_limited_gradient<LIM, true>(LIM, x, y), two_sided<LIM, true>(x, y));
 }
 
 int main() {
@@ -31,10 +33,10 @@ int main() {
   while (std::scanf("%" SCNx64 " %" SCNx64, &a, &b) == 2) {
     const double x = from_bits(a), y = from_bits(b);
     div += !same(mh_quot(x, mh_recip(y)), x / y);
-    bool bad = false;
     const MhRecip r = mh_recip(y);
+    bool bad = mh_doubt(r);
     const double q = mh_div(x, r, bad);
-    if (!bad && !r.bad) div += !same(q, x / y);
+    if (!bad) div += !equal(q, x / y);
     lim += !gradient<0>(x, y) + !gradient<1>(x, y) + !gradient<2>(x, y) + !gradient<3>(x, y);
     ++pairs;
   }

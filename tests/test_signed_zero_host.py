@@ -1,6 +1,6 @@
-"""Signs of zero in the shared-denominator quotients and the one-division limited gradients of the
-sweeps, on the host as the kernels are built (g++, -ffp-contract=off): the bits of plain division and
-of the two-sided limiter formula (UtilesRemap.cc:325-357), zeros included."""
+"""Zeros in the shared-denominator quotients and the one-division limited gradients of the sweeps, on
+the host as the kernels are built (g++, -ffp-contract=off): the bits of plain division, the sign of a
+zero included, and the values of the two-sided limiter formula (UtilesRemap.cc:325-357)."""
 import os
 import shutil
 import subprocess
