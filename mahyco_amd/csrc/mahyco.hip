@@ -500,10 +500,11 @@ void tune_store(const std::string& k, int v) {
   g_tune[k] = v;
 }
 
-// Kernel variants of a single case as one number v = node + 4 cell + 16 sweep, every one of
-// which gives the same bits: node 0 the flat node kernel, 1 / 2 / 3 the z-marching one with 12 /
-// the mesh's own (node_tile_depth) / 16 node planes per block; cell 0 the flat cell kernel, 1 / 2 / 3 the LDS-staged one with
-// 12 / 8 / 16 cell planes per block; sweep 0 row segments and tiles, 1 one thread per item.
+// Kernel variants of a single case as one number v = node + 4 cell + 16 sweep + 32 march, every one of
+// which gives the same bits: node 0 the 3D node kernel over wavefronts (an ensemble's and 2D: one thread
+// per node), 1 / 2 / 3 the z-marching one with 12 / the mesh's own (node_tile_depth) / 16 node planes per
+// block; cell 0 the flat cell kernel, 1 / 2 / 3 the LDS-staged one with 12 / 8 / 16 cell planes per
+// block; sweep 0 row and register segments, marching threads and tiles, 1 one thread per item.
 const int kTileDepth[4] = {0, 12, 8, 16};
 // target segment lengths of the marching y / z dual sweeps, by variant code bits 5-7
 constexpr int kMarchLen[5] = {10, 6, 8, 4, 12};
@@ -1747,8 +1748,8 @@ int mahyco_ensemble_autotune(MhEnsemble* e, int cycles, int* bpc_out, double* ms
 }
 
 // Times `cycles` iterations (hipGraph replays of 6, after one untimed graph) of the case
-// itself with each kernel variant (tiled or flat node kernel, tiled or flat cell kernel,
-// row/tile or one-thread-per-item sweeps; only the sweep variants in 2D) and keeps the
+// itself with each kernel variant (3D node kernel over wavefronts or z-marching, tiled or flat cell
+// kernel, row/tile or one-thread-per-item sweeps; only the sweep variants in 2D) and keeps the
 // fastest, also for later cases of the same dimensions and options.  The iterations are the
 // case's own: every variant gives the same bits.  Stops at the case's final time or an error.
 int mahyco_autotune(MhHandle* h, int cycles, int* variant_out, double* ms_per_cycle_out) {
@@ -1783,16 +1784,17 @@ int mahyco_autotune(MhHandle* h, int cycles, int* variant_out, double* ms_per_cy
     }
     return MH_OK;
   };
-  // one coordinate at a time: the sweep variant, then (3D) the node kernel and its tile depth,
-  // then the cell kernel and its tile depth, each with the best of the others so far
-  const int dflt = h->g.dim == 3 ? 2 : 0;  // tiled node kernel of the mesh's depth, flat cell kernel, tiled sweeps
-  for (int sw = 0; sw < 2 && st == MH_OK && !stopped; ++sw) st = timed((dflt & 15) | (sw << 4));
-  if (h->g.dim == 3 && h->opt.with_projection) {
+  // one coordinate at a time, each with the best of the others so far, from the variant in place, which
+  // is timed first: the sweep variant (remap loop), then in 3D the node kernel and its tile depth and
+  // (remap loop) the cell kernel and its tile depth.  A coordinate that is not timed stays as it is
+  st = timed(keep);
+  if (h->opt.with_projection && st == MH_OK && !stopped) st = timed(keep ^ 16);
+  if (h->g.dim == 3) {
     for (int node = 0; node < 4 && st == MH_OK && !stopped; ++node) {
       const int v = (best & ~3) | node;
       if (v != best) st = timed(v);
     }
-    for (int cell = 0; cell < 4 && st == MH_OK && !stopped; ++cell) {
+    for (int cell = 0; cell < 4 && h->opt.with_projection && st == MH_OK && !stopped; ++cell) {
       const int v = (best & ~12) | (cell << 2);
       if (v != best) st = timed(v);
     }
