@@ -218,9 +218,10 @@ int mahyco_ensemble_autotune(MhEnsemble* e, int cycles, int* blocks_per_cu_out, 
  * (over wavefronts, or z-marching with 12, 16 or the mesh's own count of node planes per block) and
  * the remap loop's cell kernel (flat, or LDS-staged with 8, 12 or 16 cell planes per block), then the
  * segment length of the marching y / z dual sweeps.  Keeps the fastest, also for later cases of the
- * same dimensions and options in this process.  variant = node + 4 cell + 16 sweep + 32 march with the
- * codes below.  The iterations count as the case's own (every variant gives the same bits); tuning
- * stops early at the final time or an error. */
+ * same dimensions and options in this process (members of an ensemble take the cell kernel and the
+ * sweeps from it).  variant = node + 4 cell + 16 sweep + 32 march with the codes below.  The iterations
+ * count as the case's own (every variant gives the same bits); tuning stops early at the final time or
+ * an error. */
 int mahyco_autotune(MhHandle* h, int cycles, int* variant_out, double* ms_per_cycle_out);
 
 /* The kernel-variant code of a case (the code mahyco_autotune returns): node 0 over wavefronts (2D:

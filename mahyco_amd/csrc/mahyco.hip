@@ -851,7 +851,10 @@ static int create_case(const MhMesh* mesh, const MhEnvironment* envs, int nb_env
   }
   {
     const int tuned = tune_lookup(case_key_dims(h));
-    if (tuned >= 0) set_variant(h, tuned);
+    // an ensemble's launches hold many meshes: its members keep their own node kernel and march length,
+    // whose codes were timed on one mesh alone
+    const int own = 3 | (7 << 5);
+    if (tuned >= 0) set_variant(h, ext_sc ? (tuned & ~own) | (get_variant(h) & own) : tuned);
   }
   HostInit I;
   st = host_init(h, I);
