@@ -128,7 +128,7 @@ struct ReadPoolUser {
   ~ReadPoolUser() { pool.leave(); }
 };
 // what a read of n bytes gains by the pinned route, in us: one array, and values formed per cell
-inline double array_gain(size_t n) { return n < HostStage::kArray ? 0. : n / 1048576. * 80.; }
+inline double array_gain(size_t n) { return n < HostStage::kArray ? 0. : n / 1048576. * 110.; }
 inline double formed_gain(size_t n) { return 40. + n / 1048576. * 450.; }
 
 // n bytes to dst through the ring's slots: fill(pinned, offset, length) enqueues one slot's worth on the
