@@ -200,10 +200,9 @@ inline int seg_blocks(MhHandle* h, int D, int len) {
 }
 // blocks of the pente-borne / generalised-limiter sweep, a multiple of 8
 inline int gen_blocks(MhHandle* h, int D) {
-  const long na = D == 1 ? h->g.ny : h->g.nz;
-  const long b = D == 0 ? (h->g.nc + MH_BLOCK - 2) / (MH_BLOCK - 1)
-                        : (h->g.nx + MH_GEN_TX - 1) / MH_GEN_TX * ((na + MH_GEN_TY - 2) / (MH_GEN_TY - 1)) *
-                              (D == 1 ? (long)h->g.nz : (long)h->g.ny);
+  const MhGrid& g = h->g;
+  const long b = D == 0 ? (g.nc + MH_BLOCK - 2) / (MH_BLOCK - 1)
+                        : GenTile(g.nx, D == 1 ? g.nz : g.ny, D == 1 ? g.ny : g.nz).blocks();
   return (int)((b + 7) / 8 * 8);
 }
 inline int tile_blocks(MhHandle* h, int D) {

@@ -1971,12 +1971,11 @@ __device__ __forceinline__ double pb_flux(int type, double y0, double yplus, dou
 // then the update of its cell from its own face and the next one.  A flux leaves through a face
 // from one side only, so a face forms the slope and the flux of its upwind cell alone (of both
 // cells where the face velocity is not a number).  A block takes MH_BLOCK faces: 255 cells in
-// memory order for D = x, 32 x 7 cells of a plane for y and z.  Bound by the FP64 instructions and
+// memory order for D = x, 32 x 7 cells of a plane for y and z  Bound by the FP64 instructions and
 // the latency of one face's chain of slots, whose loads run one slot ahead; with a thread per cell,
 // four fluxes per slot and all slots in registers (354: one wavefront per SIMD) it took 76 / 74 us for
 // y / x on 420x180 cells and three environments, now 25 / 29.
-#define MH_GEN_TX 32  // y / z: cells along x of a block's tile
-#define MH_GEN_TY (MH_BLOCK / MH_GEN_TX)  // faces along D, one more than cells
+// (GenTile: tiles of fewer columns and more rows on meshes narrower than 32 cells).
 template <int DIM, int D, int M>
 __device__ __forceinline__ void k_sweep_cell_gen_body(const MhDev& S, int lb, int usel, int first) {
   constexpr int NV = 3 * M + 1;
@@ -1992,7 +1991,7 @@ __device__ __forceinline__ void k_sweep_cell_gen_body(const MhDev& S, int lb, in
   // the thread's cell (i, j, k), and whether it has one (a face only: the last row of the tile)
   int i, j, k;
   bool face, cell;
-  constexpr int next = D == 0 ? 1 : MH_GEN_TX;  // thread of the face ahead
+  int next = 1;  // thread of the face ahead
   if (D == 0) {
     const long c = (long)lb * (MH_BLOCK - 1) + tid;
     face = c < nc;
@@ -2002,14 +2001,13 @@ __device__ __forceinline__ void k_sweep_cell_gen_body(const MhDev& S, int lb, in
     j = (int)(r % ny);
     k = (int)(r / ny);
   } else {
-    const int tilesx = (nx + MH_GEN_TX - 1) / MH_GEN_TX, tilesd = (na + MH_GEN_TY - 2) / (MH_GEN_TY - 1);
-    i = lb % tilesx * MH_GEN_TX + tid % MH_GEN_TX;
-    const int r = lb / tilesx;
-    const int ad = r % tilesd * (MH_GEN_TY - 1) + tid / MH_GEN_TX, t = r / tilesd;
+    const GenTile tile(nx, D == 1 ? nz : ny, na);
+    int ad, t;
+    face = tile.face(lb, tid, i, t, ad);
+    cell = face && tile.cell(tid);
+    next = 1 << tile.lx;
     j = D == 1 ? ad : t;
     k = D == 1 ? t : ad;
-    face = i < nx && ad < na && t < (D == 1 ? nz : ny);
-    cell = face && tid / MH_GEN_TX < MH_GEN_TY - 1;
   }
   const int a = D == 0 ? i : D == 1 ? j : k;
   const long c = i + (long)nx * (j + (long)ny * k);
