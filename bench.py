@@ -24,8 +24,9 @@ HBM_PEAK_GBS = 8000.0
 
 
 def algorithmic_words(nc, nn, m, d):
-    """Compulsory FP64 words per cycle of the minimal fused schedule:
-    cells W_c = 2(6m+4) + 2(d+1)(3m+1), nodes W_n = 2(2d+1) + 2(d+1)(d+2) + d(d+2)."""
+    """FP64 words per cycle of a fixed accounting, by which cycles of different code compare:
+    cells W_c = 2(6m+4) + 2(d+1)(3m+1), nodes W_n = 2(2d+1) + 2(d+1)(d+2) + d(d+2).  (It carries a
+    stored phi of the dual remap and every slot of every cell; the kernels move fewer of both.)"""
     wc = 2 * (6 * m + 4) + 2 * (d + 1) * (3 * m + 1)
     wn = 2 * (2 * d + 1) + 2 * (d + 1) * (d + 2) + d * (d + 2)
     return nc * wc + nn * wn
@@ -44,8 +45,8 @@ def kernel_bytes(kind, nc, nn, m, d):
         "k_cell_lag": nn * d + nc * (5 + nv + 2),
         # read U (3m+1) and the node coordinates / velocity along the sweep; write U, mass fluxes (m)
         "k_sweep_cell": nc * (2 * nv + m) + nn * (d + 1),
-        # read and write the dual state (d+1) and phi (d); read x along the sweep and the mass fluxes
-        "k_sweep_node": nn * (2 * (d + 1) + 2 * d + 1) + nc * m,
+        # read and write the dual state (d+1); read x along the sweep and the mass fluxes
+        "k_sweep_node": nn * (2 * (d + 1) + 1) + nc * m,
         # read U (3m+1), V_E, L, u (d per node); write rho, e, p, c, q, M, f
         "k_finalize": nc * (nv + 2 + 7) + nn * d,
         "k_node_velocity": nn * (d + 1 + d),

@@ -163,7 +163,8 @@ MH_HD D3 cqs_hex_corner(const D3* x) {
 // to the centre, the component of each half cross product 0.5 (a_U b_W - a_W b_U) (U = C+1,
 // W = C+2 mod 3) and the corner sums t (5 (..) + (..)) in the same order.  Every rounded
 // operation of cqs_hex acts on one component, so q[l] is bit for bit cqs_hex's q[l].C, and
-// only one component's terms are live at a time.
+// only one component's terms are live at a time.  No kernel calls this form or the next: hex_volume
+// took their place, and the host check of the corner vectors compares all of them.
 template <int C>
 MH_HD void cqs_hex_comp(const D3* x, double* q) {
   constexpr int U = (C + 1) % 3, W = (C + 2) % 3;

@@ -34,19 +34,24 @@ enum {
   KN_COUNT
 };
 
-// sweep variants: one thread per cell / node; row segments along x and LDS tiles along y / z
+// sweep variants: one thread per cell / node; or row segments along x and, along y / z, register
+// segments, marching threads and LDS tiles
 enum { MH_SWEEP_FLAT = 0, MH_SWEEP_TILE = 1 };
-// Sizes below which a single mesh takes the variants of the row/tile sweeps that need fewer
-// wavefronts to hide their latency; both sides measured around each line:
-// y / z cell sweeps: 2-cell register segments (k_sweep_cell_seg) below, marching threads or LDS tiles
-// (k_sweep_cell_march) above.  Tile
-// against segments, two environments: 27 / 10 us on 181x181, 30 / 22 on 512x512, 45 / 33 on 80^3,
-// 37 / 30 on 724x724, 71 / 60 on 101^3, but 45 / 54 on 1024x1024, and 69 / 85 on 128^3 (one).
+// Sizes below which a single mesh takes the variants that need fewer wavefronts to hide their latency,
+// with both sides as they are now (event times of one launch, us).
+// y / z cell sweeps: 2-cell register segments (k_sweep_cell_seg) below; above, marching threads
+// (k_sweep_cell_march) for one environment and in 2D for two, else LDS tiles (k_sweep_cell_tile).
+// Segments / march in 2D, two environments: 21 / 38 on 512x512, 40 / 47 on 850x850, 45 / 45 on 894x894,
+// 54 / 48 on 1023x1021; one: 29 / 29 on 850x850, 33 / 30 on 894x894.  3D crosses later, at about 1.3 M
+// cells: segments / tiles, two environments, 33 / 44 on 80^3, 59 / 74 on 101^3, 83 / 84 on 110^3, 123 / 107
+// on 128^3; segments / march, one, 41 / 47 on 101^3, 53 / 53 on 110^3, 87 / 63 on 128^3.
 #define MH_SEG_CELLS 800000L
-// y / z dual sweeps: one thread per node below, marching segments above.  March (4 nodes) against
-// one per node: 17 / 8.6 us on 181x181, 25 / 20 on 64^3, 30 / 30 on 80^3, 35 / 39 on 128x96x64.
+// y / z dual sweeps: one thread per node below, marching segments above.  One per node / march of 4
+// nodes: 10 / 13 on 362x362, 18.5 / 17.5 on 700x700, 19.4 / 19.5 on 760x760, 23 / 21 on 850x850; 18 / 21 on
+// 64^3, 25.5 / 24.5 on 80^3, 45 / 40 on 101^3.
 #define MH_MARCH_NODES 600000L
-// ... and 10-node segments from here on (2.1 M nodes: 94 us with 4, 87 with 10; 1.05 M: 31 / 40)
+// ... and 10-node segments from here on.  4 / 10 nodes: 45 / 47 on 1400x1400 (2.0 M nodes), 68 / 70 on 128^3
+// (2.1 M), 90 / 83 on 144^3 (3.0 M); the autotuner tries 6 (66 on 128^3) and others.
 #define MH_MARCH_LONG_NODES 1600000L
 // 3D node kernel: the cells of a node over four wavefronts below, z-marching tiles above.  Tiles (of the
 // mesh's depth) against wavefronts: 16 / 9.3 us on 24^3, 22 / 21 on 50^3, 31 / 34 on 64^3, 41 / 54 on
@@ -166,7 +171,6 @@ inline int node_row_blocks(MhHandle* h) {
   return (int)(((waves + wpb - 1) / wpb + 7) / 8 * 8);
 }
 
-// blocks of the LDS-tiled y / z sweep (64 cells along x by MH_TILE_L along D), a multiple of 8
 // k_sweep_node_march: one thread per (x node, other transverse node, segment of about nm_len nodes along D)
 inline int node_march_blocks(MhHandle* h, int D) {
   const long na = D == 1 ? h->g.ny : h->g.nz;
@@ -174,8 +178,8 @@ inline int node_march_blocks(MhHandle* h, int D) {
   const long threads = (long)h->g.nnx * nt2 * march_nseg((int)na + 1, h->nm_len);
   return (int)(((threads + MH_BLOCK - 1) / MH_BLOCK + 7) / 8 * 8);
 }
-// k_sweep_cell_march: one thread per (x cell, other transverse cell, segment of about MH_CM_L cells along D),
-// for the meshes of its environment counts whose offsets fit 32 bits
+// k_sweep_cell_march: one thread per (x cell, other transverse cell, segment of about MH_CM_L cells along
+// D), for the meshes of its environment counts whose offsets fit 32 bits
 inline bool cell_march(const MhHandle* h) { return MH_CM_HAS(h->g.dim, h->m) && h->g.nn < MH_CM_NODES; }
 inline int cell_march_blocks(const MhHandle* h, int D) {
   const long na = D == 1 ? h->g.ny : h->g.nz;
@@ -205,6 +209,7 @@ inline int gen_blocks(MhHandle* h, int D) {
                         : GenTile(g.nx, D == 1 ? g.nz : g.ny, D == 1 ? g.ny : g.nz).blocks();
   return (int)((b + 7) / 8 * 8);
 }
+// blocks of the LDS-tiled y / z sweep (64 cells along x by MH_TILE_L along D), a multiple of 8
 inline int tile_blocks(MhHandle* h, int D) {
   const long na = D == 1 ? h->g.ny : h->g.nz;
   const long nt = D == 1 ? (h->g.dim == 3 ? h->g.nz : 1) : h->g.ny;

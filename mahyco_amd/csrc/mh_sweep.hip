@@ -129,7 +129,7 @@ void launch_sweeps_t(MhHandle* h) {
     dirs[nd++] = idir;
   }
   const bool o3 = S.order2 == 2;
-  // pente-borne or generalised limiters: one thread per cell and node, limiter read at run time
+  // pente-borne or generalised limiters: one thread per face and per node, limiter read at run time
   const bool gen = !o3 && (S.pb || (S.order2 && S.limiter >= MH_MINMOD_G));
   if (S.csts) LAUNCH(h, KN_NODE_FWD, (k_node_fwd<DIM>), h->nblk_n, MH_BLOCK, S);  // PrepareRemap.cc:210
   if (S.hc && nd > 0) LAUNCH(h, KN_HCELL, (k_hcell<DIM>), h->nblk_c, MH_BLOCK, S);
