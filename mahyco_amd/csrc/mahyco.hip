@@ -1220,7 +1220,7 @@ static int read_array(MhHandle* h, const double* d, double* out, long n) {
                        (double*)pin, k);
     return hipGetLastError();
   };
-  auto plain = [&] { return hipMemcpy(out, d, bytes, hipMemcpyDeviceToHost); };
+  auto plain = [&] { return hipMemcpyWithStream(out, d, bytes, hipMemcpyDeviceToHost, h->stream); };
   return hip_check(read_back(read_pool(), h->stream, (char*)out, bytes, array_gain(bytes), fill, plain), "read back");
 }
 // Values formed per cell (field_value) from the membership, g [nc] and e [ne].
@@ -1237,9 +1237,9 @@ static int read_formed(MhHandle* h, int field, int env, const double* g, const d
     std::unique_ptr<uint8_t[]> mask(new (std::nothrow) uint8_t[nc]);
     std::unique_ptr<double[]> hg(new (std::nothrow) double[g ? nc : 1]), he(new (std::nothrow) double[e ? ne : 1]);
     if (!mask || !hg || !he) return hipErrorOutOfMemory;
-    hipError_t r = hipMemcpy(mask.get(), h->dev.mask, nc, hipMemcpyDeviceToHost);
-    if (r == hipSuccess && g) r = hipMemcpy(hg.get(), g, bytes, hipMemcpyDeviceToHost);
-    if (r == hipSuccess && e) r = hipMemcpy(he.get(), e, ne * sizeof(double), hipMemcpyDeviceToHost);
+    hipError_t r = hipMemcpyWithStream(mask.get(), h->dev.mask, nc, hipMemcpyDeviceToHost, h->stream);
+    if (r == hipSuccess && g) r = hipMemcpyWithStream(hg.get(), g, bytes, hipMemcpyDeviceToHost, h->stream);
+    if (r == hipSuccess && e) r = hipMemcpyWithStream(he.get(), e, ne * sizeof(double), hipMemcpyDeviceToHost, h->stream);
     if (r != hipSuccess) return r;
     for (long c = 0; c < nc; ++c) out[c] = field_value(field, env, h->m, nc, mask[c], hg.get(), e ? he.get() : nullptr, c);
     return hipSuccess;

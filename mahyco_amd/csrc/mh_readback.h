@@ -7,12 +7,13 @@
 // One thread below 4 MB (two copy 1 MB no faster than one), one more per 2 MB, eight at most (12 are
 // slower); 4 MB slots at most (57 MB with 2 MB ones: 3.8 ms instead of 3.4).
 //
-// Plain / pinned, us, one array into pages used before: 29 KB 34 / 35, 262 KB 41 / 45, 1 MB 85 / 85, 2 MB
-// 270 / 120, 4 MB 600 / 190, 8 MB 1200 / 255, 34 MB 5400 / 775 (into new pages 262 KB 85 / 85, 4 MB 1350 /
-// 1000, 34 MB 12900 / 7500).  Formed values: 4.6 KB 60 / 32, 262 KB 85 / 43, 2 MB 960 / 115.  Pinning itself takes 0.1 ms for
-// 64 KB and 1.3 ms from 2 MB on, once.  So one array below 256 KB always takes the plain route, and slots
-// are pinned only when the reads since they were last given back would have gained by them what they cost:
-// a case that reads one field of 2 MB takes 270 us for it, where pinning first took 1200.
+// Plain / pinned, us, one array into pages used before: 29 KB 34 / 35, 262 KB 41 / 45 (140 / 50 among a
+// process's first reads), 1 MB 85 / 85, 2 MB 270 / 120, 4 MB 600 / 190, 8 MB 1200 / 255, 34 MB 5400 / 775;
+// into new pages: 262 KB 85 / 85, 4 MB 1350 / 1000, 34 MB 12900 / 7500.  Formed values: 4.6 KB 60 / 32,
+// 262 KB 85 / 43, 2 MB 960 / 115.  Pinning itself takes 0.1 ms for 64 KB and 1.3 ms from 2 MB on, once.  So
+// one array below 64 KB always takes the plain route, and slots are pinned only when the reads since
+// they were last given back would have gained by them what they cost: a case that reads one field of
+// 2 MB takes 270 us for it, where pinning first took 1200.
 //
 // The slots belong to the process: at most two rings of 16 MB, each with one reader at a time (a read
 // that finds none free takes the plain route), given back with the last case and ensemble.
@@ -33,7 +34,7 @@
 // A ring of pinned slots.
 struct HostStage {
   static constexpr int kSlots = 4;
-  static constexpr size_t kArray = 256u << 10;  // one array: by the pinned route from here on
+  static constexpr size_t kArray = 64u << 10;  // one array: by the pinned route from here on
   char* pin = nullptr;
   size_t slot = 0;  // bytes of a slot
   int slots = 0;
@@ -128,7 +129,7 @@ struct ReadPoolUser {
   ~ReadPoolUser() { pool.leave(); }
 };
 // what a read of n bytes gains by the pinned route, in us: one array, and values formed per cell
-inline double array_gain(size_t n) { return n < HostStage::kArray ? 0. : n / 1048576. * 110.; }
+inline double array_gain(size_t n) { return n < HostStage::kArray ? 0. : 20. + n / 1048576. * 110.; }
 inline double formed_gain(size_t n) { return 40. + n / 1048576. * 450.; }
 
 // n bytes to dst through the ring's slots: fill(pinned, offset, length) enqueues one slot's worth on the
