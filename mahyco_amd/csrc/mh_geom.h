@@ -316,7 +316,11 @@ MH_HD double hex_volume(const D3* x) {
   e[7] = dot3(x[7], t * (5. * A[7] + B[7]));
   double v = 0.;
   for (int l = 0; l < 8; ++l) v += e[l];
-  return mh_quot(v, MhRecip{3., 1. / 3., false});
+  const MhRecip third{3., 1. / 3., false};
+  bool bad = false;
+  double w = mh_div(v, third, bad);  // (a sum from 0 is no -0)
+  if (__builtin_expect(bad, 0)) w = v / 3.;
+  return w;
 }
 
 // Quadrangle corner vectors: half edge normals of the two edges at each corner

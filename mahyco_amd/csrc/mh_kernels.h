@@ -4163,7 +4163,13 @@ __global__ __launch_bounds__(MH_BLOCK) void k_hist_final(MhDev S) { k_hist_final
 MH_WRAP(k_node_lag, MH_NODE_FLAT_MIN_WAVES, template <int DIM>, <DIM>, , )
 MH_WRAP(k_cell_lag, MH_CELL_MIN_WAVES, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
 MH_WRAP(k_cell_lag_remap, MH_CELL_MIN_WAVES, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
-MH_WRAP(k_cell_lag_only, MH_CELL_MIN_WAVES, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
+// (Single meshes only.  LATE: blocks ask for the stop flag ahead, as above; in a few rounds of blocks at 3
+// waves per SIMD that wait shows, 46 -> 48 us on 128x96x64, so the launch asks for it from 8192 blocks on.)
+template <int DIM, int M, bool LATE>
+__global__ __launch_bounds__(MH_BLOCK, MH_CELL_MIN_WAVES) void k_cell_lag_only(MhDev S) {
+  if (LATE && late_halted(S.sc)) return;
+  k_cell_lag_only_body<DIM, M>(S, xcd_block((int)blockIdx.x, (int)gridDim.x));
+}
 MH_WRAP(k_cell_lag_csts, 1, template <int DIM MH_COMMA int M>, <DIM MH_COMMA M>, , )
 MH_WRAP(k_cell_length, 1, template <int DIM>, <DIM>, , )
 MH_WRAP(k_sweep_cell, 1, template <int DIM MH_COMMA int D MH_COMMA int M MH_COMMA int LIM>, <DIM MH_COMMA D MH_COMMA M MH_COMMA LIM>,

@@ -22,7 +22,8 @@ void launch_cell_t(MhHandle* h) {
   if (h->dev.csts) {
     LAUNCH(h, KN_CELL, (k_cell_lag_csts<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
   } else if (!h->dev.with_proj) {
-    LAUNCH(h, KN_CELL, (k_cell_lag_only<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
+    if (h->nblk_c >= 8192) LAUNCH(h, KN_CELL, (k_cell_lag_only<DIM, M, true>), h->nblk_c, MH_BLOCK, h->dev);
+    else LAUNCH(h, KN_CELL, (k_cell_lag_only<DIM, M, false>), h->nblk_c, MH_BLOCK, h->dev);
   } else if (h->dev.sans_lagrange || h->staged) {
     LAUNCH(h, KN_CELL, (k_cell_lag<DIM, M>), h->nblk_c, MH_BLOCK, h->dev);
   } else if (DIM == 3 && h->cell_tiled) {
