@@ -1686,7 +1686,7 @@ __device__ __forceinline__ void k_sweep_cell3_body(const MhDev& S, int lb, int u
       d = 0.;
       for (int kk = 0; kk < M; ++kk) d += Uin[kk * nc + line + cs[r]];
     }
-    den[r] = mh_recip(d);
+    den[r] = mh_denom(d);
     h[r] = S.hc[D * nc + line + cs[r]];
   }
   // flags of the cells beside the faces: rows 2 .. L+3
@@ -1699,7 +1699,7 @@ __device__ __forceinline__ void k_sweep_cell3_body(const MhDev& S, int lb, int u
     for (int o = 0; o < L + 2; ++o) {
       int cnt = 0, pur = -1;
       for (int v = 0; v < M; ++v)
-        if (mh_quot(Uin[v * nc + line + cs[o + 2]], den[o + 2]) > 0.) {
+        if (mh_ratio(Uin[v * nc + line + cs[o + 2]], den[o + 2]) > 0.) {
           cnt++;
           pur = v;
         }
@@ -1741,7 +1741,7 @@ __device__ __forceinline__ void k_sweep_cell3_body(const MhDev& S, int lb, int u
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const double uv = Uin[v * nc + line + cs[r]];
-      bad |= mh_doubt(den[r]);
+      bad |= den[r].bad;
       y[r] = mh_div(uv, den[r], bad);
       if (r >= 3 && r < 3 + L) u[r - 3] = uv;
     }
@@ -2451,7 +2451,7 @@ __device__ __forceinline__ void dual_store(const MhDev& S, long n, const double*
   }
   if (!last || S.dec) dual_out_m<DIM>(S, psel)[n] = U[DIM];
   if (last && U[DIM] != 0.) {
-    const MhRecip rm = mh_recip(U[DIM]);
+    const MhRecip rm = mh_denom(U[DIM]);
 #pragma unroll
     for (int cc = 0; cc < DIM; ++cc) S.u[cc][n] = mh_quot(U[cc], rm);
   }
@@ -2522,19 +2522,19 @@ __device__ __forceinline__ void k_sweep_node_row_body(const MhDev& S, int lb, in
 #pragma unroll
   for (int cc = 0; cc < NC; ++cc) P[cc] = valid ? v[cc] : 0.;
   if (!kept && valid) {
-    const MhRecip rm = mh_recip(m);
+    const MhRecip rm = mh_denom(m);
 #pragma unroll
-    for (int cc = 0; cc < NC; ++cc) P[cc] = mh_quot(v[cc], rm);
+    for (int cc = 0; cc < NC; ++cc) P[cc] = mh_ratio(v[cc], rm);
   }
   const bool inner = valid && i >= 1 && i <= na - 1;
   const double Xm = lane_back(X), Xp = lane_front(X);
   double Pm[NC], Pp[NC], G0[NC], Gm[NC], Gp[NC];
-  const MhRecip rX = mh_recip(X - Xm);
+  const MhRecip rX = mh_denom(X - Xm);
 #pragma unroll
   for (int cc = 0; cc < NC; ++cc) {
     Pm[cc] = lane_back(P[cc]);
     Pp[cc] = lane_front(P[cc]);
-    const double eb = (valid && validp) ? mh_quot(P[cc] - Pm[cc], rX) : 0.;  // edge i-1/2
+    const double eb = (valid && validp) ? mh_ratio(P[cc] - Pm[cc], rX) : 0.;  // edge i-1/2
     const double ef = lane_front(eb);                                        // edge i+1/2
     G0[cc] = (S.order2 && inner) ? dual_limited<LIM>(S, eb, ef) : 0.;
     Gm[cc] = lane_back(G0[cc]);
@@ -2948,14 +2948,14 @@ __device__ __forceinline__ void k_sweep_cell_march_body(const MhDev& S, int lb, 
     const double w = inn ? wP : 0.;
     const bool irregular = val && (!mh_finite_nonzero(den) || (inn && (!mh_finite_nonzero(dxr) || !mh_finite(w) || !mh_finite(hh))));
     const unsigned here = sparse && __ballot(irregular) == 0 ? heldc : (1u << M) - 1u;
-    const MhRecip rden = mh_recip(den), rdx = mh_recip(dxr);
+    const MhRecip rden = mh_denom(den), rdx = mh_denom(dxr);
     const bool out = a - 2 >= a0 && a - 2 < a1;
     const bool inb = a - 2 > 0, inf = a - 2 < na - 1;
     const unsigned c = crow(a - 2);
     unsigned holds = 0;
     auto slot = [&](int v) {
-      const double phi = mh_quot(U[v], rden);
-      const double gf = inn ? mh_quot(phi - phiP[v], rdx) : 0.;
+      const double phi = mh_ratio(U[v], rden);
+      const double gf = inn ? mh_ratio(phi - phiP[v], rdx) : 0.;
       const double sl = S.order2 && valp ? mh_limited_gradient<LIM>(S.limiter, gP[v], gf) : 0.;
       const double F = innA ? wA * (upA ? pfb[v] : phiP[v] + hhA * sl) : 0.;
       const double fb = -kept(v, 2), U2 = kept(v, st & 1);
@@ -3100,11 +3100,11 @@ __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, in
     if (FEW || inner(f)) face_quant<DIM, D>(S, nl + row(f) * nD, area[f], xf[f], vf[f]);
   if (FEW && halted) return;
 #pragma unroll
-  for (int r = 0; r < R; ++r) den[r] = mh_recip(valid(r) ? d[r] : 1.);
+  for (int r = 0; r < R; ++r) den[r] = mh_denom(valid(r) ? d[r] : 1.);
 #pragma unroll
   for (int f = 1; f < R; ++f) {
     const double dxf = inner(f) ? xc[f] - xc[f - 1] : 1.;
-    dx[f] = mh_recip(dxf);
+    dx[f] = mh_denom(dxf);
     w[f] = 0.;
     hh[f] = 0.;
     if (f >= 2 && f <= R - 2 && inner(f)) {
@@ -3124,7 +3124,7 @@ __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, in
     bool bad = false;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      bad |= mh_doubt(den[r]);
+      bad |= den[r].bad;
       phi[r] = mh_div(u[r], den[r], bad);
     }
     if (__builtin_expect(bad, 0))
@@ -3133,7 +3133,7 @@ __device__ __forceinline__ void k_sweep_cell_seg_body(const MhDev& S, int lb, in
     bad = false;
 #pragma unroll
     for (int f = 1; f < R; ++f) {
-      bad |= mh_doubt(dx[f]);
+      bad |= dx[f].bad;
       gr[f] = mh_div(phi[f] - phi[f - 1], dx[f], bad);
     }
     if (__builtin_expect(bad, 0))
@@ -3234,9 +3234,9 @@ __device__ __forceinline__ void k_sweep_node_at(const MhDev& S, long n, int psel
   for (int o = -2; o <= 2; ++o) {
     const int bb = a + o;
     if (!kept) {
-      const MhRecip rm = mh_recip(mm[o + 2]);
+      const MhRecip rm = mh_denom(mm[o + 2]);
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = mh_quot(P[o + 2][cc], rm);
+      for (int cc = 0; cc < NC; ++cc) P[o + 2][cc] = mh_ratio(P[o + 2][cc], rm);
     }
     if (bb < 0 || bb > na) {
 #pragma unroll
@@ -3360,9 +3360,9 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
 #pragma unroll
     for (int cc = 0; cc < NC; ++cc) P[cc] = v[cc];
     if (!kept) {
-      const MhRecip rm = mh_recip(m);
+      const MhRecip rm = mh_denom(m);
 #pragma unroll
-      for (int cc = 0; cc < NC; ++cc) P[cc] = mh_quot(v[cc], rm);
+      for (int cc = 0; cc < NC; ++cc) P[cc] = mh_ratio(v[cc], rm);
     }
     if (b < 0 || b > na) {
 #pragma unroll
@@ -3381,9 +3381,9 @@ __device__ __forceinline__ void k_sweep_node_march_body(const MhDev& S, int lb, 
   // edge gradient between nodes b and b+1 (formed only where a limited gradient reads it)
   auto edge = [&](int b, const double* P0, double X0, const double* P1, double X1, double* E) {
     const bool used = S.order2 && b >= 0 && b + 1 <= na && (b >= 1 || b + 1 <= na - 1);
-    const MhRecip rX = mh_recip(X1 - X0);
+    const MhRecip rX = mh_denom(X1 - X0);
 #pragma unroll
-    for (int cc = 0; cc < NC; ++cc) E[cc] = used ? mh_quot(P1[cc] - P0[cc], rX) : 0.;
+    for (int cc = 0; cc < NC; ++cc) E[cc] = used ? mh_ratio(P1[cc] - P0[cc], rX) : 0.;
   };
   // window: P and X of nodes a-1 .. a+2 (slots 0..3), edges (a-1/2, a+1/2, a+3/2), G of a-1, a, a+1
   double P[4][NC], X[4], E[3][NC], G[3][NC];
@@ -4155,7 +4155,7 @@ __global__ __launch_bounds__(MH_BLOCK) void k_hist_final(MhDev S) { k_hist_final
     const int n = *nwork;                                                                    \
     for (int w = (int)blockIdx.x; w < n; w += (int)gridDim.x) {                              \
       const int2 bm = bmap[w];                                                               \
-      if (!mh_halted(tab[bm.x].sc)) NAME##_body TARGS(tab[bm.x], bm.y ARGS);                 \
+      if (w < MH_FIRST_BLOCKS || !mh_halted(tab[bm.x].sc)) NAME##_body TARGS(tab[bm.x], bm.y ARGS); \
       __syncthreads();                                                                       \
     }                                                                                        \
   }

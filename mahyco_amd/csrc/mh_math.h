@@ -44,13 +44,13 @@ MH_HD double mh_pow_half(double x) { return std::sqrt(x); }
 // last steps of the division sequence itself, so each is the correctly rounded a / b, in 6
 // instructions instead of 11, one of them a quarter-rate reciprocal.  Those steps hold while
 // nothing leaves the normal range: a remainder that is not a number, infinite or subnormal
-// (zero or infinite b, NaN, overflow) or an a below 2^-900, whose remainder may round to 0,
+// (zero or infinite b, NaN, overflow) or an a below 2^-950, whose remainder may round to 0,
 // sets `bad`, and the caller forms that group of quotients again by division.  (An advected
-// bubble leaves densities down to 2^-1074 behind, so such operands do occur.)  So it does for a b above
-// 2^120 (mh_doubt): with both bounds q is no smaller than 2^-1020, where a subnormal quotient may lie
+// bubble leaves densities down to 2^-1074 behind, so such operands do occur.)  mh_denom also rules out
+// a b above 2^70: with both bounds q is no smaller than 2^-1020, where a subnormal quotient may lie
 // at a tie that q + e y misses.  The bound is b's because a second one on every quotient costs 4 % of
-// the sweeps, and a's is not higher because velocities ahead of a blast fall to 2^-520 (2.5 % of its
-// dual sweeps).
+// the sweeps, and a's is not higher because what moves ahead of a wave falls through all magnitudes
+// (at 2^-520 2.5 % of a blast's dual sweeps).
 struct MhRecip {
   double b, y;
   bool bad;  // y itself is outside the normal range
@@ -63,7 +63,7 @@ MH_HD bool mh_unsafe(double e) {  // NaN, infinite or subnormal
   return c != FP_NORMAL && c != FP_ZERO;
 #endif
 }
-MH_HD bool mh_tiny(double a) { return std::fabs(a) < 0x1p-900 && a != 0.; }
+MH_HD bool mh_tiny(double a) { return std::fabs(a) < 0x1p-950 && a != 0.; }
 MH_HD MhRecip mh_recip(double b) {
   MhRecip r;
   r.b = b;
@@ -71,19 +71,29 @@ MH_HD MhRecip mh_recip(double b) {
   r.bad = mh_unsafe(r.y);
   return r;
 }
-// quotients of this denominator are to be formed by division
-MH_HD bool mh_doubt(const MhRecip& r) { return r.bad | (std::fabs(r.b) > 0x1p120); }
-// A zero quotient may have either sign (the remainder of -0 is +0): for values that only enter sums
-// from 0, as those of the cell sweeps do.
+// the denominator of a group of quotients; where it is bad they are formed by division
+MH_HD MhRecip mh_denom(double b) {
+  MhRecip r = mh_recip(b);
+  r.bad |= std::fabs(b) > 0x1p70;
+  return r;
+}
 MH_HD double mh_div(double a, const MhRecip& r, bool& bad) {
   const double q = a * r.y;
   const double e = std::fma(-r.b, q, a);
   bad |= mh_unsafe(e) | mh_tiny(a);
   return std::fma(e, r.y, q);
 }
-// one quotient, formed again by division where it has to be, with the bits of a / b
+// One quotient, formed again by division where it has to be.  mh_quot has the bits of a / b; a zero of
+// mh_ratio, as one of mh_div, may have either sign (the remainder of -0 is +0): for values that only
+// enter sums from 0, as those of the sweeps do.
+MH_HD double mh_ratio(double a, const MhRecip& r) {
+  bool bad = r.bad;
+  double q = mh_div(a, r, bad);
+  if (__builtin_expect(bad, 0)) q = a / r.b;
+  return q;
+}
 MH_HD double mh_quot(double a, const MhRecip& r) {
-  bool bad = mh_doubt(r);
+  bool bad = r.bad;
   double q = std::copysign(mh_div(a, r, bad), a * r.y);
   if (__builtin_expect(bad, 0)) q = a / r.b;
   return q;

@@ -32,9 +32,9 @@ int main() {
   uint64_t a, b;
   while (std::scanf("%" SCNx64 " %" SCNx64, &a, &b) == 2) {
     const double x = from_bits(a), y = from_bits(b);
-    div += !same(mh_quot(x, mh_recip(y)), x / y);
-    const MhRecip r = mh_recip(y);
-    bool bad = mh_doubt(r);
+    div += !same(mh_quot(x, mh_denom(y)), x / y) + !equal(mh_ratio(x, mh_denom(y)), x / y);
+    const MhRecip r = mh_denom(y);
+    bool bad = r.bad;
     const double q = mh_div(x, r, bad);
     if (!bad) div += !equal(q, x / y);
     lim += !gradient<0>(x, y) + !gradient<1>(x, y) + !gradient<2>(x, y) + !gradient<3>(x, y);
