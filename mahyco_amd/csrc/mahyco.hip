@@ -1008,6 +1008,7 @@ static int create_case(const MhMesh* mesh, const MhEnvironment* envs, int nb_env
   }
   S.nblk_c = h->nblk_c;
   S.nt_kc = h->nt_kc;
+  S.cm_len = cell_march_len(g);
   S.ct_k = h->ct_k;
   S.nm_len = h->nm_len;
   S.nblk_n = h->nblk_n;

@@ -181,9 +181,15 @@ inline int node_march_blocks(MhHandle* h, int D) {
 // k_sweep_cell_march: one thread per (x cell, other transverse cell, segment of about MH_CM_L cells along
 // D), for the meshes of its environment counts whose offsets fit 32 bits
 inline bool cell_march(const MhHandle* h) { return MH_CM_HAS(h->g.dim, h->m) && h->g.nn < MH_CM_NODES; }
+// Cells per segment, about.  Meshes of fewer than 4096 cells take 2: few threads march there, and each waits
+// for its rows in turn.  Ensembles, us an iteration at 2 / 8 cells in 2D with two environments: 113 / 131
+// for 128 meshes of 12x12, 129 / 172 for 128 of 24x24, 103 / 125 for 64 of 48x48, but 131 / 133 for 16 of
+// 128x128 and 204 / 193 for 16 of 200x200; at 2 / 16 cells in 3D with one: 152 / 172 for 64 of 8^3,
+// 179 / 219 for 64 of 12^3, but 468 / 433 for 8 of 48^3.
+inline int cell_march_len(const MhGrid& g) { return g.nc < 4096 ? 2 : MH_CM_L(g.dim); }
 inline int cell_march_blocks(const MhHandle* h, int D) {
   const long na = D == 1 ? h->g.ny : h->g.nz;
-  const long threads = h->g.nc / na * march_nseg((int)na, MH_CM_L(h->g.dim));
+  const long threads = h->g.nc / na * march_nseg((int)na, h->dev.cm_len);
   return (int)(((threads + MH_BLOCK - 1) / MH_BLOCK + 7) / 8 * 8);
 }
 // the y / z variants a single mesh takes (an ensemble's launches are filled by its many cases)

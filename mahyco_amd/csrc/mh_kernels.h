@@ -2775,7 +2775,7 @@ __device__ __forceinline__ void k_sweep_cell_tile_body(const MhDev& S, int lb_, 
 // cells: 201, 191 us in 3D, 46 and 80 us in 2D, which runs out of threads.  Two environments in 3D
 // hold 220 registers (187 us on the 256x128x128 tube, tiles 182; with 168 they spill: 690 us), so
 // they and more environments keep the tiles.  Same formulas in the same order as k_sweep_cell_body.
-#define MH_CM_L(DIM) ((DIM) == 3 ? 16 : 8)  // cells along D per segment, about
+#define MH_CM_L(DIM) ((DIM) == 3 ? 16 : 8)  // cells along D per segment, about (cell_march_len: 2 on small meshes)
 #define MH_CM_HAS(DIM, M) ((M) == 1 || ((DIM) == 2 && (M) == 2))
 #define MH_CM_NODES (1L << 29)  // meshes of fewer nodes: 32-bit byte offsets
 template <int DIM, int D, int M, int LIM>
@@ -2784,7 +2784,7 @@ __device__ __forceinline__ void k_sweep_cell_march_body(const MhDev& S, int lb, 
   const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
   const int na = D == 1 ? ny : nz;
   const int nt = D == 1 ? (DIM == 3 ? nz : 1) : ny;
-  const int nseg = march_nseg(na, MH_CM_L(DIM));
+  const int nseg = march_nseg(na, S.cm_len);
   const long g = lb * (long)blockDim.x + threadIdx.x;
   if (g >= (long)nx * nseg * nt) return;
   if (mh_halted(S.sc)) return;
