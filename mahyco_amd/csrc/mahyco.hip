@@ -1001,7 +1001,7 @@ static int create_case(const MhMesh* mesh, const MhEnvironment* envs, int nb_env
   S.Pa = h->Pa;
   S.Pb = h->Pb;
   // the presence bytes of the two U buffers lie behind the dual masses in Pb (3 nn words, of which
-  // the masses take nn); large single meshes and ensembles of two environments or more keep them
+  // the masses take nn), for the meshes of presence_bytes()
   if (presence_bytes(h)) {
     S.pm[0] = (uint8_t*)(h->Pb + nn);
     S.pm[1] = S.pm[0] + nc;

@@ -196,11 +196,19 @@ inline int cell_march_blocks(const MhHandle* h, int D) {
 inline bool seg_sweep(const MhHandle* h) { return !h->sweep_large && h->g.nc < MH_SEG_CELLS; }
 inline bool march_sweep(const MhHandle* h) { return h->sweep_large || h->g.nn >= MH_MARCH_NODES; }
 // whether the case keeps presence bytes (MhDev::pm): its sweeps are the row and tile ones.  Small
-// meshes are bound by latency, and their segment sweeps do not use them.
+// meshes are bound by latency, and their segment sweeps do not use them.  Nor do the tiles of 3D members
+// of an ensemble gain from them with two environments below 10^6 cells, us an iteration with / without:
+// 428 / 414 for 16 of 32^3, 593 / 567 for 8 of 48^3, 368 / 351 for 16 of 120x120x2, 1119 / 1111 for 2 of
+// 100^3, but 3907 / 3939 for 2 of 160^3.  Rows of a few cells do, 2105 / 2385 for 16 of 2x120x120 and
+// 1602 / 1776 for 8 of 8x8x2000, and so do more environments: 440 / 452 for 8 of 40^3 with three, 457 / 505
+// with four.
+inline bool presence_member(const MhHandle* h) {
+  return h->m > 2 || h->g.dim == 2 || h->g.nx < 16 || h->g.nc >= 1000000;
+}
 inline bool presence_bytes(const MhHandle* h) {
   const MhDev& S = h->dev;
   return h->m > 1 && h->opt.with_projection && S.order2 != 2 && !S.pb && !(S.order2 && S.limiter >= MH_MINMOD_G) &&
-         (h->ext_sc || !seg_sweep(h));
+         (h->ext_sc ? presence_member(h) : !seg_sweep(h));
 }
 // blocks of the sweeps over segments (one thread per len cells of a line along D), a multiple of 8
 inline int seg_blocks(MhHandle* h, int D, int len) {

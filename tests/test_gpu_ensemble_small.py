@@ -1,5 +1,5 @@
-"""Small members of an ensemble at the lengths their marching cell sweeps change segments, and at the edges
-of these, bit for bit against the oracle."""
+"""Members of an ensemble on both sides of the lines at which their cell sweeps change, bit for bit against
+the oracle: the segments of the marching sweeps on small meshes, the presence bytes of 3D members."""
 import pytest
 
 from tests.helpers import bitwise_equal, fields
@@ -25,13 +25,21 @@ def one_environment(c):
 @pytest.mark.parametrize("m", [1, 2])
 @pytest.mark.parametrize("dim", [2, 3])
 def test_small_members(dim, m):
-    from mahyco_amd.lib import Ensemble
-    from oracle.pyoracle import OracleCase
     sizes = {2: [(2, 2), (5, 7), (12, 13), (3, 331), (333, 3), (25, 40), (63, 65), (64, 64), (65, 64)],
              3: [(2, 2, 2), (3, 5, 7), (8, 9, 10), (15, 16, 17), (16, 16, 16), (2, 33, 17), (17, 16, 16)]}[dim]
     cases = [moving_tube(n, 1) for n in sizes]
-    if m == 1:
-        cases = [one_environment(c) for c in cases]
+    check([one_environment(c) for c in cases] if m == 1 else cases, m, dim)
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_presence_bytes(seed):
+    check([moving_tube(n, seed) for n in ((15, 16, 17), (16, 15, 17), (2, 40, 40), (40, 40, 2), (99, 100, 101),
+                                          (100, 100, 100))], 2, 3)
+
+
+def check(cases, m, dim):
+    from mahyco_amd.lib import Ensemble
+    from oracle.pyoracle import OracleCase
     e = Ensemble(len(cases), 8 << 30)
     slots = [e.add(c) for c in cases]
     e.step(7)
