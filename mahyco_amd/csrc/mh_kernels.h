@@ -4144,7 +4144,10 @@ __global__ __launch_bounds__(MH_BLOCK) void k_hist_final(MhDev S) { k_hist_final
 #endif
 // Batched variants are persistent: a fixed grid walks the work list bmap[0 .. *nwork) (one
 // entry per (case, block) of every case of a batch group) with a grid stride, so the list and
-// its length can change between launches of a captured graph without re-capture.
+// its length can change between launches of a captured graph without re-capture.  An entry of a mesh
+// whose run has ended is passed over: 32 meshes of 200^2 with half of them ended take 231 us an iteration
+// instead of 266, with all of them 25 instead of 107, at the same 366 us with none.  (With the first entries
+// let through as in late_halted, 241, 36 and 378 us.)
 #define MH_WRAP(NAME, WAVES, TPL, TARGS, PARAMS, ARGS)                                      \
   TPL __global__ __launch_bounds__(MH_BLOCK, WAVES) void NAME(MhDev S PARAMS) {              \
     if (late_halted(S.sc)) return;                                                           \
@@ -4155,7 +4158,7 @@ __global__ __launch_bounds__(MH_BLOCK) void k_hist_final(MhDev S) { k_hist_final
     const int n = *nwork;                                                                    \
     for (int w = (int)blockIdx.x; w < n; w += (int)gridDim.x) {                              \
       const int2 bm = bmap[w];                                                               \
-      if (w < MH_FIRST_BLOCKS || !mh_halted(tab[bm.x].sc)) NAME##_body TARGS(tab[bm.x], bm.y ARGS); \
+      if (!mh_halted(tab[bm.x].sc)) NAME##_body TARGS(tab[bm.x], bm.y ARGS);                 \
       __syncthreads();                                                                       \
     }                                                                                        \
   }
