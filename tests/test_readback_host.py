@@ -10,7 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def program(tmp_path_factory):
     if shutil.which("g++") is None:
         pytest.skip("g++ not available")
     exe = str(tmp_path_factory.mktemp("readback") / "readback_check")
@@ -19,27 +19,27 @@ def checker(tmp_path_factory):
     return exe
 
 
-def _run(checker, check):
-    r = subprocess.run([checker, check], capture_output=True, text=True, timeout=60)
+def _run(program, check):
+    r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
     return tuple(map(int, r.stdout.split()))
 
 
-def test_threads_share_the_slots(checker):
+def test_threads_share_the_slots(program):
     """Reads by several threads: each gets its own field, whatever the others read."""
-    assert _run(checker, "threads") == (48, 0)
+    assert _run(program, "threads") == (48, 0)
 
 
-def test_what_reads_pin(checker):
+def test_what_reads_pin(program):
     """A single read pins no more than it gains; pinned memory is bounded and given back."""
-    assert _run(checker, "pinning") == (66, 0)
+    assert _run(program, "pinning") == (66, 0)
 
 
-def test_pinned_memory_is_short(checker):
+def test_pinned_memory_is_short(program):
     """Where pinned memory is not to be had, or not enough, the field is read all the same."""
-    assert _run(checker, "short") == (9, 0)
+    assert _run(program, "short") == (9, 0)
 
 
-def test_thread_of_another_device(checker):
+def test_thread_of_another_device(program):
     """A case is read by threads whose current device is another than the case's (a new thread's is 0)."""
-    assert _run(checker, "device") == (4, 0)
+    assert _run(program, "device") == (4, 0)
